@@ -100,4 +100,35 @@ struct RkqHeadArgs {
 };
 snhip_status launch_rkq_heads(const RkqHeadArgs& a, int B, hipStream_t st);
 
+// ---- chunked prefill (rkprefill.hip): T consecutive tokens of one sequence as
+// T rows, leaving what stepping them one by one leaves, bit for bit.
+constexpr int kRkpMaxDim = 4096;
+constexpr int kRkpPack = 5 * 64;   // floats of `pack` per (token, head)
+
+// xn = LN(x[t]); out[t] = xn + lerp[s] (xn[t - 1] - xn) for s < mixes (6: the
+// time mix, 1: the channel mix), xn[-1] = shift; shift_next = the last xn.
+struct RkpLnArgs {
+    int T, D, mixes;
+    float eps;
+    const float* x;                // (T, D)
+    const float *g, *c, *lerp;     // gain, bias; (mixes, D)
+    const float* shift;            // (D)
+    float* shift_next;             // (D), not `shift`
+    float* out;                    // (T, mixes, D)
+};
+snhip_status launch_rkp_ln(const RkpLnArgs& a, hipStream_t st);
+
+// The heads of one layer over the chunk (rwkv7.c:143-189, 228-299): v becomes
+// the residual-mixed value, y the gated read-out, S the state after the chunk.
+struct RkpHeadArgs {
+    int T, D, NH, first;
+    const float *r, *k, *dw, *da, *dv, *g;   // (T, D); dv unused in layer 0
+    float *v, *vfirst, *y;                    // (T, D)
+    const float *w0, *a0, *v0, *kk_w, *ka_w, *rk_w, *lnx_w, *lnx_b;   // (D)
+    float* S;                                 // (NH, 64, 64)
+    float* pack;                              // (T, NH, kRkpPack)
+    float* dot;                               // (T, NH)
+};
+snhip_status launch_rkp_heads(const RkpHeadArgs& a, hipStream_t st);
+
 }  // namespace snhip

@@ -146,6 +146,7 @@ struct SnHipRwkv7 {
           *dw = nullptr, *da = nullptr, *dv = nullptr, *g = nullptr, *y = nullptr, *vfirst = nullptr,
           *xk2 = nullptr, *ck = nullptr, *nrm = nullptr, *logits = nullptr;
     int32_t* tok = nullptr;
+    float* pf = nullptr;   // chunked prefill workspace of kPfRows tokens, on first use
     unsigned long long* best = nullptr;
     int32_t *counter = nullptr, *done = nullptr, *tok_hist = nullptr;
     int hist_cap = 0;
@@ -384,42 +385,39 @@ void setup_rk_persist(SnHipRwkv7* m) {
 }
 
 // The tiled fp32 form of every layer matrix (rkseq.h: block -1), for the
-// per-kernel steps: their products then run one independent wave per 64
-// rows and 4-16 sequences, streaming 1 KiB weight blocks, with no producer
-// waves and no barrier per 64 inputs. Made when some batch size up to
-// max_batch steps per kernel (SNHIP_RKQ_W4=0: never); each is 4 bytes per
-// weight (plus 64 KiB of padding). The vocabulary head keeps its own format.
+// per-kernel steps and the chunked prefill: their products then run one
+// independent wave per 64 rows and 4-16 sequences, streaming 1 KiB weight
+// blocks, with no producer waves and no barrier per 64 inputs
+// (SNHIP_RKQ_W4=0: never). 4 bytes per weight plus 64 KiB of padding each, in
+// one allocation. The vocabulary head keeps its own format.
 void setup_rkq_w4(SnHipRwkv7* m) {
     if (env_unsigned("SNHIP_RKQ_W4", 1, 0) == 0) return;
-    const int one_launch = m->p_grid > 0 ? std::max(1, m->p_mi_max) : 0;
-    if (m->max_batch <= one_launch) return;
-    bool ok = true;
-    auto make = [&](RMat& M) {
-        if (!ok || M.M <= 0 || M.Kd <= 0 || M.Kd % 4 || (!M.q && !M.w) ||
-            rkq_tiled_floats(M.M, M.Kd) * sizeof(float) >= ((size_t)1 << 31))   // the kernel's 32-bit offsets
-            return;
-        float* w4 = ralloc<float>(m, rkq_tiled_floats(M.M, M.Kd));
-        if (!w4 || launch_rkq_block4(M.w, M.q, M.sc, M.q ? M.block : 0, M.M, M.Kd, w4, nullptr) != SNHIP_OK) {
-            ok = false;
-            return;
-        }
-        M.w4 = w4;
-    };
+    std::vector<RMat*> mats;
+    size_t floats = 0;
     for (int l = 0; l < m->L; ++l) {
         RkLayer& A = m->layers[l];
         for (RMat* M : {&A.r, &A.k, &A.v, &A.o, &A.w1, &A.w2, &A.a1, &A.a2, &A.v1, &A.v2, &A.g1, &A.g2,
-                        &A.cmk, &A.cmv})
-            make(*M);
-    }
-    if (hipDeviceSynchronize() != hipSuccess) ok = false;
-    if (!ok) {
-        // all or nothing: the products then keep the stored format
-        for (int l = 0; l < m->L; ++l) {
-            RkLayer& A = m->layers[l];
-            for (RMat* M : {&A.r, &A.k, &A.v, &A.o, &A.w1, &A.w2, &A.a1, &A.a2, &A.v1, &A.v2, &A.g1, &A.g2,
-                            &A.cmk, &A.cmv})
-                M->w4 = nullptr;
+                        &A.cmk, &A.cmv}) {
+            if (M->M <= 0 || M->Kd <= 0 || M->Kd % 4 || (!M->q && !M->w) ||
+                rkq_tiled_floats(M->M, M->Kd) * sizeof(float) >= ((size_t)1 << 31))   // the kernel's 32-bit offsets
+                continue;
+            mats.push_back(M);
+            floats += rkq_tiled_floats(M->M, M->Kd);
         }
+    }
+    float* w4 = floats ? ralloc<float>(m, floats) : nullptr;
+    if (!w4) return;   // the products keep the stored format
+    bool ok = true;
+    float* at = w4;
+    for (RMat* M : mats) {
+        ok = ok && launch_rkq_block4(M->w, M->q, M->sc, M->q ? M->block : 0, M->M, M->Kd, at, nullptr) == SNHIP_OK;
+        at += rkq_tiled_floats(M->M, M->Kd);
+    }
+    if (!ok || hipDeviceSynchronize() != hipSuccess) return;
+    at = w4;
+    for (RMat* M : mats) {
+        M->w4 = at;
+        at += rkq_tiled_floats(M->M, M->Kd);
     }
 }
 
@@ -846,14 +844,149 @@ snhip_status step_host(SnHipRwkv7* m, const int32_t* tokens, int B, float* logit
     return SNHIP_OK;
 }
 
+// Chunked prefill of sequence 0 (rkprefill.hip). Its products use whichever
+// form the matrices have; prompts shorter than kPfMin step token by token.
+// Measured on 12 x 768 INT4 g32, host call: a chunk of 4 to 16 tokens 1.4 ms, a
+// step 0.68 ms (3 tokens 2.0 ms), so the line lies at three tokens; 512 tokens
+// 4.8 ms in one chunk against 345 ms stepped.
+constexpr int kPfRows = 512;   // tokens per chunk
+constexpr int kPfMin = 3;
+
+// Floats of the workspace's parts per token, in PfWs's order.
+struct PfWs {
+    float *x, *X6, *r, *k, *v, *lo, *dw, *da, *dv, *g, *y, *vfirst, *xk2, *ck, *pack, *dot, *shift;
+    int32_t* tok;
+};
+size_t pf_layout(const SnHipRwkv7* m, float* base, PfWs* ws) {
+    const size_t T = kPfRows, D = m->D;
+    size_t at = 0;
+    auto take = [&](float*& p, size_t n) {
+        if (base) p = base + at;
+        at += (n + 63) / 64 * 64;
+    };
+    PfWs w{};
+    take(w.x, T * D);
+    take(w.X6, T * 6 * D);
+    take(w.r, T * D);
+    take(w.k, T * D);
+    take(w.v, T * D);
+    take(w.lo, T * 4 * kMaxRank);
+    take(w.dw, T * D);
+    take(w.da, T * D);
+    take(w.dv, T * D);
+    take(w.g, T * D);
+    take(w.y, T * D);
+    take(w.vfirst, T * D);
+    take(w.xk2, T * D);
+    take(w.ck, T * m->F);
+    take(w.pack, T * m->NH * kRkpPack);
+    take(w.dot, T * m->NH);
+    take(w.shift, (size_t)m->L * 2 * D);
+    float* tk = nullptr;
+    take(tk, T);
+    w.tok = reinterpret_cast<int32_t*>(tk);
+    if (ws) *ws = w;
+    return at;
+}
+
+// T <= kPfRows tokens (in ws.tok) of sequence 0 from its current state; the
+// last token's logits to logits_out unless null.
+snhip_status enqueue_chunk(SnHipRwkv7* m, const PfWs& ws, int T, float* logits_out, hipStream_t st) {
+    const int D = m->D, F = m->F, NH = m->NH;
+    const int ldl = 4 * kMaxRank, ld6 = 6 * D;
+    float* lw = ws.lo;
+    float* la = ws.lo + kMaxRank;
+    float* lv = ws.lo + 2 * kMaxRank;
+    float* lg = ws.lo + 3 * kMaxRank;
+    snhip_status rc;
+    RkqLnArgs ln{};
+    ln.D = D; ln.vocab = m->vocab; ln.eps = m->eps;
+    ln.mode = RKQ_LN_EMBED;
+    ln.tok = ws.tok; ln.embed = m->embed; ln.g = m->en_w; ln.c = m->en_b; ln.out = ws.x;
+    if ((rc = launch_rkq_ln(ln, T, st)) != SNHIP_OK) return rc;
+    MMList mm{T};
+    for (int l = 0; l < m->L; ++l) {
+        const RkLayer& A = m->layers[l];
+        const size_t sh = (size_t)l * 2 * D;
+        RkpLnArgs N{};
+        N.T = T; N.D = D; N.eps = m->eps; N.x = ws.x;
+        N.mixes = 6; N.g = A.ln1w; N.c = A.ln1b; N.lerp = A.lerp; N.out = ws.X6;
+        N.shift = m->shift + sh; N.shift_next = ws.shift + sh;
+        if ((rc = launch_rkp_ln(N, st)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.r, ws.X6, ld6, ws.r, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.k, ws.X6 + 2 * D, ld6, ws.k, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.v, ws.X6 + 3 * D, ld6, ws.v, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.w1, ws.X6 + D, ld6, lw, ldl, RKQ_TANH)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.a1, ws.X6 + 4 * D, ld6, la, ldl, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.g1, ws.X6 + 5 * D, ld6, lg, ldl, RKQ_SIGMOID)) != SNHIP_OK) return rc;
+        if (l > 0 && (rc = mm.add(A.v1, ws.X6 + 3 * D, ld6, lv, ldl, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.w2, lw, ldl, ws.dw, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.a2, la, ldl, ws.da, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.g2, lg, ldl, ws.g, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if (l > 0 && (rc = mm.add(A.v2, lv, ldl, ws.dv, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
+        RkpHeadArgs H{};
+        H.T = T; H.D = D; H.NH = NH; H.first = l == 0;
+        H.r = ws.r; H.k = ws.k; H.v = ws.v; H.dw = ws.dw; H.da = ws.da; H.dv = ws.dv; H.g = ws.g;
+        H.vfirst = ws.vfirst; H.y = ws.y;
+        H.w0 = A.w0; H.a0 = A.a0; H.v0 = A.v0; H.kk_w = A.kk; H.ka_w = A.ka; H.rk_w = A.rk;
+        H.lnx_w = A.lnxw; H.lnx_b = A.lnxb;
+        H.S = m->S + (size_t)l * NH * m->HS * m->HS;
+        H.pack = ws.pack; H.dot = ws.dot;
+        if ((rc = launch_rkp_heads(H, st)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.o, ws.y, D, ws.x, D, RKQ_ADD)) != SNHIP_OK) return rc;
+        if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
+        N.mixes = 1; N.g = A.ln2w; N.c = A.ln2b; N.lerp = A.cmk_lerp; N.out = ws.xk2;
+        N.shift = m->shift + sh + D; N.shift_next = ws.shift + sh + D;
+        if ((rc = launch_rkp_ln(N, st)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.cmk, ws.xk2, D, ws.ck, F, RKQ_RELU2)) != SNHIP_OK) return rc;
+        if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.cmv, ws.ck, F, ws.x, D, RKQ_ADD)) != SNHIP_OK) return rc;
+        if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
+    }
+    SNHIP_CHECK(hipMemcpyAsync(m->shift, ws.shift, (size_t)m->L * 2 * D * sizeof(float), hipMemcpyDeviceToDevice, st));
+    if (!logits_out) return SNHIP_OK;
+    ln.mode = RKQ_LN_PLAIN;
+    ln.x = ws.x + (size_t)(T - 1) * D; ln.g = m->on_w; ln.c = m->on_b; ln.out = m->nrm;
+    if ((rc = launch_rkq_ln(ln, 1, st)) != SNHIP_OK) return rc;
+    MMList head{1};
+    if ((rc = head.add(m->head, m->nrm, D, logits_out, m->vocab, RKQ_STORE)) != SNHIP_OK) return rc;
+    return head.flush(st);
+}
+
+snhip_status run_prefill(SnHipRwkv7* m, const int32_t* tokens, int n, float* logits_out) {
+    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (!m->pf) m->pf = ralloc<float>(m, pf_layout(m, nullptr, nullptr));
+    if (!m->pf) { set_last_error("out of device memory (prefill)"); return SNHIP_E_NOMEM; }
+    PfWs ws;
+    pf_layout(m, m->pf, &ws);
+    SNHIP_CHECK(hipEventRecord(m->ev_in, m->stream));
+    SNHIP_CHECK(hipStreamWaitEvent(m->work, m->ev_in, 0));
+    for (int c0 = 0; c0 < n; c0 += kPfRows) {
+        const int T = std::min(kPfRows, n - c0);
+        SNHIP_CHECK(hipMemcpyAsync(ws.tok, tokens + c0, T * sizeof(int32_t), hipMemcpyHostToDevice, m->work));
+        const snhip_status rc = enqueue_chunk(m, ws, T, c0 + T == n ? logits_out : nullptr, m->work);
+        if (rc != SNHIP_OK) return rc;
+    }
+    SNHIP_CHECK(hipEventRecord(m->ev_out, m->work));
+    SNHIP_CHECK(hipStreamWaitEvent(m->stream, m->ev_out, 0));
+    return SNHIP_OK;
+}
+
 snhip_status prefill_host(SnHipRwkv7* m, const int32_t* tokens, int n, float* logits) {
     if (!m || !tokens || n <= 0 || !logits) return SNHIP_E_INVAL;
     if (!tokens_ok(m, tokens, n)) return SNHIP_E_INVAL;
-    // rwkv7.c:362-364: the step, once per token, in order.
-    for (int i = 0; i < n; ++i) {
-        SNHIP_CHECK(hipMemcpyAsync(m->tok, tokens + i, sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
-        const snhip_status rc = run_steps(m, 1, m->logits, false, 1);
+    if (n >= kPfMin) {
+        const snhip_status rc = run_prefill(m, tokens, n, m->logits);
         if (rc != SNHIP_OK) return rc;
+    } else {
+        // rwkv7.c:362-364: the step, once per token, in order.
+        for (int i = 0; i < n; ++i) {
+            SNHIP_CHECK(hipMemcpyAsync(m->tok, tokens + i, sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
+            const snhip_status rc = run_steps(m, 1, m->logits, false, 1);
+            if (rc != SNHIP_OK) return rc;
+        }
     }
     SNHIP_CHECK(hipMemcpyAsync(logits, m->logits, (size_t)m->vocab * sizeof(float),
                                hipMemcpyDeviceToHost, m->stream));
