@@ -11,7 +11,7 @@
 // one wave per (token, head). What is left for the recurrence is 8 multiply-adds
 // of the read, one of the update and 8 of the read-out per state element.
 //
-// Measured (12 x 768, INT4 g32, 512-token prompt): 4.8 ms, where the
+// Measured (12 x 768, INT4 g32, 512-token prompt): 3.4 ms, where the
 // token-by-token prefill took 345 ms (512 one-launch steps of 673 us).
 #include <algorithm>
 #include <type_traits>
@@ -105,15 +105,18 @@ __global__ __launch_bounds__(64 * (kLnRows + 1)) void k_rkp_ln(RkpLnArgs A) {
     if (w == 0 || row >= A.T) return;
     const float4* prev = rows4 + (size_t)(w - 1) * n4;
     const float4* l4 = reinterpret_cast<const float4*>(A.lerp);
-    float4* o4 = reinterpret_cast<float4*>(A.out) + (size_t)row * A.mixes * n4;
+    const size_t mat = x16_floats(A.T, D);
     float4* nx = row == A.T - 1 ? reinterpret_cast<float4*>(A.shift_next) : nullptr;
     for (int q = l; q < n4; q += 64) {
         const float4 xn = own[q], p = prev[q];
         const float4 d = make_float4(p.x - xn.x, p.y - xn.y, p.z - xn.z, p.w - xn.w);
         for (int s = 0; s < A.mixes; ++s) {
             const float4 lp = l4[(size_t)s * n4 + q];
-            o4[(size_t)s * n4 + q] = make_float4(xn.x + lp.x * d.x, xn.y + lp.y * d.y, xn.z + lp.z * d.z,
-                                                 xn.w + lp.w * d.w);
+            float* o = A.out + s * mat + x16_at(row, 4 * q, D / 16);   // the four inputs are 64 floats apart
+            o[0] = xn.x + lp.x * d.x;
+            o[64] = xn.y + lp.y * d.y;
+            o[128] = xn.z + lp.z * d.z;
+            o[192] = xn.w + lp.w * d.w;
         }
         if (nx) nx[q] = xn;
     }
@@ -218,7 +221,7 @@ __global__ __launch_bounds__(64) void k_rkp_scan(RkpHeadArgs A) {
     const float4* p4 = reinterpret_cast<const float4*>(A.pack + (size_t)h * kRkpPack) + 2 * lam;
     const size_t pstride = (size_t)A.NH * kRkpPack / 4;
     const float* vp = A.v + h * kHS + row;
-    float* yp = A.y + h * kHS + row;
+    float* yp = A.ys + h * kHS + row;
     auto load = [&](TokIn& I, int tok) {
         const int t = min(tok, A.T - 1);   // past the end: the last token again, never used
         const float4* p = p4 + (size_t)t * pstride;
@@ -273,7 +276,7 @@ __global__ __launch_bounds__(256) void k_rkp_gate(RkpHeadArgs A) {
     if (tok >= A.T) return;   // no workgroup barrier below
     const int c = h * kHS + t;
     const size_t at = (size_t)tok * A.D + c;
-    const float yy = A.y[at], vv = A.v[at], gv = A.g[at];
+    const float yy = A.ys[at], vv = A.v[at], gv = A.g[at];
     const float lnw = A.lnx_w[c], lnb = A.lnx_b[c], dot = A.dot[(size_t)tok * A.NH + h];
     float* ys = reinterpret_cast<float*>(y_[wv]);
     ys[t] = yy;
@@ -301,13 +304,13 @@ __global__ __launch_bounds__(256) void k_rkp_gate(RkpHeadArgs A) {
     }
     const float rstd = 1.0f / sqrtf(var / (float)kHS + kEpsGroup);
     const float n = (yy - mean) * rstd * lnw + lnb;
-    A.y[at] = (n + dot * vv) * gv;
+    A.y[x16_at(tok, c, A.D / 16)] = (n + dot * vv) * gv;
 }
 
 }  // namespace
 
 snhip_status launch_rkp_ln(const RkpLnArgs& a, hipStream_t st) {
-    if (a.T <= 0 || a.D <= 0 || a.D > kRkpMaxDim || a.D % 4 || (a.mixes != 1 && a.mixes != 6)) return SNHIP_E_INVAL;
+    if (a.T <= 0 || a.D <= 0 || a.D > kRkpMaxDim || a.D % 16 || (a.mixes != 1 && a.mixes != 6)) return SNHIP_E_INVAL;
     const dim3 grid((a.T + kLnRows - 1) / kLnRows), blk(64 * (kLnRows + 1));
     const size_t shm = (size_t)(kLnRows + 1) * a.D * sizeof(float);   // at most 64 KiB
     switch (a.D % 256 ? 0 : a.D / 256) {

@@ -16,15 +16,25 @@ enum RkqEpi {
     RKQ_SIGMOID = 4,   // Y = 1 / (1 + expf(-y)) (rwkv7.c:256)
 };
 
-// One product Y[b] = W X[b] for the batch's rows b: W (M, Kd) row-major, fp32
-// (w) or INT4 codes + scales in quant.c's packing (q, sc). Each output is the
-// reference's chain acc = fmaf(X[b][k], W[j][k], acc) over k = 0 .. Kd-1 from
-// acc = 0 (outputs j >= M & ~7 take acc = acc + X W, two roundings, as the
-// reference's scalar column tail does). Kd is a multiple of 4 (fp32) or of the
-// group size (INT4); X rows 16-byte aligned.
+// Order in which the products read their inputs: rows in tiles of 16, inputs in
+// blocks of 16 (nkb of them, the last padded with zeros); float4 l of block kb of
+// tile t, at ((t nkb + kb) 64 + l) 4, holds inputs 16 kb + 4 j + l / 16 (j = 0..3)
+// of row 16 t + l % 16: what lane l supplies to the block's four 16x16x4 steps.
+__host__ __device__ inline size_t x16_at(int row, int k, int nkb) {
+    return ((((size_t)(row >> 4) * nkb + (k >> 4)) * 64 + (size_t)(k & 3) * 16 + (row & 15)) << 2) + ((k >> 2) & 3);
+}
+__host__ __device__ inline size_t x16_floats(int rows, int k) {
+    return (size_t)((rows + 15) / 16) * ((k + 15) / 16) * 256;
+}
+
+// One product Y[b] = W X[b] for the batch's rows b: X in x16 order, W (M, Kd)
+// row-major fp32 (w), INT4 codes + scales in quant.c's packing (q, sc), or
+// tiled. Each output is the reference's chain acc = fmaf(X[b][k], W[j][k], acc)
+// over k = 0 .. Kd-1 from acc = 0 (outputs j >= M & ~7 take acc = acc + X W, two
+// roundings, as the reference's scalar column tail does). Kd is a multiple of 4
+// (fp32) or of the group size (INT4). Y row-major (ldy), or x16 order (y16).
 struct RkqJob {
     const float* X;
-    int ldx;
     const float* w;
     const uint8_t* q;
     const float* sc;
@@ -32,25 +42,18 @@ struct RkqJob {
     float* Y;
     int ldy;
     int epi;
+    int y16;
 };
 constexpr int kRkqMaxJobs = 8;
 
 // Jobs share the weight format: block 0 = fp32 rows, 32 or 64 = INT4 group,
-// -1 = tiled fp32 (float4 (t * Kd / 4 + kb) * 64 + l = inputs 4 kb .. 4 kb + 3
-// of row 64 t + l, then a zeroed pad; launch_rkq_block4 makes them).
+// -1 = tiled fp32 (launch_rkq_tile).
 snhip_status launch_rkq_mm(const RkqJob* jobs, int n, int B, int block, hipStream_t st);
-// floats of the tiled fp32 form of an M x Kd matrix, pad included
-size_t rkq_tiled_floats(int M, int Kd);
-// out (rkq_tiled_floats) = the tiled fp32 form of an M x Kd matrix given as
-// fp32 rows w (block 0) or INT4 codes q and scales sc (block 32 or 64), each
-// value the one the products multiply by.
-snhip_status launch_rkq_block4(const float* w, const uint8_t* q, const float* sc, int block, int M, int Kd,
-                               float* out, hipStream_t st);
-// The same with the INT4 workgroup shape given: nc consumer waves of s chains
-// of 4 sequences (nc in {1, 2, 4}, s in {1, 2}, not 4 x 2), or s = 16: one
-// 16x16x1 chain of 16 sequences per consumer; 0 = chosen by B and the grid.
-snhip_status launch_rkq_mm_cfg(const RkqJob* jobs, int n, int B, int block, int nc, int s,
-                               hipStream_t st);
+// out (x16_floats(M, Kd)) = the tiled fp32 form of an M x Kd matrix given as
+// fp32 rows w (block 0) or INT4 codes q and scales sc (block 32 or 64): x16
+// order, outputs for rows, each value the one the products multiply by.
+snhip_status launch_rkq_tile(const float* w, const uint8_t* q, const float* sc, int block, int M, int Kd,
+                             float* out, hipStream_t st);
 
 // Row LayerNorm (rwkv7.c:127-140: sequential sums, two passes) over D <= 4096,
 // then one of the step's uses of it.
@@ -70,7 +73,7 @@ struct RkqLnArgs {
     const float* lerp;       // MIX1: (6, D); MIX2: (D)
     float* shift;            // MIX1: shift_0 row of sequence b at shift + b * shift_bstride; MIX2: shift_1
     size_t shift_bstride;
-    float* out;              // EMBED: x; MIX1: X6 (B, 6, D); MIX2: xk2 (B, D); PLAIN: y (B, D)
+    float* out;              // EMBED: x (B, D); else x16 order: MIX1 the six mixes one after the other, MIX2 xk2, PLAIN y
 };
 snhip_status launch_rkq_ln(const RkqLnArgs& a, int B, hipStream_t st);
 
@@ -83,9 +86,9 @@ struct RkqHeadArgs {
     const float *w0, *a0, *v0, *kk_w, *ka_w, *rk_w, *lnx_w, *lnx_b;
     float* S;            // layer base; sequence b at S + b * s_bstride, head h at + h * 64 * 64
     size_t s_bstride;
-    float* y;            // (B, D)
+    float* y;            // (B, D) in x16 order
     int D, NH, first;
-    float* dbg;          // if set: sequence 0's k, v, a, ww at dbg + 2D, 3D, 4D, 6D (rwkv7.c:308-319)
+    float* dbg;          // if set: sequence 0's k, v, a, ww, y at dbg + 2D, 3D, 4D, 6D, 7D (rwkv7.c:308-319)
     // The LoRA up-projections w2, a2, g2, v2 computed here from their INT4
     // codes (up_blk 32 or 64, ranks up_k <= 128; v2 not in layer 0) instead
     // of read from dw, da, g, dv (up_blk 0): inputs lw, la, lg, lv of
@@ -114,7 +117,7 @@ struct RkpLnArgs {
     const float *g, *c, *lerp;     // gain, bias; (mixes, D)
     const float* shift;            // (D)
     float* shift_next;             // (D), not `shift`
-    float* out;                    // (T, mixes, D)
+    float* out;                    // `mixes` matrices (T, D) in x16 order, one after the other
 };
 snhip_status launch_rkp_ln(const RkpLnArgs& a, hipStream_t st);
 
@@ -123,7 +126,8 @@ snhip_status launch_rkp_ln(const RkpLnArgs& a, hipStream_t st);
 struct RkpHeadArgs {
     int T, D, NH, first;
     const float *r, *k, *dw, *da, *dv, *g;   // (T, D); dv unused in layer 0
-    float *v, *vfirst, *y;                    // (T, D)
+    float *v, *vfirst, *ys;                   // (T, D); ys: the read-out before norm and gate
+    float* y;                                 // (T, D) in x16 order
     const float *w0, *a0, *v0, *kk_w, *ka_w, *rk_w, *lnx_w, *lnx_b;   // (D)
     float* S;                                 // (NH, 64, 64)
     float* pack;                              // (T, NH, kRkpPack)

@@ -6,15 +6,10 @@
 // dots use eight stride-8 partial sums folded as ((0+4)+(1+5))+((2+6)+(3+7)),
 // and expf / tanhf are glibc's. The kernels here repeat exactly that:
 //
-// * Products run on the matrix cores with v_mfma_f32_4x4x1_16b_f32. With one
-//   product per output per instruction, each instruction is acc + x w with a
-//   single rounding (checked on gfx950: equal to fmaf on every output, and a
-//   chain of them in k order equal to the sequential fmaf chain), so issuing
-//   them in k order gives the reference's chain. A wave owns 64 output rows
-//   (lane l supplies row out0 + l as the B operand and holds that column of
-//   every 4 x 4 block) and S groups of 4 sequences (the A operands); INT4
-//   weights are dequantized in registers as fma(q, s, -8 s), which equals
-//   quant.c's (q - 8) s.
+// * Products run on the matrix cores with v_mfma_f32_16x16x4_f32, whose four
+//   products are added in order with one rounding each (k_rkq_mm): issued in k
+//   order they give the reference's chain. INT4 weights are dequantized in
+//   registers as fma(q, s, -8 s), which equals quant.c's (q - 8) s.
 // * LayerNorm: one wave per row, the row in LDS, one lane running each
 //   sequential sum while the others prepare the squared deviations.
 // * Heads: one wave per (head, sequence), lane i owning state row i.
@@ -33,7 +28,6 @@ namespace snhip {
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
 
 constexpr float kR2 = 0.6065306597126334f;   // 1/sqrt(e), rwkv7.c:38
@@ -170,7 +164,12 @@ __global__ __launch_bounds__(LT) void k_rkq_ln(RkqLnArgs A) {
         __syncthreads();
     }
     const float mean = stat[0], rstd = stat[1];
-    float4* o4 = reinterpret_cast<float4*>(A.out);
+    const size_t mat = x16_floats((int)gridDim.x, D);   // one matrix of all rows
+    // float4 q of this row in x16 order (its four inputs are 64 floats apart)
+    auto put = [&](float* m, int q, float4 v) {
+        float* p = m + x16_at(b, 4 * q, D / 16);
+        p[0] = v.x; p[64] = v.y; p[128] = v.z; p[192] = v.w;
+    };
     auto norm = [&](float x, float g, float c) { return (x - mean) * rstd * g + c; };
     auto emit = [&](int q, float4 g, float4 c, float4 sh, const float4* lp) {
         const float4 x = xs4[q];
@@ -185,17 +184,19 @@ __global__ __launch_bounds__(LT) void k_rkq_ln(RkqLnArgs A) {
                 float4 r;
                 r.x = xn.x + lp[s6].x * d.x; r.y = xn.y + lp[s6].y * d.y;
                 r.z = xn.z + lp[s6].z * d.z; r.w = xn.w + lp[s6].w * d.w;
-                o4[(size_t)b * 6 * n4 + (size_t)s6 * n4 + q] = r;
+                put(A.out + s6 * mat, q, r);
             }
             sh4[q] = xn;
         } else if (mix2) {
             float4 r;
             r.x = xn.x + lp[0].x * (sh.x - xn.x); r.y = xn.y + lp[0].y * (sh.y - xn.y);
             r.z = xn.z + lp[0].z * (sh.z - xn.z); r.w = xn.w + lp[0].w * (sh.w - xn.w);
-            o4[(size_t)b * n4 + q] = r;
+            put(A.out, q, r);
             sh4[q] = xn;
+        } else if (A.mode == RKQ_LN_PLAIN) {
+            put(A.out, q, xn);
         } else {
-            o4[(size_t)b * n4 + q] = xn;
+            reinterpret_cast<float4*>(A.out)[(size_t)b * n4 + q] = xn;
         }
     };
     if (regs) {
@@ -222,17 +223,43 @@ __global__ __launch_bounds__(LT) void k_rkq_ln(RkqLnArgs A) {
 }
 
 // ------------------------------------------------------------- products
+// Y[b] = W X[b], every output the reference's chain acc = fmaf(x[k], w[k], acc)
+// over k in order. v_mfma_f32_16x16x4_f32 adds its four products one after the
+// other, each with one rounding, lowest k first (checked on gfx950: 51,200
+// random outputs of it, and of 32x32x2, equal the sequential fmaf chain bit for
+// bit, none equals another order or a single rounding throughout), so a chain
+// of them in k order is that chain. A dependent one issues every 36 cycles, 9
+// per input (4x4x1 chains: 13 to 19), and a wave holds only 16 outputs x 16
+// sequences per chain, so a batch of 16 already spreads over many waves.
+//
+// One wave per 16 O outputs x 16 S sequences, one wave per workgroup, nothing
+// shared and no barrier. Lane (n, g) = (l % 16, l / 16) supplies input 4 i + g
+// of step i: output n's weight (A) and sequence n's x (B), and then holds
+// outputs 4 g .. 4 g + 3 of sequence n. With one wave per SIMD a chain leaves
+// room for about six other instructions per MFMA (one issues every ~5.4
+// cycles), so both operands come in the order the steps use them (x16_at): one
+// coalesced 1 KiB load each per 16 inputs, PF of them ahead in registers. Every
+// producer writes its rows that way, and a product's own outputs are in that
+// order already. The first version, which dequantized INT4 codes and transposed
+// row-major x in the wave (11 instructions per MFMA), took 28 us for the
+// channel-mix value at B = 64; this one takes 15 (the 4x4x1 chains it replaced:
+// 26). The step at B = 64: 1,350 -> 1,030 us (12 x 768 INT4 g32); a 512-token
+// prefill chunk 4.8 -> 3.4 ms.
+//
+// Weights (BLK): -1, tiled fp32 copies of the layer matrices, made at load
+// (k_rkq_tile); 32 / 64, INT4 codes: byte g of dword i of a group is exactly
+// lane group g's input, so the wave dequantizes its operand in registers
+// (fma(q, s, -8 s), quant.c's (q - 8) s), which the vocabulary head's eight
+// chains hide; 0, fp32 rows, transposed between the lane groups.
 struct RkqMMArgs {
     RkqJob j[kRkqMaxJobs];
     int start[kRkqMaxJobs + 1];   // first workgroup of each job
-    int tiles_out[kRkqMaxJobs];   // 64-row tiles of each job
     int n, B, seq_tiles;
-    int xs_per_wave;              // tiled fp32: float4 of LDS per wave
 };
 
+// One weight, as the products multiply it.
 __device__ __forceinline__ float dequant_at(const RkqJob& J, int row, int k, int blk) {
-    if (blk < 0)   // tiled fp32 (k_rkq_mm_w4)
-        return J.w[(((size_t)(row >> 6) * (size_t)(J.Kd >> 2) + (size_t)(k >> 2)) * 64 + (row & 63)) * 4 + (k & 3)];
+    if (blk < 0) return J.w[x16_at(row, k, (J.Kd + 15) / 16)];
     if (!blk) return J.w[(size_t)row * J.Kd + k];
     const int half = blk / 2, g = k / blk, e = k % blk;
     const uint8_t byte = J.q[(size_t)row * (J.Kd / 2) + (size_t)g * half + (e % half)];
@@ -240,46 +267,6 @@ __device__ __forceinline__ float dequant_at(const RkqJob& J, int row, int k, int
     const int qv = e < half ? (byte & 0x0F) : (byte >> 4);
     return fmaf((float)qv, sc, -8.0f * sc);
 }
-
-template <int S>
-__device__ __forceinline__ void mfma_k(const float (&xv)[S], float wv, v4f (&acc)[S]) {
-#pragma unroll
-    for (int s = 0; s < S; ++s) acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(xv[s], wv, acc[s], 0, 0, 0);
-}
-
-template <int S>
-__device__ __forceinline__ void step4(const float4 (&x4)[S], float w0, float w1, float w2, float w3,
-                                      v4f (&acc)[S]) {
-    float xv[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) xv[s] = x4[s].x;
-    mfma_k<S>(xv, w0, acc);
-#pragma unroll
-    for (int s = 0; s < S; ++s) xv[s] = x4[s].y;
-    mfma_k<S>(xv, w1, acc);
-#pragma unroll
-    for (int s = 0; s < S; ++s) xv[s] = x4[s].z;
-    mfma_k<S>(xv, w2, acc);
-#pragma unroll
-    for (int s = 0; s < S; ++s) xv[s] = x4[s].w;
-    mfma_k<S>(xv, w3, acc);
-}
-
-template <int S>
-__device__ __forceinline__ void step4(const v4f (&x4)[S], float w0, float w1, float w2, float w3, v4f (&acc)[S]) {
-    float xv[S];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) xv[s] = x4[s][c];
-        mfma_k<S>(xv, c == 0 ? w0 : c == 1 ? w1 : c == 2 ? w2 : w3, acc);
-    }
-}
-
-// Inputs per chunk staged in LDS at once (X rows; INT4 codes in registers).
-constexpr int kRkqKC = 768;
-constexpr int kRkqU = 64;                  // INT4: inputs per pipeline unit (two producer halves of 32)
-constexpr int kRkqNP = 2;                  // producer waves of an INT4 workgroup
 
 // This workgroup's job (uniform selects: no dynamic index into the arguments).
 // The first workgroup of the job is selected in the same pass as the job
@@ -297,649 +284,224 @@ __device__ __forceinline__ void rkq_job_at(const RkqMMArgs& A, int wg, RkqJob& J
         if (i == ji) J = A.j[i];
     u0 = wg - j0;
 }
-__device__ __forceinline__ void rkq_job(const RkqMMArgs& A, RkqJob& J, int& u0) {
-    rkq_job_at(A, (int)blockIdx.x, J, u0);
+
+__device__ __forceinline__ float rkq_epi(int epi, float y, float v) {
+    switch (epi) {
+    case RKQ_ADD: return y + v;
+    case RKQ_RELU2: { const float r = v > 0.0f ? v : 0.0f; return r * r; }
+    case RKQ_TANH: return refmath::tanhf(v);
+    case RKQ_SIGMOID: return refmath::sigmoid(v);
+    default: return v;
+    }
 }
 
-// Tail columns and the epilogue of one lane's 4 sequences (seq0 .. seq0+3)
-// of output column `out`. Columns past the last multiple of 8 take the
-// reference's scalar tail (acc + x * w, two roundings).
-__device__ __forceinline__ void rkq_finish(const RkqJob& J, int B, int blk, int seq0, int out,
-                                           v4f acc) {
-    if (out >= J.M) return;
-    if (out >= (J.M & ~7)) {
+// A lane's outputs out0 .. out0 + 3 (out0 % 4 == 0) of sequence sq: columns
+// past the last multiple of 8 take the reference's scalar tail (acc + x * w,
+// two roundings), then the epilogue. In x16 order the outputs that pad the last
+// block of 16 are written as zeros.
+__device__ __forceinline__ void rkq_finish(const RkqJob& J, int B, int blk, int sq, int out0, v4f acc) {
+    if (sq >= B || out0 >= (J.M + 15) / 16 * 16) return;
+    if (out0 + 4 > (J.M & ~7)) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int sq = seq0 + i;
-            if (sq >= B) continue;
-            const float* x = J.X + (size_t)sq * J.ldx;
-            float a2 = 0.0f;
-            for (int k = 0; k < J.Kd; ++k) a2 = a2 + x[k] * dequant_at(J, out, k, blk);
-            acc[i] = a2;
+            const int out = out0 + i;
+            if (out < (J.M & ~7) || out >= J.M) continue;
+            float v = 0.0f;
+            for (int k = 0; k < J.Kd; ++k)
+                v = v + J.X[x16_at(sq, k, (J.Kd + 15) / 16)] * dequant_at(J, out, k, blk);
+            acc[i] = v;
         }
     }
+    if (J.y16) {   // never RKQ_ADD
+        float* y = J.Y + x16_at(sq, out0, (J.M + 15) / 16);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int sq = seq0 + i;
-        if (sq >= B) continue;
-        float* y = J.Y + (size_t)sq * J.ldy + out;
-        const float v = acc[i];
-        switch (J.epi) {
-        case RKQ_ADD: *y = *y + v; break;
-        case RKQ_RELU2: { const float r = v > 0.0f ? v : 0.0f; *y = r * r; break; }
-        case RKQ_TANH: *y = refmath::tanhf(v); break;
-        case RKQ_SIGMOID: *y = refmath::sigmoid(v); break;
-        default: *y = v; break;
-        }
+        for (int i = 0; i < 4; ++i) y[64 * i] = out0 + i < J.M ? rkq_epi(J.epi, 0.0f, acc[i]) : 0.0f;
+        return;
     }
-}
-
-// One output (sequence sq, column out) of a chain sum v: the scalar tail
-// past the last multiple of 8 as in rkq_finish, then the epilogue.
-__device__ __forceinline__ void rkq_finish1(const RkqJob& J, int B, int blk, int sq, int out, float v) {
-    if (out >= J.M || sq >= B) return;
-    if (out >= (J.M & ~7)) {
-        const float* x = J.X + (size_t)sq * J.ldx;
-        float a2 = 0.0f;
-        for (int k = 0; k < J.Kd; ++k) a2 = a2 + x[k] * dequant_at(J, out, k, blk);
-        v = a2;
-    }
-    float* y = J.Y + (size_t)sq * J.ldy + out;
-    switch (J.epi) {
-    case RKQ_ADD: *y = *y + v; break;
-    case RKQ_RELU2: { const float r = v > 0.0f ? v : 0.0f; *y = r * r; break; }
-    case RKQ_TANH: *y = refmath::tanhf(v); break;
-    case RKQ_SIGMOID: *y = refmath::sigmoid(v); break;
-    default: *y = v; break;
-    }
-}
-
-// fp32 weights: one wave per 64 rows x S groups of 4 sequences; X of the
-// chunk in LDS, the lane's weight row read 32 inputs ahead.
-template <int S>
-__global__ __launch_bounds__(64) void k_rkq_mm_f32(const RkqMMArgs A) {
-    __shared__ float4 xs4[4 * S * (kRkqKC / 4)];   // X row (4 s + r) at (4 s + r) * KC
-    RkqJob J;
-    int u0;
-    rkq_job(A, J, u0);
-    const int ot = u0 / A.seq_tiles, st = u0 % A.seq_tiles;
-    const int l = threadIdx.x, r4 = l & 3;
-    const int out = ot * 64 + l;
-    const int orow = out < J.M ? out : J.M - 1;
-    const int seq0 = st * 4 * S;
-    v4f acc[S];
+    float* y = J.Y + (size_t)sq * J.ldy + out0;
+    if (out0 + 4 <= J.M && ((reinterpret_cast<uintptr_t>(J.Y) | (uintptr_t)J.ldy * 4) & 15) == 0) {
+        v4f old = v4f{0.f, 0.f, 0.f, 0.f};
+        if (J.epi == RKQ_ADD) old = *reinterpret_cast<const v4f*>(y);
+        v4f r;
 #pragma unroll
-    for (int s = 0; s < S; ++s) acc[s] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < J.Kd; k0 += kRkqKC) {
-        const int kc = min(kRkqKC, J.Kd - k0);
-        __syncthreads();
-        const int nq = kc / 4;
-        for (int idx = l; idx < 4 * S * nq; idx += 64) {
-            const int row = idx / nq, q = idx - row * nq;
-            const int sq = seq0 + row;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (sq < A.B) v = *reinterpret_cast<const float4*>(J.X + (size_t)sq * J.ldx + k0 + 4 * q);
-            xs4[row * (kRkqKC / 4) + q] = v;
-        }
-        const float4* xl = xs4 + r4 * (kRkqKC / 4);
-        const float* wr = J.w + (size_t)orow * J.Kd + k0;
-        float4 wc[8], wn[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (4 * i < kc) wc[i] = *reinterpret_cast<const float4*>(wr + 4 * i);
-        __syncthreads();
-        for (int kb = 0; kb < kc; kb += 32) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                if (kb + 32 + 4 * i < kc) wn[i] = *reinterpret_cast<const float4*>(wr + kb + 32 + 4 * i);
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                if (kb + 4 * i < kc) {
-                    float4 x4[S];
-#pragma unroll
-                    for (int s = 0; s < S; ++s) x4[s] = xl[4 * s * (kRkqKC / 4) + kb / 4 + i];
-                    step4<S>(x4, wc[i].x, wc[i].y, wc[i].z, wc[i].w, acc);
-                }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) wc[i] = wn[i];
-        }
+        for (int i = 0; i < 4; ++i) r[i] = rkq_epi(J.epi, old[i], acc[i]);
+        *reinterpret_cast<v4f*>(y) = r;
+        return;
     }
 #pragma unroll
-    for (int s = 0; s < S; ++s) rkq_finish(J, A.B, 0, seq0 + 4 * s, out, acc[s]);
+    for (int i = 0; i < 4; ++i)
+        if (out0 + i < J.M) y[i] = rkq_epi(J.epi, J.epi == RKQ_ADD ? y[i] : 0.0f, acc[i]);
 }
 
-// Tiled fp32 weights (block = -1), made at load from the INT4 codes with the
-// producers' dequantization, or from fp32 rows: float4 (t * nb + kb) * 64 + l
-// holds inputs 4 kb .. 4 kb + 3 of row 64 t + l (rows past M repeat row
-// M - 1), nb = Kd / 4, followed by kRkwPad float4 that loads past the end
-// may touch. One wave per 64 rows x S groups of 4 sequences (one wave per
-// workgroup unless a tuning shape groups NW of an output tile's waves),
-// nothing shared between waves, so no barrier paces its chains. A chain
-// step is one dependent v_mfma_f32_4x4x1_16b_f32 (~13 cycles on gfx950),
-// and every other instruction of the wave lengthens it (measured: X read from
-// LDS once per 4 inputs, 13.3 -> 15.3 cycles per input; with 64-bit address
-// arithmetic for a weight load added, 21), so a block of 4 inputs issues
-// only its MFMAs, one buffer load of the next weights (1 KiB of consecutive
-// memory; the scalar offset advances, the lane offset and the immediate stay
-// fixed) and one LDS read of X at an immediate offset from the lane's base.
-// The wave's X rows go straight into LDS at the start (one load latency);
-// its weight blocks run PF blocks ahead in registers. Workgroups are
-// renumbered so that consecutive numbers run on one XCD (dispatch is
-// round-robin over the 8 XCDs): the sequence tiles of an output tile then
-// read its weights from one L2.
-// Weight blocks in flight per wave (PF): chosen by the launcher, 48 while
-// the launch's waves fit one per CU and 16 beyond, when each CU's loads in
-// flight are several waves' worth (measured on the RWKV-7 step, cfg4 INT4:
-// at B = 16 48 beat 24 by 2 % and 56 by 1 %; at B = 64, on the launches of
-// 656 - 768 waves, 24 beat 48 by 2 % and 16 beat 24 by 0.4 %).
-constexpr int kRkwXA = 4;          // X blocks read from LDS ahead of the MFMAs
-constexpr int kRkwXMax = 4096;     // float4 of X per workgroup (64 KiB): S * Kd <= this
-constexpr int kRkwPad = 64 * 64;   // float4 after a tiled matrix (64 blocks: the stream reads up to PF - 1 past a tile)
-// s_waitcnt vmcnt(n) (expcnt, lgkmcnt at their maximum; gfx9 split vmcnt field)
-constexpr int rkw_vmcnt(int n) { return ((n >> 4) & 3) << 14 | 0x0F70 | (n & 15); }
-
-// Direct-to-LDS loads the compiler does not see (inline asm): lane l's 16
-// (4) bytes at gaddr go to LDS byte lds + 16 l (4 l), lds wave-uniform. M0,
-// which holds the LDS base, is saved and restored around the load, and one
-// wait state separates its write from the load. Seen by the compiler
-// (builtin), these writes to LDS counted as pending at every later LDS read
-// of the kernel's chain loop, which then waited for all loads at the top of
-// each trip and drained the weight prefetch; in a function of their own,
-// the call boundary waited for every load. The caller waits for them itself:
-// before its first read of what they bring, and for all of them before the
-// wave ends (its LDS may then go to another workgroup).
-__device__ __forceinline__ void dma_lds16(const void* gaddr, uint32_t lds) {
-    uint32_t save;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %2\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(save)
-        : "v"(gaddr), "s"(lds)
-        : "memory");
-}
-__device__ __forceinline__ void dma_lds4(const void* gaddr, uint32_t lds) {
-    uint32_t save;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %2\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dword %1, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(save)
-        : "v"(gaddr), "s"(lds)
-        : "memory");
-}
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return (uint32_t)(size_t)(const __attribute__((address_space(3))) char*)p;
+// r[j] of lane group g <- r[g] of lane group j (groups of 16 lanes).
+__device__ __forceinline__ void group_transpose(float (&r)[4]) {
+    auto swap32 = [](float& a, float& b) {
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(p[0]);
+        b = __uint_as_float(p[1]);
+    };
+    auto swap16 = [](float& a, float& b) {
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(p[0]);
+        b = __uint_as_float(p[1]);
+    };
+    swap32(r[0], r[2]);
+    swap32(r[1], r[3]);
+    swap16(r[0], r[1]);
+    swap16(r[2], r[3]);
 }
 
-// An LDS address (LDS-typed, so reads through it are ds_read, counted by
-// lgkmcnt only) held in a vector register as far as the compiler knows, so
-// that reads through it keep their whole address in the one register and
-// take the rest as an immediate offset.
-typedef __attribute__((address_space(3))) const v4f lds_f4;
-__device__ __forceinline__ const lds_f4* lds_vbase(const float4* p) {
-    uint32_t a = (uint32_t)(size_t)(const lds_f4*)p;
-    asm volatile("" : "+v"(a));
-    return (const lds_f4*)(size_t)a;
+// A copy the compiler cannot merge with its source: the swaps of the transpose
+// work in place, and the copies it would make itself, of a loaded group's
+// registers, it placed right behind the load, where they wait for it.
+__device__ __forceinline__ float fresh(float v) {
+    float r;
+    asm("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
 }
 
-template <int S, int NW, int PF>
-__global__ __launch_bounds__(64 * NW) void k_rkq_mm_w4(const RkqMMArgs A) {
-    constexpr int R = 4 * S;   // sequences of the wave
-    static_assert(PF % kRkwXA == 0, "the X ring restarts with each weight group");
-    extern __shared__ float4 xsh[];
-    // NW independent waves per workgroup (one per SIMD): sequence tiles
-    // NW u0 .. NW u0 + NW - 1 of one output tile; a wave past the last tile
-    // has no work (nothing here waits on another wave)
+// A unit's weights of a lane for one output tile: 16 inputs of fp32, or one
+// INT4 group.
+template <int BLK> struct RkqW { uint4 q[BLK / 32]; float sc; };
+template <> struct RkqW<0> { float4 w; };
+template <> struct RkqW<-1> { float4 w; };
+
+template <int BLK, int O, int S, int PF>
+__global__ __launch_bounds__(64) void k_rkq_mm(const RkqMMArgs A) {
+    constexpr int U = BLK > 0 ? BLK : 16, UB = U / 16;   // inputs and 16-input blocks of a unit
+    // Consecutive numbers run on one XCD (dispatch is round-robin over the 8):
+    // an output tile's sequence tiles read its weights from one L2.
     const int T = (int)gridDim.x, b = (int)blockIdx.x, q8 = T / 8, r8 = T % 8, x8 = b % 8;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     RkqJob J;
     int u0;
     rkq_job_at(A, x8 * q8 + min(x8, r8) + b / 8, J, u0);
-    const int wg_per_tile = (A.seq_tiles + NW - 1) / NW;
-    const int ot = u0 / wg_per_tile, st = (u0 % wg_per_tile) * NW + wv;
-    if (st >= A.seq_tiles) return;
-    float4* xs = xsh + (size_t)wv * (A.xs_per_wave);
-    const int l = threadIdx.x & 63, r4 = l & 3;
-    const int out = ot * 64 + l;
-    const int seq0 = st * R;
-    const int nb = J.Kd / 4;
-    // the whole tiled matrix with its padding; block kb of this tile at
-    // scalar offset (ot * nb + kb) * 1 KiB, lane offset 16 l
-    const uint32_t bytes = (uint32_t)(((size_t)((J.M + 63) / 64) * nb * 64 + kRkwPad) * sizeof(float4));
-    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(J.w), (short)0, (int)bytes,
-                                                                        0x00020000);
-    const int vo = 16 * l;
-    const int sob = ot * nb * 1024;
-    auto ldw = [&](int kb) -> float4 {
-        const u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(rw, vo, sob + kb * 1024, 0);
+    const int ot = u0 / A.seq_tiles * O, st = u0 % A.seq_tiles * S;
+    const int l = threadIdx.x, n = l & 15, g = l >> 4;
+    const int Kd = J.Kd, nkb = (Kd + 15) / 16, nu = (Kd + U - 1) / U;
+    const int mt = (J.M + 15) / 16, xt = (A.B + 15) / 16;   // output and sequence tiles there are
+    // x (and tiled weights) through buffer resources: block kb of tile t is the
+    // KiB at scalar offset (t nkb + kb) 1024, lane l's float4 at 16 l. Tiles
+    // past the end read the last one; their results are never stored.
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(J.X), (short)0, (int)((uint32_t)xt * nkb * 1024u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(J.w), (short)0, (int)(BLK < 0 ? (uint32_t)mt * nkb * 1024u : 0u), 0x00020000);
+    auto ldf = [&](const __amdgpu_buffer_rsrc_t& r, int so) -> float4 {
+        const u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(r, 16 * l, so, 0);
         return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
     };
-    // The wave's X rows into LDS (float4 f = kb * R + row: lane l of pass f0
-    // brings float4 f0 + l; past the end the last one again, into the
-    // padding of the launch's LDS size).
-    const int nx = nb * R;
-    for (int f0 = 0; f0 < nx; f0 += 64) {
-        const int f = min(f0 + l, nx - 1);
-        const int kb = f / R, row = f - kb * R;
-        dma_lds16(J.X + (size_t)min(seq0 + row, A.B - 1) * (size_t)J.ldx + 4 * kb, lds_addr(xs + f0));
+    int xo[S], wo[O];
+    const float* wr[O];
+    const uint8_t* qr[O];
+    const float* sr[O];
+#pragma unroll
+    for (int s = 0; s < S; ++s) xo[s] = min(st + s, xt - 1) * nkb * 1024;
+#pragma unroll
+    for (int o = 0; o < O; ++o) {
+        wo[o] = min(ot + o, mt - 1) * nkb * 1024;
+        const int row = min((ot + o) * 16 + n, J.M - 1);
+        wr[o] = BLK == 0 ? J.w + (size_t)row * Kd : nullptr;
+        qr[o] = BLK > 0 ? J.q + (size_t)row * (size_t)(Kd / 2) : nullptr;
+        sr[o] = BLK > 0 ? J.sc + (size_t)row * (size_t)(Kd / U) : nullptr;
     }
-    float4 w[PF];
+    RkqW<BLK> w[PF][O];
+    float4 x[PF][S][UB];
+    auto load = [&](int p, int u_) {
+        const int u = min(u_, nu - 1);               // past the end: the last unit again, never used
 #pragma unroll
-    for (int i = 0; i < PF; ++i) w[i] = ldw(i);
-    // X in: every load but the PF weight loads above
-    __builtin_amdgcn_s_waitcnt(rkw_vmcnt(PF));
-    __builtin_amdgcn_sched_barrier(0);
-    // The L2 prefetch, issued once X is in (so the chains do not wait for
-    // it): this sequence tile's share of the output tile's weights past the
-    // first PF blocks (at most 63 - PF blocks, so that the wave's loads in
-    // flight fit the wait counter; lane l touches bytes 16 l .. + 4 of each
-    // 1 KiB block, so every 128-byte line) into a 256-byte LDS slot nothing
-    // reads. The sequence tiles of an output tile each take their own part,
-    // so its weights leave HBM together rather than block by block as every
-    // chain reaches them.
-    {
-        const int rest = max(nb - PF, 0), share = (rest + A.seq_tiles - 1) / A.seq_tiles;
-        const int pf0 = PF + min(st * share, rest);
-        // only in the shallow form (several waves per CU): with one wave per
-        // CU the deep stream alone was faster (B = 16 1,145 -> 1,125 us/step
-        // without it; B = 64 1,304 -> 1,297 with it on the shallow launches only)
-        const int npf = PF < 48 ? min(min(share, nb - pf0), 63 - PF) : 0;
-        const char* wb = reinterpret_cast<const char*>(J.w) + (size_t)(sob + pf0 * 1024) + 16 * l;
-        const uint32_t dump = lds_addr(xs + A.xs_per_wave - 16);
-        for (int j = 0; j < npf; ++j) dma_lds4(wb + 1024 * j, dump);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    v4f xa[kRkwXA][S];
-    v4f acc[S];
+        for (int o = 0; o < O; ++o) {
+            if constexpr (BLK < 0) {
+                w[p][o].w = ldf(rw, wo[o] + u * 1024);
+            } else if constexpr (BLK == 0) {
+                w[p][o].w = *reinterpret_cast<const float4*>(wr[o] + min(u * U + 4 * g, Kd - 4));
+            } else {
 #pragma unroll
-    for (int s = 0; s < S; ++s) acc[s] = v4f{0.f, 0.f, 0.f, 0.f};
-    {
-        const lds_f4* xq = lds_vbase(xs + r4);   // block kb of group s: xq[kb * R + 4 s]
+                for (int i = 0; i < BLK / 32; ++i)
+                    w[p][o].q[i] = *reinterpret_cast<const uint4*>(qr[o] + u * (BLK / 2) + 16 * i);
+                w[p][o].sc = sr[o][u];
+            }
+        }
 #pragma unroll
-        for (int j = 0; j < kRkwXA; ++j)
+        for (int s = 0; s < S; ++s)
 #pragma unroll
-            for (int s = 0; s < S; ++s) xa[j][s] = xq[j * R + 4 * s];
-    }
-    // X past block nb - 1 is read from the launch's LDS padding and weights
-    // past the tile from the next tile or the padding, never used.
-    int b0 = 0;
-    for (; b0 + PF <= nb; b0 += PF) {
-        const lds_f4* xq = lds_vbase(xs + r4 + b0 * R);
+            for (int i = 0; i < UB; ++i) x[p][s][i] = ldf(rx, xo[s] + (u * UB + i) * 1024);
+    };
+    v4f acc[O][S];
 #pragma unroll
-        for (int i = 0; i < PF; ++i) {
-            step4<S>(xa[i % kRkwXA], w[i].x, w[i].y, w[i].z, w[i].w, acc);
-            w[i] = ldw(b0 + PF + i);
+    for (int o = 0; o < O; ++o)
 #pragma unroll
-            for (int s = 0; s < S; ++s) xa[i % kRkwXA][s] = xq[(i + kRkwXA) * R + 4 * s];
-            // each block's refill stays with it (the scheduler otherwise sank
-            // the group's weight loads below its last MFMA)
-            __builtin_amdgcn_sched_barrier(0);
+        for (int s = 0; s < S; ++s) acc[o][s] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto unit = [&](int p, int u) {
+#pragma unroll
+        for (int i = 0; i < UB; ++i) {
+            float wv[O][4];
+#pragma unroll
+            for (int o = 0; o < O; ++o) {
+                if constexpr (BLK < 0) {
+                    const float4 v = w[p][o].w;
+                    wv[o][0] = v.x; wv[o][1] = v.y; wv[o][2] = v.z; wv[o][3] = v.w;
+                } else if constexpr (BLK == 0) {
+                    const bool in = u * U + 4 * g < Kd;   // a short last unit is padded with zeros
+                    const float4 v = w[p][o].w;
+                    wv[o][0] = in ? fresh(v.x) : 0.0f; wv[o][1] = in ? fresh(v.y) : 0.0f;
+                    wv[o][2] = in ? fresh(v.z) : 0.0f; wv[o][3] = in ? fresh(v.w) : 0.0f;
+                    group_transpose(wv[o]);
+                } else {
+                    // step 4 i + j: dword 4 i + j of the low nibbles, then of the high
+                    constexpr int HB = UB / 2;
+                    const float sc = w[p][o].sc, m8 = -8.0f * sc;
+                    const uint4 q = w[p][o].q[i % HB];
+                    const uint32_t sh = 8 * g + (i < HB ? 0 : 4);
+                    wv[o][0] = fmaf((float)((q.x >> sh) & 0xFu), sc, m8);
+                    wv[o][1] = fmaf((float)((q.y >> sh) & 0xFu), sc, m8);
+                    wv[o][2] = fmaf((float)((q.z >> sh) & 0xFu), sc, m8);
+                    wv[o][3] = fmaf((float)((q.w >> sh) & 0xFu), sc, m8);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int o = 0; o < O; ++o)
+#pragma unroll
+                    for (int s = 0; s < S; ++s) {
+                        const float4 v = x[p][s][i];
+                        const float xv = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
+                        acc[o][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[o][j], xv, acc[o][s], 0, 0, 0);
+                    }
+        }
+    };
+#pragma unroll
+    for (int p = 0; p < PF; ++p) load(p, p);
+    int ub = 0;
+    for (; ub + PF <= nu; ub += PF) {
+#pragma unroll
+        for (int p = 0; p < PF; ++p) {
+            unit(p, ub + p);
+            load(p, ub + p + PF);
+            __builtin_amdgcn_sched_barrier(0);       // a unit's loads stay with it
         }
     }
-    const int rem = nb - b0;   // < PF blocks, already in registers
-    const lds_f4* xq = lds_vbase(xs + r4 + b0 * R);
 #pragma unroll
-    for (int i = 0; i < PF; ++i) {
-        if (i < rem) {
-            step4<S>(xa[i % kRkwXA], w[i].x, w[i].y, w[i].z, w[i].w, acc);
+    for (int p = 0; p < PF; ++p)
+        if (ub + p < nu) unit(p, ub + p);
 #pragma unroll
-            for (int s = 0; s < S; ++s) xa[i % kRkwXA][s] = xq[(i + kRkwXA) * R + 4 * s];
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(rkw_vmcnt(0));   // the L2 prefetch's writes to LDS, before the wave can end
+    for (int o = 0; o < O; ++o)
 #pragma unroll
-    for (int s = 0; s < S; ++s) rkq_finish(J, A.B, -1, seq0 + 4 * s, out, acc[s]);
+        for (int s = 0; s < S; ++s)
+            rkq_finish(J, A.B, BLK, (st + s) * 16 + n, (ot + o) * 16 + 4 * g, acc[o][s]);
 }
 
-// The tiled form (above) of an M x Kd matrix: each value the one the
-// products use (dequant_at: fp32 rows, or INT4 codes dequantized as the
-// producers do); the padding is zeroed.
-__global__ __launch_bounds__(256) void k_rkq_block4(RkqJob J, int blk, float4* out) {
-    const int nb = J.Kd / 4;
-    const size_t n = (size_t)((J.M + 63) / 64) * nb * 64;
+// The tiled fp32 form of an M x Kd matrix: x16 order with the output in the
+// row's place, each value the one the products use, zeros past Kd; rows past M
+// repeat row M - 1.
+__global__ __launch_bounds__(256) void k_rkq_tile(RkqJob J, int blk, float* out) {
+    const int nkb = (J.Kd + 15) / 16;
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n + kRkwPad) return;
-    if (i >= n) {
-        out[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        return;
-    }
-    const int l = (int)(i % 64), kb = (int)((i / 64) % nb), t = (int)(i / 64 / nb);
-    const int o = min(64 * t + l, J.M - 1);
-    float4 v;
-    v.x = dequant_at(J, o, 4 * kb, blk);
-    v.y = dequant_at(J, o, 4 * kb + 1, blk);
-    v.z = dequant_at(J, o, 4 * kb + 2, blk);
-    v.w = dequant_at(J, o, 4 * kb + 3, blk);
-    out[i] = v;
-}
-
-// INT4 weights: a workgroup of kRkqNP producer waves and NC consumer waves
-// per 64 rows x 4 S NC sequences.
-//
-// Producer wave h dequantizes half h (32 inputs) of every 64-input unit of
-// the rows: at step t it converts unit t from codes and scales it loaded
-// kRkqPF units earlier into slot t % 3 of an LDS ring ([block][row] float4,
-// conflict-free). Consumer c multiplies unit t - 2 at step t, S independent
-// k-ordered MFMA chains of 4 sequences each sharing the weight operand. Its
-// weight window runs kRkqWD blocks of 4 inputs ahead of the MFMAs and
-// crosses into unit t - 1 (complete since the previous step), and its X
-// operands come from global memory one unit ahead, so the chains wait on
-// neither LDS nor global memory. One workgroup barrier per step, waiting on
-// LDS only; every weight is dequantized once per workgroup.
-constexpr int kRkqPF = 4;     // producer code prefetch, units
-constexpr int kRkqWD = 8;     // consumer weight window, blocks of 4 inputs (a half unit)
-
-// Producer wave h (0 or 1) of an INT4 product workgroup: converts half h of
-// every 64-input unit of rows orow.. into slot t % 3 of the LDS ring at
-// step t, one workgroup barrier per step, nsteps steps in all.
-template <int BLK>
-__device__ __forceinline__ void rkq_produce(const RkqJob& J, int h, int l, int orow, int nu, int nsteps,
-                                            float4 (*wring)[kRkqU / 4][64]) {
-    const int Kd = J.Kd;
-    constexpr int NQ = BLK / 32;
-    const uint8_t* qrow = J.q + (size_t)orow * (size_t)(Kd / 2);
-    const float* srow = J.sc + (size_t)orow * (size_t)(Kd / BLK);
-    uint4 qw[kRkqPF][NQ];
-    float sw[kRkqPF];
-    // Branch-free loads: a unit past the end reads the last half again
-    // (never converted), so no wait depends on control flow.
-    auto load = [&](int u, uint4 (&q)[NQ], float& s) {
-        const int k = min(u * kRkqU + 32 * h, Kd - 32);
-        if (BLK == 32) {
-            q[0] = *reinterpret_cast<const uint4*>(qrow + k / 2);
-            s = srow[k / 32];
-        } else {
-            const int g = k / 64;
-#pragma unroll
-            for (int i = 0; i < NQ; ++i) q[i] = *reinterpret_cast<const uint4*>(qrow + g * 32 + 16 * i);
-            s = srow[g];
-        }
-    };
-#pragma unroll
-    for (int p = 0; p < kRkqPF; ++p) load(p, qw[p], sw[p]);
-    // Groups of kRkqPF steps: a group first issues the loads of the next
-    // group's units, then converts its own (loaded one group earlier), so
-    // every wait on codes covers loads a whole group old.
-    for (int t0 = 0; t0 < nsteps; t0 += kRkqPF) {
-        uint4 qn[kRkqPF][NQ];
-        float sn[kRkqPF];
-#pragma unroll
-        for (int p = 0; p < kRkqPF; ++p) load(t0 + kRkqPF + p, qn[p], sn[p]);
-#pragma unroll
-        for (int p = 0; p < kRkqPF; ++p) {
-            const int t = t0 + p;
-            // Converted unconditionally: past the last unit (or the
-            // missing half of a half unit) this writes leftovers to slot
-            // t % 3, which the consumers do not read at or after step t.
-            const float scg = sw[p], m8 = -8.0f * scg;
-            // Block i of the half: inputs 4i .. 4i+3. BLK 64: nibble h of
-            // bytes 4i .. 4i+3; BLK 32: low nibbles of word i for i < 4,
-            // high nibbles of word i - 4 after.
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const uint4 v = BLK == 32 ? qw[p][0] : qw[p][(i >> 2) % NQ];
-                const int wi = i & 3;
-                const uint32_t word = wi == 0 ? v.x : wi == 1 ? v.y : wi == 2 ? v.z : v.w;
-                const bool hi = BLK == 32 ? i >= 4 : h == 1;
-                uint32_t nib = (hi ? (word >> 4) : word) & 0x0F0F0F0Fu;
-                // Opaque to the compiler, so that each byte converts with
-                // one v_cvt_f32_ubyteN (no field extraction).
-                asm volatile("" : "+v"(nib));
-                float4 w;
-                w.x = fmaf((float)(nib & 0xFFu), scg, m8);
-                w.y = fmaf((float)((nib >> 8) & 0xFFu), scg, m8);
-                w.z = fmaf((float)((nib >> 16) & 0xFFu), scg, m8);
-                w.w = fmaf((float)(nib >> 24), scg, m8);
-                wring[t % 3][8 * h + i][l] = w;
-            }
-            __syncthreads();
-            // keep each step's conversion after its barrier
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int p = 0; p < kRkqPF; ++p) {
-#pragma unroll
-            for (int i = 0; i < NQ; ++i) qw[p][i] = qn[p][i];
-            sw[p] = sn[p];
-        }
-    }
-}
-
-// X rows staged in LDS (XD = 0) take at most 64 KiB: rows of up to
-// kRkqXLF / (sequences per workgroup) inputs.
-constexpr int kRkqXLF = 16384;
-
-template <int BLK, int NC, int S, int XD>
-__global__ __launch_bounds__(64 * (NC + kRkqNP)) void k_rkq_mm_q4(const RkqMMArgs A) {
-    constexpr int U4 = kRkqU / 4;                      // blocks per unit
-    static_assert(U4 % kRkqWD == 0 && kRkqWD == U4 / 2, "the weight window is a half unit");
-    constexpr int XR = XD > 0 ? XD : 1;                // X register sets
-    constexpr int NSQ = 4 * S * NC;                    // sequences of the workgroup
-    __shared__ float4 wring[3][U4][64];
-    constexpr int XLK = kRkqXLF / NSQ;                 // inputs per staged row
-    constexpr int XLS = XLK / 4 + 1;                   // row stride in float4 (padded: rows on distinct banks)
-    __shared__ float4 xlds[XD == 0 ? NSQ * XLS : 1];
-    RkqJob J;
-    int u0;
-    rkq_job(A, J, u0);
-    const int ot = u0 / A.seq_tiles, st = u0 % A.seq_tiles;
-    // wave index in a scalar register: every branch on the role is uniform
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, r4 = l & 3;
-    const int out = ot * 64 + l;
-    const int orow = out < J.M ? out : J.M - 1;
-    const int Kd = J.Kd;
-    const int nu = (Kd + kRkqU - 1) / kRkqU;            // the last unit is half when Kd % 64 == 32
-    const bool half_last = (Kd % kRkqU) != 0;
-    // Steps (one barrier each) for both roles: units 0 .. nu - 1 are written
-    // at steps 0 .. nu - 1 and multiplied at steps 2 .. nu + 1; the count is
-    // rounded up to the producer's prefetch depth (idle steps at the end).
-    const int nsteps = (nu + 2 + kRkqPF - 1) / kRkqPF * kRkqPF;
-    if constexpr (XD == 0) {
-        // The X rows of the workgroup's sequences into LDS, by every wave
-        // (Kd <= XLK; rows past the batch repeat the last sequence's).
-        const int kq = Kd / 4;
-        for (int idx = threadIdx.x; idx < NSQ * kq; idx += 64 * (NC + kRkqNP)) {
-            const int sq = idx / kq, q = idx - sq * kq;
-            xlds[sq * XLS + q] =
-                *reinterpret_cast<const float4*>(J.X + (size_t)min(st * NSQ + sq, A.B - 1) * (size_t)J.ldx + 4 * q);
-        }
-        __syncthreads();
-    }
-    if (wv < kRkqNP) {
-        rkq_produce<BLK>(J, wv, l, orow, nu, nsteps, wring);
-        return;
-    }
-    // ---- consumer c: sequences seqb + 4 s + (0..3), lane row r4 of each chain.
-    // Rows past the batch read the last sequence's X (their outputs are not
-    // stored), and loads past the end re-read the last block, so every load
-    // is unconditional and no wait depends on control flow.
-    const int c = wv - kRkqNP;
-    const int seqb = st * (4 * S * NC) + c * (4 * S);
-    const float* xr[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s)
-        xr[s] = J.X + (size_t)min(seqb + 4 * s + r4, A.B - 1) * (size_t)J.ldx;
-    // X operands run XR units ahead of the MFMAs, from global memory (XD = 1;
-    // XD = 2 in launches of at most one workgroup per CU, whose chains then
-    // wait on X less: the second set's registers would keep larger grids
-    // from residing at three workgroups per CU) or from the rows staged in
-    // LDS (XD = 0).
-    static_assert(XD >= 0 && XD <= 2, "X depth");
-    auto ldx = [&](int s, int k) -> float4 {
-        if constexpr (XD == 0) return xlds[(c * 4 * S + 4 * s + r4) * XLS + (k >> 2)];
-        else return *reinterpret_cast<const float4*>(xr[s] + k);
-    };
-    float4 xw[XR][S][U4];   // unit u's block i in xw[u % XR]; refilled with unit u + XR's
-    float4 ww[kRkqWD];      // weight blocks, slot = block % kRkqWD
-    v4f acc[S];
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-        acc[s] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int d = 0; d < XR; ++d)
-#pragma unroll
-            for (int i = 0; i < U4; ++i) xw[d][s][i] = ldx(s, min(d * kRkqU + 4 * i, Kd - 4));
-    }
-    // Steps 0 and 1: the producers write units 0 and 1; the window takes
-    // unit 0's first half once it is complete.
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kRkqWD; ++j) ww[j] = wring[0][j][l];
-    __syncthreads();
-    // One full unit from X set P: block i's MFMAs, then its refills (weight
-    // block i + kRkqWD, from the next unit's slot for the last half; X block i
-    // of unit u + XD). Straight-line, so the window stays in place.
-    auto full_unit = [&](auto par, int slot, int nslot, int knext) {
-        constexpr int P = decltype(par)::value;
-#pragma unroll
-        for (int i = 0; i < U4; ++i) {
-            const float4 wc = ww[i % kRkqWD];
-#pragma unroll
-            for (int s = 0; s < S; ++s) acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(xw[P][s][i].x, wc.x, acc[s], 0, 0, 0);
-#pragma unroll
-            for (int s = 0; s < S; ++s) acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(xw[P][s][i].y, wc.y, acc[s], 0, 0, 0);
-#pragma unroll
-            for (int s = 0; s < S; ++s) acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(xw[P][s][i].z, wc.z, acc[s], 0, 0, 0);
-#pragma unroll
-            for (int s = 0; s < S; ++s) acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(xw[P][s][i].w, wc.w, acc[s], 0, 0, 0);
-            ww[i % kRkqWD] = i + kRkqWD < U4 ? wring[slot][i + kRkqWD][l] : wring[nslot][i + kRkqWD - U4][l];
-            const int kx = min(knext + 4 * i, Kd - 4);
-#pragma unroll
-            for (int s = 0; s < S; ++s) xw[P][s][i] = ldx(s, kx);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    auto half_unit = [&](auto par) {
-        constexpr int P = decltype(par)::value;
-#pragma unroll
-        for (int i = 0; i < U4 / 2; ++i) {
-            const float4 wc = ww[i % kRkqWD];
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(xw[P][s][i].x, wc.x, acc[s], 0, 0, 0);
-                acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(xw[P][s][i].y, wc.y, acc[s], 0, 0, 0);
-                acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(xw[P][s][i].z, wc.z, acc[s], 0, 0, 0);
-                acc[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(xw[P][s][i].w, wc.w, acc[s], 0, 0, 0);
-            }
-        }
-    };
-    constexpr std::integral_constant<int, 0> x0{};
-    constexpr std::integral_constant<int, XR - 1> x1{};
-    // Steps 2 .. nu: units 0 .. nu - 2, each followed by another; two at a
-    // time, so that the X set of each is fixed at compile time.
-    int u = 0;
-    for (; u + 2 <= nu - 1; u += 2) {
-        full_unit(x0, u % 3, (u + 1) % 3, (u + XR) * kRkqU);
-        __syncthreads();
-        full_unit(x1, (u + 1) % 3, (u + 2) % 3, (u + 1 + XR) * kRkqU);
-        __syncthreads();
-    }
-    if (u < nu - 1) {   // one more (u even: set 0)
-        full_unit(x0, u % 3, (u + 1) % 3, (u + XR) * kRkqU);
-        __syncthreads();
-        ++u;
-    }
-    // Step nu + 1: the last unit, u = nu - 1 (its refills read in-bounds
-    // leftovers).
-    if ((u & 1) == 0 || XR == 1) {
-        if (!half_last) full_unit(x0, u % 3, (u + 1) % 3, Kd);
-        else half_unit(x0);
-    } else {
-        if (!half_last) full_unit(x1, u % 3, (u + 1) % 3, Kd);
-        else half_unit(x1);
-    }
-    __syncthreads();
-    for (int t = nu + 2; t < nsteps; ++t) __syncthreads();
-#pragma unroll
-    for (int s = 0; s < S; ++s) rkq_finish(J, A.B, BLK, seqb + 4 * s, out, acc[s]);
-}
-
-// INT4 weights, wide form: as k_rkq_mm_q4, but each consumer wave runs one
-// chain of v_mfma_f32_16x16x1_4b_f32 over 16 sequences. That instruction also
-// holds one product per output per instruction and rounds once (checked on
-// gfx950: a chain of them in k order equals the sequential fmaf chain), and
-// one chain of it keeps a SIMD's matrix pipe busy (a dependent one issues
-// every ~32.5 cycles, independent ones every ~32), so a wave covers 16
-// sequences x 64 rows with one accumulator. Lane l supplies weight row
-// out0 + l (B, block l / 16, column l % 16) and the input of sequence l % 16
-// (A, the same rows in every block); it then holds, in register 4 b + r,
-// sequence 4 (l / 16) + r of row out0 + 16 b + l % 16.
-template <int BLK, int NC>
-__global__ __launch_bounds__(64 * (NC + kRkqNP)) void k_rkq_mm_q4w(const RkqMMArgs A) {
-    constexpr int U4 = kRkqU / 4;
-    __shared__ float4 wring[3][U4][64];
-    RkqJob J;
-    int u0;
-    rkq_job(A, J, u0);
-    const int ot = u0 / A.seq_tiles, st = u0 % A.seq_tiles;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
-    const int out = ot * 64 + l;
-    const int orow = out < J.M ? out : J.M - 1;
-    const int Kd = J.Kd;
-    const int nu = (Kd + kRkqU - 1) / kRkqU;
-    const bool half_last = (Kd % kRkqU) != 0;
-    const int nsteps = (nu + 2 + kRkqPF - 1) / kRkqPF * kRkqPF;
-    if (wv < kRkqNP) {
-        rkq_produce<BLK>(J, wv, l, orow, nu, nsteps, wring);
-        return;
-    }
-    const int c = wv - kRkqNP;
-    const int seqb = st * (16 * NC) + 16 * c;
-    const float* xr = J.X + (size_t)min(seqb + (l & 15), A.B - 1) * (size_t)J.ldx;
-    // (X rows staged in LDS, as the one-chain kernel does for large grids,
-    // made the channel-mix key at B = 64 slower: its chains wait on the
-    // 16x16x1 issue rate, not on X.)
-    float4 xw[U4];
-    float4 ww[kRkqWD];
-    v16f acc = {};
-#pragma unroll
-    for (int i = 0; i < U4; ++i) xw[i] = *reinterpret_cast<const float4*>(xr + min(4 * i, Kd - 4));
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kRkqWD; ++j) ww[j] = wring[0][j][l];
-    __syncthreads();
-    auto full_unit = [&](int slot, int nslot, int knext) {
-#pragma unroll
-        for (int i = 0; i < U4; ++i) {
-            const float4 wc = ww[i % kRkqWD];
-            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(xw[i].x, wc.x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(xw[i].y, wc.y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(xw[i].z, wc.z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(xw[i].w, wc.w, acc, 0, 0, 0);
-            ww[i % kRkqWD] = i + kRkqWD < U4 ? wring[slot][i + kRkqWD][l] : wring[nslot][i + kRkqWD - U4][l];
-            xw[i] = *reinterpret_cast<const float4*>(xr + min(knext + 4 * i, Kd - 4));
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    for (int u = 0; u < nu - 1; ++u) {
-        full_unit(u % 3, (u + 1) % 3, (u + 1) * kRkqU);
-        __syncthreads();
-    }
-    const int ul = nu - 1;
-    if (!half_last) {
-        full_unit(ul % 3, (ul + 1) % 3, Kd);
-    } else {
-#pragma unroll
-        for (int i = 0; i < U4 / 2; ++i) {
-            const float4 wc = ww[i % kRkqWD];
-            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(xw[i].x, wc.x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(xw[i].y, wc.y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(xw[i].z, wc.z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(xw[i].w, wc.w, acc, 0, 0, 0);
-        }
-    }
-    __syncthreads();
-    for (int t = nu + 2; t < nsteps; ++t) __syncthreads();
-    const int sq0 = seqb + 4 * (l >> 4), col = ot * 64 + (l & 15);
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) rkq_finish1(J, A.B, BLK, sq0 + r, col + 16 * b, acc[4 * b + r]);
+    if (i >= (size_t)((J.M + 15) / 16) * nkb * 256) return;
+    const int j = i & 3, l = (i >> 2) & 63;
+    const size_t t = i >> 8;
+    const int k = (int)(t % nkb) * 16 + 4 * j + (l >> 4), row = min((int)(t / nkb) * 16 + (l & 15), J.M - 1);
+    out[i] = k < J.Kd ? dequant_at(J, row, k, blk) : 0.0f;
 }
 
 // ---------------------------------------------------------------- heads
@@ -1137,7 +699,9 @@ __global__ __launch_bounds__(64 * NWV) void k_rkq_heads(RkqHeadArgs A) {
     }
     sync();
     const float n = (yy - mean) * stat[0] * lnw + lnb;
-    A.y[row + c] = (n + dot * vv) * gv;
+    const float yg = (n + dot * vv) * gv;
+    A.y[x16_at(b, c, A.D / 16)] = yg;
+    if (A.dbg && b == 0) A.dbg[(size_t)7 * A.D + c] = yg;
 }
 
 __global__ void k_refmath(const float* __restrict__ x, float* __restrict__ e, float* __restrict__ th,
@@ -1152,7 +716,7 @@ __global__ void k_refmath(const float* __restrict__ x, float* __restrict__ e, fl
 }  // namespace
 
 snhip_status launch_rkq_ln(const RkqLnArgs& a, int B, hipStream_t st) {
-    if (a.D <= 0 || a.D > kLnMax || a.D % 4 || B <= 0) return SNHIP_E_INVAL;
+    if (a.D <= 0 || a.D > kLnMax || a.D % 16 || B <= 0) return SNHIP_E_INVAL;
     hipLaunchKernelGGL(k_rkq_ln<kLnT>, dim3(B), dim3(kLnT), 0, st, a);
     SNHIP_CHECK(hipGetLastError());
     return SNHIP_OK;
@@ -1191,215 +755,73 @@ int cu_count() {
     return cached[dev];
 }
 
-// nc, s: INT4 consumer waves per workgroup and chains per consumer (0: chosen
-// here); fp32 rows: s groups of 4 sequences per wave; tiled fp32: nc waves
-// per workgroup, s groups of 4 sequences per wave.
-snhip_status launch_rkq_mm_cfg(const RkqJob* jobs, int n, int B, int block, int nc, int s,
-                               hipStream_t st) {
+snhip_status launch_rkq_mm(const RkqJob* jobs, int n, int B, int block, hipStream_t st) {
     if (n <= 0 || n > kRkqMaxJobs || B <= 0 || (block != -1 && block != 0 && block != 32 && block != 64))
         return SNHIP_E_INVAL;
     RkqMMArgs a{};
-    int tiles1 = 0, kmax = 0;
+    const long seqs = (B + 15) / 16;
     for (int i = 0; i < n; ++i) {
         const RkqJob& J = jobs[i];
-        const int kq = block > 0 ? block : 4;
-        if (J.M <= 0 || J.Kd <= 0 || J.Kd % kq || J.ldx % 4 || !J.X || !J.Y ||
-            (block > 0 ? (!J.q || !J.sc || J.Kd % 32) : !J.w))
+        if (J.M <= 0 || J.Kd <= 0 || J.Kd % (block > 0 ? block : 4) || !J.X || !J.Y ||
+            (block > 0 ? (!J.q || !J.sc) : !J.w) || (J.y16 && J.epi == RKQ_ADD) ||
+            seqs * ((J.Kd + 15) / 16) >= (1 << 21))   // x within 32-bit offsets
             return SNHIP_E_INVAL;
         a.j[i] = J;
-        a.tiles_out[i] = (J.M + 63) / 64;
-        tiles1 += a.tiles_out[i];
-        kmax = std::max(kmax, J.Kd);
     }
-    int per;   // sequences per workgroup
-    int S = 1, NC = 1;
-    bool xl = false;   // INT4: four one-chain consumers per workgroup, X staged in LDS
-    size_t shm = 0;
-    int NW = 1;   // tiled fp32: waves per workgroup
-    bool wdeep = true;   // tiled fp32: the deeper weight stream (at most one wave per CU)
-    if (block < 0) {
-        // One chain per wave; the waves of one output tile's sequence tiles
-        // in workgroups of NW (one per SIMD) once there are more waves than
-        // CUs; more than four per CU: two chains per wave, and so on.
-        const long cus = cu_count();
-        auto waves = [&](int s_) { return (long)tiles1 * ((B + 4 * s_ - 1) / (4 * s_)); };
-        // SNHIP_RKQ_W4_SHAPE=S,NW (tuning): that shape wherever it fits
-        if (!s && !nc)
-            if (const char* e = getenv("SNHIP_RKQ_W4_SHAPE")) {
-                int s_ = 0, n_ = 0;
-                if (sscanf(e, "%d,%d", &s_, &n_) == 2 && (s_ == 1 || s_ == 2 || s_ == 4) &&
-                    (n_ == 1 || n_ == 2 || n_ == 4) && s_ * kmax <= kRkwXMax &&
-                    (size_t)n_ * ((s_ * kmax + 63) / 64 * 64 + kRkwXA * 4 * s_ + 16) * sizeof(float4) <= 65536) {
-                    s = s_;
-                    nc = n_;
-                }
-            }
-        S = 1;
-        if (s) S = s;
-        else
-            while (S < 4 && waves(S) > 4 * cus) S *= 2;
-        while (!s && S > 1 && S * kmax > kRkwXMax) S /= 2;
-        if ((S != 1 && S != 2 && S != 4) || S * kmax > kRkwXMax) return SNHIP_E_INVAL;
-        // One wave per workgroup (grouping an output tile's waves 2 or 4 per
-        // workgroup measured 2 % slower at B = 64 once the stream depth
-        // follows the waves per CU); NW only when forced.
-        NW = nc ? nc : 1;
-        wdeep = waves(S) <= cus;
-        // per wave: X (S Kd float4, rounded up to the staging's 64) and the
-        // read-ahead past the last block; at most 64 KiB per workgroup
-        a.xs_per_wave = (S * kmax + 63) / 64 * 64 + kRkwXA * 4 * S + 16;   // + the prefetch's dump slot
-        while (!nc && NW > 1 && (size_t)NW * a.xs_per_wave * sizeof(float4) > 65536) NW /= 2;
-        shm = (size_t)NW * a.xs_per_wave * sizeof(float4);
-        if ((NW != 1 && NW != 2 && NW != 4) || shm > 65536) return SNHIP_E_INVAL;
-        per = 4 * S;
-    } else if (block == 0) {
-        const long waves1 = (long)tiles1 * ((B + 3) / 4);
-        S = s ? s : (B > 8 && waves1 / 4 >= 1024) ? 4 : (B > 4 && waves1 / 2 >= 1024) ? 2 : 1;
-        if (S != 1 && S != 2 && S != 4) return SNHIP_E_INVAL;
-        per = 4 * S;
-    } else {
-        // Measured on MI355X (K = 768 / 3072 products, B = 1 / 8 / 64): one
-        // consumer of one chain is fastest while the grid of such workgroups
-        // stays within ~1024 (up to 3 reside per CU); larger grids (the
-        // vocabulary head) share the dequantized units among more chains.
-        // S = 16 selects the wide kernel (one 16x16x1 chain of 16 sequences
-        // per consumer), used from B = 8 once the one-chain grid exceeds 256
-        // workgroups (SNHIP_RKQ_WIDE_GRID): the products are then bound by
-        // matrix-core throughput, not chain latency. NC then keeps the grid at
-        // >= ~512 workgroups. Measured on the RWKV-7 step (B = 64): head
-        // 376 -> 112 us, channel-mix key 26 -> 21 us.
-        const long wg11 = (long)tiles1 * ((B + 3) / 4);
-        int nc0 = wg11 <= 1024 ? 1 : 2, s0 = wg11 <= 1024 || B < 16 ? 1 : 2;
-        // Not for launches with a tanh / sigmoid epilogue (a wide lane finishes
-        // 16 outputs, not 4) or with a short K (fill-bound).
-        bool wide_ok = true;
-        for (int i = 0; i < n; ++i)
-            wide_ok = wide_ok && jobs[i].Kd >= 256 && jobs[i].epi != RKQ_TANH && jobs[i].epi != RKQ_SIGMOID;
-        if (wide_ok && B >= 8 && wg11 > (long)env_unsigned("SNHIP_RKQ_WIDE_GRID", 256, 0)) {
-            s0 = 16;
-            nc0 = B > 32 ? 4 : B > 16 ? 2 : 1;   // chains of 16 per workgroup: 1, 2 or 4 (instantiated)
-            while (nc0 > 1 && (long)tiles1 * ((B + 16 * nc0 - 1) / (16 * nc0)) < 512) nc0 /= 2;
-        }
-        NC = nc ? nc : nc0;
-        S = s ? s : s0;
-        if (!((NC == 1 || NC == 2 || NC == 4) && (S == 1 || S == 2 || S == 16)) || (NC == 4 && S == 2))
-            return SNHIP_E_INVAL;
-        // One-chain launches of more than one workgroup per CU instead run
-        // one workgroup of four consumers per 16 sequences with their X rows
-        // staged in LDS once (each consumer lane otherwise loads its X from
-        // global memory one unit ahead, and at three workgroups per CU those
-        // loads' latency held the chains back). Measured on the RWKV-7 step
-        // at B = 64 (r, k, v and the LoRA downs, 656 -> 164 workgroups):
-        // 31.3 -> 21.9 us; the LoRA ups 7.3 -> 6.5. Staging the rows of
-        // smaller grids (one workgroup of one consumer per CU) was slower
-        // (B = 8 step 1384 -> 1504 us).
-        if (!nc && !s && NC == 1 && S == 1 && B >= 16 && wg11 > (long)cu_count() &&
-            env_unsigned("SNHIP_RKQ_XL", 1, 0)) {
-            bool fits = true;
-            for (int i = 0; i < n; ++i) fits = fits && jobs[i].Kd <= kRkqXLF / 16;
-            if (fits) {
-                NC = 4;
-                xl = true;
-            }
-        }
-        per = (S == 16 ? 16 : 4 * S) * NC;
+    // Output x sequence tiles per wave: the fewest rounds of chains over the
+    // SIMDs (four per CU; each runs its waves' chains at 8 cycles per input, a
+    // lone chain at 9); where shapes come out even, the larger one reads its
+    // operands less often.
+    const long simds = 4L * cu_count();
+    static constexpr int kShape[4][2] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}};
+    int shape = 0;
+    double best = 0.0;
+    auto waves = [&](int i) { return (jobs[i].M + 15) / 16; };
+    for (int h = 0; h < 4; ++h) {
+        const int O = kShape[h][0], S = kShape[h][1];
+        long tiles = 0;
+        for (int i = 0; i < n; ++i) tiles += (waves(i) + O - 1) / O;
+        const long rounds = (tiles * ((seqs + S - 1) / S) + simds - 1) / simds;
+        const double cost = rounds * O * S == 1 ? 1.125 : (double)(rounds * O * S);
+        if (h == 0 || cost <= best) { shape = h; best = cost; }
     }
+    const int O = kShape[shape][0], S = kShape[shape][1];
     a.n = n;
     a.B = B;
-    a.seq_tiles = (B + per - 1) / per;
+    a.seq_tiles = (int)((seqs + S - 1) / S);
     int total = 0;
     for (int i = 0; i < n; ++i) {
         a.start[i] = total;
-        total += a.tiles_out[i] * ((a.seq_tiles + NW - 1) / NW);
+        total += (waves(i) + O - 1) / O * a.seq_tiles;
     }
-    a.start[n] = total;
-    for (int i = n + 1; i <= kRkqMaxJobs; ++i) a.start[i] = total;
-    // Measured on the RWKV-7 step at B = 64: X two units ahead takes W_o and
-    // the channel-mix value (192 workgroups) 1.5 us faster each, and makes
-    // the 656- and 768-workgroup launches 1.9 us slower.
-    const bool deep = total <= cu_count();
-#define SNHIP_RKQ_F32(S_) hipLaunchKernelGGL((k_rkq_mm_f32<S_>), dim3(total), dim3(64), 0, st, a)
-#define SNHIP_RKQ_Q4(B_, N_, S_) \
-    hipLaunchKernelGGL((k_rkq_mm_q4<B_, N_, S_, 1>), dim3(total), dim3(64 * (N_ + kRkqNP)), 0, st, a)
-#define SNHIP_RKQ_Q4D(B_) \
-    hipLaunchKernelGGL((k_rkq_mm_q4<B_, 1, 1, 2>), dim3(total), dim3(64 * (1 + kRkqNP)), 0, st, a)
-#define SNHIP_RKQ_Q4L(B_, N_) \
-    hipLaunchKernelGGL((k_rkq_mm_q4<B_, N_, 1, 0>), dim3(total), dim3(64 * (N_ + kRkqNP)), 0, st, a)
-#define SNHIP_RKQ_Q4W(B_, N_) \
-    hipLaunchKernelGGL((k_rkq_mm_q4w<B_, N_>), dim3(total), dim3(64 * (N_ + kRkqNP)), 0, st, a)
-#define SNHIP_RKQ_Q4B(B_)                                 \
-    do {                                                  \
-        if (S == 16) {                                    \
-            if (NC == 1) SNHIP_RKQ_Q4W(B_, 1);            \
-            else if (NC == 2) SNHIP_RKQ_Q4W(B_, 2);       \
-            else SNHIP_RKQ_Q4W(B_, 4);                    \
-        } else if (xl) SNHIP_RKQ_Q4L(B_, 4);             \
-        else if (NC == 1 && S == 1 && deep) SNHIP_RKQ_Q4D(B_); \
-        else if (NC == 1 && S == 1) SNHIP_RKQ_Q4(B_, 1, 1); \
-        else if (NC == 2 && S == 1) SNHIP_RKQ_Q4(B_, 2, 1); \
-        else if (NC == 4) SNHIP_RKQ_Q4(B_, 4, 1);        \
-        else if (NC == 1) SNHIP_RKQ_Q4(B_, 1, 2);        \
-        else SNHIP_RKQ_Q4(B_, 2, 2);                     \
+    for (int i = n; i <= kRkqMaxJobs; ++i) a.start[i] = total;
+#define SNHIP_RKQ(B_, O_, S_, P_) hipLaunchKernelGGL((k_rkq_mm<B_, O_, S_, P_>), dim3(total), dim3(64), 0, st, a)
+    // read-ahead: about 100 registers of operands per wave
+#define SNHIP_RKQ4(B_, P0, P1, P2, P3)              \
+    do {                                            \
+        if (shape == 0) SNHIP_RKQ(B_, 1, 1, P0);    \
+        else if (shape == 1) SNHIP_RKQ(B_, 1, 2, P1); \
+        else if (shape == 2) SNHIP_RKQ(B_, 2, 2, P2); \
+        else SNHIP_RKQ(B_, 2, 4, P3);               \
     } while (0)
-    if (block < 0) {
-#define SNHIP_RKW(S_, N_, P_) \
-    hipLaunchKernelGGL((k_rkq_mm_w4<S_, N_, P_>), dim3(total), dim3(64 * N_), shm, st, a)
-        if (S == 1) {
-            if (NW == 1) {
-                if (wdeep) SNHIP_RKW(1, 1, 48);
-                else SNHIP_RKW(1, 1, 16);
-            } else if (NW == 2) {
-                SNHIP_RKW(1, 2, 40);
-            } else {
-                SNHIP_RKW(1, 4, 24);
-            }
-        } else if (S == 2) {
-            if (NW == 1) SNHIP_RKW(2, 1, 40);
-            else if (NW == 2) SNHIP_RKW(2, 2, 40);
-            else SNHIP_RKW(2, 4, 40);
-        } else {
-            if (NW == 1) SNHIP_RKW(4, 1, 24);
-            else if (NW == 2) SNHIP_RKW(4, 2, 24);
-            else SNHIP_RKW(4, 4, 24);
-        }
-#undef SNHIP_RKW
-    } else if (block == 0) {
-        if (S == 1) SNHIP_RKQ_F32(1);
-        else if (S == 2) SNHIP_RKQ_F32(2);
-        else SNHIP_RKQ_F32(4);
-    } else if (block == 32) {
-        SNHIP_RKQ_Q4B(32);
-    } else {
-        SNHIP_RKQ_Q4B(64);
-    }
-#undef SNHIP_RKQ_F32
-#undef SNHIP_RKQ_Q4
-#undef SNHIP_RKQ_Q4D
-#undef SNHIP_RKQ_Q4L
-#undef SNHIP_RKQ_Q4B
-#undef SNHIP_RKQ_Q4W
+    if (block < 0) SNHIP_RKQ4(-1, 16, 8, 6, 4);
+    else if (block == 0) SNHIP_RKQ4(0, 12, 8, 6, 4);
+    else if (block == 32) SNHIP_RKQ4(32, 8, 4, 3, 2);
+    else SNHIP_RKQ4(64, 4, 3, 2, 1);
+#undef SNHIP_RKQ4
+#undef SNHIP_RKQ
     SNHIP_CHECK(hipGetLastError());
     return SNHIP_OK;
 }
 
-snhip_status launch_rkq_mm(const RkqJob* jobs, int n, int B, int block, hipStream_t st) {
-    return launch_rkq_mm_cfg(jobs, n, B, block, 0, 0, st);
-}
-
-size_t rkq_tiled_floats(int M, int Kd) {
-    return ((size_t)((M + 63) / 64) * (size_t)(Kd / 4) * 64 + kRkwPad) * 4;
-}
-
-snhip_status launch_rkq_block4(const float* w, const uint8_t* q, const float* sc, int block, int M, int Kd,
-                               float* out, hipStream_t st) {
+snhip_status launch_rkq_tile(const float* w, const uint8_t* q, const float* sc, int block, int M, int Kd,
+                             float* out, hipStream_t st) {
     if (M <= 0 || Kd <= 0 || Kd % 4 || !out || (block != 0 && block != 32 && block != 64) ||
         (block ? (!q || !sc || Kd % block) : !w))
         return SNHIP_E_INVAL;
     RkqJob J{};
     J.w = w; J.q = q; J.sc = sc; J.M = M; J.Kd = Kd;
-    const size_t n = rkq_tiled_floats(M, Kd) / 4;
-    hipLaunchKernelGGL(k_rkq_block4, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, J, block,
-                       reinterpret_cast<float4*>(out));
+    hipLaunchKernelGGL(k_rkq_tile, dim3((unsigned)((x16_floats(M, Kd) + 255) / 256)), dim3(256), 0, st, J, block, out);
     SNHIP_CHECK(hipGetLastError());
     return SNHIP_OK;
 }

@@ -123,7 +123,7 @@ struct RMat {
     uint8_t* q = nullptr;
     float* sc = nullptr;
     int block = 0;
-    float* w4 = nullptr;   // the tiled fp32 form the per-kernel steps multiply (or null)
+    float* wt = nullptr;   // the tiled fp32 form the products multiply (or null)
 };
 
 struct RkLayer {
@@ -384,13 +384,11 @@ void setup_rk_persist(SnHipRwkv7* m) {
     m->p_exact = exact;
 }
 
-// The tiled fp32 form of every layer matrix (rkseq.h: block -1), for the
-// per-kernel steps and the chunked prefill: their products then run one
-// independent wave per 64 rows and 4-16 sequences, streaming 1 KiB weight
-// blocks, with no producer waves and no barrier per 64 inputs
-// (SNHIP_RKQ_W4=0: never). 4 bytes per weight plus 64 KiB of padding each, in
-// one allocation. The vocabulary head keeps its own format.
-void setup_rkq_w4(SnHipRwkv7* m) {
+// The tiled fp32 form of every layer matrix (rkseq.h: block -1), which the
+// per-kernel step and the chunked prefill multiply: 4 bytes per weight, in one
+// allocation (SNHIP_RKQ_W4=0: never; the products then take the stored format).
+// The vocabulary head keeps its own format.
+void setup_rkq_tiles(SnHipRwkv7* m) {
     if (env_unsigned("SNHIP_RKQ_W4", 1, 0) == 0) return;
     std::vector<RMat*> mats;
     size_t floats = 0;
@@ -398,27 +396,21 @@ void setup_rkq_w4(SnHipRwkv7* m) {
         RkLayer& A = m->layers[l];
         for (RMat* M : {&A.r, &A.k, &A.v, &A.o, &A.w1, &A.w2, &A.a1, &A.a2, &A.v1, &A.v2, &A.g1, &A.g2,
                         &A.cmk, &A.cmv}) {
-            if (M->M <= 0 || M->Kd <= 0 || M->Kd % 4 || (!M->q && !M->w) ||
-                rkq_tiled_floats(M->M, M->Kd) * sizeof(float) >= ((size_t)1 << 31))   // the kernel's 32-bit offsets
-                continue;
+            if (x16_floats(M->M, M->Kd) * sizeof(float) >= ((size_t)1 << 31)) continue;   // 32-bit offsets
             mats.push_back(M);
-            floats += rkq_tiled_floats(M->M, M->Kd);
+            floats += x16_floats(M->M, M->Kd);
         }
     }
-    float* w4 = floats ? ralloc<float>(m, floats) : nullptr;
-    if (!w4) return;   // the products keep the stored format
-    bool ok = true;
-    float* at = w4;
+    float* at = floats ? ralloc<float>(m, floats) : nullptr;
+    if (!at) return;
+    std::vector<float*> tiles;
     for (RMat* M : mats) {
-        ok = ok && launch_rkq_block4(M->w, M->q, M->sc, M->q ? M->block : 0, M->M, M->Kd, at, nullptr) == SNHIP_OK;
-        at += rkq_tiled_floats(M->M, M->Kd);
+        if (launch_rkq_tile(M->w, M->q, M->sc, M->q ? M->block : 0, M->M, M->Kd, at, nullptr) != SNHIP_OK) return;
+        tiles.push_back(at);
+        at += x16_floats(M->M, M->Kd);
     }
-    if (!ok || hipDeviceSynchronize() != hipSuccess) return;
-    at = w4;
-    for (RMat* M : mats) {
-        M->w4 = at;
-        at += rkq_tiled_floats(M->M, M->Kd);
-    }
+    if (hipDeviceSynchronize() != hipSuccess) return;
+    for (size_t i = 0; i < mats.size(); ++i) mats[i]->wt = tiles[i];
 }
 
 // Do steps of B sequences run as B slices of the persistent kernel?
@@ -585,20 +577,21 @@ SnHipRwkv7* load_rk(const char* path, int max_batch, int wfmt, int block) {
     m->S = ralloc<float>(m, B * L * NH * HS * HS);
     m->shift = ralloc<float>(m, B * L * 2 * D);
     m->x = ralloc<float>(m, B * D);
-    m->X6 = ralloc<float>(m, B * 6 * D);
+    const size_t B16 = (B + 15) / 16 * 16;   // the products' inputs: whole tiles of 16 rows
+    m->X6 = ralloc<float>(m, B16 * 6 * D);
     m->r = ralloc<float>(m, B * D);
     m->k = ralloc<float>(m, B * D);
     m->v = ralloc<float>(m, B * D);
-    m->lo = ralloc<float>(m, B * 4 * kMaxRank);
+    m->lo = ralloc<float>(m, B16 * 4 * kMaxRank);
     m->dw = ralloc<float>(m, B * D);
     m->da = ralloc<float>(m, B * D);
     m->dv = ralloc<float>(m, B * D);
     m->g = ralloc<float>(m, B * D);
-    m->y = ralloc<float>(m, B * D);
+    m->y = ralloc<float>(m, B16 * D);
     m->vfirst = ralloc<float>(m, B * D);
-    m->xk2 = ralloc<float>(m, B * D);
-    m->ck = ralloc<float>(m, B * F);
-    m->nrm = ralloc<float>(m, B * D);
+    m->xk2 = ralloc<float>(m, B16 * D);
+    m->ck = ralloc<float>(m, x16_floats(B, F));
+    m->nrm = ralloc<float>(m, B16 * D);
     m->logits = ralloc<float>(m, B * V);
     m->tok = ralloc<int32_t>(m, B);
     m->best = ralloc<unsigned long long>(m, B * 4096);
@@ -621,7 +614,7 @@ SnHipRwkv7* load_rk(const char* path, int max_batch, int wfmt, int block) {
     if (const char* e = getenv("SNHIP_NO_GRAPH")) m->use_graphs = !(e[0] == '1');
     m->fuse_ups = env_unsigned("SNHIP_RKQ_FUSE_UPS", 1, 0) != 0;
     setup_rk_persist(m);
-    setup_rkq_w4(m);
+    setup_rkq_tiles(m);
     m->ready = 1;
     return m;
 }
@@ -634,16 +627,17 @@ struct MMList {
     int blk[kRkqMaxJobs];
     int n = 0;
 
-    snhip_status add(const RMat& W, const float* X, int ldx, float* Y, int ldy, int epi) {
+    // Y = W X; ldy 0: Y in x16 order
+    snhip_status add(const RMat& W, const float* X, float* Y, int ldy, int epi) {
         if (n == kRkqMaxJobs) return SNHIP_E_INVAL;
         RkqJob j{};
-        j.X = X; j.ldx = ldx;
-        j.w = W.w4 ? W.w4 : W.w; j.q = W.w4 ? nullptr : W.q; j.sc = W.w4 ? nullptr : W.sc;
+        j.X = X;
+        j.w = W.wt ? W.wt : W.w; j.q = W.wt ? nullptr : W.q; j.sc = W.wt ? nullptr : W.sc;
         j.M = W.M; j.Kd = W.Kd;
-        j.Y = Y; j.ldy = ldy;
+        j.Y = Y; j.ldy = ldy; j.y16 = ldy == 0;
         j.epi = epi;
         jobs[n] = j;
-        blk[n] = W.w4 ? -1 : W.q ? W.block : 0;
+        blk[n] = W.wt ? -1 : W.q ? W.block : 0;
         ++n;
         return SNHIP_OK;
     }
@@ -668,13 +662,8 @@ struct MMList {
 // 0's intermediates of that layer there in the reference's order (rwkv7.c:308-319).
 snhip_status enqueue_step(SnHipRwkv7* m, int B, float* logits_out, bool greedy, hipStream_t st,
                           int dbg_layer = -1, float* dbg = nullptr) {
-    const int D = m->D, F = m->F, NH = m->NH, L = m->L, HS = m->HS;
+    const int D = m->D, NH = m->NH, L = m->L, HS = m->HS;
     const size_t s_bstride = (size_t)L * NH * HS * HS, sh_bstride = (size_t)L * 2 * D;
-    const int ldl = 4 * kMaxRank;
-    float* lw = m->lo;
-    float* la = m->lo + kMaxRank;
-    float* lv = m->lo + 2 * kMaxRank;
-    float* lg = m->lo + 3 * kMaxRank;
     snhip_status rc;
     RkqLnArgs ln{};
     ln.D = D; ln.vocab = m->vocab; ln.eps = m->eps; ln.shift_bstride = sh_bstride;
@@ -690,21 +679,6 @@ snhip_status enqueue_step(SnHipRwkv7* m, int B, float* logits_out, bool greedy, 
         ln.mode = RKQ_LN_MIX1;
         ln.x = m->x; ln.g = A.ln1w; ln.c = A.ln1b; ln.lerp = A.lerp; ln.shift = sh; ln.out = m->X6;
         if ((rc = launch_rkq_ln(ln, B, st)) != SNHIP_OK) return rc;
-        const float* xr = m->X6;
-        const float* xw = m->X6 + D;
-        const float* xk = m->X6 + 2 * D;
-        const float* xv = m->X6 + 3 * D;
-        const float* xa = m->X6 + 4 * D;
-        const float* xg = m->X6 + 5 * D;
-        const int ld6 = 6 * D;
-        if ((rc = mm.add(A.r, xr, ld6, m->r, D, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.k, xk, ld6, m->k, D, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.v, xv, ld6, m->v, D, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.w1, xw, ld6, lw, ldl, RKQ_TANH)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.a1, xa, ld6, la, ldl, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.g1, xg, ld6, lg, ldl, RKQ_SIGMOID)) != SNHIP_OK) return rc;
-        if (l > 0 && (rc = mm.add(A.v1, xv, ld6, lv, ldl, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
         // The LoRA up-projections run inside the heads kernel when they are
         // INT4 of one group size with ranks up to 128 (SNHIP_RKQ_FUSE_UPS=0:
         // never): it computes each channel's four short chains from the
@@ -716,11 +690,28 @@ snhip_status enqueue_step(SnHipRwkv7* m, int B, float* logits_out, bool greedy, 
                           A.w2.Kd % A.w2.block == 0 && A.a2.Kd % A.w2.block == 0 &&
                           A.g2.Kd % A.w2.block == 0 && (l == 0 || A.v2.Kd % A.w2.block == 0) &&
                           A.w2.M == D && A.a2.M == D && A.g2.M == D && (l == 0 || A.v2.M == D);
+        // the middles in row-major order for the heads kernel, else as the
+        // products read them
+        const size_t lo1 = fuse ? (size_t)kMaxRank : x16_floats(B, kMaxRank);
+        const int ldl = fuse ? 4 * kMaxRank : 0;
+        float* lw = m->lo;
+        float* la = m->lo + lo1;
+        float* lv = m->lo + 2 * lo1;
+        float* lg = m->lo + 3 * lo1;
+        const size_t x1 = x16_floats(B, D);
+        if ((rc = mm.add(A.r, m->X6, m->r, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.k, m->X6 + 2 * x1, m->k, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.v, m->X6 + 3 * x1, m->v, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.w1, m->X6 + x1, lw, ldl, RKQ_TANH)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.a1, m->X6 + 4 * x1, la, ldl, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.g1, m->X6 + 5 * x1, lg, ldl, RKQ_SIGMOID)) != SNHIP_OK) return rc;
+        if (l > 0 && (rc = mm.add(A.v1, m->X6 + 3 * x1, lv, ldl, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
         if (!fuse) {
-            if ((rc = mm.add(A.w2, lw, ldl, m->dw, D, RKQ_STORE)) != SNHIP_OK) return rc;
-            if ((rc = mm.add(A.a2, la, ldl, m->da, D, RKQ_STORE)) != SNHIP_OK) return rc;
-            if ((rc = mm.add(A.g2, lg, ldl, m->g, D, RKQ_STORE)) != SNHIP_OK) return rc;
-            if (l > 0 && (rc = mm.add(A.v2, lv, ldl, m->dv, D, RKQ_STORE)) != SNHIP_OK) return rc;
+            if ((rc = mm.add(A.w2, lw, m->dw, D, RKQ_STORE)) != SNHIP_OK) return rc;
+            if ((rc = mm.add(A.a2, la, m->da, D, RKQ_STORE)) != SNHIP_OK) return rc;
+            if ((rc = mm.add(A.g2, lg, m->g, D, RKQ_STORE)) != SNHIP_OK) return rc;
+            if (l > 0 && (rc = mm.add(A.v2, lv, m->dv, D, RKQ_STORE)) != SNHIP_OK) return rc;
             if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
         }
         RkqHeadArgs H{};
@@ -749,22 +740,22 @@ snhip_status enqueue_step(SnHipRwkv7* m, int B, float* logits_out, bool greedy, 
         H.first = l == 0;
         H.dbg = dl;
         if ((rc = launch_rkq_heads(H, B, st)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.o, m->y, D, m->x, D, RKQ_ADD)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.o, m->y, m->x, D, RKQ_ADD)) != SNHIP_OK) return rc;
         if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
         ln.mode = RKQ_LN_MIX2;
         ln.x = m->x; ln.g = A.ln2w; ln.c = A.ln2b; ln.lerp = A.cmk_lerp; ln.shift = sh + D; ln.out = m->xk2;
         if ((rc = launch_rkq_ln(ln, B, st)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.cmk, m->xk2, D, m->ck, F, RKQ_RELU2)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.cmk, m->xk2, m->ck, 0, RKQ_RELU2)) != SNHIP_OK) return rc;
         if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.cmv, m->ck, F, m->x, D, RKQ_ADD)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.cmv, m->ck, m->x, D, RKQ_ADD)) != SNHIP_OK) return rc;
         if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
         if (dl) {
-            // xn (the LayerNorm output, kept as shift_0), r, g, y and the layer's x
+            // xn (the LayerNorm output, kept as shift_0), r, g and the layer's x
+            // (the heads kernel has written the others)
             const size_t n = (size_t)D * sizeof(float);
             SNHIP_CHECK(hipMemcpyAsync(dl, sh, n, hipMemcpyDeviceToDevice, st));
             SNHIP_CHECK(hipMemcpyAsync(dl + D, m->r, n, hipMemcpyDeviceToDevice, st));
             SNHIP_CHECK(hipMemcpyAsync(dl + 5 * D, m->g, n, hipMemcpyDeviceToDevice, st));
-            SNHIP_CHECK(hipMemcpyAsync(dl + 7 * D, m->y, n, hipMemcpyDeviceToDevice, st));
             SNHIP_CHECK(hipMemcpyAsync(dl + 8 * D, m->x, n, hipMemcpyDeviceToDevice, st));
             return SNHIP_OK;
         }
@@ -772,7 +763,7 @@ snhip_status enqueue_step(SnHipRwkv7* m, int B, float* logits_out, bool greedy, 
     ln.mode = RKQ_LN_PLAIN;
     ln.x = m->x; ln.g = m->on_w; ln.c = m->on_b; ln.out = m->nrm;
     if ((rc = launch_rkq_ln(ln, B, st)) != SNHIP_OK) return rc;
-    if ((rc = mm.add(m->head, m->nrm, D, logits_out, m->vocab, RKQ_STORE)) != SNHIP_OK) return rc;
+    if ((rc = mm.add(m->head, m->nrm, logits_out, m->vocab, RKQ_STORE)) != SNHIP_OK) return rc;
     if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
     if (greedy) {
         const int nblk = 64;
@@ -846,15 +837,15 @@ snhip_status step_host(SnHipRwkv7* m, const int32_t* tokens, int B, float* logit
 
 // Chunked prefill of sequence 0 (rkprefill.hip). Its products use whichever
 // form the matrices have; prompts shorter than kPfMin step token by token.
-// Measured on 12 x 768 INT4 g32, host call: a chunk of 4 to 16 tokens 1.4 ms, a
-// step 0.68 ms (3 tokens 2.0 ms), so the line lies at three tokens; 512 tokens
-// 4.8 ms in one chunk against 345 ms stepped.
+// Measured on 12 x 768 INT4 g32, host call: a chunk of 2 to 16 tokens 1.1 ms, a
+// step 0.71 ms, so the line lies at two tokens; 512 tokens 3.4 ms in one chunk
+// against 345 ms stepped.
 constexpr int kPfRows = 512;   // tokens per chunk
-constexpr int kPfMin = 3;
+constexpr int kPfMin = 2;
 
 // Floats of the workspace's parts per token, in PfWs's order.
 struct PfWs {
-    float *x, *X6, *r, *k, *v, *lo, *dw, *da, *dv, *g, *y, *vfirst, *xk2, *ck, *pack, *dot, *shift;
+    float *x, *X6, *r, *k, *v, *lo, *dw, *da, *dv, *g, *ys, *y, *vfirst, *xk2, *ck, *pack, *dot, *shift;
     int32_t* tok;
 };
 size_t pf_layout(const SnHipRwkv7* m, float* base, PfWs* ws) {
@@ -875,10 +866,11 @@ size_t pf_layout(const SnHipRwkv7* m, float* base, PfWs* ws) {
     take(w.da, T * D);
     take(w.dv, T * D);
     take(w.g, T * D);
+    take(w.ys, T * D);
     take(w.y, T * D);
     take(w.vfirst, T * D);
     take(w.xk2, T * D);
-    take(w.ck, T * m->F);
+    take(w.ck, x16_floats(T, m->F));
     take(w.pack, T * m->NH * kRkpPack);
     take(w.dot, T * m->NH);
     take(w.shift, (size_t)m->L * 2 * D);
@@ -892,12 +884,12 @@ size_t pf_layout(const SnHipRwkv7* m, float* base, PfWs* ws) {
 // T <= kPfRows tokens (in ws.tok) of sequence 0 from its current state; the
 // last token's logits to logits_out unless null.
 snhip_status enqueue_chunk(SnHipRwkv7* m, const PfWs& ws, int T, float* logits_out, hipStream_t st) {
-    const int D = m->D, F = m->F, NH = m->NH;
-    const int ldl = 4 * kMaxRank, ld6 = 6 * D;
+    const int D = m->D, NH = m->NH;
+    const size_t x1 = x16_floats(T, D), lo1 = x16_floats(T, kMaxRank);
     float* lw = ws.lo;
-    float* la = ws.lo + kMaxRank;
-    float* lv = ws.lo + 2 * kMaxRank;
-    float* lg = ws.lo + 3 * kMaxRank;
+    float* la = ws.lo + lo1;
+    float* lv = ws.lo + 2 * lo1;
+    float* lg = ws.lo + 3 * lo1;
     snhip_status rc;
     RkqLnArgs ln{};
     ln.D = D; ln.vocab = m->vocab; ln.eps = m->eps;
@@ -913,36 +905,36 @@ snhip_status enqueue_chunk(SnHipRwkv7* m, const PfWs& ws, int T, float* logits_o
         N.mixes = 6; N.g = A.ln1w; N.c = A.ln1b; N.lerp = A.lerp; N.out = ws.X6;
         N.shift = m->shift + sh; N.shift_next = ws.shift + sh;
         if ((rc = launch_rkp_ln(N, st)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.r, ws.X6, ld6, ws.r, D, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.k, ws.X6 + 2 * D, ld6, ws.k, D, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.v, ws.X6 + 3 * D, ld6, ws.v, D, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.w1, ws.X6 + D, ld6, lw, ldl, RKQ_TANH)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.a1, ws.X6 + 4 * D, ld6, la, ldl, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.g1, ws.X6 + 5 * D, ld6, lg, ldl, RKQ_SIGMOID)) != SNHIP_OK) return rc;
-        if (l > 0 && (rc = mm.add(A.v1, ws.X6 + 3 * D, ld6, lv, ldl, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.r, ws.X6, ws.r, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.k, ws.X6 + 2 * x1, ws.k, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.v, ws.X6 + 3 * x1, ws.v, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.w1, ws.X6 + x1, lw, 0, RKQ_TANH)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.a1, ws.X6 + 4 * x1, la, 0, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.g1, ws.X6 + 5 * x1, lg, 0, RKQ_SIGMOID)) != SNHIP_OK) return rc;
+        if (l > 0 && (rc = mm.add(A.v1, ws.X6 + 3 * x1, lv, 0, RKQ_STORE)) != SNHIP_OK) return rc;
         if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.w2, lw, ldl, ws.dw, D, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.a2, la, ldl, ws.da, D, RKQ_STORE)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.g2, lg, ldl, ws.g, D, RKQ_STORE)) != SNHIP_OK) return rc;
-        if (l > 0 && (rc = mm.add(A.v2, lv, ldl, ws.dv, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.w2, lw, ws.dw, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.a2, la, ws.da, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.g2, lg, ws.g, D, RKQ_STORE)) != SNHIP_OK) return rc;
+        if (l > 0 && (rc = mm.add(A.v2, lv, ws.dv, D, RKQ_STORE)) != SNHIP_OK) return rc;
         if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
         RkpHeadArgs H{};
         H.T = T; H.D = D; H.NH = NH; H.first = l == 0;
         H.r = ws.r; H.k = ws.k; H.v = ws.v; H.dw = ws.dw; H.da = ws.da; H.dv = ws.dv; H.g = ws.g;
-        H.vfirst = ws.vfirst; H.y = ws.y;
+        H.vfirst = ws.vfirst; H.ys = ws.ys; H.y = ws.y;
         H.w0 = A.w0; H.a0 = A.a0; H.v0 = A.v0; H.kk_w = A.kk; H.ka_w = A.ka; H.rk_w = A.rk;
         H.lnx_w = A.lnxw; H.lnx_b = A.lnxb;
         H.S = m->S + (size_t)l * NH * m->HS * m->HS;
         H.pack = ws.pack; H.dot = ws.dot;
         if ((rc = launch_rkp_heads(H, st)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.o, ws.y, D, ws.x, D, RKQ_ADD)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.o, ws.y, ws.x, D, RKQ_ADD)) != SNHIP_OK) return rc;
         if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
         N.mixes = 1; N.g = A.ln2w; N.c = A.ln2b; N.lerp = A.cmk_lerp; N.out = ws.xk2;
         N.shift = m->shift + sh + D; N.shift_next = ws.shift + sh + D;
         if ((rc = launch_rkp_ln(N, st)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.cmk, ws.xk2, D, ws.ck, F, RKQ_RELU2)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.cmk, ws.xk2, ws.ck, 0, RKQ_RELU2)) != SNHIP_OK) return rc;
         if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
-        if ((rc = mm.add(A.cmv, ws.ck, F, ws.x, D, RKQ_ADD)) != SNHIP_OK) return rc;
+        if ((rc = mm.add(A.cmv, ws.ck, ws.x, D, RKQ_ADD)) != SNHIP_OK) return rc;
         if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
     }
     SNHIP_CHECK(hipMemcpyAsync(m->shift, ws.shift, (size_t)m->L * 2 * D * sizeof(float), hipMemcpyDeviceToDevice, st));
@@ -951,7 +943,7 @@ snhip_status enqueue_chunk(SnHipRwkv7* m, const PfWs& ws, int T, float* logits_o
     ln.x = ws.x + (size_t)(T - 1) * D; ln.g = m->on_w; ln.c = m->on_b; ln.out = m->nrm;
     if ((rc = launch_rkq_ln(ln, 1, st)) != SNHIP_OK) return rc;
     MMList head{1};
-    if ((rc = head.add(m->head, m->nrm, D, logits_out, m->vocab, RKQ_STORE)) != SNHIP_OK) return rc;
+    if ((rc = head.add(m->head, m->nrm, logits_out, m->vocab, RKQ_STORE)) != SNHIP_OK) return rc;
     return head.flush(st);
 }
 

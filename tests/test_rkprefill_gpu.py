@@ -21,7 +21,7 @@ CFGS = {128: RwkvConfig(layers=2, dim=128, head_size=64, ff=256, vocab=512, rank
 
 
 @pytest.mark.parametrize("dim,int4,T,env", [
-    (128, False, 3, {}), (128, False, 5, {}), (128, True, 65, {}), (128, True, 513, {}),
+    (128, False, 2, {}), (128, False, 5, {}), (128, True, 65, {}), (128, True, 513, {}),
     (128, True, 30, {"SNHIP_RKQ_W4": "0"}), (128, False, 30, {"SNHIP_RKQ_W4": "0"}),
     (128, False, 31, {"SNHIP_RK_EXACT": "0"}),
     (768, False, 7, {}), (768, True, 6, {}), (768, True, 130, {}), (768, True, 1025, {}),
