@@ -26,6 +26,7 @@ namespace {
 constexpr float kR2 = 0.6065306597126334f;   // 1/sqrt(e), rwkv7.c:38
 constexpr float kEpsGroup = 6.4e-4f;          // rwkv7.c:39
 constexpr int kHS = 64;
+typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
 
 // The wave's own LDS operations complete in order; this keeps the compiler
 // from moving them across.
@@ -218,50 +219,78 @@ __global__ __launch_bounds__(64) void k_rkp_scan(RkpHeadArgs A) {
     float s[8];
 #pragma unroll
     for (int m = 0; m < 8; ++m) s[m] = Sr[8 * m];
-    const float4* p4 = reinterpret_cast<const float4*>(A.pack + (size_t)h * kRkpPack) + 2 * lam;
-    const size_t pstride = (size_t)A.NH * kRkpPack / 4;
-    const float* vp = A.v + h * kHS + row;
-    float* yp = A.ys + h * kHS + row;
+    // Through buffer resources: a token costs one scalar offset per array.
+    const int D4 = A.D * 4, pbytes = A.NH * kRkpPack * 4;
+    auto rsrc = [&](const float* base, int bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, bytes, 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rp = rsrc(A.pack, A.T * pbytes), rv = rsrc(A.v, A.T * D4), ry = rsrc(A.ys, A.T * D4);
+    const int po = h * kRkpPack * 4 + 32 * lam, vo = (h * kHS + row) * 4;
+    auto ld4 = [&](int so, int imm) -> float4 {
+        const u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(rp, po + imm, so, 0);
+        return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
+    };
     auto load = [&](TokIn& I, int tok) {
-        const int t = min(tok, A.T - 1);   // past the end: the last token again, never used
-        const float4* p = p4 + (size_t)t * pstride;
-        I.n[0] = p[16]; I.n[1] = p[17];
-        I.na[0] = p[32]; I.na[1] = p[33];
-        I.w[0] = p[0]; I.w[1] = p[1];
-        I.k[0] = p[48]; I.k[1] = p[49];
-        I.r[0] = p[64]; I.r[1] = p[65];
-        I.v = vp[(size_t)t * A.D];
+        const int t = min(tok, A.T - 1), so = t * pbytes;   // past the end: the last token again, never used
+        I.n[0] = ld4(so, 256); I.n[1] = ld4(so, 272);
+        I.na[0] = ld4(so, 512); I.na[1] = ld4(so, 528);
+        I.w[0] = ld4(so, 0); I.w[1] = ld4(so, 16);
+        I.k[0] = ld4(so, 768); I.k[1] = ld4(so, 784);
+        I.r[0] = ld4(so, 1024); I.r[1] = ld4(so, 1040);
+        I.v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rv, vo, t * D4, 0));
+    };
+    // the row's eight lanes hold the same sum: all of them store it, no branch
+    auto put = [&](int t, float y) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), ry, vo, t * D4, 0);
     };
     auto el = [](const float4 (&x)[2], int m) {
         const float4 v = x[m >> 2];
         return (m & 3) == 0 ? v.x : (m & 3) == 1 ? v.y : (m & 3) == 2 ? v.z : v.w;
     };
-    TokIn I[kAhead];
+    // Step t reads the state before token t twice: for its own read and for
+    // token t - 1's read-out, so the two chains of eight run interleaved (each
+    // alone left the issue slot waiting: 125 us per 512-token layer). Step 0
+    // writes to row 0 what step 1 then writes over.
+    auto step = [&](const TokIn& X, const float4 (&r)[2], int t) {
+        float pv = 0.0f, ya = 0.0f;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            pv = fmaf(s[m], el(X.n, m), pv);
+            ya = fmaf(s[m], el(r, m), ya);
+        }
+        pv = fold8(pv);
+        ya = fold8(ya);
+        put(max(t - 1, 0), ya);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const float vk = X.v * el(X.k, m);
+            s[m] = fmaf(s[m], el(X.w, m), vk - pv * el(X.na, m));
+        }
+    };
+    TokIn I[kAhead];   // slot t % kAhead; a token's slot is refilled in the step after it, which reads its r
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) load(I[i], i);
-    for (int t0 = 0; t0 < A.T; t0 += kAhead) {
+    I[kAhead - 1].r[0] = I[kAhead - 1].r[1] = make_float4(0.f, 0.f, 0.f, 0.f);   // before token 0
+    int t0 = 0;
+    for (; t0 + kAhead <= A.T; t0 += kAhead) {
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) {
-            const int t = t0 + i;
-            if (t >= A.T) break;
-            const TokIn& X = I[i];
-            float pv = 0.0f;
-#pragma unroll
-            for (int m = 0; m < 8; ++m) pv = fmaf(s[m], el(X.n, m), pv);
-            pv = fold8(pv);
-            float ya = 0.0f;
-#pragma unroll
-            for (int m = 0; m < 8; ++m) {
-                const float vk = X.v * el(X.k, m);
-                s[m] = fmaf(s[m], el(X.w, m), vk - pv * el(X.na, m));
-                ya = fmaf(s[m], el(X.r, m), ya);
-            }
-            ya = fold8(ya);
-            if (lam == 0) yp[(size_t)t * A.D] = ya;
-            load(I[i], t + kAhead);
+            TokIn& P = I[(i + kAhead - 1) % kAhead];
+            step(I[i], P.r, t0 + i);
+            load(P, t0 + i + kAhead - 1);
             __builtin_amdgcn_sched_barrier(0);   // the loads stay with their token
         }
     }
+#pragma unroll
+    for (int i = 0; i < kAhead - 1; ++i)
+        if (t0 + i < A.T) step(I[i], I[(i + kAhead - 1) % kAhead].r, t0 + i);
+    // the last token's read-out; its r is read again (its slot is not a fixed one)
+    const int sl = (A.T - 1) * pbytes;
+    const float4 rl[2] = {ld4(sl, 1024), ld4(sl, 1040)};
+    float ya = 0.0f;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) ya = fmaf(s[m], el(rl, m), ya);
+    put(A.T - 1, fold8(ya));
 #pragma unroll
     for (int m = 0; m < 8; ++m) Sr[8 * m] = s[m];
 }
