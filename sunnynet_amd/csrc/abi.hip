@@ -3,9 +3,11 @@
 // and version rules; the recurrence and INT4 primitives run on the GPU.
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <set>
 #include <thread>
 #include <utility>
+#include <vector>
 
 #include "common.h"
 
@@ -20,6 +22,85 @@ int host_threads() {
     if (g_threads > 0) return g_threads;
     const unsigned n = std::thread::hardware_concurrency();
     return n > 0 ? (int)n : 1;
+}
+
+namespace {
+// The streams of the calls in flight that run persistent kernels, per device.
+struct Flight {
+    int dev;
+    hipStream_t st;
+};
+std::mutex g_flight_mu;
+std::vector<Flight> g_flight;
+}  // namespace
+
+PersistCall::PersistCall(hipStream_t st) : st_(st) {
+    (void)hipGetDevice(&dev_);
+    std::lock_guard<std::mutex> lock(g_flight_mu);
+    g_flight.push_back(Flight{dev_, st_});
+}
+hipError_t PersistCall::finish() {
+    done_ = true;
+    return hipStreamSynchronize(st_);
+}
+PersistCall::~PersistCall() {
+    if (!done_) (void)hipStreamSynchronize(st_);
+    std::lock_guard<std::mutex> lock(g_flight_mu);
+    for (size_t i = 0; i < g_flight.size(); ++i)
+        if (g_flight[i].dev == dev_ && g_flight[i].st == st_) {
+            g_flight.erase(g_flight.begin() + (long)i);
+            break;
+        }
+}
+
+hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st) {
+    if (env_unsigned("SNHIP_COOP", 0, 0) != 0) return hipLaunchCooperativeKernel(k, grid, block, args, 0, st);
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    // Held over the launch: of two calls, the later one sees the earlier one's
+    // kernel on its stream (a call stays listed until its kernels are done).
+    std::lock_guard<std::mutex> lock(g_flight_mu);
+    for (const Flight& f : g_flight) {
+        if (e != hipSuccess) return e;
+        if (f.dev != dev || f.st == st) continue;
+        hipEvent_t ev = nullptr;
+        if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
+        e = hipEventRecord(ev, f.st);
+        if (e == hipSuccess) e = hipStreamWaitEvent(st, ev, 0);
+        (void)hipEventDestroy(ev);
+    }
+    return e != hipSuccess ? e : hipLaunchKernel(k, grid, block, args, 0, st);
+}
+
+hipError_t StreamOrder::mark(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(st, &cs);
+    set_ = false;
+    if (e != hipSuccess || cs != hipStreamCaptureStatusNone) return e;
+    if (!ev_) e = hipEventCreateWithFlags(&ev_, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(ev_, st);
+    set_ = e == hipSuccess;
+    return e;
+}
+hipError_t StreamOrder::follow(hipStream_t st) {
+    const bool wait = set_;
+    set_ = false;
+    return wait ? hipStreamWaitEvent(st, ev_, 0) : hipSuccess;
+}
+
+bool stream_has_all_cus(hipStream_t st) {
+    if (!st) return true;
+    int dev = 0, ncu = 0;
+    uint32_t mask[32] = {};
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipExtStreamGetCUMask(st, 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    int n = 0;
+    for (uint32_t w : mask) n += __builtin_popcount(w);
+    return n == 0 || n >= ncu;   // 0: no mask
 }
 }  // namespace snhip
 

@@ -267,14 +267,15 @@ __device__ __forceinline__ void publish_tiles(unsigned* f, int wg, int G, int T,
 // The reader's half: until each of the n flags f[0 .. n) holds `want`; true
 // if the launch is abandoned (a wait timed out, here or in another
 // workgroup).
-__device__ __forceinline__ bool await(const unsigned* f, int n, unsigned want, unsigned* err, unsigned limit,
-                                      int* sdead) {
+__device__ __forceinline__ bool await(const unsigned* f, int n, unsigned want, unsigned* err, unsigned* herr,
+                                      unsigned limit, int* sdead) {
     int dead = 0;
     for (int i = threadIdx.x; i < n && !dead; i += NT) {
         unsigned k = 0;
         while (__hip_atomic_load(const_cast<unsigned*>(f + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != want) {
             if (++k > limit) {
                 __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(herr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 dead = 1;
                 break;
             }
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(NT) void k_decode_batch(BatchArgs a) {
         if (ph == 3) return f;
         return f + (size_t)mb * N3;
     };
-    auto wait = [&](const unsigned* f, int n) { return await(f, n, want, a.err, a.spin_limit, &sdead); };
+    auto wait = [&](const unsigned* f, int n) { return await(f, n, want, a.err, a.herr, a.spin_limit, &sdead); };
 
     WF<BLK> wa[NCM];
     if (wg < T1) load_w<BLK, NCD, FULL>(wa, mat(ltab[0].VW, R + D, D), tile_of(wg, mb, N1).n0, wv, lane);

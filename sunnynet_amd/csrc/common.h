@@ -50,15 +50,50 @@ inline unsigned env_unsigned(const char* name, unsigned dflt, unsigned lo) {
     return v < (long)lo ? lo : (unsigned)v;
 }
 
+// A call that runs grid-synchronizing persistent kernels on `st`: from before
+// its first launch until those kernels have finished (the destructor waits for
+// them unless finish() has). See launch_persistent.
+class PersistCall {
+public:
+    explicit PersistCall(hipStream_t st);
+    ~PersistCall();
+    hipError_t finish();   // waits for the stream
+    PersistCall(const PersistCall&) = delete;
+    PersistCall& operator=(const PersistCall&) = delete;
+
+private:
+    hipStream_t st_;
+    int dev_ = 0;
+    bool done_ = false;
+};
+
 // Launches a grid-synchronizing persistent kernel whose grid is sized to
-// co-reside: cooperatively (the runtime checks residency), or, with
-// SNHIP_COOP=0, as an ordinary launch of the same grid (for tools that do not
-// handle cooperative launches; every grid-wide wait in these kernels is
-// bounded, so a grid that did not co-reside ends in a reported time-out).
-inline hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st) {
-    if (env_unsigned("SNHIP_COOP", 1, 0) == 0) return hipLaunchKernel(k, grid, block, args, 0, st);
-    return hipLaunchCooperativeKernel(k, grid, block, args, 0, st);
-}
+// co-reside (checked against the kernel's occupancy when the handle is set up),
+// inside a PersistCall on `st`. It is an ordinary launch: a cooperative one goes
+// through a queue of its own with host-side waits on both ends, about 60 us per
+// call (SunnyNet-100M fp32 B = 1 step 315 -> 258 us). What the cooperative queue
+// also gave, that no two such kernels share the device, is kept by ordering each
+// launch after the work queued by every other call in flight on the device.
+// SNHIP_COOP=1 launches cooperatively.
+hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st);
+
+// Steps and prefills of one handle are in order also across a change of the
+// caller's stream: each that returns before its work is done marks its end on
+// the stream it ran on, and a new stream waits for the mark.
+class StreamOrder {
+public:
+    ~StreamOrder() { if (ev_) (void)hipEventDestroy(ev_); }
+    hipError_t mark(hipStream_t st);      // (not while st is being captured)
+    hipError_t follow(hipStream_t st);
+
+private:
+    hipEvent_t ev_ = nullptr;
+    bool set_ = false;
+};
+
+// Whether `st` may use every CU (a stream made with a CU mask may not, and a
+// grid sized for the whole device would not co-reside on it).
+bool stream_has_all_cus(hipStream_t st);
 
 // Waits for this wave's outstanding LDS operations only (gfx9 s_waitcnt
 // encoding: vmcnt = 63, expcnt = 7, lgkmcnt = 0); global loads stay in flight.

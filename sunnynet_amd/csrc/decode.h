@@ -44,9 +44,13 @@ struct PersistArgs {
     float* s;               // (L, D) state: read at the first step, written back after the last
     float* hist;            // (L, kh, D) conv history, newest first: same
     float* ring;            // (grid, L, kh, D) each workgroup's recent LN_in outputs
-    unsigned long long* ex; // (2, kPersistExWords) exchange words, zeroed before the launch
-    unsigned long long* sx; // (L, 2, D) new-state words, zeroed before the launch
-    unsigned* err;          // set on a poll time-out
+    // Words of earlier launches keep their (smaller) epochs: nothing is cleared
+    // between launches.
+    unsigned long long* ex; // (2, kPersistExWords) exchange words
+    unsigned long long* sx; // (L, 2, D) new-state words
+    unsigned ep0, st0;      // last epochs used in ex (one per exchange) and sx (one per step)
+    unsigned* err;          // set on a poll time-out, zero before the launch
+    unsigned* herr;         // the same for the host (pinned)
     const int32_t* tok_in;  // first input token (device)
     int32_t* out_tok;       // greedy: token chosen after each step (n_steps)
     float* logits;          // if not NULL: logits of the last step (vocab)
@@ -108,7 +112,8 @@ struct BatchArgs {
     float* nrm;             // (B, D) LN_out of the last residual (the head's input)
     unsigned* flags;        // batch_flag_words(L, B, ...) dataflow flags, zeroed once
     unsigned epoch;         // this launch's epoch (> 0, one more per launch)
-    unsigned* err;          // set on a wait's time-out
+    unsigned* err;          // set on a wait's time-out, zero before the launch
+    unsigned* herr;         // the same for the host (pinned)
     unsigned spin_limit;    // polls before a wait gives up
     unsigned stall;         // added to every awaited epoch: > 0 only to test the time-out path
 };

@@ -18,6 +18,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <optional>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -573,8 +574,9 @@ struct SnHipModel {
     int hist_cap = 0;                     // capacity of tok_hist in tokens
     std::vector<void*> allocs;
     hipStream_t stream = nullptr;         // caller's stream
-    hipStream_t work = nullptr;           // internal stream that runs the step graphs
-    hipEvent_t ev_in = nullptr, ev_out = nullptr;
+    snhip::StreamOrder order;
+    bool all_cus = true;                  // it may use every CU: the persistent kernels need them
+    hipStream_t cap = nullptr;            // graphs are captured here
     // Captured step graphs keyed by (B, logits pointer, greedy).
     std::map<std::tuple<int, const void*, int>, hipGraphExec_t> graphs;
     bool use_graphs = true;
@@ -605,7 +607,9 @@ struct SnHipModel {
     unsigned long long* psx = nullptr;    // new-state words (L x 2 x D)
     float* pring = nullptr;               // per-workgroup LN_in history rings
     unsigned* perr = nullptr;             // time-out flag
-    unsigned* h_err = nullptr;            // pinned copies of the time-out flags: [0] perr, [1] berr
+    unsigned* h_err = nullptr;            // pinned time-out flags, written by the kernel: [0] beside perr, [1] berr
+    unsigned persist_ep = 0, persist_st = 0;   // last epochs used in pex and psx
+    int persist_nseq = 1;                 // sequences whose words pex and psx hold
     unsigned persist_spin = 1u << 22;     // poll limit (SNHIP_PERSIST_SPIN)
     unsigned persist_stall = 0;           // SNHIP_PERSIST_STALL: forces time-outs (tests), read per call
     // A persistent step timed out after some workgroups had written their part
@@ -641,9 +645,7 @@ void free_model(SnHipModel* m) {
     if (!m) return;
     if (m->h_err) (void)hipHostFree(m->h_err);
     for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
-    if (m->ev_in) (void)hipEventDestroy(m->ev_in);
-    if (m->ev_out) (void)hipEventDestroy(m->ev_out);
-    if (m->work) (void)hipStreamDestroy(m->work);
+    if (m->cap) (void)hipStreamDestroy(m->cap);
     for (void* p : m->allocs) (void)hipFree(p);
     delete m;
 }
@@ -862,7 +864,7 @@ bool layer_table(SnHipModel* m) {
     return true;
 }
 
-// Pinned host copies of the persistent kernels' time-out flags.
+// Pinned host time-out flags of the persistent kernels.
 bool host_err(SnHipModel* m) {
     if (m->h_err) return true;
     if (hipHostMalloc((void**)&m->h_err, 2 * sizeof(unsigned), 0) != hipSuccess) {
@@ -931,14 +933,17 @@ void setup_persist(SnHipModel* m) {
     for (int g = cap; g >= 1 && !nwg; --g)
         if (persist_grid_ok(g, m->D, m->I, m->R, m->vocab)) nwg = g;
     if (nwg < 1) return;
-    const int nseq = setup_persist_mi(m, ncu, cap);
+    const int nseq = m->persist_nseq = setup_persist_mi(m, ncu, cap);
     int ring_wg = nwg;
     for (int b = 2; b <= m->mi_max; ++b) ring_wg = std::max(ring_wg, b * m->mi_grid[b]);
     m->pex = dalloc<unsigned long long>(m, 2 * (size_t)kPersistExWords * nseq);
     m->psx = dalloc<unsigned long long>(m, (size_t)m->L * 2 * m->D * nseq);
     m->pring = dalloc<float>(m, (size_t)ring_wg * m->L * m->kh * m->D);
     m->perr = dalloc<unsigned>(m, 1);
-    if (!m->pex || !m->psx || !m->pring || !m->perr || !layer_table(m) || !host_err(m)) {
+    if (!m->pex || !m->psx || !m->pring || !m->perr || !layer_table(m) || !host_err(m) ||
+        hipMemset(m->pex, 0, 2 * (size_t)kPersistExWords * nseq * sizeof(unsigned long long)) != hipSuccess ||
+        hipMemset(m->psx, 0, (size_t)m->L * 2 * m->D * nseq * sizeof(unsigned long long)) != hipSuccess ||
+        hipMemset(m->perr, 0, sizeof(unsigned)) != hipSuccess) {
         m->mi_max = 0;
         return;
     }
@@ -1144,9 +1149,7 @@ SnHipModel* load_model(const char* path, int vocab, int dim, int inner, int rank
         hipMemset(m->hist, 0, B * layers * (m->kh ? m->kh : 1) * D * sizeof(float)) != hipSuccess ||
         hipMemset(m->counter, 0, sizeof(int32_t)) != hipSuccess ||
         hipMemset(m->done, 0, sizeof(int32_t)) != hipSuccess ||
-        hipStreamCreateWithFlags(&m->work, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&m->ev_in, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&m->ev_out, hipEventDisableTiming) != hipSuccess) {
+        hipStreamCreateWithFlags(&m->cap, hipStreamNonBlocking) != hipSuccess) {
         set_last_error("device setup failed");
         free_model(m);
         return nullptr;
@@ -1225,7 +1228,7 @@ __global__ void k_copy_rows(const float* __restrict__ src, long lds, float* __re
 // Final norm, LM head and (greedy) token selection for B rows of x.
 // Does a step of B sequences run as the batched persistent kernel?
 bool uses_batch(const SnHipModel* m, int B) {
-    return m->batch_wg > 0 && B >= m->gemm_min_batch && B <= std::min(m->max_batch, m->batch_max);
+    return m->batch_wg > 0 && m->all_cus && B >= m->gemm_min_batch && B <= std::min(m->max_batch, m->batch_max);
 }
 
 snhip_status enqueue_head(SnHipModel* m, int B, const float* x, float* logits_out, bool greedy,
@@ -1293,10 +1296,10 @@ snhip_status enqueue_layer_gemv(SnHipModel* m, int B, int l, hipStream_t st) {
     return SNHIP_OK;
 }
 
-// Enqueue one decode step for sequences [0, B) on `st`; tokens in m->tok.
+// Enqueue one decode step for sequences [0, B) on `st`; tokens in tok (device).
 // greedy: the head also reduces the first maximal logit per sequence and a
 // final kernel writes it to m->tok (the next step's input) and m->tok_hist.
-snhip_status enqueue_step(SnHipModel* m, int B, float* logits_out, bool greedy, hipStream_t st) {
+snhip_status enqueue_step(SnHipModel* m, const int32_t* tok, int B, float* logits_out, bool greedy, hipStream_t st) {
     const int D = m->D, I = m->I, R = m->R, L = m->L;
     const size_t sbs = (size_t)L * D;                               // s batch stride
     const size_t hbs = (size_t)L * (m->kh ? m->kh : 1) * D;         // hist batch stride
@@ -1308,7 +1311,7 @@ snhip_status enqueue_step(SnHipModel* m, int B, float* logits_out, bool greedy, 
         a.L = L; a.B = B; a.D = D; a.I = I; a.R = R; a.K = m->K; a.kh = m->kh;
         a.clamp = m->clamp; a.eps = m->eps; a.p_floor = m->p_floor;
         a.no_g = m->no_g; a.no_c = m->no_c;
-        a.tok = m->tok; a.embed = m->embed; a.vocab = m->vocab;
+        a.tok = tok; a.embed = m->embed; a.vocab = m->vocab;
         float* p = m->bbuf;
         const size_t LB = (size_t)L * B;
         a.xs = p; p += LB * D;
@@ -1319,7 +1322,7 @@ snhip_status enqueue_step(SnHipModel* m, int B, float* logits_out, bool greedy, 
         a.z = p; p += LB * I;
         a.sn = p;
         a.s = m->s; a.hist = m->hist; a.nrm = m->nrm;
-        a.flags = m->bflags; a.err = m->berr; a.spin_limit = m->persist_spin; a.stall = m->persist_stall;
+        a.flags = m->bflags; a.err = m->berr; a.herr = m->h_err + 1; a.spin_limit = m->persist_spin; a.stall = m->persist_stall;
         if (m->batch_epoch == 0xFFFFFFFFu) {
             // epochs start over from clean flags
             SNHIP_CHECK(hipMemsetAsync(m->bflags, 0, m->bflag_words * sizeof(unsigned), st));
@@ -1330,7 +1333,7 @@ snhip_status enqueue_step(SnHipModel* m, int B, float* logits_out, bool greedy, 
         if (rc != SNHIP_OK) return rc;
         return enqueue_head(m, B, nullptr, logits_out, greedy, st, true);
     }
-    hipLaunchKernelGGL(k_embed, dim3(B), dim3(256), 0, st, m->tok, m->embed, m->x, D, m->vocab);
+    hipLaunchKernelGGL(k_embed, dim3(B), dim3(256), 0, st, tok, m->embed, m->x, D, m->vocab);
     const bool mm = B >= m->gemm_min_batch;
     for (int l = 0; l < L; ++l) {
         const Layer& A = m->layers[l];
@@ -1388,6 +1391,8 @@ snhip_status persist_status(SnHipModel* m, int rows) {
     if (!single && !batched) return SNHIP_OK;
     m->h_err[0] = m->h_err[1] = 0;
     m->poisoned = std::max(m->poisoned, rows);
+    if (m->perr) SNHIP_CHECK(hipMemsetAsync(m->perr, 0, sizeof(unsigned), m->stream));
+    if (m->berr) SNHIP_CHECK(hipMemsetAsync(m->berr, 0, sizeof(unsigned), m->stream));
     set_last_error(single ? "persistent decode: exchange wait timed out"
                           : "batched persistent decode: a dataflow wait timed out");
     return SNHIP_E_DEVICE;
@@ -1403,30 +1408,40 @@ snhip_status check_usable(const SnHipModel* m) {
     return SNHIP_OK;
 }
 
-// Runs `reps` decode steps on the internal stream, ordered after the work
-// already queued on the caller's stream and before anything queued on it
-// later. The step's kernels are captured once per (B, logits, greedy) into a
-// HIP graph and replayed.
-snhip_status run_steps(SnHipModel* m, int B, float* logits_out, bool greedy, int reps) {
-    SNHIP_CHECK(hipEventRecord(m->ev_in, m->stream));
-    SNHIP_CHECK(hipStreamWaitEvent(m->work, m->ev_in, 0));
+// Copies B tokens into m->tok on the caller's stream.
+snhip_status put_tokens(SnHipModel* m, const int32_t* t, int B, hipMemcpyKind kind) {
+    SNHIP_CHECK(hipMemcpyAsync(m->tok, t, B * sizeof(int32_t), kind, m->stream));
+    return SNHIP_OK;
+}
+
+// Runs `reps` decode steps on the caller's stream, the first on tok (device).
+// (An internal stream, ordered by events, cost each call two cross-queue waits
+// of about 20 us.) The step's kernels are captured once per (B, logits, greedy)
+// into a HIP graph, which reads m->tok, and replayed.
+snhip_status run_steps(SnHipModel* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps) {
     const bool batch = uses_batch(m, B);
+    if (tok != m->tok && (!batch || greedy)) {
+        // greedy steps write the next tokens to m->tok
+        const snhip_status rc = put_tokens(m, tok, B, hipMemcpyDeviceToDevice);
+        if (rc != SNHIP_OK) return rc;
+        tok = m->tok;
+    }
     if (!m->use_graphs || batch) {
         // The batched persistent step is a handful of launches per step: they
-        // are queued directly (a cooperative launch is not captured).
+        // are queued directly (ordered against other calls' persistent launches).
+        std::optional<PersistCall> call;
         if (batch) {
             m->persist_stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
-            SNHIP_CHECK(hipMemsetAsync(m->berr, 0, sizeof(unsigned), m->work));
+            call.emplace(m->stream);
         }
         for (int i = 0; i < reps; ++i) {
-            const snhip_status rc = enqueue_step(m, B, logits_out, greedy, m->work);
+            const snhip_status rc = enqueue_step(m, tok, B, logits_out, greedy, m->stream);
             if (rc != SNHIP_OK) return rc;
         }
         if (batch) {
             // The call returns once its launches have finished, so that a
             // barrier time-out is reported by this call, not a later one.
-            SNHIP_CHECK(hipMemcpyAsync(m->h_err + 1, m->berr, sizeof(unsigned), hipMemcpyDeviceToHost, m->work));
-            SNHIP_CHECK(hipStreamSynchronize(m->work));
+            SNHIP_CHECK(call->finish());
             const snhip_status st = persist_status(m, B);
             if (st != SNHIP_OK) return st;
         }
@@ -1439,9 +1454,9 @@ snhip_status run_steps(SnHipModel* m, int B, float* logits_out, bool greedy, int
                 m->graphs.clear();
             }
             hipGraph_t g = nullptr;
-            SNHIP_CHECK(hipStreamBeginCapture(m->work, hipStreamCaptureModeThreadLocal));
-            const snhip_status rc = enqueue_step(m, B, logits_out, greedy, m->work);
-            const hipError_t ec = hipStreamEndCapture(m->work, &g);
+            SNHIP_CHECK(hipStreamBeginCapture(m->cap, hipStreamCaptureModeThreadLocal));
+            const snhip_status rc = enqueue_step(m, tok, B, logits_out, greedy, m->cap);
+            const hipError_t ec = hipStreamEndCapture(m->cap, &g);
             if (rc != SNHIP_OK) { if (g) (void)hipGraphDestroy(g); return rc; }
             SNHIP_CHECK(ec);
             hipGraphExec_t ex = nullptr;
@@ -1450,16 +1465,9 @@ snhip_status run_steps(SnHipModel* m, int B, float* logits_out, bool greedy, int
             SNHIP_CHECK(ei);
             it = m->graphs.emplace(key, ex).first;
         }
-        for (int i = 0; i < reps; ++i) SNHIP_CHECK(hipGraphLaunch(it->second, m->work));
+        for (int i = 0; i < reps; ++i) SNHIP_CHECK(hipGraphLaunch(it->second, m->stream));
     }
-    SNHIP_CHECK(hipEventRecord(m->ev_out, m->work));
-    SNHIP_CHECK(hipStreamWaitEvent(m->stream, m->ev_out, 0));
-    return SNHIP_OK;
-}
-
-// Copies B tokens into m->tok on the caller's stream.
-snhip_status put_tokens(SnHipModel* m, const int32_t* t, int B, hipMemcpyKind kind) {
-    SNHIP_CHECK(hipMemcpyAsync(m->tok, t, B * sizeof(int32_t), kind, m->stream));
+    SNHIP_CHECK(m->order.mark(m->stream));
     return SNHIP_OK;
 }
 
@@ -1467,7 +1475,6 @@ snhip_status put_tokens(SnHipModel* m, const int32_t* t, int B, hipMemcpyKind ki
 snhip_status ensure_prefill_ws(SnHipModel* m, int chunk) {
     if (m->pf_chunk >= chunk) return SNHIP_OK;
     SNHIP_CHECK(hipStreamSynchronize(m->stream));
-    SNHIP_CHECK(hipStreamSynchronize(m->work));
     float** bufs[] = {&m->pf_x, &m->pf_raw, &m->pf_at, &m->pf_v, &m->pf_q, &m->pf_u,
                       &m->pf_st, &m->pf_z, &m->pf_yn, &m->pf_sfb, &m->pf_send, &m->pf_pa, &m->pf_pb};
     for (float** b : bufs)
@@ -1611,26 +1618,23 @@ snhip_status run_prefill(SnHipModel* m, const int32_t* tokens_dev, int B, int T,
     chunk = std::min(chunk, T);
     snhip_status rc = ensure_prefill_ws(m, chunk);
     if (rc != SNHIP_OK) return rc;
-    SNHIP_CHECK(hipEventRecord(m->ev_in, m->stream));
-    SNHIP_CHECK(hipStreamWaitEvent(m->work, m->ev_in, 0));
     for (int c0 = 0; c0 < T; c0 += chunk) {
         const int Tc = std::min(chunk, T - c0);
         SNHIP_CHECK(hipMemcpy2DAsync(m->pf_tok, (size_t)Tc * sizeof(int32_t), tokens_dev + c0,
                                      (size_t)T * sizeof(int32_t), (size_t)Tc * sizeof(int32_t), B,
-                                     hipMemcpyDeviceToDevice, m->work));
-        rc = enqueue_prefill_chunk(m, B, Tc, c0 + Tc >= T ? logits_out : nullptr, m->work,
+                                     hipMemcpyDeviceToDevice, m->stream));
+        rc = enqueue_prefill_chunk(m, B, Tc, c0 + Tc >= T ? logits_out : nullptr, m->stream,
                                    all_logits, T, c0);
         if (rc != SNHIP_OK) return rc;
     }
-    SNHIP_CHECK(hipEventRecord(m->ev_out, m->work));
-    SNHIP_CHECK(hipStreamWaitEvent(m->stream, m->ev_out, 0));
+    SNHIP_CHECK(m->order.mark(m->stream));
     return SNHIP_OK;
 }
 
 // n_steps decode steps of sequences [0, B) in persistent launches on the
-// internal stream (ordered like run_steps): B = 1 on the persist_wg grid, else
+// caller's stream: B = 1 on the persist_wg grid, else
 // (2 <= B <= mi_max) each sequence on its own mi_grid[B] workgroups of one
-// launch. The first input tokens are in m->tok. greedy: out_tok (n_steps, B)
+// launch. The first input tokens are in tok (device). greedy: out_tok (n_steps, B)
 // receives each step's argmax tokens, fed to the next step; otherwise n_steps
 // must be 1. logits (B, vocab, device), if not NULL, gets the last step's.
 // The call returns once the launches have finished and reports an exchange
@@ -1638,12 +1642,10 @@ snhip_status run_prefill(SnHipModel* m, const int32_t* tokens_dev, int B, int T,
 // after its own last wait, so a time-out can leave the sequences part-stepped:
 // the handle then refuses steps until reset or set. *launch_failed is set when the
 // first cooperative launch could not be queued at all (nothing ran).
-snhip_status run_persist(SnHipModel* m, int B, int n_steps, bool greedy, int32_t* out_tok,
+snhip_status run_persist(SnHipModel* m, const int32_t* tok, int B, int n_steps, bool greedy, int32_t* out_tok,
                          float* logits, bool* launch_failed) {
     constexpr int kMaxStepsPerLaunch = 1 << 20;   // keeps exchange epochs far from wrapping
-    SNHIP_CHECK(hipEventRecord(m->ev_in, m->stream));
-    SNHIP_CHECK(hipStreamWaitEvent(m->work, m->ev_in, 0));
-    SNHIP_CHECK(hipMemsetAsync(m->perr, 0, sizeof(unsigned), m->work));
+    PersistCall call(m->stream);
     PersistArgs a{};
     a.layers = m->dlayers;
     a.L = m->L; a.D = m->D; a.I = m->I; a.R = m->R; a.K = m->K; a.kh = m->kh;
@@ -1651,7 +1653,7 @@ snhip_status run_persist(SnHipModel* m, int B, int n_steps, bool greedy, int32_t
     a.embed = m->embed; a.no_g = m->no_g; a.no_c = m->no_c;
     a.head = pmat(m->head);
     a.s = m->s; a.hist = m->hist;
-    a.ring = m->pring; a.ex = m->pex; a.sx = m->psx; a.err = m->perr;
+    a.ring = m->pring; a.ex = m->pex; a.sx = m->psx; a.err = m->perr; a.herr = m->h_err;
     a.greedy = greedy ? 1 : 0;
     a.spin_limit = m->persist_spin;
     a.stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
@@ -1660,58 +1662,65 @@ snhip_status run_persist(SnHipModel* m, int B, int n_steps, bool greedy, int32_t
     const int grid = B == 1 ? m->persist_wg : B * m->mi_grid[B];
     for (int done = 0; done < n_steps;) {
         const int n = std::min(n_steps - done, kMaxStepsPerLaunch);
-        // Epochs restart at 1 in every launch: clear the words of the last one.
-        SNHIP_CHECK(hipMemsetAsync(m->pex, 0, 2 * (size_t)kPersistExWords * B * sizeof(unsigned long long), m->work));
-        SNHIP_CHECK(hipMemsetAsync(m->psx, 0, (size_t)m->L * 2 * m->D * B * sizeof(unsigned long long), m->work));
-        a.tok_in = done == 0 ? m->tok : out_tok + (size_t)(done - 1) * B;
+        // A launch uses 4 L + 1 exchange epochs and one state epoch per step;
+        // before they would wrap, the words start over from zero.
+        const uint64_t n_ep = (uint64_t)n * (4 * (uint64_t)m->L + 1) + 2;
+        if (m->persist_ep + n_ep > 0xFFFFFFFFull || (uint64_t)m->persist_st + n > 0xFFFFFFFFull) {
+            const size_t nseq = (size_t)m->persist_nseq;
+            SNHIP_CHECK(hipMemsetAsync(m->pex, 0, 2 * (size_t)kPersistExWords * nseq * sizeof(unsigned long long), m->stream));
+            SNHIP_CHECK(hipMemsetAsync(m->psx, 0, (size_t)m->L * 2 * m->D * nseq * sizeof(unsigned long long), m->stream));
+            m->persist_ep = m->persist_st = 0;
+        }
+        a.ep0 = m->persist_ep;
+        a.st0 = m->persist_st;
+        m->persist_ep += (unsigned)n_ep;
+        m->persist_st += (unsigned)n;
+        a.tok_in = done == 0 ? tok : out_tok + (size_t)(done - 1) * B;
         a.out_tok = greedy ? out_tok + (size_t)done * B : nullptr;
         a.logits = done + n == n_steps ? logits : nullptr;
         a.n_steps = n;
-        const snhip_status rc = launch_decode_persist(a, grid, blk, m->work);
+        const snhip_status rc = launch_decode_persist(a, grid, blk, m->stream);
         if (rc != SNHIP_OK) {
             if (done == 0 && launch_failed) *launch_failed = true;
             return rc;
         }
         done += n;
     }
-    SNHIP_CHECK(hipMemcpyAsync(m->h_err, m->perr, sizeof(unsigned), hipMemcpyDeviceToHost, m->work));
-    SNHIP_CHECK(hipEventRecord(m->ev_out, m->work));
-    SNHIP_CHECK(hipStreamWaitEvent(m->stream, m->ev_out, 0));
-    SNHIP_CHECK(hipStreamSynchronize(m->work));
+    SNHIP_CHECK(call.finish());
     return persist_status(m, B);
 }
 
 // Does a step of B >= 2 sequences run as B instances of the single-sequence
 // persistent kernel in one launch?
-bool uses_mi(const SnHipModel* m, int B) { return m->persist_wg > 0 && B >= 2 && B <= m->mi_max; }
+bool uses_mi(const SnHipModel* m, int B) { return m->persist_wg > 0 && m->all_cus && B >= 2 && B <= m->mi_max; }
 
-// One step of sequences [0, B), B >= 2 (tokens in m->tok): the single-sequence
+// One step of sequences [0, B), B >= 2, on tok (device): the single-sequence
 // persistent kernel on a slice of the grid per sequence when it takes B, else
 // the per-kernel or batched step. A failed cooperative launch turns the
 // persistent path for B >= 2 off and falls back.
-snhip_status step_many(SnHipModel* m, int B, float* logits_out) {
+snhip_status step_many(SnHipModel* m, const int32_t* tok, int B, float* logits_out) {
     if (uses_mi(m, B)) {
         bool launch_failed = false;
-        const snhip_status rc = run_persist(m, B, 1, false, nullptr, logits_out, &launch_failed);
+        const snhip_status rc = run_persist(m, tok, B, 1, false, nullptr, logits_out, &launch_failed);
         if (!launch_failed) return rc;
         m->mi_max = 0;
         (void)hipGetLastError();
     }
-    return run_steps(m, B, logits_out, false, 1);
+    return run_steps(m, tok, B, logits_out, false, 1);
 }
 
-// One step of sequence 0 (tokens already in m->tok): the persistent kernel
+// One step of sequence 0 on tok (device): the persistent kernel
 // when enabled, else the captured per-kernel step. A failed cooperative launch
 // turns the persistent path off for this handle and falls back.
-snhip_status step_one(SnHipModel* m, float* logits_out) {
-    if (m->persist_wg) {
+snhip_status step_one(SnHipModel* m, const int32_t* tok, float* logits_out) {
+    if (m->persist_wg && m->all_cus) {
         bool launch_failed = false;
-        const snhip_status rc = run_persist(m, 1, 1, false, nullptr, logits_out, &launch_failed);
+        const snhip_status rc = run_persist(m, tok, 1, 1, false, nullptr, logits_out, &launch_failed);
         if (!launch_failed) return rc;
         m->persist_wg = 0;
         (void)hipGetLastError();
     }
-    return run_steps(m, 1, logits_out, false, 1);
+    return run_steps(m, tok, 1, logits_out, false, 1);
 }
 
 bool tokens_ok(const SnHipModel* m, const int32_t* t, int n) {
@@ -1748,9 +1757,8 @@ SnHipModel* snhip_load_ex(const char* path, int vocab, int dim, int inner, int r
 
 void snhip_free(SnHipModel* m) {
     if (!m) return;
-    // Only this handle's work is waited for: its internal stream and the
-    // caller's stream it was bound to (NULL = the null stream).
-    if (m->work) (void)hipStreamSynchronize(m->work);
+    // Only this handle's work is waited for: the caller's stream it was bound
+    // to (NULL = the null stream).
     (void)hipStreamSynchronize(m->stream);
     free_model(m);
 }
@@ -1780,7 +1788,10 @@ int32_t snhip_batch_grid(const SnHipModel* m) { return m ? m->batch_wg : 0; }
 
 snhip_status snhip_set_stream(SnHipModel* m, void* stream) {
     if (!m) return SNHIP_E_INVAL;
+    if (m->stream == as_stream(stream)) return SNHIP_OK;
     m->stream = as_stream(stream);
+    m->all_cus = stream_has_all_cus(m->stream);
+    SNHIP_CHECK(m->order.follow(m->stream));
     return SNHIP_OK;
 }
 
@@ -1788,9 +1799,7 @@ snhip_status snhip_step_batch_dev(SnHipModel* m, const int32_t* tokens_dev, int3
                                   float* logits_dev) {
     if (!m || !tokens_dev || !logits_dev || B <= 0 || B > m->max_batch) return SNHIP_E_INVAL;
     if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
-    const snhip_status rc = put_tokens(m, tokens_dev, B, hipMemcpyDeviceToDevice);
-    if (rc != SNHIP_OK) return rc;
-    return B == 1 ? step_one(m, logits_dev) : step_many(m, B, logits_dev);
+    return B == 1 ? step_one(m, tokens_dev, logits_dev) : step_many(m, tokens_dev, B, logits_dev);
 }
 
 snhip_status snhip_step_batch(SnHipModel* m, const int32_t* tokens, int32_t B, float* logits) {
@@ -1798,7 +1807,7 @@ snhip_status snhip_step_batch(SnHipModel* m, const int32_t* tokens, int32_t B, f
     if (!tokens_ok(m, tokens, B)) return SNHIP_E_INVAL;
     if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     snhip_status rc = put_tokens(m, tokens, B, hipMemcpyHostToDevice);
-    if (rc == SNHIP_OK) rc = B == 1 ? step_one(m, m->logits) : step_many(m, B, m->logits);
+    if (rc == SNHIP_OK) rc = B == 1 ? step_one(m, m->tok, m->logits) : step_many(m, m->tok, B, m->logits);
     if (rc != SNHIP_OK) return rc;
     SNHIP_CHECK(hipMemcpyAsync(logits, m->logits, (size_t)B * m->vocab * sizeof(float),
                                hipMemcpyDeviceToHost, m->stream));
@@ -1826,8 +1835,7 @@ snhip_status snhip_prefill_host(SnHipModel* m, const int32_t* tokens, int32_t n,
         rc = run_prefill(m, dt, 1, n, m->logits);
     } else {
         for (int i = 0; i < n && rc == SNHIP_OK; ++i) {   // the reference's step loop (sunnynet.c:347-349)
-            rc = put_tokens(m, dt + i, 1, hipMemcpyDeviceToDevice);
-            if (rc == SNHIP_OK) rc = run_steps(m, 1, m->logits, false, 1);
+            rc = run_steps(m, dt + i, 1, m->logits, false, 1);
         }
     }
     if (rc == SNHIP_OK &&
@@ -1857,9 +1865,7 @@ snhip_status snhip_dbg_layer(SnHipModel* m, int32_t token, int32_t layer, float*
     if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     const int D = m->D, I = m->I, R = m->R;
     const size_t hbs = (size_t)m->L * (m->kh ? m->kh : 1) * D;
-    hipStream_t st = m->work;
-    SNHIP_CHECK(hipEventRecord(m->ev_in, m->stream));
-    SNHIP_CHECK(hipStreamWaitEvent(st, m->ev_in, 0));
+    hipStream_t st = m->stream;
     SNHIP_CHECK(hipMemcpyAsync(m->tok, &token, sizeof(int32_t), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_embed, dim3(1), dim3(256), 0, st, m->tok, m->embed, m->x, D, m->vocab);
     for (int l = 0; l <= layer; ++l) {
@@ -1907,20 +1913,16 @@ snhip_status snhip_decode_greedy_dev(SnHipModel* m, const int32_t* tokens_dev, i
     if (!m || !tokens_dev || !out_tokens_dev || B <= 0 || B > m->max_batch || n_steps <= 0)
         return SNHIP_E_INVAL;
     if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
-    if (B == 1 && m->persist_wg) {
-        snhip_status rc = put_tokens(m, tokens_dev, 1, hipMemcpyDeviceToDevice);
-        if (rc != SNHIP_OK) return rc;
+    if (B == 1 && m->persist_wg && m->all_cus) {
         bool launch_failed = false;
-        rc = run_persist(m, 1, n_steps, true, out_tokens_dev, logits_dev, &launch_failed);
+        const snhip_status rc = run_persist(m, tokens_dev, 1, n_steps, true, out_tokens_dev, logits_dev, &launch_failed);
         if (!launch_failed) return rc;
         m->persist_wg = 0;
         (void)hipGetLastError();
     }
     if (uses_mi(m, B)) {
-        snhip_status rc = put_tokens(m, tokens_dev, B, hipMemcpyDeviceToDevice);
-        if (rc != SNHIP_OK) return rc;
         bool launch_failed = false;
-        rc = run_persist(m, B, n_steps, true, out_tokens_dev, logits_dev, &launch_failed);
+        const snhip_status rc = run_persist(m, tokens_dev, B, n_steps, true, out_tokens_dev, logits_dev, &launch_failed);
         if (!launch_failed) return rc;
         m->mi_max = 0;
         (void)hipGetLastError();
@@ -1928,7 +1930,6 @@ snhip_status snhip_decode_greedy_dev(SnHipModel* m, const int32_t* tokens_dev, i
     if ((long)n_steps * B > (long)m->hist_cap || !m->tok_hist) {
         // Grow the token history; graphs bake its address, so drop them.
         SNHIP_CHECK(hipStreamSynchronize(m->stream));
-        SNHIP_CHECK(hipStreamSynchronize(m->work));
         for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
         m->graphs.clear();
         long cap = 256L * m->max_batch;
@@ -1945,11 +1946,9 @@ snhip_status snhip_decode_greedy_dev(SnHipModel* m, const int32_t* tokens_dev, i
         m->allocs.push_back(h);
         m->hist_cap = (int)cap;
     }
-    snhip_status rc = put_tokens(m, tokens_dev, B, hipMemcpyDeviceToDevice);
-    if (rc != SNHIP_OK) return rc;
     SNHIP_CHECK(hipMemsetAsync(m->counter, 0, sizeof(int32_t), m->stream));
     float* lg = logits_dev ? logits_dev : m->logits;
-    rc = run_steps(m, B, lg, true, n_steps);
+    const snhip_status rc = run_steps(m, tokens_dev, B, lg, true, n_steps);
     if (rc != SNHIP_OK) return rc;
     SNHIP_CHECK(hipMemcpyAsync(out_tokens_dev, m->tok_hist, (size_t)n_steps * B * sizeof(int32_t),
                                hipMemcpyDeviceToDevice, m->stream));

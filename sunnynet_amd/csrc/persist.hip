@@ -26,8 +26,9 @@
 // Words are double-buffered by epoch parity. A writer of epoch e + 2 has read
 // epoch e + 1 from every workgroup, and each of those read all of epoch e
 // before writing e + 1, so no reader is still on the slot being overwritten
-// (every workgroup produces and reads every exchange). Buffers are zeroed
-// before each launch and epochs start at 1.
+// (every workgroup produces and reads every exchange). Epochs grow from launch
+// to launch (a launch starts after the one before it has finished), so the
+// buffers are cleared only when they would wrap.
 //
 // Ownership. Workgroup w owns channels [w cpw, (w + 1) cpw): their state s,
 // the W_eff and W_c rows, and the residual x. Everything a channel needs in

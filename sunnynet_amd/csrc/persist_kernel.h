@@ -70,7 +70,7 @@ __device__ __forceinline__ float ll_f(u64 w) { return __uint_as_float((uint32_t)
 __device__ __forceinline__ u64 ll_ready(float v, unsigned ep) { return ((u64)ep << 32) | __float_as_uint(v); }
 
 struct PollCtl {
-    unsigned* err;
+    unsigned *err, *herr;
     unsigned limit;
 };
 
@@ -89,6 +89,7 @@ __device__ __forceinline__ bool ll_spin(u64 (&w)[W], Addr&& addr, Want&& want, c
             if (__hip_atomic_load(pc.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
             if (spins > pc.limit) {
                 __hip_atomic_store(pc.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(pc.herr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 return false;
             }
         }
@@ -575,7 +576,7 @@ __global__ __launch_bounds__(NT) void k_decode_persist(PersistArgs a) {
     }
     const int cpw = D / G, c0 = wg * cpw;                     // owned channels
     const int grp0 = c0 >> 3, ngrp = cpw >= 8 ? cpw >> 3 : 1; // owned channel groups
-    const PollCtl pc{a.err, a.spin_limit};
+    const PollCtl pc{a.err, a.herr, a.spin_limit};
     for (int i = tid; i < L * (int)sizeof(PLayer) / 4; i += NT)
         ((uint32_t*)ltab)[i] = ((const uint32_t*)a.layers)[i];
     const PLayer* lt = ltab;
@@ -627,7 +628,7 @@ __global__ __launch_bounds__(NT) void k_decode_persist(PersistArgs a) {
     Pool<BLK> p0, p1;   // p1: fp32 jobs of more than one batch
     prefetch_job<BLK>(job(0), p0, lane);
 
-    unsigned ep = 0;                  // epoch of the last exchange produced
+    unsigned ep = a.ep0;              // epoch of the last exchange produced
     const unsigned stall = a.stall;   // > 0 only to test the time-out path
     int tok = a.tok_in[0];
     float* ring_wg = a.ring + (size_t)blockIdx.x * L * KH * D;
@@ -647,7 +648,7 @@ __global__ __launch_bounds__(NT) void k_decode_persist(PersistArgs a) {
             // ---- the phase's input: the vector it multiplies (A: x, B: v,
             // C: u, D: z, H: x), for A also the old state s (words PD..)
             const int n0 = t == 1 ? R : t == 3 ? I : D;
-            const unsigned e0 = ep + stall, e1 = (unsigned)step + stall;
+            const unsigned e0 = ep + stall, e1 = a.st0 + (unsigned)step + stall;
             const u64* s0 = exs(ep);
             const u64* s1 = a.sx + ((size_t)l * 2 + ((step - 1) & 1)) * D;
             const bool plain0 = t == 0 && l == 0;          // x = the token's embedding row
@@ -775,7 +776,7 @@ __global__ __launch_bounds__(NT) void k_decode_persist(PersistArgs a) {
                     if (a.clamp && pg < a.p_floor) pg = a.p_floor;
                     const float sn = pg * xs2[sidx<BLK>(i, D)] + (1.0f - pg) * uu;
                     ll_putf(out + i, uu, epv);
-                    ll_putf(sout + i, sn, (unsigned)step + 1);
+                    ll_putf(sout + i, sn, a.st0 + (unsigned)step + 1);
                     sown[c] = sn;
                 }
             } else if (t == 2) {

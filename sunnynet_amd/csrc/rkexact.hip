@@ -721,6 +721,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         A.xch += (size_t)sqi * A.words;
         A.keys += (size_t)sqi * A.words;
         A.tok += sqi;
+        A.tok_in += sqi;
         A.logits += (size_t)sqi * A.vocab;
     }
     if (tid == 0) sdead = 0;
@@ -738,7 +739,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
             reinterpret_cast<int*>(&Ls2[l & 1])[tid] = reinterpret_cast<const int*>(A.layers + l)[tid];
     };
     float vfo = 0.0f;   // head owners, thread c < 64: v_first of channel c (layer 0's v)
-    int tok = *A.tok;
+    int tok = *A.tok_in;
     const int cnt0 = A.hist0;
     Pend pend;
         // A head owner's P2 operands into LDS: the 64 x 64 state (loaded into
@@ -788,7 +789,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         const bool owners_skip = NH * 4 <= G;   // the head owners take no P1 rows
         const size_t slab = rkp_slab(D, F);
         const unsigned ep = A.epoch + (unsigned)st;
-        const PollCtl pc{A.err, A.spin_limit, ep + A.stall};
+        const PollCtl pc{A.err, A.herr, A.spin_limit, ep + A.stall};
         const bool last = st + 1 == A.nsteps;
 
         // x = LN_0(E[tok]) (rwkv7.c:351-352); NaN for an out-of-range id.

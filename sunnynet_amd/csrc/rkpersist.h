@@ -33,7 +33,8 @@ struct RkPArgs {
     unsigned long long* xch;  // per-layer exchange slabs, rkp_slab(D, F) words each
     float* logits;            // (vocab)
     unsigned long long* keys; // (2 grid) exchange words of the argmax keys
-    int32_t* tok;             // the step's input token (and, greedy, the next one)
+    const int32_t* tok_in;    // the launch's first input token
+    int32_t* tok;             // receives the last token (greedy: the next launch's input)
     int32_t* tok_hist;        // greedy: (steps, ni) tokens, from row hist0 on
     int32_t* counter;         // set to hist0 + nsteps after a greedy launch
     int hist_cap, greedy;
@@ -41,14 +42,15 @@ struct RkPArgs {
     // Independent sequences, one per equal slice of the grid (0 or 1: one).
     // Sequence q runs on workgroups [q G, (q+1) G), G = grid / ni, with its
     // own state (S + q L NH 64 64, shift + q L 2 D, vfirst + q D), exchange
-    // and key words (xch and keys + q words), token tok[q], token column q of
+    // and key words (xch and keys + q words), tokens tok_in[q] and tok[q], column q of
     // tok_hist and logits + q vocab.
     int ni;
     size_t words;
     unsigned epoch;           // the epoch of the launch's first step (> 0; step st uses epoch + st, and
                               // no epoch is used twice between two clearings of the words)
     int nsteps;               // steps of the launch (greedy; 1 otherwise)
-    unsigned* err;
+    unsigned* err;            // set on a time-out, zero before the launch
+    unsigned* herr;           // the same for the host (pinned)
     unsigned spin_limit;
     unsigned stall;           // added to every wait target: tests force time-outs with it
 };

@@ -468,6 +468,7 @@ __global__ __launch_bounds__(NT) void k_rk_persist(RkPArgs A) {
         A.xch += (size_t)sq * A.words;
         A.keys += (size_t)sq * A.words;
         A.tok += sq;
+        A.tok_in += sq;
         A.logits += (size_t)sq * A.vocab;
     }
     if (tid == 0) sdead = 0;
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(NT) void k_rk_persist(RkPArgs A) {
         return sdead == 0;
     };
     float vfo = 0.0f;   // head owners, thread c < 64: v_first of channel c (layer 0's v)
-    int tok = *A.tok;
+    int tok = *A.tok_in;
     const int cnt0 = A.hist0;
 
     // Greedy launches run nsteps steps, step st with epoch A.epoch + st; every
@@ -494,7 +495,7 @@ __global__ __launch_bounds__(NT) void k_rk_persist(RkPArgs A) {
         asm volatile("" : "+s"(D), "+s"(F), "+s"(L), "+s"(NH), "+s"(G));
         const size_t slab = rkp_slab(D, F);
         const unsigned ep = A.epoch + (unsigned)st;
-        const PollCtl pc{A.err, A.spin_limit, ep + A.stall};
+        const PollCtl pc{A.err, A.herr, A.spin_limit, ep + A.stall};
         const bool last = st + 1 == A.nsteps;
 
         // x = LN_0(E[tok]) (rwkv7.c:351-352); NaN for an out-of-range id. From

@@ -25,7 +25,7 @@ __device__ __forceinline__ bool ex_ok(u64 w, unsigned ep) { return (uint32_t)(w 
 __device__ __forceinline__ float ex_f(u64 w) { return __uint_as_float((uint32_t)w); }
 
 struct PollCtl {
-    unsigned* err;
+    unsigned *err, *herr;
     unsigned limit;
     unsigned want;   // the step's epoch (plus the test stall)
 };
@@ -48,6 +48,7 @@ __device__ __forceinline__ bool ex_spin(u64 (&w)[W], const u64* const (&src)[W],
             if (__hip_atomic_load(pc.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
             if (spins > pc.limit) {
                 __hip_atomic_store(pc.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(pc.herr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 return false;
             }
         }

@@ -151,9 +151,11 @@ struct SnHipRwkv7 {
     int32_t *counter = nullptr, *done = nullptr, *tok_hist = nullptr;
     int hist_cap = 0;
     std::vector<void*> allocs;
-    hipStream_t stream = nullptr, work = nullptr;
-    hipEvent_t ev_in = nullptr, ev_out = nullptr;
-    std::map<std::tuple<int, const void*, int>, hipGraphExec_t> graphs;
+    hipStream_t stream = nullptr;         // the caller's
+    snhip::StreamOrder order;
+    bool all_cus = true;                  // it may use every CU: the one-launch steps need them
+    hipStream_t cap = nullptr;            // graphs are captured here
+    std::map<int, hipGraphExec_t> graphs;   // the captured layers, by batch size
     bool use_graphs = true;
     bool fuse_ups = true;   // LoRA up-projections inside the heads kernel (SNHIP_RKQ_FUSE_UPS=0: apart)
     // One-sequence steps as one cooperative launch each (rkpersist.hip);
@@ -170,7 +172,8 @@ struct SnHipRwkv7 {
     unsigned p_epoch = 0;                 // the last epoch a persistent launch used
     unsigned long long* p_words = nullptr;   // exchange slabs and key words (zeroed: epoch 0)
     size_t p_nwords = 0;
-    unsigned* p_err = nullptr;
+    unsigned* p_err = nullptr;            // time-out flag of a launch's workgroups (zero between calls)
+    unsigned* h_err = nullptr;            // the same for the host: pinned, written by the kernel that times out
     unsigned p_spin = 1u << 22;
     // A persistent step timed out after some layers had written S and shift in
     // place: every stepping call fails until snhip_rk_reset or set_state.
@@ -192,9 +195,8 @@ T* ralloc(SnHipRwkv7* m, size_t n) {
 void free_rk(SnHipRwkv7* m) {
     if (!m) return;
     for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
-    if (m->ev_in) (void)hipEventDestroy(m->ev_in);
-    if (m->ev_out) (void)hipEventDestroy(m->ev_out);
-    if (m->work) (void)hipStreamDestroy(m->work);
+    if (m->cap) (void)hipStreamDestroy(m->cap);
+    if (m->h_err) (void)hipHostFree(m->h_err);
     for (void* p : m->allocs) (void)hipFree(p);
     delete m;
 }
@@ -368,8 +370,11 @@ void setup_rk_persist(SnHipRwkv7* m) {
     m->p_err = ralloc<unsigned>(m, 1);
     if (!dtab || !m->p_words || !m->p_err ||
         hipMemcpy(dtab, tab.data(), tab.size() * sizeof(RkPLayer), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(m->p_words, 0, m->p_nwords * sizeof(unsigned long long)) != hipSuccess)
+        hipMemset(m->p_words, 0, m->p_nwords * sizeof(unsigned long long)) != hipSuccess ||
+        hipMemset(m->p_err, 0, sizeof(unsigned)) != hipSuccess ||
+        hipHostMalloc((void**)&m->h_err, sizeof(unsigned), 0) != hipSuccess)
         return;
+    *m->h_err = 0;
     unsigned long long* xch = m->p_words;
     unsigned long long* keys = xch + (size_t)m->L * rkp_slab(m->D, m->F);
     RkPArgs& a = m->p_args;
@@ -378,7 +383,7 @@ void setup_rk_persist(SnHipRwkv7* m) {
     a.head = pmat(m->head);
     a.S = m->S; a.shift = m->shift; a.vfirst = m->vfirst; a.xch = xch; a.keys = keys;
     a.tok = m->tok; a.counter = m->counter;
-    a.err = m->p_err; a.spin_limit = m->p_spin; a.stall = 0;
+    a.err = m->p_err; a.herr = m->h_err; a.spin_limit = m->p_spin; a.stall = 0;
     a.words = m->p_seq_words;
     m->p_grid = G;
     m->p_exact = exact;
@@ -414,17 +419,18 @@ void setup_rkq_tiles(SnHipRwkv7* m) {
 }
 
 // Do steps of B sequences run as B slices of the persistent kernel?
-bool uses_mi(const SnHipRwkv7* m, int B) { return m->p_grid > 0 && B >= 2 && B <= m->p_mi_max; }
+bool uses_mi(const SnHipRwkv7* m, int B) { return m->p_grid > 0 && m->all_cus && B >= 2 && B <= m->p_mi_max; }
 
-// reps persistent steps of sequences [0, B) (B = 1, or 2..p_mi_max on a grid
-// slice each): greedy, one launch of up to kRkPStepsPerLaunch steps at a
+// reps persistent steps of sequences [0, B) on tok (device; B = 1, or
+// 2..p_mi_max on a grid slice each): greedy, one launch of up to kRkPStepsPerLaunch steps at a
 // time, otherwise one launch per step; every step has its own epoch. The
 // call waits for them and reports a time-out of an exchange wait as an error.
 // The kernel updates S and shift in place layer by layer, so a time-out
 // leaves them part-stepped: the handle is then refused for stepping until its
 // state is reset or set.
 constexpr int kRkPStepsPerLaunch = 1024;
-snhip_status run_persist(SnHipRwkv7* m, int B, float* logits_out, bool greedy, int reps) {
+snhip_status run_persist(SnHipRwkv7* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps) {
+    PersistCall call(m->stream);
     RkPArgs a = m->p_args;
     a.stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
     a.logits = logits_out;
@@ -433,27 +439,27 @@ snhip_status run_persist(SnHipRwkv7* m, int B, float* logits_out, bool greedy, i
     a.hist_cap = m->hist_cap;
     a.ni = B;
     const int grid = B == 1 ? m->p_grid : B * m->p_mi_grid[B];
-    SNHIP_CHECK(hipMemsetAsync(m->p_err, 0, sizeof(unsigned), m->work));
     for (int i = 0; i < reps;) {
         const int n = greedy ? std::min(reps - i, kRkPStepsPerLaunch) : 1;
         if (m->p_epoch > 0xFFFFFFFFu - (unsigned)n) {
             // epochs start over from clean words
-            SNHIP_CHECK(hipMemsetAsync(m->p_words, 0, m->p_nwords * sizeof(unsigned long long), m->work));
+            SNHIP_CHECK(hipMemsetAsync(m->p_words, 0, m->p_nwords * sizeof(unsigned long long), m->stream));
             m->p_epoch = 0;
         }
         a.epoch = m->p_epoch + 1;
         a.nsteps = n;
         a.hist0 = i;
         m->p_epoch += (unsigned)n;
-        const snhip_status rc = m->p_exact ? launch_rk_exact(a, grid, m->work) : launch_rk_persist(a, grid, m->work);
+        a.tok_in = i == 0 ? tok : m->tok;
+        const snhip_status rc = m->p_exact ? launch_rk_exact(a, grid, m->stream) : launch_rk_persist(a, grid, m->stream);
         if (rc != SNHIP_OK) return rc;
         i += n;
     }
-    unsigned err = 0;
-    SNHIP_CHECK(hipMemcpyAsync(&err, m->p_err, sizeof(unsigned), hipMemcpyDeviceToHost, m->work));
-    SNHIP_CHECK(hipStreamSynchronize(m->work));
-    if (err) {
+    SNHIP_CHECK(call.finish());
+    if (*m->h_err) {
+        *m->h_err = 0;
         m->poisoned = 1;
+        SNHIP_CHECK(hipMemsetAsync(m->p_err, 0, sizeof(unsigned), m->stream));
         set_last_error("RWKV-7 persistent step: an exchange wait timed out");
         return SNHIP_E_DEVICE;
     }
@@ -604,9 +610,7 @@ SnHipRwkv7* load_rk(const char* path, int max_batch, int wfmt, int block) {
         hipMemset(m->shift, 0, B * L * 2 * D * sizeof(float)) != hipSuccess ||
         hipMemset(m->counter, 0, sizeof(int32_t)) != hipSuccess ||
         hipMemset(m->done, 0, sizeof(int32_t)) != hipSuccess ||
-        hipStreamCreateWithFlags(&m->work, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&m->ev_in, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&m->ev_out, hipEventDisableTiming) != hipSuccess) {
+        hipStreamCreateWithFlags(&m->cap, hipStreamNonBlocking) != hipSuccess) {
         set_last_error("device setup failed");
         free_rk(m);
         return nullptr;
@@ -660,8 +664,7 @@ struct MMList {
 
 // dbg (device, 9 D floats): run layers 0..dbg_layer only and leave sequence
 // 0's intermediates of that layer there in the reference's order (rwkv7.c:308-319).
-snhip_status enqueue_step(SnHipRwkv7* m, int B, float* logits_out, bool greedy, hipStream_t st,
-                          int dbg_layer = -1, float* dbg = nullptr) {
+snhip_status enqueue_layers(SnHipRwkv7* m, int B, hipStream_t st, int dbg_layer = -1, float* dbg = nullptr) {
     const int D = m->D, NH = m->NH, L = m->L, HS = m->HS;
     const size_t s_bstride = (size_t)L * NH * HS * HS, sh_bstride = (size_t)L * 2 * D;
     snhip_status rc;
@@ -763,6 +766,15 @@ snhip_status enqueue_step(SnHipRwkv7* m, int B, float* logits_out, bool greedy, 
     ln.mode = RKQ_LN_PLAIN;
     ln.x = m->x; ln.g = m->on_w; ln.c = m->on_b; ln.out = m->nrm;
     if ((rc = launch_rkq_ln(ln, B, st)) != SNHIP_OK) return rc;
+    SNHIP_CHECK(hipGetLastError());
+    return SNHIP_OK;
+}
+
+// The step's vocabulary head over the final norm in m->nrm, and with greedy the
+// next tokens.
+snhip_status enqueue_head(SnHipRwkv7* m, int B, float* logits_out, bool greedy, hipStream_t st) {
+    MMList mm{B};
+    snhip_status rc;
     if ((rc = mm.add(m->head, m->nrm, logits_out, m->vocab, RKQ_STORE)) != SNHIP_OK) return rc;
     if ((rc = mm.flush(st)) != SNHIP_OK) return rc;
     if (greedy) {
@@ -776,44 +788,50 @@ snhip_status enqueue_step(SnHipRwkv7* m, int B, float* logits_out, bool greedy, 
     return SNHIP_OK;
 }
 
-// reps steps on the internal stream, ordered after the caller's stream;
-// captured once per (B, logits, greedy) into a graph and replayed.
-snhip_status run_steps(SnHipRwkv7* m, int B, float* logits_out, bool greedy, int reps) {
+// reps steps on the caller's stream, the first on tok (device; null: m->tok).
+// (An internal stream, ordered by events, cost each call two cross-queue waits
+// of about 20 us, and once a process had launched cooperatively a stream could
+// land on a queue where every kernel took about 20 us more.) The
+// layers are captured once per batch size into a graph and replayed; the head
+// is launched behind it, so that a call's logits buffer is not part of the
+// graph (with the pointer in its key, a caller that gave a new buffer each step
+// paid captures: up to 0.6 ms per step at B = 64).
+snhip_status run_steps(SnHipRwkv7* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps) {
     if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
-    SNHIP_CHECK(hipEventRecord(m->ev_in, m->stream));
-    SNHIP_CHECK(hipStreamWaitEvent(m->work, m->ev_in, 0));
-    if ((B == 1 && m->p_grid > 0) || uses_mi(m, B)) {
-        const snhip_status rc = run_persist(m, B, logits_out, greedy, reps);
-        if (rc != SNHIP_OK) return rc;
-    } else if (!m->use_graphs) {
+    if ((B == 1 && m->p_grid > 0 && m->all_cus) || uses_mi(m, B)) {
+        return run_persist(m, tok ? tok : m->tok, B, logits_out, greedy, reps);
+    } else {
+        if (tok) SNHIP_CHECK(hipMemcpyAsync(m->tok, tok, B * sizeof(int32_t), hipMemcpyDeviceToDevice, m->stream));
+        hipGraphExec_t ex = nullptr;
+        if (m->use_graphs) {
+            auto it = m->graphs.find(B);
+            if (it == m->graphs.end()) {
+                if (m->graphs.size() >= 16) {
+                    for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
+                    m->graphs.clear();
+                }
+                hipGraph_t g = nullptr;
+                SNHIP_CHECK(hipStreamBeginCapture(m->cap, hipStreamCaptureModeThreadLocal));
+                const snhip_status rc = enqueue_layers(m, B, m->cap);
+                const hipError_t ec = hipStreamEndCapture(m->cap, &g);
+                if (rc != SNHIP_OK) { if (g) (void)hipGraphDestroy(g); return rc; }
+                SNHIP_CHECK(ec);
+                const hipError_t ei = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
+                (void)hipGraphDestroy(g);
+                SNHIP_CHECK(ei);
+                it = m->graphs.emplace(B, ex).first;
+            }
+            ex = it->second;
+        }
         for (int i = 0; i < reps; ++i) {
-            const snhip_status rc = enqueue_step(m, B, logits_out, greedy, m->work);
+            snhip_status rc = SNHIP_OK;
+            if (ex) SNHIP_CHECK(hipGraphLaunch(ex, m->stream));
+            else rc = enqueue_layers(m, B, m->stream);
+            if (rc == SNHIP_OK) rc = enqueue_head(m, B, logits_out, greedy, m->stream);
             if (rc != SNHIP_OK) return rc;
         }
-    } else {
-        const auto key = std::make_tuple(B, (const void*)logits_out, greedy ? 1 : 0);
-        auto it = m->graphs.find(key);
-        if (it == m->graphs.end()) {
-            if (m->graphs.size() >= 16) {
-                for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
-                m->graphs.clear();
-            }
-            hipGraph_t g = nullptr;
-            SNHIP_CHECK(hipStreamBeginCapture(m->work, hipStreamCaptureModeThreadLocal));
-            const snhip_status rc = enqueue_step(m, B, logits_out, greedy, m->work);
-            const hipError_t ec = hipStreamEndCapture(m->work, &g);
-            if (rc != SNHIP_OK) { if (g) (void)hipGraphDestroy(g); return rc; }
-            SNHIP_CHECK(ec);
-            hipGraphExec_t ex = nullptr;
-            const hipError_t ei = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(g);
-            SNHIP_CHECK(ei);
-            it = m->graphs.emplace(key, ex).first;
-        }
-        for (int i = 0; i < reps; ++i) SNHIP_CHECK(hipGraphLaunch(it->second, m->work));
     }
-    SNHIP_CHECK(hipEventRecord(m->ev_out, m->work));
-    SNHIP_CHECK(hipStreamWaitEvent(m->stream, m->ev_out, 0));
+    SNHIP_CHECK(m->order.mark(m->stream));
     return SNHIP_OK;
 }
 
@@ -827,7 +845,7 @@ snhip_status step_host(SnHipRwkv7* m, const int32_t* tokens, int B, float* logit
     if (!m || !tokens || !logits || B <= 0 || B > m->max_batch) return SNHIP_E_INVAL;
     if (!tokens_ok(m, tokens, B)) return SNHIP_E_INVAL;
     SNHIP_CHECK(hipMemcpyAsync(m->tok, tokens, B * sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
-    const snhip_status rc = run_steps(m, B, m->logits, false, 1);
+    const snhip_status rc = run_steps(m, nullptr, B, m->logits, false, 1);
     if (rc != SNHIP_OK) return rc;
     SNHIP_CHECK(hipMemcpyAsync(logits, m->logits, (size_t)B * m->vocab * sizeof(float),
                                hipMemcpyDeviceToHost, m->stream));
@@ -942,9 +960,7 @@ snhip_status enqueue_chunk(SnHipRwkv7* m, const PfWs& ws, int T, float* logits_o
     ln.mode = RKQ_LN_PLAIN;
     ln.x = ws.x + (size_t)(T - 1) * D; ln.g = m->on_w; ln.c = m->on_b; ln.out = m->nrm;
     if ((rc = launch_rkq_ln(ln, 1, st)) != SNHIP_OK) return rc;
-    MMList head{1};
-    if ((rc = head.add(m->head, m->nrm, logits_out, m->vocab, RKQ_STORE)) != SNHIP_OK) return rc;
-    return head.flush(st);
+    return enqueue_head(m, 1, logits_out, false, st);
 }
 
 snhip_status run_prefill(SnHipRwkv7* m, const int32_t* tokens, int n, float* logits_out) {
@@ -953,16 +969,12 @@ snhip_status run_prefill(SnHipRwkv7* m, const int32_t* tokens, int n, float* log
     if (!m->pf) { set_last_error("out of device memory (prefill)"); return SNHIP_E_NOMEM; }
     PfWs ws;
     pf_layout(m, m->pf, &ws);
-    SNHIP_CHECK(hipEventRecord(m->ev_in, m->stream));
-    SNHIP_CHECK(hipStreamWaitEvent(m->work, m->ev_in, 0));
     for (int c0 = 0; c0 < n; c0 += kPfRows) {
         const int T = std::min(kPfRows, n - c0);
-        SNHIP_CHECK(hipMemcpyAsync(ws.tok, tokens + c0, T * sizeof(int32_t), hipMemcpyHostToDevice, m->work));
-        const snhip_status rc = enqueue_chunk(m, ws, T, c0 + T == n ? logits_out : nullptr, m->work);
+        SNHIP_CHECK(hipMemcpyAsync(ws.tok, tokens + c0, T * sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
+        const snhip_status rc = enqueue_chunk(m, ws, T, c0 + T == n ? logits_out : nullptr, m->stream);
         if (rc != SNHIP_OK) return rc;
     }
-    SNHIP_CHECK(hipEventRecord(m->ev_out, m->work));
-    SNHIP_CHECK(hipStreamWaitEvent(m->stream, m->ev_out, 0));
     return SNHIP_OK;
 }
 
@@ -976,7 +988,7 @@ snhip_status prefill_host(SnHipRwkv7* m, const int32_t* tokens, int n, float* lo
         // rwkv7.c:362-364: the step, once per token, in order.
         for (int i = 0; i < n; ++i) {
             SNHIP_CHECK(hipMemcpyAsync(m->tok, tokens + i, sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
-            const snhip_status rc = run_steps(m, 1, m->logits, false, 1);
+            const snhip_status rc = run_steps(m, nullptr, 1, m->logits, false, 1);
             if (rc != SNHIP_OK) return rc;
         }
     }
@@ -1005,7 +1017,6 @@ SnHipRwkv7* snhip_rk_load_ex(const char* path, int32_t max_batch, int32_t weight
 void snhip_rk_free(SnHipRwkv7* m) {
     if (!m) return;
     // Only this handle's work is waited for (see snhip_free).
-    if (m->work) (void)hipStreamSynchronize(m->work);
     (void)hipStreamSynchronize(m->stream);
     free_rk(m);
 }
@@ -1036,14 +1047,13 @@ snhip_status snhip_rk_dbg(SnHipRwkv7* m, int token, int layer, float* out) {
     if (!d) return SNHIP_E_NOMEM;
     const int32_t t = token;
     snhip_status rc = SNHIP_OK;
-    if (hipMemcpyAsync(m->tok, &t, sizeof(int32_t), hipMemcpyHostToDevice, m->stream) != hipSuccess ||
-        hipEventRecord(m->ev_in, m->stream) != hipSuccess || hipStreamWaitEvent(m->work, m->ev_in, 0) != hipSuccess)
+    if (hipMemcpyAsync(m->tok, &t, sizeof(int32_t), hipMemcpyHostToDevice, m->stream) != hipSuccess)
         rc = SNHIP_E_DEVICE;
-    if (rc == SNHIP_OK) rc = enqueue_step(m, 1, m->logits, false, m->work, layer, d);
-    if (rc == SNHIP_OK && (hipMemcpyAsync(out, d, n * sizeof(float), hipMemcpyDeviceToHost, m->work) != hipSuccess ||
-                           hipStreamSynchronize(m->work) != hipSuccess))
+    if (rc == SNHIP_OK) rc = enqueue_layers(m, 1, m->stream, layer, d);
+    if (rc == SNHIP_OK && (hipMemcpyAsync(out, d, n * sizeof(float), hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
+                           hipStreamSynchronize(m->stream) != hipSuccess))
         rc = SNHIP_E_DEVICE;
-    (void)hipStreamSynchronize(m->work);
+    (void)hipStreamSynchronize(m->stream);
     for (auto it = m->allocs.begin(); it != m->allocs.end(); ++it)
         if (*it == d) { (void)hipFree(d); m->allocs.erase(it); break; }
     return rc;
@@ -1054,7 +1064,10 @@ int snhip_rk_ready(const SnHipRwkv7* m) { return m && m->ready; }
 
 snhip_status snhip_rk_set_stream(SnHipRwkv7* m, void* stream) {
     if (!m) return SNHIP_E_INVAL;
+    if (m->stream == as_stream(stream)) return SNHIP_OK;
     m->stream = as_stream(stream);
+    m->all_cus = stream_has_all_cus(m->stream);
+    SNHIP_CHECK(m->order.follow(m->stream));
     return SNHIP_OK;
 }
 
@@ -1073,8 +1086,7 @@ int32_t snhip_rk_persist_grid_batch(const SnHipRwkv7* m, int32_t B) {
 snhip_status snhip_rk_step_batch_dev(SnHipRwkv7* m, const int32_t* tokens_dev, int32_t B,
                                      float* logits_dev) {
     if (!m || !tokens_dev || !logits_dev || B <= 0 || B > m->max_batch) return SNHIP_E_INVAL;
-    SNHIP_CHECK(hipMemcpyAsync(m->tok, tokens_dev, B * sizeof(int32_t), hipMemcpyDeviceToDevice, m->stream));
-    return run_steps(m, B, logits_dev, false, 1);
+    return run_steps(m, tokens_dev, B, logits_dev, false, 1);
 }
 
 snhip_status snhip_rk_decode_greedy_dev(SnHipRwkv7* m, const int32_t* tokens_dev, int32_t B,
@@ -1083,11 +1095,8 @@ snhip_status snhip_rk_decode_greedy_dev(SnHipRwkv7* m, const int32_t* tokens_dev
     if (!m || !tokens_dev || !out_tokens_dev || B <= 0 || B > m->max_batch || n_steps <= 0)
         return SNHIP_E_INVAL;
     if ((long)n_steps * B > (long)m->hist_cap || !m->tok_hist) {
-        // Grow the token history; graphs bake its address, so drop them.
+        // Grow the token history.
         SNHIP_CHECK(hipStreamSynchronize(m->stream));
-        SNHIP_CHECK(hipStreamSynchronize(m->work));
-        for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
-        m->graphs.clear();
         long cap = 256L * m->max_batch;
         while (cap < (long)n_steps * B) cap *= 2;
         if (cap > (1L << 30)) return SNHIP_E_INVAL;
@@ -1102,9 +1111,8 @@ snhip_status snhip_rk_decode_greedy_dev(SnHipRwkv7* m, const int32_t* tokens_dev
         m->allocs.push_back(hbuf);
         m->hist_cap = (int)cap;
     }
-    SNHIP_CHECK(hipMemcpyAsync(m->tok, tokens_dev, B * sizeof(int32_t), hipMemcpyDeviceToDevice, m->stream));
     SNHIP_CHECK(hipMemsetAsync(m->counter, 0, sizeof(int32_t), m->stream));
-    const snhip_status rc = run_steps(m, B, logits_dev ? logits_dev : m->logits, true, n_steps);
+    const snhip_status rc = run_steps(m, tokens_dev, B, logits_dev ? logits_dev : m->logits, true, n_steps);
     if (rc != SNHIP_OK) return rc;
     SNHIP_CHECK(hipMemcpyAsync(out_tokens_dev, m->tok_hist, (size_t)n_steps * B * sizeof(int32_t),
                                hipMemcpyDeviceToDevice, m->stream));

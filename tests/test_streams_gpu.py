@@ -1,0 +1,85 @@
+"""Persistent steps on the caller's streams: two handles stepped from two threads
+on two streams at once give what each gives alone (their kernels must not share
+the device), and a handle that moves between streams goes on from its state."""
+from __future__ import annotations
+
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+from sunnynet_amd.blob import pack_sunny_blob
+from sunnynet_amd.config import SMALL
+from sunnynet_amd.runtime.model import HipModel
+from sunnynet_amd.runtime.rwkv7 import HipRwkv7
+from sunnynet_amd.rwkv7 import RWKV_TINY, init_rwkv7, pack_rwkv7_blob
+from sunnynet_amd.weights import init_sunnynet
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def paths(tmp_path_factory):
+    d = tmp_path_factory.mktemp("streams")
+    (d / "s.bin").write_bytes(pack_sunny_blob(init_sunnynet(SMALL, 0)))
+    (d / "r.bin").write_bytes(pack_rwkv7_blob(init_rwkv7(RWKV_TINY, 2)))
+    return d / "s.bin", d / "r.bin"
+
+
+def _make(kind, paths):
+    if kind.startswith("rwkv"):
+        return HipRwkv7(paths[1], max_batch=int(kind[4:]))
+    c = SMALL
+    B = {"sunny1": 1, "sunny4": 4, "sunny20": 20}[kind]
+    return HipModel(paths[0], c.vocab_size, c.dim, c.inner, c.rank, c.taps, c.layers, max_batch=B)
+
+
+def _run(h, kind, n, streams):
+    B, V = h.max_batch, h.vocab
+    rng = np.random.default_rng(5)
+    out = []
+    for i in range(n):
+        with torch.cuda.stream(streams[i % len(streams)]):
+            t = torch.from_numpy(rng.integers(0, V, B).astype(np.int32)).cuda()
+            out.append(h.step_batch(t).cpu())
+    return out
+
+
+@pytest.mark.parametrize("a,b", [("sunny1", "rwkv1"), ("sunny4", "sunny20"), ("sunny1", "sunny20")])
+def test_two_threads_two_streams(gpu, paths, a, b):
+    print("two threads, two streams:", a, b, flush=True)
+    n = 24
+    alone = {}
+    for k in (a, b):
+        h = _make(k, paths)
+        alone[k] = _run(h, k, n, [torch.cuda.current_stream()])
+        h.close()
+    got, errs = {}, []
+
+    def work(k):
+        try:
+            h = _make(k, paths)
+            got[k] = _run(h, k, n, [torch.cuda.Stream()])
+            h.close()
+        except Exception as e:      # reported below: a thread's exception is lost
+            errs.append(e)
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in (a, b)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not errs, errs
+    for k in (a, b):
+        assert all(torch.equal(x, y) for x, y in zip(got[k], alone[k])), k
+
+
+@pytest.mark.parametrize("kind", ["sunny1", "sunny4", "rwkv1", "rwkv12"])
+def test_moves_between_streams(gpu, paths, kind):
+    print("steps alternating between two streams:", kind, flush=True)
+    h = _make(kind, paths)
+    ref = _run(h, kind, 6, [torch.cuda.current_stream()])
+    h.reset()
+    got = _run(h, kind, 6, [torch.cuda.Stream(), torch.cuda.current_stream(), torch.cuda.Stream()])
+    assert all(torch.equal(x, y) for x, y in zip(got, ref))
