@@ -298,6 +298,197 @@ void k_recur_scan_buf(const float* __restrict__ a, const float* __restrict__ b,
     }
 }
 
+// Ring form, for few channels: chains of T steps on so few lanes that their
+// latency, not HBM, sets the time. One lane per channel, up to 64 channels (of
+// any rows: flat index b N + n) per workgroup of W waves; wave w owns steps
+// [w TC, (w + 1) TC) of every tile. On the ring's critical path a wave runs
+// only its slot's chain from registers and hands the result on through LDS
+// (value, then sequence word; LDS operations of a wave complete in order, so
+// who sees the word sees the value); it then runs the chain again from the same
+// start and stores, while the next waves are in their slots. Each wave holds
+// two tiles of inputs: tile i + 1 is loaded before tile i is processed. Rows
+// are uniform offsets: a step costs one scalar add. What is left bounds it by the
+// loads a CU keeps in flight (63 per wave): 4 waves of 32 or 64 steps, and 32
+// backward, measure the same as 8 of 32 (16 backward). A whole call on 4096
+// channels of 2048 steps, forward 55 -> 30 us (one workgroup per 64 channels, a
+// barrier per slot before), backward 961 -> 54 us (one lane per channel straight
+// through time before); 2331 channels of 333 steps 19 -> 12 us forward.
+//   SCAN_FMA, SCAN_GATED: x0 = a, x1 = b; y0 = out, end = send (steps forward)
+//   SCAN_BWD: x0 = p, x1 = dout, x2 = nu, x3 = out; y0 = dp, y1 = dnu, end = ds0
+//   SCAN_DS:  x0 = p, x1 = dstate; y0 = ds before each step's decay, end = ds0
+// The last two walk time backwards from 0, in scan_avx2.c:50-99's and
+// core_avx2.c:78-149's order: ds += x1; (outputs); ds *= p.
+enum { SCAN_FMA, SCAN_GATED, SCAN_BWD, SCAN_DS };
+struct RingArgs {
+    const float *x0, *x1, *x2, *x3, *s0;
+    float *y0, *y1, *end;
+    int T, N, N8;      // channels from N8 on take two roundings (forward)
+    int total;         // B N
+    int ch;            // channels of a workgroup (at most 64; the other lanes idle)
+    int yT, yrow, yoff;   // y0: floats per batch row, per step, and before channel 0
+    unsigned bytes, ybytes;
+};
+
+typedef __attribute__((address_space(3))) volatile int lds_word;
+typedef __attribute__((address_space(3))) volatile float lds_val;
+constexpr int kRingPolls = 1 << 26;   // bounded all the same: the waves of a workgroup are resident together
+
+template <int MODE, int TC>
+struct RingBuf {
+    float a[TC], b[TC];
+    float c[MODE == SCAN_BWD ? TC : 1], d[MODE == SCAN_BWD ? TC : 1];
+};
+
+template <int MODE, bool ALLFUSED, int W, int TC>
+__global__ __launch_bounds__(64 * W) void k_scan_ring(const RingArgs A) {
+    constexpr bool BACK = MODE == SCAN_BWD || MODE == SCAN_DS;
+    __shared__ float carry[64];
+    __shared__ int seq;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // consecutive numbers run on one XCD: neighbours share the lines of its L2
+    const int G = (int)gridDim.x, g = (int)blockIdx.x, q8 = G / 8, r8 = G % 8, x8 = g % 8;
+    const int raw = (x8 * q8 + min(x8, r8) + g / 8) * A.ch + lane;
+    const bool valid = lane < A.ch && raw < A.total;
+    // lanes without a channel load a neighbour's and store nothing
+    const int ch = min(min(raw, raw - lane + A.ch - 1), A.total - 1);
+    const int bb = ch / A.N, n = ch - bb * A.N;
+    const int T = A.T, rowb = A.N * 4;
+    const bool fused = ALLFUSED || n < A.N8;
+    auto rsrc = [](const float* p, unsigned bytes) { return make_rsrc(p, bytes); };
+    const __amdgpu_buffer_rsrc_t r0 = rsrc(A.x0, A.bytes), r1 = rsrc(A.x1, A.bytes);
+    const __amdgpu_buffer_rsrc_t r2 = rsrc(MODE == SCAN_BWD ? A.x2 : A.x0, A.bytes);
+    const __amdgpu_buffer_rsrc_t r3 = rsrc(MODE == SCAN_BWD ? A.x3 : A.x0, A.bytes);
+    const __amdgpu_buffer_rsrc_t w0 = rsrc(A.y0, A.ybytes);
+    const __amdgpu_buffer_rsrc_t w1 = rsrc(MODE == SCAN_BWD ? A.y1 : A.y0, A.ybytes);
+    const int vo = (bb * T * A.N + n) * 4;
+    // out of range for lanes without a channel: the store is dropped
+    const int yo = valid ? (bb * A.yT + A.yoff + n) * 4 : 0x7fffffff;
+    const int yrowb = A.yrow * 4;
+    constexpr int TILE = W * TC;
+    const int ntiles = (T + TILE - 1) / TILE;
+    auto ld1 = [](const __amdgpu_buffer_rsrc_t& r, int v, int so) {
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, v, so, 0));
+    };
+    // Step k of this wave's slot of `tile` is time t_of; steps past the end load
+    // a step within it and are not run.
+    auto t_of = [&](int tile, int k) {
+        const int i = tile * TILE + w * TC + k;
+        return BACK ? T - 1 - i : i;
+    };
+    float sz = 0.0f;
+    if (MODE == SCAN_BWD || !BACK) sz = A.s0[ch];
+    auto load = [&](RingBuf<MODE, TC>& X, int tile) {
+#pragma unroll
+        for (int k = 0; k < TC; ++k) {
+            const int t = min(max(t_of(tile, k), 0), T - 1), so = t * rowb;
+            X.a[k] = ld1(r0, vo, so);
+            X.b[k] = ld1(r1, vo, so);
+            if constexpr (MODE == SCAN_BWD) {
+                X.c[k] = ld1(r2, vo, so);
+                X.d[k] = ld1(r3, vo, max(t - 1, 0) * rowb);
+            }
+        }
+    };
+    auto prep = [&](RingBuf<MODE, TC>& X, int tile) {
+        if constexpr (MODE == SCAN_GATED) {
+#pragma unroll
+            for (int k = 0; k < TC; ++k) {
+                X.b[k] = mul_rn(sub_rn(1.0f, X.a[k]), X.b[k]);
+                asm volatile("" : "+v"(X.b[k]));   // here, not after the wait for the carry
+            }
+        } else if constexpr (MODE == SCAN_BWD) {
+#pragma unroll
+            for (int k = 0; k < TC; ++k) {
+                X.c[k] = sub_rn(t_of(tile, k) == 0 ? sz : X.d[k], X.c[k]);   // s_{-1} is s0
+                X.d[k] = sub_rn(1.0f, X.a[k]);
+                asm volatile("" : "+v"(X.c[k]), "+v"(X.d[k]));
+            }
+        } else {
+            // (the chain's inputs are in before the wait)
+#pragma unroll
+            for (int k = 0; k < TC; ++k) asm volatile("" : "+v"(X.a[k]), "+v"(X.b[k]));
+        }
+    };
+    auto step = [&](float s, const RingBuf<MODE, TC>& X, int k) {
+        if constexpr (BACK) return mul_rn(add_rn(X.b[k], s), X.a[k]);
+        else if constexpr (ALLFUSED) return fmaf(X.a[k], s, X.b[k]);
+        else return fused ? fmaf(X.a[k], s, X.b[k]) : add_rn(mul_rn(X.a[k], s), X.b[k]);
+    };
+    auto emit = [&](float s, const RingBuf<MODE, TC>& X, int k, int t) {
+        auto st1 = [&](const __amdgpu_buffer_rsrc_t& r, float v) {
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, yo, t * yrowb, 0);
+        };
+        if constexpr (MODE == SCAN_BWD) {
+            const float ds = add_rn(X.b[k], s);
+            st1(w1, mul_rn(ds, X.d[k]));
+            st1(w0, mul_rn(ds, X.c[k]));
+            return mul_rn(ds, X.a[k]);
+        } else if constexpr (MODE == SCAN_DS) {
+            const float ds = add_rn(X.b[k], s);
+            st1(w0, ds);
+            return mul_rn(ds, X.a[k]);
+        } else {
+            const float o = step(s, X, k);
+            st1(w0, o);
+            return o;
+        }
+    };
+    auto run = [&](RingBuf<MODE, TC>& X, int tile) {
+        prep(X, tile);
+        const int want = tile * W + w, left = T - want * TC;   // steps from this slot's first on
+        float s = 0.0f;
+        for (int i = 0; i < kRingPolls; ++i) {
+            const int q = __builtin_amdgcn_readfirstlane(*(lds_word*)&seq);
+            s = *(lds_val*)&carry[lane];
+            if (q == want) break;
+            if (q + 1 < want) __builtin_amdgcn_s_sleep(1);   // not next: leave the issue slots alone
+        }
+        __builtin_amdgcn_s_setprio(3);   // the chain goes ahead of the SIMD's other wave
+        __builtin_amdgcn_sched_barrier(0);
+        float e = s;
+        if (left >= TC) {
+#pragma unroll
+            for (int k = 0; k < TC; ++k) e = step(e, X, k);
+        } else {
+#pragma unroll
+            for (int k = 0; k < TC; ++k)
+                if (k < left) e = step(e, X, k);
+        }
+        *(lds_val*)&carry[lane] = e;
+        *(lds_word*)&seq = want + 1;
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < TC; ++k)
+            if (k < left) s = emit(s, X, k, t_of(tile, k));
+    };
+    // keeps a tile's loads where they are written, ahead of the tile before it
+    auto issued = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (w == 0) {
+        carry[lane] = BACK ? 0.0f : sz;
+        if (lane == 0) seq = 0;
+    }
+    __syncthreads();
+    RingBuf<MODE, TC> P, Q;
+    load(P, 0);
+    int tile = 0;
+    for (; tile + 2 <= ntiles; tile += 2) {
+        load(Q, tile + 1);
+        issued();
+        run(P, tile);
+        load(P, min(tile + 2, ntiles - 1));
+        issued();
+        run(Q, tile + 1);
+    }
+    if (tile < ntiles) run(P, tile);
+    __syncthreads();
+    if (w == 0 && valid && A.end) A.end[ch] = carry[lane];
+}
+
 template <bool GATED>
 __global__ void k_recur_step(const float* __restrict__ a, const float* __restrict__ b,
                              float* __restrict__ s, long total, int N, int N8) {
@@ -336,6 +527,19 @@ hipError_t launch_cfg(const float* a, const float* b, const float* s0, float* ou
 }
 
 bool aligned(const void* p, size_t n) { return (reinterpret_cast<uintptr_t>(p) % n) == 0; }
+
+// Below this many channels (B N; up to it backward) a scan takes the ring form,
+// and at any number where the layout is not the buffer kernels'. Gated, 2048
+// steps, us, ring / buffer kernels: 4096 channels 30 / 58, 8192 35 / 62, 12288
+// 64 / 66, 16384 86 / 70; backward 4096 54 / 118 (961 in the one-lane kernel),
+// 16384 165 / 230, 32768 269 / 262. 16 rows of 2047 channels, 777 steps: ring 72,
+// one-lane-per-channel tiles 138.
+constexpr long kRingChannels = 16384;
+// Channels of a ring workgroup: half a wave where that still spreads the call over
+// at most one workgroup per CU. 32 / 64 of them, us: 8192 channels backward 90 /
+// 106, forward 35 / 36; 2331 channels of 333 steps backward 13 / 28; but 12288
+// channels forward 73 / 64, backward 143 / 133.
+int ring_ch(long chans) { return chans <= 32 * 256 ? 32 : 64; }
 }  // namespace
 
 template <int CPL, int W, int TC>
@@ -351,9 +555,34 @@ hipError_t launch_buf(const float* a, const float* b, const float* s0, float* ou
     return hipGetLastError();
 }
 
-// Launch-shape selection. SNHIP_SCAN_SHAPE="kind,cpl,w,tc" (kind "buf" or
-// "gen") pins one compiled shape for the tuning sweep and tests; otherwise the
-// buffer kernel when the layout allows it, else the generic kernel.
+// The ring form's 32-bit offsets: every array, with a tile past its end, below
+// 2 GiB.
+bool ring_ok(int B, int T, int N, int row) { return ((long)B * T + 1024) * row * 4 < (1L << 31) && (long)B * N < (1L << 24); }
+
+template <int MODE, int TC>
+hipError_t launch_ring(RingArgs a, int B, hipStream_t st) {
+    constexpr int W = 8;
+    a.total = B * a.N;
+    const unsigned grid = (unsigned)((a.total + a.ch - 1) / a.ch);
+    if (a.N8 == a.N) hipLaunchKernelGGL((k_scan_ring<MODE, true, W, TC>), dim3(grid), dim3(64 * W), 0, st, a);
+    else hipLaunchKernelGGL((k_scan_ring<MODE, false, W, TC>), dim3(grid), dim3(64 * W), 0, st, a);
+    return hipGetLastError();
+}
+
+RingArgs ring_args(const float* x0, const float* x1, const float* s0, float* y0, float* end, int B, int T, int N) {
+    RingArgs a{};
+    a.x0 = x0; a.x1 = x1; a.s0 = s0; a.y0 = y0; a.end = end;
+    a.T = T; a.N = N; a.N8 = N;
+    a.yT = T * N; a.yrow = N;
+    a.bytes = a.ybytes = (unsigned)((size_t)B * T * N * 4);
+    return a;
+}
+
+// Launch-shape selection. SNHIP_SCAN_SHAPE="kind,cpl,w,tc" (kind "buf", "gen" or
+// "ring"; for "ring" w is the channels of a workgroup) pins one compiled shape for
+// the tuning sweep and tests; otherwise the ring form for few channels, the buffer
+// kernel when the layout allows it, else the ring form again; the generic kernel
+// where an array is past the ring's 32-bit offsets.
 snhip_status launch_recur_scan(const float* a, const float* b, const float* s0,
                                float* out, float* send, int B, int T, int N,
                                int gated, hipStream_t st) {
@@ -369,19 +598,27 @@ snhip_status launch_recur_scan(const float* a, const float* b, const float* s0,
     char kind = 'g';
     int cpl = 1, w = 8, tc = 16;
     if (N % 2 == 0 && al8 && chans / 128 >= 192) cpl = 2;
-    if (buf_ok(2, 2 * 32) && chans / 128 >= 128) { kind = 'b'; cpl = 2; w = 2; tc = 32; }
+    if (buf_ok(2, 2 * 32) && chans / 128 >= 192) { kind = 'b'; cpl = 2; w = 2; tc = 32; }
     else if (buf_ok(1, 4 * 32)) { kind = 'b'; cpl = 1; w = 4; tc = 32; }
+    if ((chans < kRingChannels || kind == 'g') && ring_ok(B, T, N, N)) { kind = 'r'; cpl = 1; w = ring_ch(chans); tc = 32; }
     if (const char* env = getenv("SNHIP_SCAN_SHAPE")) {
         char k[8] = {0};
         int c = 0, ww = 0, t = 0;
-        if (sscanf(env, "%3[a-z],%d,%d,%d", k, &c, &ww, &t) == 4) {
+        if (sscanf(env, "%7[a-z],%d,%d,%d", k, &c, &ww, &t) == 4) {
             kind = k[0]; cpl = c; w = ww; tc = t;
         }
         if (kind == 'b' && !buf_ok(cpl, w * tc)) return SNHIP_E_INVAL;
+        if (kind == 'r' && !ring_ok(B, T, N, N)) return SNHIP_E_INVAL;
         if (kind == 'g' && ((cpl == 2 && (N % 2 || !al8)) || (cpl == 4 && (N % 4 || !al16))))
             return SNHIP_E_INVAL;
     }
     hipError_t e = hipErrorInvalidValue;
+    if (kind == 'r' && cpl == 1 && w >= 1 && w <= 64 && tc == 32) {
+        RingArgs r = ring_args(a, b, s0, out, send, B, T, N);
+        r.N8 = N & ~7;
+        r.ch = w;
+        e = gated ? launch_ring<SCAN_GATED, 32>(r, B, st) : launch_ring<SCAN_FMA, 32>(r, B, st);
+    } else
 #define SNHIP_GEN_CASE(C, WW, TT)                                                   \
     if (kind == 'g' && cpl == C && w == WW && tc == TT)                             \
         e = launch_cfg<C, WW, TT>(a, b, s0, out, send, B, T, N, gated, st);         \
@@ -571,9 +808,17 @@ snhip_status launch_scan_bwd(const float* p, const float* nu, const float* s0, c
     const bool al8 = aligned(p, 8) && aligned(nu, 8) && aligned(s0, 8) && aligned(out, 8) &&
                      aligned(dout, 8) && aligned(dp, 8) && aligned(dnu, 8) && aligned(ds0, 8);
     constexpr int C = 2, WW = 2, TT = 16;
-    const bool buf = N % (64 * C) == 0 && al8 && (long)T * N * 4 < (1L << 31) &&
-                     (long)B * N / 128 >= 128;
-    if (buf) {
+    const bool buf = N % (64 * C) == 0 && al8 && (long)T * N * 4 < (1L << 31);
+    if (((long)B * N <= kRingChannels || !buf) && ring_ok(B, T, N, N)) {
+        RingArgs r = ring_args(p, dout, s0, dp, ds0, B, T, N);
+        r.x2 = nu; r.x3 = out; r.y1 = dnu;
+        r.ch = ring_ch((long)B * N);
+        const hipError_t e = launch_ring<SCAN_BWD, 16>(r, B, st);
+        if (e != hipSuccess) {
+            set_last_error(std::string("scan_bwd launch: ") + hipGetErrorString(e));
+            return SNHIP_E_DEVICE;
+        }
+    } else if (buf) {
         const unsigned grid = (unsigned)((long)B * N / (64 * C));
         hipLaunchKernelGGL((k_scan_bwd_buf<C, WW, TT>), dim3(grid), dim3(64 * WW), 0, st, p, nu, s0, out,
                            dout, dp, dnu, ds0, T, N);
