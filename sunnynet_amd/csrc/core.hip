@@ -28,8 +28,15 @@
 // tiles of inputs in registers: the loads for tile i+1 are issued before
 // tile i is processed, a whole tile period ahead of their use. The fast path
 // needs D % 128 == 0 and T % (W TC) == 0 (the reference's block pads T to its
-// scan chunk before it calls the kernel); any other shape takes a one lane per
-// channel kernel.
+// scan chunk before it calls the kernel). Any other shape, and few channels, take
+// the split form: the heavy part as an elementwise kernel over all steps at once
+// (after the chain in the backward), the chain as a ring scan over u and p
+// (forward) or over p and dstate (backward, ds passing through dq). It moves
+// 28 B forward and 48 B backward per channel and step where the fused kernels
+// move 20 and 36, but neither part waits for the other's latency: on 8192
+// channels of 2048 steps the fused kernels' 64 workgroups leave three CUs in four
+// idle. Arrays past the ring's 32-bit offsets and outputs that overlap inputs take
+// a one lane per channel kernel.
 #include <mutex>
 #include <string>
 
@@ -424,13 +431,200 @@ __global__ void k_core_bwd_gen(const float* __restrict__ q, const float* __restr
     dacc_out[i] = dacc;
 }
 
-// ddelta[d] += sum over rows b of dacc[b, d], rows in order.
-__global__ void k_core_ddelta(const float* __restrict__ dacc, float* __restrict__ ddelta, int B, int D) {
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    if (d >= D) return;
+// ---- the split form: the gates element by element over the whole chip, the
+// chain as a ring scan (scan.hip). A lane owns 4 channels (a group is a lane
+// pair) over the L steps of one chunk of time; lanes run over channels, then
+// chunks, then rows. VEC: 16-byte accesses, else one float at a time (arrays
+// that are not 16-byte aligned). Bound by HBM (8 steps of a lane give 8192
+// wavefronts at 8192 channels of 2048 steps, R steps' loads in flight in each).
+template <bool VEC>
+__device__ __forceinline__ void ld4(float (&v)[4], const float* p) {
+    if constexpr (VEC) {
+        const float4 x = *reinterpret_cast<const float4*>(p);
+        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = p[c];
+    }
+}
+template <bool VEC>
+__device__ __forceinline__ void st4(float* p, const float (&v)[4]) {
+    if constexpr (VEC) {
+        *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) p[c] = v[c];
+    }
+}
+// The other lane of the pair (DPP quad_perm 1,0,3,2).
+__device__ __forceinline__ float pair_swap(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, false));
+}
+struct Gate4 {
+    float sig[4], s1[4], s2[4];
+};
+__device__ __forceinline__ Gate4 gate4_of(const float (&g)[4]) {
+    Gate4 r;
+    float e[6];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) e[c] = expf(sub_rn(0.0f, g[c]));
+    e[4] = pair_swap(e[0]);
+    e[5] = pair_swap(e[1]);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        r.sig[c] = div_rn(1.0f, add_rn(1.0f, e[c]));
+        r.s1[c] = div_rn(1.0f, add_rn(1.0f, div_rn(e[c], e[c + 1])));
+        r.s2[c] = div_rn(1.0f, add_rn(1.0f, div_rn(e[c], e[c + 2])));
+    }
+    return r;
+}
+// Row, first step and channel of a lane; false past the end (pairs are in or out
+// together: D / 4 is even).
+struct GateAt {
+    int b, chunk, d;
+};
+__device__ __forceinline__ bool gate_at(GateAt& a, int B, int D, int nch) {
+    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x, D4 = (unsigned)D / 4;
+    const unsigned r = i / D4;
+    a.d = (int)(i - r * D4) * 4;
+    a.b = (int)(r / (unsigned)nch);
+    a.chunk = (int)(r - (unsigned)a.b * (unsigned)nch);
+    return a.b < B;
+}
+
+// u and p of L steps.
+template <bool VEC>
+__global__ __launch_bounds__(256)
+void k_core_gate(const float* __restrict__ q, const float* __restrict__ delta, float* __restrict__ uo,
+                 float* __restrict__ po, int B, int T, int D, int L, int nch) {
+    GateAt at;
+    if (!gate_at(at, B, D, nch)) return;
+    float dl[4], base[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        dl[c] = delta[at.d + c];
+        base[c] = sub_rn(1.0f, dl[c]);
+    }
+    const size_t row = (size_t)at.b * T;
+    const int t0 = at.chunk * L, t1 = min(t0 + L, T);
+    constexpr int R = 4;
+    for (int tb = t0; tb < t1; tb += R) {
+        float ur[R][4], g[R][4];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const float* x = q + (row + min(tb + k, T - 1)) * 2 * D + at.d;
+            ld4<VEC>(ur[k], x);
+            ld4<VEC>(g[k], x + D);
+        }
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const Gate4 G = gate4_of(g[k]);
+            float u[4], p[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                u[c] = mul_rn(ur[k][c], mul_rn(G.s1[c], G.s2[c]));
+                p[c] = fmaf(dl[c], G.sig[c], base[c]);
+            }
+            if (tb + k < t1) {
+                const size_t o = (row + tb + k) * D + at.d;
+                st4<VEC>(uo + o, u);
+                st4<VEC>(po + o, p);
+            }
+        }
+    }
+}
+
+// dq of L steps, whose gate half holds ds (before the step's decay) on entry; the
+// steps' ddelta terms, summed backwards in time, go to dacc[(b nch + chunk) D + d].
+template <bool VEC>
+__global__ __launch_bounds__(256)
+void k_core_gate_bwd(const float* __restrict__ q, const float* __restrict__ delta, const float* __restrict__ s0,
+                     const float* __restrict__ states, const float* __restrict__ uo,
+                     const float* __restrict__ po, const float* __restrict__ du_in, float* __restrict__ dq,
+                     float* __restrict__ dacc, int B, int T, int D, int L, int nch) {
+    GateAt at;
+    if (!gate_at(at, B, D, nch)) return;
+    float dl[4], acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) dl[c] = delta[at.d + c];
+    const size_t row = (size_t)at.b * T;
+    const int t0 = at.chunk * L, t1 = min(t0 + L, T);
+    constexpr int R = 2;
+    for (int tb = t1 - 1; tb >= t0; tb -= R) {
+        float ur[R][4], g[R][4], ds[R][4], u[R][4], p[R][4], sp[R][4], di[R][4];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int t = max(tb - k, t0);
+            const size_t o = (row + t) * D + at.d, oq = (row + t) * 2 * D + at.d;
+            ld4<VEC>(ds[k], dq + oq + D);
+            ld4<VEC>(ur[k], q + oq);
+            ld4<VEC>(g[k], q + oq + D);
+            ld4<VEC>(u[k], uo + o);
+            ld4<VEC>(p[k], po + o);
+            if (t > 0) ld4<VEC>(sp[k], states + o - D);
+            else
+#pragma unroll
+                for (int c = 0; c < 4; ++c) sp[k][c] = s0[(size_t)at.b * D + at.d + c];   // s_{-1}
+            ld4<VEC>(di[k], du_in + o);
+        }
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const Gate4 G = gate4_of(g[k]);
+            float dur[4], a1[4], a2[4], dp[4], dg[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                dp[c] = mul_rn(ds[k][c], sub_rn(sp[k][c], u[k][c]));
+                const float du = fmaf(ds[k][c], sub_rn(1.0f, p[k][c]), di[k][c]);
+                dur[c] = mul_rn(du, mul_rn(G.s1[c], G.s2[c]));
+                const float dw = mul_rn(du, ur[k][c]);
+                a1[c] = mul_rn(mul_rn(dw, G.s2[c]), mul_rn(G.s1[c], sub_rn(1.0f, G.s1[c])));
+                a2[c] = mul_rn(mul_rn(dw, G.s1[c]), mul_rn(G.s2[c], sub_rn(1.0f, G.s2[c])));
+            }
+            // a1[i - 1] and a2[i - 2] around the group
+            const float m1[4] = {pair_swap(a1[3]), a1[0], a1[1], a1[2]};
+            const float m2[4] = {pair_swap(a2[2]), pair_swap(a2[3]), a2[0], a2[1]};
+            const bool in = tb - k >= t0;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float v = sub_rn(sub_rn(add_rn(a1[c], a2[c]), m1[c]), m2[c]);
+                dg[c] = fmaf(mul_rn(dp[c], dl[c]), mul_rn(G.sig[c], sub_rn(1.0f, G.sig[c])), v);
+                if (in) acc[c] = fmaf(dp[c], sub_rn(G.sig[c], 1.0f), acc[c]);
+            }
+            if (in) {
+                const size_t oq = (row + tb - k) * 2 * D + at.d;
+                st4<VEC>(dq + oq, dur);
+                st4<VEC>(dq + oq + D, dg);
+            }
+        }
+    }
+    float* o = dacc + ((size_t)at.b * nch + at.chunk) * D + at.d;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o[c] = acc[c];
+}
+
+// ddelta[d] += sum over the n partial rows of dacc[r, d]: kDdSlots running sums of
+// every kDdSlots-th row in order, then those in order (n <= kDdSlots: the rows in
+// order).
+constexpr int kDdSlots = 64, kDdChans = 16;
+__global__ __launch_bounds__(kDdSlots * kDdChans)
+void k_core_ddelta(const float* __restrict__ dacc, float* __restrict__ ddelta, int n, int D) {
+    __shared__ float part[kDdSlots][kDdChans];
+    const int c = threadIdx.x % kDdChans, j = threadIdx.x / kDdChans;
+    const int d = blockIdx.x * kDdChans + c;
     float r = 0.0f;
-    for (int b = 0; b < B; ++b) r = add_rn(r, dacc[(size_t)b * D + d]);
-    ddelta[d] = add_rn(ddelta[d], r);
+    if (d < D) {
+#pragma unroll 4
+        for (int i = j; i < n; i += kDdSlots) r = add_rn(r, dacc[(size_t)i * D + d]);
+    }
+    part[j][c] = r;
+    __syncthreads();
+    if (j == 0 && d < D) {
+        r = 0.0f;
+#pragma unroll 8
+        for (int i = 0; i < kDdSlots; ++i)
+            if (i < n) r = add_rn(r, part[i][c]);
+        ddelta[d] = add_rn(ddelta[d], r);
+    }
 }
 
 // Ring shapes (waves per workgroup, steps per slot), from a sweep on the
@@ -453,11 +647,71 @@ bool fast_ok(int B, int T, int D, int tile, std::initializer_list<const void*> p
     return true;
 }
 
+
+// The split form is taken by calls whose shape or alignment the fused kernels do
+// not run, and by long ones with few channels (B D). Split / fused, us, forward
+// and backward, at 2048 steps: 1024 channels 45 / 163 and 58 / 339, 8192 104 / 170
+// and 179 / 343, 12288 148 / 179 and 269 / 346, 16384 188 / 182 and 350 / 345,
+// 32768 366 / 227 and 671 / 417 (the fused kernels read and write each array once);
+// at 8192 channels of 128 steps 14.6 / 14.3 and 32 / 36 (launches), of 256 18 / 24
+// and 34 / 56. Against one lane per channel, 600 channels of 777 steps: 319 -> 24
+// and 450 -> 42.
+bool split_pays(bool fused, int B, int T, int D) {
+    return !fused || ((long)B * D < 16384 && T >= 256);
+}
+
+bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+struct Span {
+    const float* p;
+    size_t n;
+};
+// No output of the call overlaps one of its inputs (the fused kernels read each
+// element before they write the same place, the split form does not).
+bool apart(std::initializer_list<Span> out, std::initializer_list<Span> in) {
+    for (const Span& o : out)
+        for (const Span& i : in)
+            if (o.p != i.p ? (o.p < i.p ? o.p + o.n > i.p : i.p + i.n > o.p) : true) return false;
+    return true;
+}
+
+// The split kernels' grid: 4-channel lanes over `nch` chunks of every row.
+bool split_grid(int B, int D, int nch, unsigned* grid) {
+    const size_t lanes = (size_t)B * nch * (D / 4);
+    *grid = (unsigned)((lanes + 255) / 256);
+    return lanes < (1ull << 31);
+}
+constexpr int kGateSteps = 8;   // steps of a lane of k_core_gate
+
+// Floats the backward's ddelta partials may take, and what a call takes: a row per
+// chunk of time and batch row.
+constexpr size_t kCoreBwdScratchFloats = (size_t)1 << 20;
+int bwd_chunks(int B, int T, int D) {
+    const size_t rows = kCoreBwdScratchFloats / ((size_t)B * D);
+    const int want = (T + kGateSteps - 1) / kGateSteps;
+    return rows < 1 ? 1 : rows < (size_t)want ? (int)rows : want;
+}
 }  // namespace
 
 snhip_status launch_core_fwd(const float* q, const float* delta, const float* s0, float* states,
                              float* uo, float* po, int B, int T, int D, hipStream_t st) {
-    if (fast_ok(B, T, D, kFW * kFTC, {q, states, uo, po})) {
+    const bool fused = fast_ok(B, T, D, kFW * kFTC, {q, states, uo, po});
+    const size_t n = (size_t)B * T * D, c = (size_t)B * D;
+    const int nch = (T + kGateSteps - 1) / kGateSteps;
+    unsigned grid = 0;
+    if (split_pays(fused, B, T, D) && ring_scan_ok(B, T, D, D) && split_grid(B, D, nch, &grid) &&
+        apart({{uo, n}, {po, n}, {states, n}}, {{q, 2 * n}, {delta, (size_t)D}, {s0, c}}) &&
+        apart({{uo, n}}, {{po, n}}) && apart({{states, n}}, {{po, n}, {uo, n}})) {
+        if (al16(q) && al16(uo) && al16(po))
+            hipLaunchKernelGGL((k_core_gate<true>), dim3(grid), dim3(256), 0, st, q, delta, uo, po, B, T, D,
+                               kGateSteps, nch);
+        else
+            hipLaunchKernelGGL((k_core_gate<false>), dim3(grid), dim3(256), 0, st, q, delta, uo, po, B, T, D,
+                               kGateSteps, nch);
+        SNHIP_CHECK(hipGetLastError());
+        return launch_ring_gated(po, uo, s0, states, B, T, D, st);
+    }
+    if (fused) {
         const unsigned grid = (unsigned)((long)B * D / 128);
         hipLaunchKernelGGL((k_core_fwd_buf<kFW, kFTC>), dim3(grid), dim3(64 * kFW), 0, st, q, delta, s0,
                            states, uo, po, T, D);
@@ -471,13 +725,32 @@ snhip_status launch_core_fwd(const float* q, const float* delta, const float* s0
 }
 
 namespace {
-// Backward kernels plus the in-order row reduction of ddelta, with the (B, D)
-// per-row partials in `acc` (every element is written before it is read).
+// Backward kernels plus the in-order reduction of ddelta, with the partials in
+// `acc` (bwd_chunks(B, T, D) B D floats; every element read is written before).
 snhip_status core_bwd_ws(const float* q, const float* delta, const float* s0, const float* states,
                          const float* uo, const float* po, const float* dstate, const float* du_in,
                          float* dq, float* ddelta, float* ds0, int B, int T, int D, float* acc,
                          hipStream_t st) {
-    if (fast_ok(B, T, D, kBW * kBTC, {q, states, uo, po, dstate, du_in, dq})) {
+    const bool fused = fast_ok(B, T, D, kBW * kBTC, {q, states, uo, po, dstate, du_in, dq});
+    const size_t n = (size_t)B * T * D, c = (size_t)B * D;
+    int parts = B;
+    const int nch = bwd_chunks(B, T, D);
+    unsigned grid = 0;
+    if (split_pays(fused, B, T, D) && ring_scan_ok(B, T, D, 2 * D) && split_grid(B, D, nch, &grid) &&
+        apart({{dq, 2 * n}, {ds0, c}}, {{q, 2 * n}, {delta, (size_t)D}, {s0, c}, {states, n}, {uo, n}, {po, n},
+                                        {dstate, n}, {du_in, n}}) &&
+        apart({{dq, 2 * n}}, {{ds0, c}})) {
+        const int L = (T + nch - 1) / nch;
+        const snhip_status rc = launch_ring_ds(po, dstate, dq + D, 2 * D, ds0, B, T, D, st);
+        if (rc != SNHIP_OK) return rc;
+        if (al16(q) && al16(states) && al16(uo) && al16(po) && al16(du_in) && al16(dq))
+            hipLaunchKernelGGL((k_core_gate_bwd<true>), dim3(grid), dim3(256), 0, st, q, delta, s0, states, uo,
+                               po, du_in, dq, acc, B, T, D, L, nch);
+        else
+            hipLaunchKernelGGL((k_core_gate_bwd<false>), dim3(grid), dim3(256), 0, st, q, delta, s0, states, uo,
+                               po, du_in, dq, acc, B, T, D, L, nch);
+        parts = B * nch;
+    } else if (fused) {
         const unsigned grid = (unsigned)((long)B * D / 128);
         hipLaunchKernelGGL((k_core_bwd_buf<kBW, kBTC>), dim3(grid), dim3(64 * kBW), 0, st, q, delta, s0,
                            states, uo, po, dstate, du_in, dq, acc, ds0, T, D);
@@ -487,16 +760,16 @@ snhip_status core_bwd_ws(const float* q, const float* delta, const float* s0, co
                            s0, states, uo, po, dstate, du_in, dq, acc, ds0, B, T, D);
     }
     SNHIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_core_ddelta, dim3((unsigned)((D + 255) / 256)), dim3(256), 0, st, acc, ddelta, B, D);
+    hipLaunchKernelGGL(k_core_ddelta, dim3((unsigned)((D + kDdChans - 1) / kDdChans)), dim3(kDdSlots * kDdChans),
+                       0, st, acc, ddelta, parts, D);
     SNHIP_CHECK(hipGetLastError());
     return SNHIP_OK;
 }
 
-// Scratch of the allocation-free backward: the (B, D) ddelta partials of
-// calls with B * D <= kCoreBwdScratchFloats (4 MiB per GPU, held for the life
-// of the process). Host code uses the per-device address from
-// hipGetSymbolAddress, never the array's name.
-constexpr size_t kCoreBwdScratchFloats = (size_t)1 << 20;
+// Scratch of the allocation-free backward: the ddelta partials of calls with
+// B * D <= kCoreBwdScratchFloats (4 MiB per GPU, held for the life of the
+// process). Host code uses the per-device address from hipGetSymbolAddress,
+// never the array's name.
 static __device__ __align__(256) float scratch[kCoreBwdScratchFloats];
 
 constexpr int kMaxDevices = 64;
@@ -525,9 +798,10 @@ snhip_status scratch_ptr(float** out) {
 snhip_status launch_core_bwd(const float* q, const float* delta, const float* s0, const float* states,
                              const float* uo, const float* po, const float* dstate, const float* du_in,
                              float* dq, float* ddelta, float* ds0, int B, int T, int D, hipStream_t st) {
-    // Per-row sums of ddelta's terms, reduced over rows in order afterwards.
+    // Partial sums of ddelta's terms, reduced in order afterwards.
     float* acc = nullptr;
-    SNHIP_CHECK(hipMallocAsync(reinterpret_cast<void**>(&acc), (size_t)B * D * sizeof(float), st));
+    SNHIP_CHECK(hipMallocAsync(reinterpret_cast<void**>(&acc),
+                               (size_t)bwd_chunks(B, T, D) * B * D * sizeof(float), st));
     const snhip_status rc = core_bwd_ws(q, delta, s0, states, uo, po, dstate, du_in, dq, ddelta, ds0,
                                         B, T, D, acc, st);
     const hipError_t f = hipFreeAsync(acc, st);

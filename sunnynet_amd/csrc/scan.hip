@@ -325,7 +325,7 @@ struct RingArgs {
     int T, N, N8;      // channels from N8 on take two roundings (forward)
     int total;         // B N
     int ch;            // channels of a workgroup (at most 64; the other lanes idle)
-    int yT, yrow, yoff;   // y0: floats per batch row, per step, and before channel 0
+    int yT, yrow;      // y0: floats per batch row and per step
     unsigned bytes, ybytes;
 };
 
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(64 * W) void k_scan_ring(const RingArgs A) {
     const __amdgpu_buffer_rsrc_t w1 = rsrc(MODE == SCAN_BWD ? A.y1 : A.y0, A.ybytes);
     const int vo = (bb * T * A.N + n) * 4;
     // out of range for lanes without a channel: the store is dropped
-    const int yo = valid ? (bb * A.yT + A.yoff + n) * 4 : 0x7fffffff;
+    const int yo = valid ? (bb * A.yT + n) * 4 : 0x7fffffff;
     const int yrowb = A.yrow * 4;
     constexpr int TILE = W * TC;
     const int ntiles = (T + TILE - 1) / TILE;
@@ -557,7 +557,9 @@ hipError_t launch_buf(const float* a, const float* b, const float* s0, float* ou
 
 // The ring form's 32-bit offsets: every array, with a tile past its end, below
 // 2 GiB.
-bool ring_ok(int B, int T, int N, int row) { return ((long)B * T + 1024) * row * 4 < (1L << 31) && (long)B * N < (1L << 24); }
+bool ring_scan_ok(int B, int T, int N, int row) {
+    return ((long)B * T + 1024) * row * 4 < (1L << 31) && (long)B * N < (1L << 24);
+}
 
 template <int MODE, int TC>
 hipError_t launch_ring(RingArgs a, int B, hipStream_t st) {
@@ -576,6 +578,25 @@ RingArgs ring_args(const float* x0, const float* x1, const float* s0, float* y0,
     a.yT = T * N; a.yrow = N;
     a.bytes = a.ybytes = (unsigned)((size_t)B * T * N * 4);
     return a;
+}
+
+snhip_status launch_ring_gated(const float* p, const float* u, const float* s0, float* states, int B, int T,
+                               int N, hipStream_t st) {
+    RingArgs r = ring_args(p, u, s0, states, nullptr, B, T, N);
+    r.ch = ring_ch((long)B * N);
+    SNHIP_CHECK((launch_ring<SCAN_GATED, 32>(r, B, st)));
+    return SNHIP_OK;
+}
+
+snhip_status launch_ring_ds(const float* p, const float* dstate, float* out, int row, float* ds0, int B, int T,
+                            int N, hipStream_t st) {
+    RingArgs r = ring_args(p, dstate, nullptr, out, ds0, B, T, N);
+    r.ch = ring_ch((long)B * N);
+    r.yT = T * row;
+    r.yrow = row;
+    r.ybytes = (unsigned)(((size_t)B * T * row - (row - N)) * 4);   // `out` starts within its first row
+    SNHIP_CHECK((launch_ring<SCAN_DS, 32>(r, B, st)));
+    return SNHIP_OK;
 }
 
 // Launch-shape selection. SNHIP_SCAN_SHAPE="kind,cpl,w,tc" (kind "buf", "gen" or
@@ -600,7 +621,7 @@ snhip_status launch_recur_scan(const float* a, const float* b, const float* s0,
     if (N % 2 == 0 && al8 && chans / 128 >= 192) cpl = 2;
     if (buf_ok(2, 2 * 32) && chans / 128 >= 192) { kind = 'b'; cpl = 2; w = 2; tc = 32; }
     else if (buf_ok(1, 4 * 32)) { kind = 'b'; cpl = 1; w = 4; tc = 32; }
-    if ((chans < kRingChannels || kind == 'g') && ring_ok(B, T, N, N)) { kind = 'r'; cpl = 1; w = ring_ch(chans); tc = 32; }
+    if ((chans < kRingChannels || kind == 'g') && ring_scan_ok(B, T, N, N)) { kind = 'r'; cpl = 1; w = ring_ch(chans); tc = 32; }
     if (const char* env = getenv("SNHIP_SCAN_SHAPE")) {
         char k[8] = {0};
         int c = 0, ww = 0, t = 0;
@@ -608,7 +629,7 @@ snhip_status launch_recur_scan(const float* a, const float* b, const float* s0,
             kind = k[0]; cpl = c; w = ww; tc = t;
         }
         if (kind == 'b' && !buf_ok(cpl, w * tc)) return SNHIP_E_INVAL;
-        if (kind == 'r' && !ring_ok(B, T, N, N)) return SNHIP_E_INVAL;
+        if (kind == 'r' && !ring_scan_ok(B, T, N, N)) return SNHIP_E_INVAL;
         if (kind == 'g' && ((cpl == 2 && (N % 2 || !al8)) || (cpl == 4 && (N % 4 || !al16))))
             return SNHIP_E_INVAL;
     }
@@ -809,7 +830,7 @@ snhip_status launch_scan_bwd(const float* p, const float* nu, const float* s0, c
                      aligned(dout, 8) && aligned(dp, 8) && aligned(dnu, 8) && aligned(ds0, 8);
     constexpr int C = 2, WW = 2, TT = 16;
     const bool buf = N % (64 * C) == 0 && al8 && (long)T * N * 4 < (1L << 31);
-    if (((long)B * N <= kRingChannels || !buf) && ring_ok(B, T, N, N)) {
+    if (((long)B * N <= kRingChannels || !buf) && ring_scan_ok(B, T, N, N)) {
         RingArgs r = ring_args(p, dout, s0, dp, ds0, B, T, N);
         r.x2 = nu; r.x3 = out; r.y1 = dnu;
         r.ch = ring_ch((long)B * N);
