@@ -131,12 +131,15 @@ snhip_status launch_core_bwd_noalloc(const float* q, const float* delta, const f
                                      const float* dstate, const float* du_in, float* dq, float* ddelta,
                                      float* ds0, int B, int T, int D, hipStream_t st);
 // The ring form of the recurrence (scan.hip) for arrays of `row` floats per step:
-// whether its 32-bit offsets reach; states of the gated form; and, walking time
-// backwards from 0, ds += dstate, out = ds, ds *= p, with out's steps `row` apart
+// whether its 32-bit offsets reach; states of the gated form; states and the last
+// one of s = p s + b with two roundings, s0's batch rows s0_stride apart; and,
+// walking time backwards from 0, ds += dstate, out = ds, ds *= p, with out's steps `row` apart
 // and ds after the first step in ds0.
 bool ring_scan_ok(int B, int T, int N, int row);
 snhip_status launch_ring_gated(const float* p, const float* u, const float* s0, float* states, int B, int T,
                                int N, hipStream_t st);
+snhip_status launch_ring_rows(const float* p, const float* b, const float* s0, size_t s0_stride, float* states,
+                              float* end, int B, int T, int N, hipStream_t st);
 snhip_status launch_ring_ds(const float* p, const float* dstate, float* out, int row, float* ds0, int B, int T,
                             int N, hipStream_t st);
 snhip_status launch_recur_scan(const float* a, const float* b, const float* s0,

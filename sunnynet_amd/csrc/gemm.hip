@@ -17,6 +17,7 @@
 // fixed order by a second kernel, so results are deterministic. Products with
 // at most 64 rows of X (batched decode) take the skinny path below instead.
 #include "gemm.h"
+#include "gemmepi.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -26,30 +27,6 @@ namespace {
 
 constexpr int BM = 64, BN = 64, BK = 32, LDSK = BK + 4;
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ const float* xrow(const GemmArgs& g, int m) {
-    if (g.shift_T > 0) {
-        const int t = m % g.shift_T;
-        return t == 0 ? g.X0 + (long)(m / g.shift_T) * g.ldx0 : g.X + (long)(m - 1) * g.ldx;
-    }
-    return g.X + (long)m * g.ldx;
-}
-
-__device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int m, int n, float acc) {
-    float* y = g.Y + (long)m * g.ldy + n;
-    if (g.epi == GEPI_STORE) {
-        *y = acc;
-    } else if (g.epi == GEPI_WEDGE) {
-        *y = acc * (1.0f + 0.5f * g.a_tanh / (1.0f + fabsf(acc)));       // sunnynet.c:270-271
-    } else if (g.epi == GEPI_RESID) {
-        *y = acc + (g.b_gain * g.s[(long)m * g.lds + n] + g.sfb[(long)m * g.ldf + n] + *y);  // :276
-    } else if (g.epi == GEPI_ADD) {
-        *y = *y + acc;                                                    // rwkv7.c:300,314
-    } else {
-        const float t = acc > 0.0f ? acc : 0.0f;                          // rwkv7.c:308-312
-        *y = t * t;
-    }
-}
 
 template <int BLK>
 __global__ __launch_bounds__(256) void k_gemm(GemmArgs g, int kchunk, float* __restrict__ part) {
@@ -71,7 +48,7 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g, int kchunk, float* __r
             const int row = (tid >> 3) + 32 * pass, c4 = tid & 7;
             const int m = m0 + row;
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (m < g.M) v = *reinterpret_cast<const float4*>(xrow(g, m) + kt + 4 * c4);
+            if (m < g.M) v = *reinterpret_cast<const float4*>(gemm_xrow(g, m) + kt + 4 * c4);
             *reinterpret_cast<float4*>(As + row * LDSK + 4 * c4) = v;
         }
         if constexpr (BLK == 0) {
@@ -555,6 +532,13 @@ __global__ __launch_bounds__(256) void k_gemm_sk(SkJobs J) {
 
 }  // namespace
 
+snhip_status launch_gemm_reduce(const GemmArgs& g, int splits, const float* part, hipStream_t st) {
+    const long MN = (long)g.M * g.N;
+    hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, st, g, splits, part);
+    SNHIP_CHECK(hipGetLastError());
+    return SNHIP_OK;
+}
+
 snhip_status launch_gemm(const GemmArgs& g, float* work, size_t work_floats, hipStream_t st) {
     if (g.M <= 0 || g.N <= 0 || g.K <= 0 || g.K % BK) {
         set_last_error("gemm: K must be a positive multiple of 32");
@@ -586,13 +570,7 @@ snhip_status launch_gemm(const GemmArgs& g, float* work, size_t work_floats, hip
     else
         hipLaunchKernelGGL(k_gemm<64>, grid, dim3(256), 0, st, g, kchunk, part);
     SNHIP_CHECK(hipGetLastError());
-    if (part) {
-        const long MN = (long)g.M * g.N;
-        hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, st, g,
-                           splits, part);
-        SNHIP_CHECK(hipGetLastError());
-    }
-    return SNHIP_OK;
+    return part ? launch_gemm_reduce(g, splits, part, st) : SNHIP_OK;
 }
 
 namespace {

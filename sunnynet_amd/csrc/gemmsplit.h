@@ -1,0 +1,36 @@
+// Products of many rows on the fp16 matrix cores at fp32 accuracy (gemmsplit.hip).
+//
+// A row x of K floats is held as 2^s x = h + l in two fp16 planes, s the power of
+// two that takes the row's largest magnitude into [2^14, 2^15): h rounds 2^s x to
+// 11 bits, l the exact remainder to 11 more, so h + l differs from 2^s x by at most
+// 2^-22 of it or 2^-25. A product is X W^T = 2^-(sx + sw) (Hx Hw + Hx Lw + Lx Hw),
+// accumulated in fp32; Lx Lw, below 2^-22 of a term, is left out.
+#pragma once
+
+#include <climits>
+
+#include "gemm.h"
+
+namespace snhip {
+
+constexpr int kSplitTile = 256;          // rows of planes are padded to this
+constexpr int kSplitNonFinite = INT_MIN; // `ex` of a row with an infinity or NaN
+
+// Planes of a matrix of rows: `pl` in fragment order (split_halfs(rows, K)
+// uint16), `ex` the rows' s (rows padded to kSplitTile).
+struct SplitMat {
+    uint16_t* pl = nullptr;
+    int* ex = nullptr;
+};
+inline size_t split_rows(size_t rows) { return (rows + kSplitTile - 1) / kSplitTile * kSplitTile; }
+inline size_t split_halfs(size_t rows, size_t K) { return split_rows(rows) * K * 2; }
+
+// Planes of g's X rows (g.M, with its shifted reads), or of its weights (g.N rows).
+snhip_status launch_split_x(const GemmArgs& g, SplitMat out, hipStream_t st);
+snhip_status launch_split_w(const GemmArgs& g, SplitMat out, hipStream_t st);
+// Y = X W^T with g's epilogue from the planes of both. `work` is scratch for
+// split-K partials as launch_gemm's.
+snhip_status launch_gemm_split(const GemmArgs& g, SplitMat x, SplitMat w, float* work, size_t work_floats,
+                               hipStream_t st);
+
+}  // namespace snhip

@@ -28,6 +28,7 @@
 #include "common.h"
 #include "decode.h"
 #include "gemm.h"
+#include "gemmsplit.h"
 #include "gemv.h"
 #include "snhip.h"
 
@@ -66,7 +67,7 @@ __device__ __forceinline__ float block_sum256(float v, float* red) {
 constexpr int kLnPer = 16;
 // Prefill: up to this many channels (max_batch x dim) the gates are computed
 // for every row in parallel and the scan only multiplies and adds
-// (k_gate_rows + k_scan_rows); above it k_core_scan fuses them.
+// (k_gate_rows + the ring scan); above it k_core_scan fuses them.
 constexpr size_t kSplitScanChannels = 16384;
 
 __global__ void k_round_f16(float* __restrict__ x, long n) {
@@ -305,6 +306,7 @@ struct Mat {
     uint8_t* q = nullptr;
     float* sc = nullptr;
     uint16_t* h = nullptr;    // fp16 bits of w (the fp16 format; read by the B=1 persistent kernel)
+    SplitMat split;           // fp16 planes for products of many rows (prefill), if built
 };
 
 struct Layer {
@@ -467,64 +469,6 @@ __global__ __launch_bounds__(256) void k_gate_rows(const float* __restrict__ q, 
     pb[idx] = (1.0f - p) * uu;
 }
 
-// s_t = p_t s_{t-1} + b_t per channel (two roundings, as the decode step) over
-// the T rows of each sequence, for 64 channels per block: in each tile of
-// W TC steps wave w holds steps [w TC, (w + 1) TC), loaded before the tile's
-// hand-off chain starts; the state passes wave to wave through LDS, and a wave
-// loads its slice of the next tile right after its turn.
-template <int W, int TC>
-__global__ __launch_bounds__(64 * W) void k_scan_rows(
-        const float* __restrict__ pa, const float* __restrict__ pb, const float* __restrict__ s_in,
-        size_t s_bstride, float* __restrict__ s_out, size_t out_bstride, float* __restrict__ states, int T,
-        int D) {
-    __shared__ float carry[64];
-    const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int gpr = D / 64;
-    const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / gpr);
-    const int i = (blockIdx.x - b * gpr) * 64 + lane;
-    // This sequence's rows as buffer resources: 32-bit byte offsets from a
-    // scalar base (raw buffer addressing, dword 3 = 0x00020000 on gfx950).
-    const size_t o = (size_t)b * T * D;
-    const int bytes = T * D * 4;
-    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(pa + o), (short)0, bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(pb + o), (short)0, bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(states + o, (short)0, bytes, 0x00020000);
-    constexpr int TILE = W * TC;
-    float P[TC], Bv[TC];
-    auto load = [&](int t0) {
-        const int ts = min(t0 + w * TC, T - 1);
-        const int kmax = T - 1 - ts;
-#pragma unroll
-        for (int k = 0; k < TC; ++k) {
-            const int vo = ((ts + min(k, kmax)) * D + i) * 4;
-            P[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ra, vo, 0, 0));
-            Bv[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rb, vo, 0, 0));
-        }
-    };
-    if (w == 0) carry[lane] = s_in[(size_t)b * s_bstride + i];
-    load(0);
-    for (int t0 = 0; t0 < T; t0 += TILE) {
-        const int ts = t0 + w * TC;
-        for (int j = 0; j < W; ++j) {
-            barrier_lds();
-            if (w == j) {
-                float s = carry[lane];
-#pragma unroll
-                for (int k = 0; k < TC; ++k)
-                    if (ts + k < T) {
-                        s = P[k] * s + Bv[k];
-                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s), rs, ((ts + k) * D + i) * 4, 0, 0);
-                    }
-                carry[lane] = s;
-                if (t0 + TILE < T) load(t0 + TILE);
-            }
-        }
-    }
-    barrier_lds();
-    if (w == 0) s_out[(size_t)b * out_bstride + i] = carry[lane];
-}
-
 // Rows t = T-1 of each sequence: dst[b] = src[b*T + T-1].
 __global__ void k_last_rows(const float* __restrict__ src, float* __restrict__ dst, int T, int D) {
     const int b = blockIdx.x;
@@ -594,6 +538,8 @@ struct SnHipModel {
           *pf_u = nullptr, *pf_st = nullptr, *pf_z = nullptr, *pf_yn = nullptr, *pf_sfb = nullptr,
           *pf_send = nullptr, *pf_pa = nullptr, *pf_pb = nullptr;
     int32_t* pf_tok = nullptr;
+    snhip::SplitMat pf_xs;                       // planes of the current product's rows
+    bool split_tried = false, split_head_tried = false;
     // Persistent single-sequence decode (persist.hip): grid size, 0 when the
     // model's shape or the device does not allow it.
     int persist_wg = 0;
@@ -1477,19 +1423,21 @@ snhip_status ensure_prefill_ws(SnHipModel* m, int chunk) {
     SNHIP_CHECK(hipStreamSynchronize(m->stream));
     float** bufs[] = {&m->pf_x, &m->pf_raw, &m->pf_at, &m->pf_v, &m->pf_q, &m->pf_u,
                       &m->pf_st, &m->pf_z, &m->pf_yn, &m->pf_sfb, &m->pf_send, &m->pf_pa, &m->pf_pb};
-    for (float** b : bufs)
-        if (*b) {
-            (void)hipFree(*b);
-            for (auto it = m->allocs.begin(); it != m->allocs.end(); ++it)
-                if (*it == *b) { m->allocs.erase(it); break; }
-            *b = nullptr;
-        }
-    if (m->pf_tok) {
-        (void)hipFree(m->pf_tok);
+    auto drop = [&](void* p) {
+        if (!p) return;
+        (void)hipFree(p);
         for (auto it = m->allocs.begin(); it != m->allocs.end(); ++it)
-            if (*it == m->pf_tok) { m->allocs.erase(it); break; }
-        m->pf_tok = nullptr;
+            if (*it == p) { m->allocs.erase(it); break; }
+    };
+    for (float** b : bufs) {
+        drop(*b);
+        *b = nullptr;
     }
+    drop(m->pf_tok);
+    drop(m->pf_xs.pl);
+    drop(m->pf_xs.ex);
+    m->pf_tok = nullptr;
+    m->pf_xs = SplitMat{};
     const size_t rows = (size_t)m->max_batch * chunk, D = m->D, I = m->I, R = m->R;
     m->pf_x = dalloc<float>(m, rows * D);
     m->pf_raw = dalloc<float>(m, rows * D);
@@ -1510,8 +1458,52 @@ snhip_status ensure_prefill_ws(SnHipModel* m, int chunk) {
     for (float** b : bufs)
         if (!*b) { m->pf_chunk = 0; set_last_error("out of device memory (prefill)"); return SNHIP_E_NOMEM; }
     if (!m->pf_tok) { m->pf_chunk = 0; return SNHIP_E_NOMEM; }
+    // Without memory for the planes the products stay on the fp32 matrix cores.
+    m->pf_xs.pl = dalloc<uint16_t>(m, split_halfs(rows, std::max({D, I, R})));
+    m->pf_xs.ex = dalloc<int>(m, split_rows(rows));
     m->pf_chunk = chunk;
     return SNHIP_OK;
+}
+
+// Planes of the matrices `mats` in one allocation, once per model; left out when
+// there is no memory for them.
+snhip_status build_split(SnHipModel* m, const std::vector<Mat*>& mats, bool* tried) {
+    if (*tried) return SNHIP_OK;
+    // nothing is allocated under a caller's capture: those products stay as they are
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    SNHIP_CHECK(hipStreamIsCapturing(m->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) return SNHIP_OK;
+    *tried = true;
+    if (const char* e = getenv("SNHIP_GEMM_SPLIT"))
+        if (atoi(e) == 0) return SNHIP_OK;
+    size_t halfs = 0, rows = 0;
+    for (const Mat* W : mats) {
+        halfs += split_halfs(W->M, W->Kd);
+        rows += split_rows(W->M);
+    }
+    uint16_t* pl = dalloc<uint16_t>(m, halfs);
+    int* ex = pl ? dalloc<int>(m, rows) : nullptr;
+    if (!ex) {
+        (void)hipGetLastError();
+        return SNHIP_OK;
+    }
+    for (Mat* W : mats) {
+        const SplitMat S{pl, ex};
+        const snhip_status rc = launch_split_w(gemm_for(m, *W, nullptr, 0, 0, nullptr, 0), S, m->stream);
+        if (rc != SNHIP_OK) return rc;
+        W->split = S;
+        pl += split_halfs(W->M, W->Kd);
+        ex += split_rows(W->M);
+    }
+    return SNHIP_OK;
+}
+
+// A prefill product: from the planes for more rows than the decode paths take.
+snhip_status run_gemm_rows(SnHipModel* m, const GemmArgs& g, const Mat& W, hipStream_t st) {
+    if (g.M <= 64 || !W.split.pl || !m->pf_xs.pl || !m->pf_xs.ex) return run_gemm(m, g, st);
+    const snhip_status rc = launch_split_x(g, m->pf_xs, st);
+    if (rc != SNHIP_OK) return rc;
+    return launch_gemm_split(g, m->pf_xs, W.split, m->gemm_work, m->gemm_work_floats, st);
 }
 
 // One chunk of Tc tokens for sequences [0, B), all layers, carrying s and
@@ -1543,16 +1535,16 @@ snhip_status enqueue_prefill_chunk(SnHipModel* m, int B, int Tc, float* logits_o
                                0, st, m->pf_raw, h_l, hbs, B, Tc, D, m->kh);
             at = m->pf_at;
         }
-        if ((rc = run_gemm(m, gemm_for(m, A.V, at, D, (int)rows, m->pf_v, R), st)) != SNHIP_OK) return rc;
-        if ((rc = run_gemm(m, gemm_for(m, A.U, m->pf_v, R, (int)rows, m->pf_q, 2 * D), st)) != SNHIP_OK) return rc;
-        if ((size_t)m->max_batch * D <= kSplitScanChannels) {
+        if ((rc = run_gemm_rows(m, gemm_for(m, A.V, at, D, (int)rows, m->pf_v, R), A.V, st)) != SNHIP_OK) return rc;
+        if ((rc = run_gemm_rows(m, gemm_for(m, A.U, m->pf_v, R, (int)rows, m->pf_q, 2 * D), A.U, st)) != SNHIP_OK) return rc;
+        if ((size_t)m->max_batch * D <= kSplitScanChannels && ring_scan_ok(B, Tc, D, D)) {
             // Few channels: the gates of every row in parallel, then a scan
             // that only multiplies and adds.
             const long n = rows * D;
             hipLaunchKernelGGL(k_gate_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m->pf_q,
                                A.delta, m->pf_u, m->pf_pa, m->pf_pb, n, D, m->clamp, m->p_floor);
-            hipLaunchKernelGGL((k_scan_rows<16, 16>), dim3((unsigned)(B * (D / 64))), dim3(1024), 0, st,
-                               m->pf_pa, m->pf_pb, s_l, sbs, m->pf_send, (size_t)D, m->pf_st, Tc, D);
+            if ((rc = launch_ring_rows(m->pf_pa, m->pf_pb, s_l, sbs, m->pf_st, m->pf_send, B, Tc, D, st)) != SNHIP_OK)
+                return rc;
         } else {
             hipLaunchKernelGGL((k_core_scan<4, 16>), dim3((unsigned)(B * (D / 64))), dim3(256), 0, st,
                                m->pf_q, A.delta, s_l, sbs, m->pf_send, (size_t)D, m->pf_u, m->pf_st,
@@ -1561,18 +1553,18 @@ snhip_status enqueue_prefill_chunk(SnHipModel* m, int B, int Tc, float* logits_o
         GemmArgs gz = gemm_for(m, A.Wz, m->pf_u, D, (int)rows, m->pf_z, I);
         gz.epi = GEPI_WEDGE;
         gz.a_tanh = A.a_tanh;
-        if ((rc = run_gemm(m, gz, st)) != SNHIP_OK) return rc;
+        if ((rc = run_gemm_rows(m, gz, A.Wz, st)) != SNHIP_OK) return rc;
         launch_ln((int)rows, m->pf_z, I, A.nm_g, A.nm_c, m->pf_yn, I, I, m->eps, st);
         // sfb_t = W_eff s_{t-1}, with s_{-1} the carried state (layers.py:208-217,243-250)
         GemmArgs gs = gemm_for(m, A.Ws, m->pf_st, D, (int)rows, m->pf_sfb, D);
         gs.X0 = s_l; gs.ldx0 = (long)sbs; gs.shift_T = Tc;
-        if ((rc = run_gemm(m, gs, st)) != SNHIP_OK) return rc;
+        if ((rc = run_gemm_rows(m, gs, A.Ws, st)) != SNHIP_OK) return rc;
         GemmArgs gc = gemm_for(m, A.Wc, m->pf_yn, I, (int)rows, m->pf_x, D);
         gc.epi = GEPI_RESID;
         gc.b_gain = A.b_gain;
         gc.s = m->pf_st; gc.lds = D;
         gc.sfb = m->pf_sfb; gc.ldf = D;
-        if ((rc = run_gemm(m, gc, st)) != SNHIP_OK) return rc;
+        if ((rc = run_gemm_rows(m, gc, A.Wc, st)) != SNHIP_OK) return rc;
         hipLaunchKernelGGL(k_copy_rows, dim3(B), dim3(256), 0, st, m->pf_send, (long)D, s_l,
                            (long)sbs, D);
     }
@@ -1584,13 +1576,13 @@ snhip_status enqueue_prefill_chunk(SnHipModel* m, int B, int Tc, float* logits_o
         launch_ln((int)rows, m->pf_x, D, m->no_g, m->no_c, m->pf_raw, D, D, m->eps, st);
         const size_t V = (size_t)m->vocab;
         if (Tc == T) {
-            if ((rc = run_gemm(m, gemm_for(m, m->head, m->pf_raw, D, (int)rows, all_logits, (long)V), st)) != SNHIP_OK)
+            if ((rc = run_gemm_rows(m, gemm_for(m, m->head, m->pf_raw, D, (int)rows, all_logits, (long)V), m->head, st)) != SNHIP_OK)
                 return rc;
         } else {
             for (int b = 0; b < B; ++b) {
                 GemmArgs gh = gemm_for(m, m->head, m->pf_raw + (size_t)b * Tc * D, D, Tc,
                                        all_logits + ((size_t)b * T + c0) * V, (long)V);
-                if ((rc = run_gemm(m, gh, st)) != SNHIP_OK) return rc;
+                if ((rc = run_gemm_rows(m, gh, m->head, st)) != SNHIP_OK) return rc;
             }
         }
     }
@@ -1618,6 +1610,13 @@ snhip_status run_prefill(SnHipModel* m, const int32_t* tokens_dev, int B, int T,
     chunk = std::min(chunk, T);
     snhip_status rc = ensure_prefill_ws(m, chunk);
     if (rc != SNHIP_OK) return rc;
+    if ((long)B * chunk > 64) {
+        std::vector<Mat*> mats;
+        for (Layer& A : m->layers)
+            for (Mat* W : {&A.V, &A.U, &A.Wz, &A.Wc, &A.Ws}) mats.push_back(W);
+        if ((rc = build_split(m, mats, &m->split_tried)) != SNHIP_OK) return rc;
+        if (all_logits && (rc = build_split(m, {&m->head}, &m->split_head_tried)) != SNHIP_OK) return rc;
+    }
     for (int c0 = 0; c0 < T; c0 += chunk) {
         const int Tc = std::min(chunk, T - c0);
         SNHIP_CHECK(hipMemcpy2DAsync(m->pf_tok, (size_t)Tc * sizeof(int32_t), tokens_dev + c0,

@@ -323,6 +323,7 @@ struct RingArgs {
     const float *x0, *x1, *x2, *x3, *s0;
     float *y0, *y1, *end;
     int T, N, N8;      // channels from N8 on take two roundings (forward)
+    size_t s0_stride;  // of a batch row of s0
     int total;         // B N
     int ch;            // channels of a workgroup (at most 64; the other lanes idle)
     int yT, yrow;      // y0: floats per batch row and per step
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(64 * W) void k_scan_ring(const RingArgs A) {
         return BACK ? T - 1 - i : i;
     };
     float sz = 0.0f;
-    if (MODE == SCAN_BWD || !BACK) sz = A.s0[ch];
+    if (MODE == SCAN_BWD || !BACK) sz = A.s0[(size_t)bb * A.s0_stride + n];
     auto load = [&](RingBuf<MODE, TC>& X, int tile) {
 #pragma unroll
         for (int k = 0; k < TC; ++k) {
@@ -574,7 +575,7 @@ hipError_t launch_ring(RingArgs a, int B, hipStream_t st) {
 RingArgs ring_args(const float* x0, const float* x1, const float* s0, float* y0, float* end, int B, int T, int N) {
     RingArgs a{};
     a.x0 = x0; a.x1 = x1; a.s0 = s0; a.y0 = y0; a.end = end;
-    a.T = T; a.N = N; a.N8 = N;
+    a.T = T; a.N = N; a.N8 = N; a.s0_stride = N;
     a.yT = T * N; a.yrow = N;
     a.bytes = a.ybytes = (unsigned)((size_t)B * T * N * 4);
     return a;
@@ -585,6 +586,16 @@ snhip_status launch_ring_gated(const float* p, const float* u, const float* s0, 
     RingArgs r = ring_args(p, u, s0, states, nullptr, B, T, N);
     r.ch = ring_ch((long)B * N);
     SNHIP_CHECK((launch_ring<SCAN_GATED, 32>(r, B, st)));
+    return SNHIP_OK;
+}
+
+snhip_status launch_ring_rows(const float* p, const float* b, const float* s0, size_t s0_stride, float* states,
+                              float* end, int B, int T, int N, hipStream_t st) {
+    RingArgs r = ring_args(p, b, s0, states, end, B, T, N);
+    r.N8 = 0;
+    r.s0_stride = s0_stride;
+    r.ch = ring_ch((long)B * N);
+    SNHIP_CHECK((launch_ring<SCAN_FMA, 32>(r, B, st)));
     return SNHIP_OK;
 }
 
