@@ -28,6 +28,32 @@ inline size_t split_halfs(size_t rows, size_t K) { return split_rows(rows) * K *
 // Planes of g's X rows (g.M, with its shifted reads), or of its weights (g.N rows).
 snhip_status launch_split_x(const GemmArgs& g, SplitMat out, hipStream_t st);
 snhip_status launch_split_w(const GemmArgs& g, SplitMat out, hipStream_t st);
+// Planes of the prefill's intermediate rows, made where they are computed, for rows
+// of at most kSplitRegs values (a multiple of 8; all arrays 16-byte aligned):
+constexpr int kSplitRegs = 2048;
+// raw + depthwise conv over the rows of each sequence of T (k_conv_rows' order);
+struct SplitConv {
+    const float *raw, *hist;
+    size_t hist_bstride;
+    const float* dw;
+    int T, D, taps;
+};
+// the gated u, with p and (1 - p) u to pa and pb (k_gate_rows' order);
+struct SplitGate {
+    const float *q, *delta;
+    float *pa, *pb;
+    int D, clamp;
+    float p_floor;
+};
+// LayerNorm of rows of n.
+struct SplitLn {
+    const float *x, *g, *c;
+    int n;
+    float eps;
+};
+snhip_status launch_split_conv(const SplitConv& c, int rows, SplitMat out, hipStream_t st);
+snhip_status launch_split_gate(const SplitGate& c, int rows, SplitMat out, hipStream_t st);
+snhip_status launch_split_ln(const SplitLn& c, int rows, SplitMat out, hipStream_t st);
 // Y = X W^T with g's epilogue from the planes of both. `work` is scratch for
 // split-K partials as launch_gemm's.
 snhip_status launch_gemm_split(const GemmArgs& g, SplitMat x, SplitMat w, float* work, size_t work_floats,

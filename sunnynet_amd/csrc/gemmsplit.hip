@@ -19,103 +19,217 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(1))) const void g_void;
 typedef __attribute__((address_space(3))) void l_void;
 
-// ---- planes. A block takes 8 rows, 32 lanes to a row; a lane splits 8 values at
+// ---- planes. A block takes 8 rows, half a wave or one to a row; a lane splits 8 values at
 // a time (16 bytes of each plane), so 8 neighbouring rows fill a 128-byte line.
 // Rows of at most kSplitRegs values are held in registers between the search for
-// the largest magnitude and the split; longer ones are read twice. Bound by HBM
-// (8192 x 1024: 18 us for 67 MB); at 999 x 1024 by the latency of one pass.
-constexpr int kSplitRegs = 2048;
-template <int BLK>
-__device__ __forceinline__ void split_load(float (&v)[8], const GemmArgs& g, bool weights, const float* xr, long n,
-                                           int k) {
-    if (BLK == 0 || !weights) {
-        const float4 a = *reinterpret_cast<const float4*>(xr + k), b = *reinterpret_cast<const float4*>(xr + k + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else {
-        // byte j of a group: k = j (low nibble) and j + BLK / 2 (high)
-        const int grp = k / BLK, in = k % BLK, sh = in >= BLK / 2 ? 4 : 0;
-        const float sc = g.sc[n * (g.K / BLK) + grp];
-        const uint8_t* q = g.q + n * (g.K / 2) + (long)grp * (BLK / 2) + in % (BLK / 2);
+// the largest magnitude and the split; longer ones are loaded twice. Bound by HBM
+// (8192 x 1024: 14 us for 67 MB); at 999 x 1024 by the latency of one pass (5 us).
+// A row comes from memory (RowSrc), or from the kernel that would otherwise write it
+// only for this pass to read it back: 8192 x 1024, conv and planes 53 -> 24 us,
+// gates and planes 51 -> 41; 8192 x 1536, LayerNorm and planes 42 -> 28.
+// Over the LPR lanes of a row.
+template <int LPR, class F>
+__device__ __forceinline__ float row_reduce(float v, F f) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (float)((int)((q[j] >> sh) & 0xFu) - 8) * sc;   // quant.c:82-83
-    }
+    for (int o = LPR / 2; o > 0; o >>= 1) v = f(v, __shfl_xor(v, o, 64));
+    return v;
 }
-
-template <int BLK, bool REGS>
-__global__ __launch_bounds__(256) void k_split_rows(GemmArgs g, int weights, uint16_t* __restrict__ pl,
-                                                    int* __restrict__ ex) {
-    const int lane = threadIdx.x & 31, rows = weights ? g.N : g.M, K = g.K, nk = K / 16;
-    const int row = blockIdx.x * 8 + (threadIdx.x >> 5);
-    if (row >= rows) return;
-    const float* xr = nullptr;
-    if (weights) {
-        if (BLK == 0) xr = g.w + (long)row * K;
-    } else {
-        xr = gemm_xrow(g, row);
+// The largest magnitude so far, infinite once there is an infinity or NaN.
+__device__ __forceinline__ float row_look(float mx, const float (&x)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float a = fabsf(x[j]);
+        mx = fmaxf(mx, a < __builtin_inff() ? a : __builtin_inff());
     }
-    constexpr int NV = REGS ? kSplitRegs / 256 : 1;
-    float v[NV][8], mx = 0.0f;
-    bool bad = false;
-    auto look = [&](const float (&x)[8]) {
+    return mx;
+}
+__device__ __forceinline__ void split_store(const float (&y)[8], int s, bool bad, uint16_t* pl, int row, int k,
+                                            int nk) {
+    half8 h, l;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        float x = ldexpf(y[j], s);
+        // such a row's products are all infinite or NaN: only those, signs and
+        // zeros count
+        if (bad && fabsf(x) < __builtin_inff()) x = x == 0.0f ? 0.0f : copysignf(1.0f, x);
+        h[j] = (_Float16)x;
+        l[j] = bad ? (_Float16)0.0f : (_Float16)(x - (float)h[j]);
+    }
+    half8* o = reinterpret_cast<half8*>(pl + (((size_t)(row >> 5) * nk + (k >> 4)) << 10)) + ((k >> 3) & 1) * 32 +
+               (row & 31);
+    o[0] = h;
+    o[64] = l;
+}
+__device__ __forceinline__ void ld8(float (&v)[8], const float* p) {
+    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ void st8(float* p, const float (&v)[8]) {
+    reinterpret_cast<float4*>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
+    reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
+}
+__device__ __forceinline__ float sgm(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+// Rows of X (with its shifted reads).
+struct XSrc {
+    GemmArgs g;
+    __device__ __forceinline__ void load(float (&v)[8], int row, int k) const { ld8(v, gemm_xrow(g, row) + k); }
+    template <int LPR, int NV> __device__ __forceinline__ void row(float (&)[NV][8], int, int) const {}
+};
+// Rows of W: fp32 (BLK 0), or INT4 groups of BLK, dequantized as quant.c:82-83.
+template <int BLK>
+struct WSrc {
+    GemmArgs g;
+    __device__ __forceinline__ void load(float (&v)[8], int row, int k) const {
+        if constexpr (BLK == 0) {
+            ld8(v, g.w + (long)row * g.K + k);
+        } else {
+            // byte j of a group: k = j (low nibble) and j + BLK / 2 (high)
+            const int grp = k / BLK, in = k % BLK, sh = in >= BLK / 2 ? 4 : 0;
+            const float sc = g.sc[(long)row * (g.K / BLK) + grp];
+            const uint8_t* q = g.q + (long)row * (g.K / 2) + (long)grp * (BLK / 2) + in % (BLK / 2);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = (float)((int)((q[j] >> sh) & 0xFu) - 8) * sc;
+        }
+    }
+    template <int LPR, int NV> __device__ __forceinline__ void row(float (&)[NV][8], int, int) const {}
+};
+struct ConvSrc {
+    SplitConv c;
+    __device__ __forceinline__ void load(float (&v)[8], int row, int k) const {
+        const int b = row / c.T, t = row - b * c.T;
+        float r[8], d[8], p[8], acc[8];
+        const float* x = c.raw + (size_t)row * c.D + k;
+        ld8(r, x);
+        ld8(d, c.dw + (size_t)(c.taps - 1) * c.D + k);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] = r[j] * d[j];
+        for (int q = 0; q < c.taps - 1; ++q) {
+            ld8(p, t - 1 - q >= 0 ? x - (size_t)(q + 1) * c.D
+                                  : c.hist + (size_t)b * c.hist_bstride + (size_t)(q - t) * c.D + k);
+            ld8(d, c.dw + (size_t)(c.taps - 2 - q) * c.D + k);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] = acc[j] + p[j] * d[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = r[j] + acc[j];
+    }
+    template <int LPR, int NV> __device__ __forceinline__ void row(float (&)[NV][8], int, int) const {}
+};
+// A lane's 8 values are one group: its gate and u rows are 16 floats side by side.
+struct GateSrc {
+    SplitGate c;
+    __device__ __forceinline__ void load(float (&v)[8], int row, int k) const {
+        float u[8], gt[8], dl[8], a[8], b[8];
+        const float* x = c.q + (size_t)row * 2 * c.D + 2 * k;
+        ld8(u, x);
+        ld8(gt, x + 8);
+        ld8(dl, c.delta + k);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            bad |= !(fabsf(x[j]) < __builtin_inff());
-            mx = fmaxf(mx, fabsf(x[j]));
+            const float gi = gt[j];
+            v[j] = u[j] * (sgm(gi - gt[(j + 1) & 7]) * sgm(gi - gt[(j + 2) & 7]));
+            float p = 1.0f - dl[j] * (1.0f - sgm(gi));
+            if (c.clamp && p < c.p_floor) p = c.p_floor;
+            a[j] = p;
+            b[j] = (1.0f - p) * v[j];
         }
-    };
+        st8(c.pa + (size_t)row * c.D + k, a);
+        st8(c.pb + (size_t)row * c.D + k, b);
+    }
+    template <int LPR, int NV> __device__ __forceinline__ void row(float (&)[NV][8], int, int) const {}
+};
+struct LnSrc {
+    SplitLn c;
+    __device__ __forceinline__ void load(float (&v)[8], int row, int k) const { ld8(v, c.x + (size_t)row * c.n + k); }
+    template <int LPR, int NV> __device__ __forceinline__ void row(float (&v)[NV][8], int lane, int K) const {
+        auto add = [](float x, float y) { return x + y; };
+        float g[NV][8], o[NV][8], t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int k = min(lane * 8 + i * LPR * 8, K - 8);
+            ld8(g[i], c.g + k);
+            ld8(o[i], c.c + k);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) t += v[i][j];                       // zeros past K
+        }
+        const float mean = row_reduce<LPR>(t, add) / (float)K;
+        t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if (lane * 8 + i * LPR * 8 < K)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float d = v[i][j] - mean;
+                    t += d * d;
+                }
+        const float rstd = 1.0f / sqrtf(row_reduce<LPR>(t, add) / (float)K + c.eps);
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if (lane * 8 + i * LPR * 8 < K)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[i][j] = (v[i][j] - mean) * rstd * g[i][j] + o[i][j];
+    }
+};
+
+template <class Src, bool REGS, int LPR>
+__global__ __launch_bounds__(8 * LPR) void k_split_rows(Src src, int rows, int K, uint16_t* __restrict__ pl,
+                                                    int* __restrict__ ex) {
+    const int lane = threadIdx.x % LPR, nk = K / 16;
+    const int row = blockIdx.x * 8 + threadIdx.x / LPR;
+    if (row >= rows) return;
+    constexpr int NV = REGS ? kSplitRegs / (LPR * 8) : 1;
+    float v[NV][8], mx = 0.0f;
+    auto most = [](float x, float y) { return fmaxf(x, y); };
     if constexpr (REGS) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const int k = lane * 8 + i * 256;
-            if (k < K) split_load<BLK>(v[i], g, weights, xr, row, k);
+            const int k = lane * 8 + i * LPR * 8;
+            if (k < K) src.load(v[i], row, k);
             else
 #pragma unroll
                 for (int j = 0; j < 8; ++j) v[i][j] = 0.0f;
         }
+        src.template row<LPR, NV>(v, lane, K);
 #pragma unroll
-        for (int i = 0; i < NV; ++i) look(v[i]);
+        for (int i = 0; i < NV; ++i) mx = row_look(mx, v[i]);
     } else {
-        for (int k = lane * 8; k < K; k += 256) {
-            split_load<BLK>(v[0], g, weights, xr, row, k);
-            look(v[0]);
+        for (int k = lane * 8; k < K; k += LPR * 8) {
+            src.load(v[0], row, k);
+            mx = row_look(mx, v[0]);
         }
     }
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) {
-        mx = fmaxf(mx, __shfl_xor(mx, o, 32));
-        bad |= __shfl_xor((int)bad, o, 32) != 0;
-    }
+    mx = row_reduce<LPR>(mx, most);
+    const bool bad = !(mx < __builtin_inff());
     int e = 0;
-    (void)frexpf(mx, &e);                         // mx in [2^(e-1), 2^e)
+    (void)frexpf(mx, &e);                        // mx in [2^(e-1), 2^e)
     const int s = bad ? 0 : (mx > 0.0f ? 15 - e : 0);
-    auto split = [&](const float (&y)[8], int k) {
-        half8 h, l;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            float x = ldexpf(y[j], s);
-            // such a row's products are all infinite or NaN: only those, signs and
-            // zeros count
-            if (bad && fabsf(x) < __builtin_inff()) x = x == 0.0f ? 0.0f : copysignf(1.0f, x);
-            h[j] = (_Float16)x;
-            l[j] = bad ? (_Float16)0.0f : (_Float16)(x - (float)h[j]);
-        }
-        half8* o = reinterpret_cast<half8*>(pl + (((size_t)(row >> 5) * nk + (k >> 4)) << 10)) +
-                   ((k >> 3) & 1) * 32 + (row & 31);
-        o[0] = h;
-        o[64] = l;
-    };
     if constexpr (REGS) {
 #pragma unroll
         for (int i = 0; i < NV; ++i)
-            if (lane * 8 + i * 256 < K) split(v[i], lane * 8 + i * 256);
+            if (lane * 8 + i * LPR * 8 < K) split_store(v[i], s, bad, pl, row, lane * 8 + i * LPR * 8, nk);
     } else {
-        for (int k = lane * 8; k < K; k += 256) {
-            split_load<BLK>(v[0], g, weights, xr, row, k);
-            split(v[0], k);
+        for (int k = lane * 8; k < K; k += LPR * 8) {
+            src.load(v[0], row, k);
+            split_store(v[0], s, bad, pl, row, k, nk);
         }
     }
     if (lane == 0) ex[row] = bad ? kSplitNonFinite : s;
+}
+
+template <bool REGS, class Src>
+snhip_status split_launch(const Src& src, int rows, int K, SplitMat out, hipStream_t st) {
+    // us per call, 32 / 64 lanes to a row: 8192 rows of 1024, planes alone 14.4 / 17.6,
+    // conv 24 / 30, gates 41 / 45; 999 rows (125 blocks) 6.0 / 5.1, 14.1 / 9.2, 14.3 / 11.2.
+    if (rows >= 4096)
+        hipLaunchKernelGGL((k_split_rows<Src, REGS, 32>), dim3((rows + 7) / 8), dim3(256), 0, st, src, rows, K, out.pl,
+                           out.ex);
+    else
+        hipLaunchKernelGGL((k_split_rows<Src, REGS, 64>), dim3((rows + 7) / 8), dim3(512), 0, st, src, rows, K, out.pl,
+                           out.ex);
+    SNHIP_CHECK(hipGetLastError());
+    return SNHIP_OK;
 }
 
 // One output of a row with an infinity or NaN in it.
@@ -287,20 +401,24 @@ __global__ __launch_bounds__(256, 2) void k_gemm_split(GemmArgs g, SplitMat X, S
 }  // namespace
 
 snhip_status launch_split_x(const GemmArgs& g, SplitMat out, hipStream_t st) {
-    const dim3 grid((g.M + 7) / 8), blk(256);
-    if (g.K <= kSplitRegs) hipLaunchKernelGGL((k_split_rows<0, true>), grid, blk, 0, st, g, 0, out.pl, out.ex);
-    else hipLaunchKernelGGL((k_split_rows<0, false>), grid, blk, 0, st, g, 0, out.pl, out.ex);
-    SNHIP_CHECK(hipGetLastError());
-    return SNHIP_OK;
+    return g.K <= kSplitRegs ? split_launch<true>(XSrc{g}, g.M, g.K, out, st)
+                             : split_launch<false>(XSrc{g}, g.M, g.K, out, st);
 }
 
 snhip_status launch_split_w(const GemmArgs& g, SplitMat out, hipStream_t st) {
-    const dim3 grid((g.N + 7) / 8), blk(256);
-    if (!g.q) hipLaunchKernelGGL((k_split_rows<0, false>), grid, blk, 0, st, g, 1, out.pl, out.ex);
-    else if (g.block == 32) hipLaunchKernelGGL((k_split_rows<32, false>), grid, blk, 0, st, g, 1, out.pl, out.ex);
-    else hipLaunchKernelGGL((k_split_rows<64, false>), grid, blk, 0, st, g, 1, out.pl, out.ex);
-    SNHIP_CHECK(hipGetLastError());
-    return SNHIP_OK;
+    if (!g.q) return split_launch<false>(WSrc<0>{g}, g.N, g.K, out, st);
+    if (g.block == 32) return split_launch<false>(WSrc<32>{g}, g.N, g.K, out, st);
+    return split_launch<false>(WSrc<64>{g}, g.N, g.K, out, st);
+}
+
+snhip_status launch_split_conv(const SplitConv& c, int rows, SplitMat out, hipStream_t st) {
+    return split_launch<true>(ConvSrc{c}, rows, c.D, out, st);
+}
+snhip_status launch_split_gate(const SplitGate& c, int rows, SplitMat out, hipStream_t st) {
+    return split_launch<true>(GateSrc{c}, rows, c.D, out, st);
+}
+snhip_status launch_split_ln(const SplitLn& c, int rows, SplitMat out, hipStream_t st) {
+    return split_launch<true>(LnSrc{c}, rows, c.n, out, st);
 }
 
 snhip_status launch_gemm_split(const GemmArgs& g, SplitMat x, SplitMat w, float* work, size_t work_floats,

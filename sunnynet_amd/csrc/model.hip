@@ -1498,11 +1498,19 @@ snhip_status build_split(SnHipModel* m, const std::vector<Mat*>& mats, bool* tri
     return SNHIP_OK;
 }
 
-// A prefill product: from the planes for more rows than the decode paths take.
-snhip_status run_gemm_rows(SnHipModel* m, const GemmArgs& g, const Mat& W, hipStream_t st) {
-    if (g.M <= 64 || !W.split.pl || !m->pf_xs.pl || !m->pf_xs.ex) return run_gemm(m, g, st);
-    const snhip_status rc = launch_split_x(g, m->pf_xs, st);
-    if (rc != SNHIP_OK) return rc;
+// Whether a prefill product of `rows` rows runs from the planes: more rows than the
+// decode paths take.
+bool split_rows_ok(const SnHipModel* m, const Mat& W, long rows) {
+    return rows > 64 && W.split.pl && m->pf_xs.pl && m->pf_xs.ex;
+}
+
+// A prefill product; `planes`: those of its rows are in pf_xs already.
+snhip_status run_gemm_rows(SnHipModel* m, const GemmArgs& g, const Mat& W, hipStream_t st, bool planes = false) {
+    if (!planes) {
+        if (!split_rows_ok(m, W, g.M)) return run_gemm(m, g, st);
+        const snhip_status rc = launch_split_x(g, m->pf_xs, st);
+        if (rc != SNHIP_OK) return rc;
+    }
     return launch_gemm_split(g, m->pf_xs, W.split, m->gemm_work, m->gemm_work_floats, st);
 }
 
@@ -1526,23 +1534,40 @@ snhip_status enqueue_prefill_chunk(SnHipModel* m, int B, int Tc, float* logits_o
         float* s_l = m->s + (size_t)l * D;
         float* h_l = m->hist + (size_t)l * (m->kh ? m->kh : 1) * D;
         launch_ln((int)rows, m->pf_x, D, A.ni_g, A.ni_c, m->pf_raw, D, D, m->eps, st);
+        // Rows that only a product reads are split into its planes as they are computed.
+        auto fuse = [&](const Mat& W) { return W.Kd <= kSplitRegs && split_rows_ok(m, W, rows); };
         const float* at = m->pf_raw;
+        bool conv_split = false, gate_split = false;
         if (m->K > 1) {
             const long n = rows * D;
-            hipLaunchKernelGGL(k_conv_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                               m->pf_raw, h_l, hbs, A.dw, m->pf_at, B, Tc, D, m->K);
+            conv_split = fuse(A.V);
+            if (conv_split) {
+                if ((rc = launch_split_conv({m->pf_raw, h_l, hbs, A.dw, Tc, D, m->K}, (int)rows, m->pf_xs, st)) != SNHIP_OK)
+                    return rc;
+            } else {
+                hipLaunchKernelGGL(k_conv_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
+                                   m->pf_raw, h_l, hbs, A.dw, m->pf_at, B, Tc, D, m->K);
+                at = m->pf_at;
+            }
             hipLaunchKernelGGL(k_hist_update, dim3((unsigned)(((long)B * D + 255) / 256)), dim3(256),
                                0, st, m->pf_raw, h_l, hbs, B, Tc, D, m->kh);
-            at = m->pf_at;
         }
-        if ((rc = run_gemm_rows(m, gemm_for(m, A.V, at, D, (int)rows, m->pf_v, R), A.V, st)) != SNHIP_OK) return rc;
+        if ((rc = run_gemm_rows(m, gemm_for(m, A.V, at, D, (int)rows, m->pf_v, R), A.V, st, conv_split)) != SNHIP_OK)
+            return rc;
         if ((rc = run_gemm_rows(m, gemm_for(m, A.U, m->pf_v, R, (int)rows, m->pf_q, 2 * D), A.U, st)) != SNHIP_OK) return rc;
         if ((size_t)m->max_batch * D <= kSplitScanChannels && ring_scan_ok(B, Tc, D, D)) {
             // Few channels: the gates of every row in parallel, then a scan
             // that only multiplies and adds.
             const long n = rows * D;
-            hipLaunchKernelGGL(k_gate_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m->pf_q,
-                               A.delta, m->pf_u, m->pf_pa, m->pf_pb, n, D, m->clamp, m->p_floor);
+            gate_split = fuse(A.Wz);
+            if (gate_split) {
+                if ((rc = launch_split_gate({m->pf_q, A.delta, m->pf_pa, m->pf_pb, D, m->clamp, m->p_floor}, (int)rows,
+                                            m->pf_xs, st)) != SNHIP_OK)
+                    return rc;
+            } else {
+                hipLaunchKernelGGL(k_gate_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m->pf_q,
+                                   A.delta, m->pf_u, m->pf_pa, m->pf_pb, n, D, m->clamp, m->p_floor);
+            }
             if ((rc = launch_ring_rows(m->pf_pa, m->pf_pb, s_l, sbs, m->pf_st, m->pf_send, B, Tc, D, st)) != SNHIP_OK)
                 return rc;
         } else {
@@ -1553,18 +1578,23 @@ snhip_status enqueue_prefill_chunk(SnHipModel* m, int B, int Tc, float* logits_o
         GemmArgs gz = gemm_for(m, A.Wz, m->pf_u, D, (int)rows, m->pf_z, I);
         gz.epi = GEPI_WEDGE;
         gz.a_tanh = A.a_tanh;
-        if ((rc = run_gemm_rows(m, gz, A.Wz, st)) != SNHIP_OK) return rc;
-        launch_ln((int)rows, m->pf_z, I, A.nm_g, A.nm_c, m->pf_yn, I, I, m->eps, st);
+        if ((rc = run_gemm_rows(m, gz, A.Wz, st, gate_split)) != SNHIP_OK) return rc;
         // sfb_t = W_eff s_{t-1}, with s_{-1} the carried state (layers.py:208-217,243-250)
         GemmArgs gs = gemm_for(m, A.Ws, m->pf_st, D, (int)rows, m->pf_sfb, D);
         gs.X0 = s_l; gs.ldx0 = (long)sbs; gs.shift_T = Tc;
         if ((rc = run_gemm_rows(m, gs, A.Ws, st)) != SNHIP_OK) return rc;
+        const bool ln_split = fuse(A.Wc);
+        if (ln_split) {
+            if ((rc = launch_split_ln({m->pf_z, A.nm_g, A.nm_c, I, m->eps}, (int)rows, m->pf_xs, st)) != SNHIP_OK) return rc;
+        } else {
+            launch_ln((int)rows, m->pf_z, I, A.nm_g, A.nm_c, m->pf_yn, I, I, m->eps, st);
+        }
         GemmArgs gc = gemm_for(m, A.Wc, m->pf_yn, I, (int)rows, m->pf_x, D);
         gc.epi = GEPI_RESID;
         gc.b_gain = A.b_gain;
         gc.s = m->pf_st; gc.lds = D;
         gc.sfb = m->pf_sfb; gc.ldf = D;
-        if ((rc = run_gemm_rows(m, gc, A.Wc, st)) != SNHIP_OK) return rc;
+        if ((rc = run_gemm_rows(m, gc, A.Wc, st, ln_split)) != SNHIP_OK) return rc;
         hipLaunchKernelGGL(k_copy_rows, dim3(B), dim3(256), 0, st, m->pf_send, (long)D, s_l,
                            (long)sbs, D);
     }
