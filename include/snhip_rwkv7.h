@@ -71,9 +71,9 @@ int snhip_rk_ready(const SnHipRwkv7* m);
 snhip_status snhip_rk_set_stream(SnHipRwkv7* m, void* stream);
 int32_t snhip_rk_max_batch(const SnHipRwkv7* m);
 /* Workgroups of the one-launch step that runs steps of a single sequence
- * (one cooperative launch per call of greedy steps, one per step otherwise),
- * or 0 when steps of one sequence take the per-kernel step (no cooperative
- * launch, a shape it does not take, or SNHIP_RK_EXACT=0 in the environment
+ * (one launch per call of greedy steps, one per step otherwise),
+ * or 0 when steps of one sequence take the per-kernel step (no co-resident
+ * grid, a shape it does not take, or SNHIP_RK_EXACT=0 in the environment
  * at load). By default it is the exact-order kernel, whose logits equal the
  * reference's sn_rk_step bit for bit. With SNHIP_RK_PERSIST=1 at load it is
  * instead a kernel that sums in parallel, not bit-exact (measured up to
