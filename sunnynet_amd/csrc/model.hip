@@ -1461,6 +1461,7 @@ snhip_status ensure_prefill_ws(SnHipModel* m, int chunk) {
     // Without memory for the planes the products stay on the fp32 matrix cores.
     m->pf_xs.pl = dalloc<uint16_t>(m, split_halfs(rows, std::max({D, I, R})));
     m->pf_xs.ex = dalloc<int>(m, split_rows(rows));
+    if (!m->pf_xs.pl || !m->pf_xs.ex) (void)hipGetLastError();   // not an error of the launches that follow
     m->pf_chunk = chunk;
     return SNHIP_OK;
 }
