@@ -72,22 +72,6 @@ hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, 
     return e != hipSuccess ? e : hipLaunchKernel(k, grid, block, args, 0, st);
 }
 
-hipError_t StreamOrder::mark(hipStream_t st) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    hipError_t e = hipStreamIsCapturing(st, &cs);
-    set_ = false;
-    if (e != hipSuccess || cs != hipStreamCaptureStatusNone) return e;
-    if (!ev_) e = hipEventCreateWithFlags(&ev_, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventRecord(ev_, st);
-    set_ = e == hipSuccess;
-    return e;
-}
-hipError_t StreamOrder::follow(hipStream_t st) {
-    const bool wait = set_;
-    set_ = false;
-    return wait ? hipStreamWaitEvent(st, ev_, 0) : hipSuccess;
-}
-
 bool stream_has_all_cus(hipStream_t st) {
     if (!st) return true;
     int dev = 0, ncu = 0;

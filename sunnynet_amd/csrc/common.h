@@ -9,6 +9,7 @@
 #include <string>
 
 #include "snhip_abi.h"
+#include "streamorder.h"
 
 namespace snhip {
 
@@ -77,19 +78,25 @@ private:
 // SNHIP_COOP=1 launches cooperatively.
 hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st);
 
-// Steps and prefills of one handle are in order also across a change of the
-// caller's stream: each that returns before its work is done marks its end on
-// the stream it ran on, and a new stream waits for the mark.
-class StreamOrder {
-public:
-    ~StreamOrder() { if (ev_) (void)hipEventDestroy(ev_); }
-    hipError_t mark(hipStream_t st);      // (not while st is being captured)
-    hipError_t follow(hipStream_t st);
-
-private:
-    hipEvent_t ev_ = nullptr;
-    bool set_ = false;
+// StreamOrderT on the device.
+struct HipEvents {
+    using Stream = hipStream_t;
+    using Event = hipEvent_t;
+    using Error = hipError_t;
+    static constexpr hipError_t ok = hipSuccess;
+    static hipError_t capturing(Stream st, bool* c) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        const hipError_t e = hipStreamIsCapturing(st, &cs);
+        *c = cs != hipStreamCaptureStatusNone;
+        return e;
+    }
+    static hipError_t create(Event* ev) { return hipEventCreateWithFlags(ev, hipEventDisableTiming); }
+    static void destroy(Event ev) { (void)hipEventDestroy(ev); }
+    static hipError_t record(Event ev, Stream st) { return hipEventRecord(ev, st); }
+    static hipError_t wait(Stream st, Event ev) { return hipStreamWaitEvent(st, ev, 0); }
+    static hipError_t host_wait(Event ev) { return hipEventSynchronize(ev); }
 };
+using StreamOrder = StreamOrderT<HipEvents>;
 
 // Whether `st` may use every CU (a stream made with a CU mask may not, and a
 // grid sized for the whole device would not co-reside on it).

@@ -1787,9 +1787,10 @@ SnHipModel* snhip_load_ex(const char* path, int vocab, int dim, int inner, int r
 
 void snhip_free(SnHipModel* m) {
     if (!m) return;
-    // Only this handle's work is waited for: the caller's stream it was bound
-    // to (NULL = the null stream).
+    // Only this handle's work is waited for: on the caller's stream it is bound
+    // to (NULL = the null stream) and on the one it last ran on.
     (void)hipStreamSynchronize(m->stream);
+    (void)m->order.drain();
     free_model(m);
 }
 
@@ -1982,6 +1983,7 @@ snhip_status snhip_decode_greedy_dev(SnHipModel* m, const int32_t* tokens_dev, i
     if (rc != SNHIP_OK) return rc;
     SNHIP_CHECK(hipMemcpyAsync(out_tokens_dev, m->tok_hist, (size_t)n_steps * B * sizeof(int32_t),
                                hipMemcpyDeviceToDevice, m->stream));
+    SNHIP_CHECK(m->order.mark(m->stream));
     return SNHIP_OK;
 }
 
@@ -1992,6 +1994,7 @@ snhip_status snhip_get_state_dev(SnHipModel* m, float* s_dev, float* hist_dev, i
     if (m->kh)
         SNHIP_CHECK(hipMemcpyAsync(hist_dev, m->hist, (size_t)B * m->L * m->kh * m->D * sizeof(float),
                                    hipMemcpyDeviceToDevice, m->stream));
+    SNHIP_CHECK(m->order.mark(m->stream));
     return SNHIP_OK;
 }
 
@@ -2003,6 +2006,7 @@ snhip_status snhip_set_state_dev(SnHipModel* m, const float* s_dev, const float*
     if (m->kh)
         SNHIP_CHECK(hipMemcpyAsync(m->hist, hist_dev, (size_t)B * m->L * m->kh * m->D * sizeof(float),
                                    hipMemcpyDeviceToDevice, m->stream));
+    SNHIP_CHECK(m->order.mark(m->stream));
     if (B >= m->poisoned) m->poisoned = 0;
     return SNHIP_OK;
 }

@@ -1018,6 +1018,7 @@ void snhip_rk_free(SnHipRwkv7* m) {
     if (!m) return;
     // Only this handle's work is waited for (see snhip_free).
     (void)hipStreamSynchronize(m->stream);
+    (void)m->order.drain();
     free_rk(m);
 }
 
@@ -1116,6 +1117,7 @@ snhip_status snhip_rk_decode_greedy_dev(SnHipRwkv7* m, const int32_t* tokens_dev
     if (rc != SNHIP_OK) return rc;
     SNHIP_CHECK(hipMemcpyAsync(out_tokens_dev, m->tok_hist, (size_t)n_steps * B * sizeof(int32_t),
                                hipMemcpyDeviceToDevice, m->stream));
+    SNHIP_CHECK(m->order.mark(m->stream));
     return SNHIP_OK;
 }
 
@@ -1125,6 +1127,7 @@ snhip_status snhip_rk_get_state_dev(SnHipRwkv7* m, float* S_dev, float* shift_de
                                hipMemcpyDeviceToDevice, m->stream));
     SNHIP_CHECK(hipMemcpyAsync(shift_dev, m->shift, (size_t)B * m->L * 2 * m->D * sizeof(float),
                                hipMemcpyDeviceToDevice, m->stream));
+    SNHIP_CHECK(m->order.mark(m->stream));
     return SNHIP_OK;
 }
 
@@ -1135,6 +1138,7 @@ snhip_status snhip_rk_set_state_dev(SnHipRwkv7* m, const float* S_dev, const flo
                                hipMemcpyDeviceToDevice, m->stream));
     SNHIP_CHECK(hipMemcpyAsync(m->shift, shift_dev, (size_t)B * m->L * 2 * m->D * sizeof(float),
                                hipMemcpyDeviceToDevice, m->stream));
+    SNHIP_CHECK(m->order.mark(m->stream));
     m->poisoned = 0;
     return SNHIP_OK;
 }

@@ -1,0 +1,42 @@
+// Order of one handle's calls across the streams they run on.
+#pragma once
+
+namespace snhip {
+
+// Calls of one handle are in order also across changes of the caller's stream:
+// each call that returns before its work is done marks the work's end on the
+// stream it ran on (mark), and every other stream the handle is bound to before
+// the next mark waits for it (follow), however many there are and whether or not
+// anything runs on them. Rt supplies streams and events, so that the rule runs
+// without a device too.
+template <class Rt>
+class StreamOrderT {
+public:
+    using Stream = typename Rt::Stream;
+    using Error = typename Rt::Error;
+
+    ~StreamOrderT() { if (ev_) Rt::destroy(ev_); }
+
+    // (not while st is being captured: nothing has run there, and the earlier
+    // mark still stands)
+    Error mark(Stream st) {
+        bool capturing = false;
+        Error e = Rt::capturing(st, &capturing);
+        if (e != Rt::ok || capturing) return e;
+        if (!ev_ && (e = Rt::create(&ev_)) != Rt::ok) return e;
+        if ((e = Rt::record(ev_, st)) != Rt::ok) return e;
+        set_ = true;
+        at_ = st;
+        return Rt::ok;
+    }
+    Error follow(Stream st) { return set_ && st != at_ ? Rt::wait(st, ev_) : Rt::ok; }
+    // The host waits for the mark.
+    Error drain() { return set_ ? Rt::host_wait(ev_) : Rt::ok; }
+
+private:
+    typename Rt::Event ev_{};
+    bool set_ = false;
+    Stream at_{};
+};
+
+}  // namespace snhip

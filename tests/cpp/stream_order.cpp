@@ -1,0 +1,65 @@
+// Runs StreamOrderT over a device of names: a stream is the set of operations
+// that have finished before whatever it is given next. Reads one command per
+// line and prints a line per operation: its number and whether every earlier
+// operation of the handle has finished before it starts.
+//   bind S     the handle is bound to stream S
+//   async      an operation of the handle that returns before it is done
+//   quiet      one that does not mark
+//   capture S  S is being captured from here on; endcapture S ends it
+//   free       the handle's last wait: prints whether all operations are done
+#include <cstdint>
+#include <iostream>
+#include <map>
+#include <string>
+
+#include "streamorder.h"
+
+struct Dev {
+    std::map<std::string, uint64_t> streams;
+    std::map<std::string, bool> cap;
+    uint64_t host = 0;
+};
+static Dev dev;
+
+struct Rt {
+    using Stream = std::string;
+    using Event = uint64_t*;
+    using Error = int;
+    static constexpr int ok = 0;
+    static int capturing(Stream s, bool* c) { *c = dev.cap[s]; return ok; }
+    static int create(Event* e) { *e = new uint64_t(0); return ok; }
+    static void destroy(Event e) { delete e; }
+    static int record(Event e, Stream s) { if (dev.cap[s]) return 1; *e = dev.streams[s]; return ok; }
+    static int wait(Stream s, Event e) { if (dev.cap[s]) return 2; dev.streams[s] |= *e; return ok; }
+    static int host_wait(Event e) { dev.host |= *e; return ok; }
+};
+
+int main() {
+    snhip::StreamOrderT<Rt> order;
+    std::string cmd, cur;
+    uint64_t all = 0;
+    int n = 0;
+    auto check = [](int e) { if (e) std::cout << "error " << e << "\n"; };
+    while (std::cin >> cmd) {
+        if (cmd == "bind") {
+            std::cin >> cur;
+            check(order.follow(cur));
+        } else if (cmd == "capture" || cmd == "endcapture") {
+            std::string s;
+            std::cin >> s;
+            dev.cap[s] = cmd == "capture";
+        } else if (cmd == "free") {
+            check(order.drain());
+            const uint64_t done = dev.host | dev.streams[cur];
+            std::cout << "free " << ((done & all) == all) << "\n";
+        } else {
+            if (!dev.cap[cur]) {
+                std::cout << n << " " << ((dev.streams[cur] & all) == all) << "\n";
+                all |= 1ull << n;
+                dev.streams[cur] |= 1ull << n;
+                ++n;
+            }
+            if (cmd == "async") check(order.mark(cur));
+        }
+    }
+}

@@ -1,6 +1,7 @@
-"""Persistent steps on the caller's streams: two handles stepped from two threads
-on two streams at once give what each gives alone (their kernels must not share
-the device), and a handle that moves between streams goes on from its state."""
+"""Steps on the caller's streams: two handles stepped from two threads on two
+streams at once give what each gives alone (their persistent kernels must not
+share the device), and a handle that moves between streams goes on from its state,
+also while its earlier calls are still running."""
 from __future__ import annotations
 
 import threading
@@ -83,3 +84,53 @@ def test_moves_between_streams(gpu, paths, kind):
     h.reset()
     got = _run(h, kind, 6, [torch.cuda.Stream(), torch.cuda.current_stream(), torch.cuda.Stream()])
     assert all(torch.equal(x, y) for x, y in zip(got, ref))
+
+
+def _calls(h, kind, toks, streams, between):
+    """A chain of calls, each on the next of `streams`, none waited for. `between`
+    binds the handle to one more stream before each call: with a read of the state
+    (which only copies), or with nothing."""
+    keep, i = [], 0
+
+    def on(f):
+        nonlocal i
+        with torch.cuda.stream(streams[i % len(streams)]):
+            keep.append(f())
+        i += 1
+
+    for t in toks:
+        if between == "state":
+            on(lambda: h.get_state(h.max_batch))
+        elif between == "bind":
+            on(h._bind_stream)
+        on(lambda: h.step_batch(t))
+        if kind == "sunny20":
+            on(lambda: h.prefill_batch(torch.stack([t, t, t, t], 1)))
+            on(lambda: h.decode_greedy(t, 3))
+    on(lambda: h.get_state(h.max_batch))
+    return keep
+
+
+@pytest.mark.parametrize("between", ["none", "bind", "state"])
+@pytest.mark.parametrize("kind", ["rwkv12", "sunny20"])
+def test_running_calls_move_between_streams(gpu, paths, monkeypatch, kind, between):
+    """Calls that return before they are done (captured steps, prefill, captured
+    greedy decoding) over three streams, synchronized once at the end."""
+    print("calls in flight over three streams:", kind, between, flush=True)
+    monkeypatch.setenv("SNHIP_BATCH_PERSIST", "0")    # read at load: the captured per-kernel step
+    h = _make(kind, paths)
+    assert kind != "sunny20" or h.batch_grid == 0
+    rng = np.random.default_rng(6)
+    toks = [torch.from_numpy(rng.integers(0, h.vocab, h.max_batch).astype(np.int32)).cuda() for _ in range(6)]
+    _calls(h, kind, toks, [torch.cuda.current_stream()], between)     # graphs captured, workspaces there
+    torch.cuda.synchronize()
+    out = []
+    for streams in ([torch.cuda.current_stream()], [torch.cuda.Stream() for _ in range(3)]):
+        h.reset()
+        out.append(_calls(h, kind, toks, streams, between))
+        torch.cuda.synchronize()
+    flat = [[x for r in o if r is not None for x in (r if isinstance(r, tuple) else (r,))] for o in out]
+    assert len(flat[0]) == len(flat[1])
+    for x, y in zip(*flat):
+        assert torch.equal(x, y), kind
+    h.close()
