@@ -94,7 +94,16 @@ struct HipEvents {
     static void destroy(Event ev) { (void)hipEventDestroy(ev); }
     static hipError_t record(Event ev, Stream st) { return hipEventRecord(ev, st); }
     static hipError_t wait(Stream st, Event ev) { return hipStreamWaitEvent(st, ev, 0); }
-    static hipError_t host_wait(Event ev) { return hipEventSynchronize(ev); }
+    // also while this thread captures a stream (in the global mode such a call
+    // ends the capture)
+    static hipError_t host_wait(Event ev) {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) return e;
+        e = hipEventSynchronize(ev);
+        const hipError_t r = hipThreadExchangeStreamCaptureMode(&mode);
+        return e != hipSuccess ? e : r;
+    }
 };
 using StreamOrder = StreamOrderT<HipEvents>;
 

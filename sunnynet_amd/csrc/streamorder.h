@@ -29,7 +29,15 @@ public:
         at_ = st;
         return Rt::ok;
     }
-    Error follow(Stream st) { return set_ && st != at_ ? Rt::wait(st, ev_) : Rt::ok; }
+    // (A stream under capture cannot wait for an event from outside the capture:
+    // the host waits instead.)
+    Error follow(Stream st) {
+        if (!set_ || st == at_) return Rt::ok;
+        bool capturing = false;
+        const Error e = Rt::capturing(st, &capturing);
+        if (e != Rt::ok) return e;
+        return capturing ? Rt::host_wait(ev_) : Rt::wait(st, ev_);
+    }
     // The host waits for the mark.
     Error drain() { return set_ ? Rt::host_wait(ev_) : Rt::ok; }
 

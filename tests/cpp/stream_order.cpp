@@ -5,7 +5,8 @@
 //   bind S     the handle is bound to stream S
 //   async      an operation of the handle that returns before it is done
 //   quiet      one that does not mark
-//   capture S  S is being captured from here on; endcapture S ends it
+//   capture S  S is being captured from here on; endcapture S ends it (a call on
+//              it prints nothing: it runs when the capture is replayed)
 //   free       the handle's last wait: prints whether all operations are done
 #include <cstdint>
 #include <iostream>
@@ -54,7 +55,8 @@ int main() {
             std::cout << "free " << ((done & all) == all) << "\n";
         } else {
             if (!dev.cap[cur]) {
-                std::cout << n << " " << ((dev.streams[cur] & all) == all) << "\n";
+                const uint64_t done = dev.host | dev.streams[cur];
+                std::cout << n << " " << ((done & all) == all) << "\n";
                 all |= 1ull << n;
                 dev.streams[cur] |= 1ull << n;
                 ++n;

@@ -47,3 +47,9 @@ def test_every_stream_waits(sim, script):
 def test_capture_keeps_the_mark(sim):
     # a call captured on B marks nothing; the work on A is still waited for
     assert _ordered(sim("bind A;async;bind B;capture B;async;endcapture B;bind C;async;free"))
+
+
+def test_capture_waits_on_the_host(sim):
+    # the capturing stream cannot wait for A's event; what it captures is
+    # replayed later, on any stream, after the work that the handle had running
+    assert _ordered(sim("bind A;async;capture B;bind B;async;endcapture B;quiet;free"))

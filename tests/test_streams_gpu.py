@@ -134,3 +134,38 @@ def test_running_calls_move_between_streams(gpu, paths, monkeypatch, kind, betwe
     for x, y in zip(*flat):
         assert torch.equal(x, y), kind
     h.close()
+
+
+@pytest.mark.parametrize("running", [False, True])
+def test_prefill_captured_on_another_stream(gpu, paths, running):
+    """A prefill captured on a stream of its own, after (or while) the handle works
+    on another: every replay goes on from the state as an eager call does."""
+    print("prefill captured on another stream, work running:", running, flush=True)
+    h, ref = _make("sunny4", paths), _make("sunny4", paths)
+    rng = np.random.default_rng(7)
+    toks = torch.from_numpy(rng.integers(0, h.vocab, (4, 40)).astype(np.int32)).cuda()
+    side, cap = torch.cuda.Stream(), torch.cuda.Stream()
+    out = [x.prefill_batch(toks) for x in (h, ref)]      # workspaces and planes are there
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=cap):
+        if running:
+            with torch.cuda.stream(side):
+                h.prefill_batch(toks, logits=False)
+        lg = h.prefill_batch(toks)
+    torch.cuda.synchronize()
+    if running:
+        ref.prefill_batch(toks, logits=False)
+    for i in range(4):
+        want = ref.prefill_batch(toks)
+        state = ref.get_state(4)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(lg, want), i
+        assert all(torch.equal(a, b) for a, b in zip(h.get_state(4), state)), i
+    # and an eager call afterwards
+    assert torch.equal(h.prefill_batch(toks), ref.prefill_batch(toks))
+    assert torch.equal(out[0], out[1])
+    h.close()
+    ref.close()
