@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -89,6 +90,12 @@ struct HipEvents {
         const hipError_t e = hipStreamIsCapturing(st, &cs);
         *c = cs != hipStreamCaptureStatusNone;
         return e;
+    }
+    static unsigned long long id(Stream st) {
+        // odd for the per-thread streams, which no handle (an address) is
+        static std::atomic<unsigned long long> threads{0};
+        thread_local const unsigned long long mine = 2 * ++threads + 1;
+        return st == hipStreamPerThread ? mine : (unsigned long long)reinterpret_cast<uintptr_t>(st);
     }
     static hipError_t create(Event* ev) { return hipEventCreateWithFlags(ev, hipEventDisableTiming); }
     static void destroy(Event ev) { (void)hipEventDestroy(ev); }

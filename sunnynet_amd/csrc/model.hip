@@ -1354,6 +1354,12 @@ snhip_status check_usable(const SnHipModel* m) {
     return SNHIP_OK;
 }
 
+// Before a call's first operation: what other streams still run for the handle.
+snhip_status follow_streams(SnHipModel* m) {
+    SNHIP_CHECK(m->order.follow(m->stream));
+    return SNHIP_OK;
+}
+
 // Copies B tokens into m->tok on the caller's stream.
 snhip_status put_tokens(SnHipModel* m, const int32_t* t, int B, hipMemcpyKind kind) {
     SNHIP_CHECK(hipMemcpyAsync(m->tok, t, B * sizeof(int32_t), kind, m->stream));
@@ -1797,6 +1803,7 @@ void snhip_free(SnHipModel* m) {
 void snhip_reset(SnHipModel* m) {
     if (!m) return;
     const size_t B = m->max_batch;
+    (void)follow_streams(m);
     (void)hipMemsetAsync(m->s, 0, B * m->L * m->D * sizeof(float), m->stream);
     (void)hipMemsetAsync(m->hist, 0, B * m->L * (m->kh ? m->kh : 1) * m->D * sizeof(float),
                          m->stream);
@@ -1819,24 +1826,22 @@ int32_t snhip_batch_grid(const SnHipModel* m) { return m ? m->batch_wg : 0; }
 
 snhip_status snhip_set_stream(SnHipModel* m, void* stream) {
     if (!m) return SNHIP_E_INVAL;
-    if (m->stream == as_stream(stream)) return SNHIP_OK;
     m->stream = as_stream(stream);
     m->all_cus = stream_has_all_cus(m->stream);
-    SNHIP_CHECK(m->order.follow(m->stream));
     return SNHIP_OK;
 }
 
 snhip_status snhip_step_batch_dev(SnHipModel* m, const int32_t* tokens_dev, int32_t B,
                                   float* logits_dev) {
     if (!m || !tokens_dev || !logits_dev || B <= 0 || B > m->max_batch) return SNHIP_E_INVAL;
-    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (check_usable(m) != SNHIP_OK || follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     return B == 1 ? step_one(m, tokens_dev, logits_dev) : step_many(m, tokens_dev, B, logits_dev);
 }
 
 snhip_status snhip_step_batch(SnHipModel* m, const int32_t* tokens, int32_t B, float* logits) {
     if (!m || !tokens || !logits || B <= 0 || B > m->max_batch) return SNHIP_E_INVAL;
     if (!tokens_ok(m, tokens, B)) return SNHIP_E_INVAL;
-    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (check_usable(m) != SNHIP_OK || follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     snhip_status rc = put_tokens(m, tokens, B, hipMemcpyHostToDevice);
     if (rc == SNHIP_OK) rc = B == 1 ? step_one(m, m->tok, m->logits) : step_many(m, m->tok, B, m->logits);
     if (rc != SNHIP_OK) return rc;
@@ -1855,7 +1860,7 @@ void snhip_step(SnHipModel* m, int token, float* logits) {
 snhip_status snhip_prefill_host(SnHipModel* m, const int32_t* tokens, int32_t n, float* logits) {
     if (!m || !tokens || n <= 0 || !logits) return SNHIP_E_INVAL;
     if (!tokens_ok(m, tokens, n)) return SNHIP_E_INVAL;
-    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (check_usable(m) != SNHIP_OK || follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     int32_t* dt = nullptr;
     SNHIP_CHECK(hipMalloc(&dt, (size_t)n * sizeof(int32_t)));
     snhip_status rc = SNHIP_OK;
@@ -1887,13 +1892,13 @@ void snhip_prefill(SnHipModel* m, const int* tokens, int n, float* logits) {
 snhip_status snhip_prefill_batch_dev(SnHipModel* m, const int32_t* tokens_dev, int32_t B,
                                      int32_t T, float* logits_dev) {
     if (!m || !tokens_dev || B <= 0 || B > m->max_batch || T <= 0) return SNHIP_E_INVAL;
-    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (check_usable(m) != SNHIP_OK || follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     return run_prefill(m, tokens_dev, B, T, logits_dev);
 }
 
 snhip_status snhip_dbg_layer(SnHipModel* m, int32_t token, int32_t layer, float* dbg) {
     if (!m || !dbg || layer < 0 || layer >= m->L || token < 0 || token >= m->vocab) return SNHIP_E_INVAL;
-    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (check_usable(m) != SNHIP_OK || follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     const int D = m->D, I = m->I, R = m->R;
     const size_t hbs = (size_t)m->L * (m->kh ? m->kh : 1) * D;
     hipStream_t st = m->stream;
@@ -1934,7 +1939,7 @@ snhip_status snhip_prefill_all_dev(SnHipModel* m, const int32_t* tokens_dev, int
                                    int32_t T, float* logits_all_dev) {
     if (!m || !tokens_dev || !logits_all_dev || B <= 0 || B > m->max_batch || T <= 0)
         return SNHIP_E_INVAL;
-    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (check_usable(m) != SNHIP_OK || follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     return run_prefill(m, tokens_dev, B, T, nullptr, logits_all_dev);
 }
 
@@ -1943,7 +1948,7 @@ snhip_status snhip_decode_greedy_dev(SnHipModel* m, const int32_t* tokens_dev, i
                                      float* logits_dev) {
     if (!m || !tokens_dev || !out_tokens_dev || B <= 0 || B > m->max_batch || n_steps <= 0)
         return SNHIP_E_INVAL;
-    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (check_usable(m) != SNHIP_OK || follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     if (B == 1 && m->persist_wg && m->all_cus) {
         bool launch_failed = false;
         const snhip_status rc = run_persist(m, tokens_dev, 1, n_steps, true, out_tokens_dev, logits_dev, &launch_failed);
@@ -1989,6 +1994,7 @@ snhip_status snhip_decode_greedy_dev(SnHipModel* m, const int32_t* tokens_dev, i
 
 snhip_status snhip_get_state_dev(SnHipModel* m, float* s_dev, float* hist_dev, int32_t B) {
     if (!m || !s_dev || B <= 0 || B > m->max_batch || (m->kh && !hist_dev)) return SNHIP_E_INVAL;
+    if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     SNHIP_CHECK(hipMemcpyAsync(s_dev, m->s, (size_t)B * m->L * m->D * sizeof(float),
                                hipMemcpyDeviceToDevice, m->stream));
     if (m->kh)
@@ -2001,6 +2007,7 @@ snhip_status snhip_get_state_dev(SnHipModel* m, float* s_dev, float* hist_dev, i
 snhip_status snhip_set_state_dev(SnHipModel* m, const float* s_dev, const float* hist_dev,
                                  int32_t B) {
     if (!m || !s_dev || B <= 0 || B > m->max_batch || (m->kh && !hist_dev)) return SNHIP_E_INVAL;
+    if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     SNHIP_CHECK(hipMemcpyAsync(m->s, s_dev, (size_t)B * m->L * m->D * sizeof(float),
                                hipMemcpyDeviceToDevice, m->stream));
     if (m->kh)

@@ -475,6 +475,12 @@ snhip_status check_usable(const SnHipRwkv7* m) {
     return SNHIP_OK;
 }
 
+// Before a call's first operation: what other streams still run for the handle.
+snhip_status follow_streams(SnHipRwkv7* m) {
+    SNHIP_CHECK(m->order.follow(m->stream));
+    return SNHIP_OK;
+}
+
 SnHipRwkv7* load_rk(const char* path, int max_batch, int wfmt, int block) {
     if (!path || max_batch <= 0 || max_batch > 1024) { set_last_error("invalid arguments"); return nullptr; }
     if (wfmt != SNHIP_WEIGHTS_F32 && wfmt != SNHIP_WEIGHTS_INT4 && wfmt != SNHIP_WEIGHTS_STORED) {
@@ -844,6 +850,7 @@ bool tokens_ok(const SnHipRwkv7* m, const int32_t* t, int n) {
 snhip_status step_host(SnHipRwkv7* m, const int32_t* tokens, int B, float* logits) {
     if (!m || !tokens || !logits || B <= 0 || B > m->max_batch) return SNHIP_E_INVAL;
     if (!tokens_ok(m, tokens, B)) return SNHIP_E_INVAL;
+    if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     SNHIP_CHECK(hipMemcpyAsync(m->tok, tokens, B * sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
     const snhip_status rc = run_steps(m, nullptr, B, m->logits, false, 1);
     if (rc != SNHIP_OK) return rc;
@@ -981,6 +988,7 @@ snhip_status run_prefill(SnHipRwkv7* m, const int32_t* tokens, int n, float* log
 snhip_status prefill_host(SnHipRwkv7* m, const int32_t* tokens, int n, float* logits) {
     if (!m || !tokens || n <= 0 || !logits) return SNHIP_E_INVAL;
     if (!tokens_ok(m, tokens, n)) return SNHIP_E_INVAL;
+    if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     if (n >= kPfMin) {
         const snhip_status rc = run_prefill(m, tokens, n, m->logits);
         if (rc != SNHIP_OK) return rc;
@@ -1025,6 +1033,7 @@ void snhip_rk_free(SnHipRwkv7* m) {
 void snhip_rk_reset(SnHipRwkv7* m) {
     if (!m) return;
     const size_t B = m->max_batch;
+    (void)follow_streams(m);
     (void)hipMemsetAsync(m->S, 0, B * m->L * m->NH * m->HS * m->HS * sizeof(float), m->stream);
     (void)hipMemsetAsync(m->shift, 0, B * m->L * 2 * m->D * sizeof(float), m->stream);
     (void)hipStreamSynchronize(m->stream);
@@ -1042,7 +1051,7 @@ void snhip_rk_prefill(SnHipRwkv7* m, const int* tokens, int n, float* logits) {
 
 snhip_status snhip_rk_dbg(SnHipRwkv7* m, int token, int layer, float* out) {
     if (!m || !out || layer < 0 || layer >= m->L || token < 0 || token >= m->vocab) return SNHIP_E_INVAL;
-    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (check_usable(m) != SNHIP_OK || follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     const size_t n = (size_t)9 * m->D;
     float* d = ralloc<float>(m, n);
     if (!d) return SNHIP_E_NOMEM;
@@ -1065,10 +1074,8 @@ int snhip_rk_ready(const SnHipRwkv7* m) { return m && m->ready; }
 
 snhip_status snhip_rk_set_stream(SnHipRwkv7* m, void* stream) {
     if (!m) return SNHIP_E_INVAL;
-    if (m->stream == as_stream(stream)) return SNHIP_OK;
     m->stream = as_stream(stream);
     m->all_cus = stream_has_all_cus(m->stream);
-    SNHIP_CHECK(m->order.follow(m->stream));
     return SNHIP_OK;
 }
 
@@ -1087,6 +1094,7 @@ int32_t snhip_rk_persist_grid_batch(const SnHipRwkv7* m, int32_t B) {
 snhip_status snhip_rk_step_batch_dev(SnHipRwkv7* m, const int32_t* tokens_dev, int32_t B,
                                      float* logits_dev) {
     if (!m || !tokens_dev || !logits_dev || B <= 0 || B > m->max_batch) return SNHIP_E_INVAL;
+    if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     return run_steps(m, tokens_dev, B, logits_dev, false, 1);
 }
 
@@ -1095,6 +1103,7 @@ snhip_status snhip_rk_decode_greedy_dev(SnHipRwkv7* m, const int32_t* tokens_dev
                                         float* logits_dev) {
     if (!m || !tokens_dev || !out_tokens_dev || B <= 0 || B > m->max_batch || n_steps <= 0)
         return SNHIP_E_INVAL;
+    if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     if ((long)n_steps * B > (long)m->hist_cap || !m->tok_hist) {
         // Grow the token history.
         SNHIP_CHECK(hipStreamSynchronize(m->stream));
@@ -1123,6 +1132,7 @@ snhip_status snhip_rk_decode_greedy_dev(SnHipRwkv7* m, const int32_t* tokens_dev
 
 snhip_status snhip_rk_get_state_dev(SnHipRwkv7* m, float* S_dev, float* shift_dev, int32_t B) {
     if (!m || !S_dev || !shift_dev || B <= 0 || B > m->max_batch) return SNHIP_E_INVAL;
+    if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     SNHIP_CHECK(hipMemcpyAsync(S_dev, m->S, (size_t)B * m->L * m->NH * m->HS * m->HS * sizeof(float),
                                hipMemcpyDeviceToDevice, m->stream));
     SNHIP_CHECK(hipMemcpyAsync(shift_dev, m->shift, (size_t)B * m->L * 2 * m->D * sizeof(float),
@@ -1134,6 +1144,7 @@ snhip_status snhip_rk_get_state_dev(SnHipRwkv7* m, float* S_dev, float* shift_de
 snhip_status snhip_rk_set_state_dev(SnHipRwkv7* m, const float* S_dev, const float* shift_dev,
                                     int32_t B) {
     if (!m || !S_dev || !shift_dev || B <= 0 || B > m->max_batch) return SNHIP_E_INVAL;
+    if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     SNHIP_CHECK(hipMemcpyAsync(m->S, S_dev, (size_t)B * m->L * m->NH * m->HS * m->HS * sizeof(float),
                                hipMemcpyDeviceToDevice, m->stream));
     SNHIP_CHECK(hipMemcpyAsync(m->shift, shift_dev, (size_t)B * m->L * 2 * m->D * sizeof(float),

@@ -5,10 +5,11 @@ namespace snhip {
 
 // Calls of one handle are in order also across changes of the caller's stream:
 // each call that returns before its work is done marks the work's end on the
-// stream it ran on (mark), and every other stream the handle is bound to before
-// the next mark waits for it (follow), however many there are and whether or not
-// anything runs on them. Rt supplies streams and events, so that the rule runs
-// without a device too.
+// stream it ran on (mark), and every call before the next mark on any other stream
+// waits for it first (follow), however many there are. Streams are told apart by
+// Rt's number for them and not by their handle: the per-thread stream has one handle
+// in every thread. Rt supplies streams and events, so that the rule runs without a
+// device too.
 template <class Rt>
 class StreamOrderT {
 public:
@@ -26,13 +27,13 @@ public:
         if (!ev_ && (e = Rt::create(&ev_)) != Rt::ok) return e;
         if ((e = Rt::record(ev_, st)) != Rt::ok) return e;
         set_ = true;
-        at_ = st;
+        at_ = Rt::id(st);
         return Rt::ok;
     }
     // (A stream under capture cannot wait for an event from outside the capture:
     // the host waits instead.)
     Error follow(Stream st) {
-        if (!set_ || st == at_) return Rt::ok;
+        if (!set_ || Rt::id(st) == at_) return Rt::ok;
         bool capturing = false;
         const Error e = Rt::capturing(st, &capturing);
         if (e != Rt::ok) return e;
@@ -44,7 +45,7 @@ public:
 private:
     typename Rt::Event ev_{};
     bool set_ = false;
-    Stream at_{};
+    unsigned long long at_ = 0;
 };
 
 }  // namespace snhip

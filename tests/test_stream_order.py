@@ -39,6 +39,8 @@ def _ordered(lines):
     # freed on the third stream
     "bind A;async;bind B;bind C;free",
     "bind A;async;async;bind B;bind A;bind C;async;free",
+    # one handle value, several streams: the per-thread stream
+    "bind P;thread 1;async;thread 2;async;thread 1;async;free",
 ])
 def test_every_stream_waits(sim, script):
     assert _ordered(sim(script)), script

@@ -5,11 +5,13 @@ also while its earlier calls are still running."""
 from __future__ import annotations
 
 import threading
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
 import torch
 
+from sunnynet_amd import _native
 from sunnynet_amd.blob import pack_sunny_blob
 from sunnynet_amd.config import SMALL
 from sunnynet_amd.runtime.model import HipModel
@@ -169,3 +171,38 @@ def test_prefill_captured_on_another_stream(gpu, paths, running):
     assert torch.equal(out[0], out[1])
     h.close()
     ref.close()
+
+
+@pytest.mark.parametrize("kind", ["rwkv12", "sunny20"])
+def test_per_thread_stream_in_two_threads(gpu, paths, monkeypatch, kind):
+    """One handle bound to the per-thread stream (one handle value, another stream in
+    every thread), its calls alternating between two threads, none waited for."""
+    print("per-thread stream, two threads:", kind, flush=True)
+    monkeypatch.setenv("SNHIP_BATCH_PERSIST", "0")
+    lib = _native.lib()
+    step, bind = ((lib.snhip_rk_step_batch_dev, lib.snhip_rk_set_stream) if kind == "rwkv12"
+                  else (lib.snhip_step_batch_dev, lib.snhip_set_stream))
+    h = _make(kind, paths)
+    rng = np.random.default_rng(8)
+    n, B = 12, h.max_batch
+    toks = torch.from_numpy(rng.integers(0, h.vocab, (n, B)).astype(np.int32)).cuda()
+    out = torch.empty(2, n, B, h.vocab, device="cuda")
+    per_thread = 2          # hipStreamPerThread
+    h.step_batch(toks[0])   # the graph is captured
+    torch.cuda.synchronize()
+    for run in range(2):
+        h.reset()
+        _native.check(bind(h._h, per_thread if run else 0), "set_stream")
+        errs = []
+
+        def call(i):
+            rc = step(h._h, toks[i].data_ptr(), B, out[run, i].data_ptr())
+            if rc:
+                errs.append((i, rc))
+        with ThreadPoolExecutor(1) as a, ThreadPoolExecutor(1) as b:
+            for i in range(n):
+                (a, b)[i % 2].submit(call, i).result()
+            assert not errs, errs
+            torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1])
+    h.close()
