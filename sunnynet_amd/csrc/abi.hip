@@ -3,13 +3,12 @@
 // and version rules; the recurrence and INT4 primitives run on the GPU.
 #include <cstdio>
 #include <cstring>
-#include <mutex>
 #include <set>
 #include <thread>
 #include <utility>
-#include <vector>
 
 #include "common.h"
+#include "devgate.h"
 
 namespace snhip {
 namespace {
@@ -25,51 +24,31 @@ int host_threads() {
 }
 
 namespace {
-// The streams of the calls in flight that run persistent kernels, per device.
-struct Flight {
-    int dev;
-    hipStream_t st;
-};
-std::mutex g_flight_mu;
-std::vector<Flight> g_flight;
+constexpr int kMaxDevices = 64;
+DeviceGate g_gate[kMaxDevices];
 }  // namespace
 
-PersistCall::PersistCall(hipStream_t st) : st_(st) {
-    (void)hipGetDevice(&dev_);
-    std::lock_guard<std::mutex> lock(g_flight_mu);
-    g_flight.push_back(Flight{dev_, st_});
+hipError_t PersistCall::enter() {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
+    if ((e = hipStreamSynchronize(st_)) != hipSuccess) return e;
+    g_gate[dev].enter();
+    gate_ = &g_gate[dev];
+    return hipSuccess;
 }
 hipError_t PersistCall::finish() {
-    done_ = true;
-    return hipStreamSynchronize(st_);
-}
-PersistCall::~PersistCall() {
-    if (!done_) (void)hipStreamSynchronize(st_);
-    std::lock_guard<std::mutex> lock(g_flight_mu);
-    for (size_t i = 0; i < g_flight.size(); ++i)
-        if (g_flight[i].dev == dev_ && g_flight[i].st == st_) {
-            g_flight.erase(g_flight.begin() + (long)i);
-            break;
-        }
+    if (!gate_) return hipSuccess;
+    const hipError_t e = hipStreamSynchronize(st_);
+    gate_->leave();
+    gate_ = nullptr;
+    return e;
 }
 
 hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st) {
     if (env_unsigned("SNHIP_COOP", 0, 0) != 0) return hipLaunchCooperativeKernel(k, grid, block, args, 0, st);
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    // Held over the launch: of two calls, the later one sees the earlier one's
-    // kernel on its stream (a call stays listed until its kernels are done).
-    std::lock_guard<std::mutex> lock(g_flight_mu);
-    for (const Flight& f : g_flight) {
-        if (e != hipSuccess) return e;
-        if (f.dev != dev || f.st == st) continue;
-        hipEvent_t ev = nullptr;
-        if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
-        e = hipEventRecord(ev, f.st);
-        if (e == hipSuccess) e = hipStreamWaitEvent(st, ev, 0);
-        (void)hipEventDestroy(ev);
-    }
-    return e != hipSuccess ? e : hipLaunchKernel(k, grid, block, args, 0, st);
+    return hipLaunchKernel(k, grid, block, args, 0, st);
 }
 
 bool stream_has_all_cus(hipStream_t st) {

@@ -52,21 +52,24 @@ inline unsigned env_unsigned(const char* name, unsigned dflt, unsigned lo) {
     return v < (long)lo ? lo : (unsigned)v;
 }
 
-// A call that runs grid-synchronizing persistent kernels on `st`: from before
-// its first launch until those kernels have finished (the destructor waits for
-// them unless finish() has). See launch_persistent.
+// A call that runs grid-synchronizing persistent kernels on `st`. enter() waits
+// until what is queued on the stream is done and then for the device's gate;
+// finish() waits for the call's kernels and opens the gate (so does the destructor).
+// Whoever holds the gate thus waits for its own kernels only: nothing on a stream,
+// of this library or not, that depends on another call's result is waited for under
+// it.
 class PersistCall {
 public:
-    explicit PersistCall(hipStream_t st);
-    ~PersistCall();
-    hipError_t finish();   // waits for the stream
+    explicit PersistCall(hipStream_t st) : st_(st) {}
+    ~PersistCall() { (void)finish(); }
+    hipError_t enter();
+    hipError_t finish();
     PersistCall(const PersistCall&) = delete;
     PersistCall& operator=(const PersistCall&) = delete;
 
 private:
     hipStream_t st_;
-    int dev_ = 0;
-    bool done_ = false;
+    class DeviceGate* gate_ = nullptr;   // held
 };
 
 // Launches a grid-synchronizing persistent kernel whose grid is sized to
@@ -74,8 +77,7 @@ private:
 // inside a PersistCall on `st`. It is an ordinary launch: a cooperative one goes
 // through a queue of its own with host-side waits on both ends, about 60 us per
 // call (SunnyNet-100M fp32 B = 1 step 315 -> 258 us). What the cooperative queue
-// also gave, that no two such kernels share the device, is kept by ordering each
-// launch after the work queued by every other call in flight on the device.
+// also gave, that no two such kernels share the device, the gate keeps.
 // SNHIP_COOP=1 launches cooperatively.
 hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st);
 

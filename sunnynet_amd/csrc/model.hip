@@ -1380,11 +1380,12 @@ snhip_status run_steps(SnHipModel* m, const int32_t* tok, int B, float* logits_o
     }
     if (!m->use_graphs || batch) {
         // The batched persistent step is a handful of launches per step: they
-        // are queued directly (ordered against other calls' persistent launches).
+        // are queued directly.
         std::optional<PersistCall> call;
         if (batch) {
             m->persist_stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
             call.emplace(m->stream);
+            SNHIP_CHECK(call->enter());
         }
         for (int i = 0; i < reps; ++i) {
             const snhip_status rc = enqueue_step(m, tok, B, logits_out, greedy, m->stream);
@@ -1682,6 +1683,7 @@ snhip_status run_persist(SnHipModel* m, const int32_t* tok, int B, int n_steps, 
                          float* logits, bool* launch_failed) {
     constexpr int kMaxStepsPerLaunch = 1 << 20;   // keeps exchange epochs far from wrapping
     PersistCall call(m->stream);
+    SNHIP_CHECK(call.enter());
     PersistArgs a{};
     a.layers = m->dlayers;
     a.L = m->L; a.D = m->D; a.I = m->I; a.R = m->R; a.K = m->K; a.kh = m->kh;

@@ -431,6 +431,7 @@ bool uses_mi(const SnHipRwkv7* m, int B) { return m->p_grid > 0 && m->all_cus &&
 constexpr int kRkPStepsPerLaunch = 1024;
 snhip_status run_persist(SnHipRwkv7* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps) {
     PersistCall call(m->stream);
+    SNHIP_CHECK(call.enter());
     RkPArgs a = m->p_args;
     a.stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
     a.logits = logits_out;

@@ -4,7 +4,9 @@ share the device), and a handle that moves between streams goes on from its stat
 also while its earlier calls are still running."""
 from __future__ import annotations
 
+import ctypes
 import threading
+import time
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -206,3 +208,90 @@ def test_per_thread_stream_in_two_threads(gpu, paths, monkeypatch, kind):
             torch.cuda.synchronize()
     assert torch.equal(out[0], out[1])
     h.close()
+
+
+@pytest.mark.parametrize("a,b", [("sunny1", "rwkv1"), ("sunny4", "sunny20")])
+def test_two_threads_per_thread_stream(gpu, paths, a, b):
+    """Two handles bound to the per-thread stream, stepped from two threads at once."""
+    print("two threads, per-thread streams:", a, b, flush=True)
+    n, per_thread = 24, 2
+    h = {k: _make(k, paths) for k in (a, b)}
+    rng = np.random.default_rng(9)
+    toks = {k: torch.from_numpy(rng.integers(0, h[k].vocab, (n, h[k].max_batch)).astype(np.int32)).cuda()
+            for k in (a, b)}
+    want = {k: torch.stack([h[k].step_batch(t) for t in toks[k]]) for k in (a, b)}
+    got = {k: torch.empty_like(want[k]) for k in (a, b)}
+    lib = _native.lib()
+    torch.cuda.synchronize()
+    errs = []
+
+    def work(k):
+        rk = "_rk" if k.startswith("rwkv") else ""
+        step, bind = getattr(lib, f"snhip{rk}_step_batch_dev"), getattr(lib, f"snhip{rk}_set_stream")
+        rc = bind(h[k]._h, per_thread)
+        for i in range(n):
+            rc = rc or step(h[k]._h, toks[k][i].data_ptr(), h[k].max_batch, got[k][i].data_ptr())
+        if rc:
+            errs.append((k, rc, _native.last_error()))
+    for k in (a, b):
+        h[k].reset()
+    torch.cuda.synchronize()
+    ts = [threading.Thread(target=work, args=(k,)) for k in (a, b)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errs, errs
+    for k in (a, b):
+        assert torch.equal(got[k], want[k]), k
+        h[k].close()
+
+
+def test_a_call_does_not_wait_for_foreign_work(gpu, paths):
+    """A call whose stream is busy with work of the caller's (here 0.6 s of it) does
+    not hold up a step of another handle on another stream: that work may be waiting
+    for the step's result."""
+    print("a step beside a call that is behind other work", flush=True)
+    ha, hb = _make("sunny1", paths), _make("rwkv1", paths)
+    t = torch.zeros(1, dtype=torch.int32, device="cuda")
+    ha.step_batch(t)
+    hb.step_batch(t)
+    n = 1_000_000
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    torch.cuda._sleep(n)
+    ev[0].record()
+    torch.cuda._sleep(n)
+    ev[1].record()
+    torch.cuda.synchronize()
+    sa, busy = torch.cuda.Stream(), torch.cuda.Event()
+    with torch.cuda.stream(sa):
+        torch.cuda._sleep(int(n * 600 / ev[0].elapsed_time(ev[1])))
+        busy.record()
+    # a stream that the runtime has not put on the busy one's hardware queue
+    sb = None
+    for c in [torch.cuda.Stream() for _ in range(8)]:
+        with torch.cuda.stream(c):
+            t.clone()
+            e = torch.cuda.Event()
+            e.record()
+        time.sleep(0.01)
+        if e.query():
+            sb = c
+            break
+    assert sb is not None and not busy.query()
+
+    def first():
+        with torch.cuda.stream(sa):
+            ha.step_batch(t)
+    th = threading.Thread(target=first)
+    th.start()
+    time.sleep(0.1)             # the first call is waiting by now
+    with torch.cuda.stream(sb):
+        hb.step_batch(t)
+    still = not busy.query()      # (the step returns when it is done)
+    th.join()
+    torch.cuda.synchronize()
+    assert still, "the second handle's step waited for the first one's stream"
+    ha.close()
+    hb.close()
