@@ -3,6 +3,9 @@
 // and version rules; the recurrence and INT4 primitives run on the GPU.
 #include <cstdio>
 #include <cstring>
+#include <map>
+#include <memory>
+#include <mutex>
 #include <set>
 #include <thread>
 #include <utility>
@@ -24,18 +27,35 @@ int host_threads() {
 }
 
 namespace {
-constexpr int kMaxDevices = 64;
-DeviceGate g_gate[kMaxDevices];
+// A gate that another process has not opened for this long is passed with a
+// cooperative launch: the longest hold is a launch of a second or so.
+constexpr double kGateSeconds = 60.0;
+thread_local bool t_shared = false;   // this thread's PersistCall holds the gate against its process only
+
+// The device's gate; its files are named by the card's PCI address.
+DeviceGate* gate_of(int dev) {
+    static std::mutex mu;
+    static std::map<int, std::unique_ptr<DeviceGate>> gates;
+    std::lock_guard<std::mutex> lock(mu);
+    std::unique_ptr<DeviceGate>& g = gates[dev];
+    if (!g) {
+        char pci[64] = "unknown";
+        if (hipDeviceGetPCIBusId(pci, sizeof pci, dev) != hipSuccess) (void)hipGetLastError();
+        const char* dir = getenv("SNHIP_LOCK_DIR");
+        g.reset(new DeviceGate(std::string(dir ? dir : "/tmp") + "/snhip-" + pci + ".lock"));
+    }
+    return g.get();
+}
 }  // namespace
 
 hipError_t PersistCall::enter() {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
     if ((e = hipStreamSynchronize(st_)) != hipSuccess) return e;
-    g_gate[dev].enter();
-    gate_ = &g_gate[dev];
+    DeviceGate* g = gate_of(dev);
+    t_shared = !g->enter(kGateSeconds);
+    gate_ = g;
     return hipSuccess;
 }
 hipError_t PersistCall::finish() {
@@ -43,11 +63,13 @@ hipError_t PersistCall::finish() {
     const hipError_t e = hipStreamSynchronize(st_);
     gate_->leave();
     gate_ = nullptr;
+    t_shared = false;
     return e;
 }
 
 hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st) {
-    if (env_unsigned("SNHIP_COOP", 0, 0) != 0) return hipLaunchCooperativeKernel(k, grid, block, args, 0, st);
+    if (t_shared || env_unsigned("SNHIP_COOP", 0, 0) != 0)
+        return hipLaunchCooperativeKernel(k, grid, block, args, 0, st);
     return hipLaunchKernel(k, grid, block, args, 0, st);
 }
 

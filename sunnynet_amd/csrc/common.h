@@ -77,9 +77,16 @@ private:
 // inside a PersistCall on `st`. It is an ordinary launch: a cooperative one goes
 // through a queue of its own with host-side waits on both ends, about 60 us per
 // call (SunnyNet-100M fp32 B = 1 step 315 -> 258 us). What the cooperative queue
-// also gave, that no two such kernels share the device, the gate keeps.
-// SNHIP_COOP=1 launches cooperatively.
+// also gave, that no two such kernels share the device, the gate keeps, among this
+// process's threads and among the processes that see its files (in SNHIP_LOCK_DIR,
+// by default /tmp; containers that share a card share that folder, or set
+// SNHIP_COOP=1). Without the files, and with SNHIP_COOP=1, the launch is cooperative.
 hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st);
+
+// Steps of one launch, or of the launches of one hold of the gate, so that other
+// callers wait for a fraction of a second and not for a whole decode: giving the
+// gate away and back costs a launch and a wait of the host, about 15 us.
+constexpr int kPersistHoldSteps = 1024;
 
 // StreamOrderT on the device.
 struct HipEvents {

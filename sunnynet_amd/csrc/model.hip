@@ -18,7 +18,6 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
-#include <optional>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -1378,25 +1377,26 @@ snhip_status run_steps(SnHipModel* m, const int32_t* tok, int B, float* logits_o
         if (rc != SNHIP_OK) return rc;
         tok = m->tok;
     }
-    if (!m->use_graphs || batch) {
+    if (batch) {
         // The batched persistent step is a handful of launches per step: they
-        // are queued directly.
-        std::optional<PersistCall> call;
-        if (batch) {
-            m->persist_stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
-            call.emplace(m->stream);
-            SNHIP_CHECK(call->enter());
+        // are queued directly. The call returns once its launches have finished,
+        // so that a barrier time-out is reported by this call, not a later one.
+        m->persist_stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
+        for (int i = 0; i < reps;) {
+            PersistCall call(m->stream);
+            SNHIP_CHECK(call.enter());
+            for (const int end = std::min(reps, i + kPersistHoldSteps); i < end; ++i) {
+                const snhip_status rc = enqueue_step(m, tok, B, logits_out, greedy, m->stream);
+                if (rc != SNHIP_OK) return rc;
+            }
+            SNHIP_CHECK(call.finish());
+            const snhip_status st = persist_status(m, B);
+            if (st != SNHIP_OK) return st;
         }
+    } else if (!m->use_graphs) {
         for (int i = 0; i < reps; ++i) {
             const snhip_status rc = enqueue_step(m, tok, B, logits_out, greedy, m->stream);
             if (rc != SNHIP_OK) return rc;
-        }
-        if (batch) {
-            // The call returns once its launches have finished, so that a
-            // barrier time-out is reported by this call, not a later one.
-            SNHIP_CHECK(call->finish());
-            const snhip_status st = persist_status(m, B);
-            if (st != SNHIP_OK) return st;
         }
     } else {
         const auto key = std::make_tuple(B, (const void*)logits_out, greedy ? 1 : 0);
@@ -1420,7 +1420,7 @@ snhip_status run_steps(SnHipModel* m, const int32_t* tok, int B, float* logits_o
         }
         for (int i = 0; i < reps; ++i) SNHIP_CHECK(hipGraphLaunch(it->second, m->stream));
     }
-    SNHIP_CHECK(m->order.mark(m->stream));
+    if (!batch) SNHIP_CHECK(m->order.mark(m->stream));   // (the batched step is done)
     return SNHIP_OK;
 }
 
@@ -1681,9 +1681,6 @@ snhip_status run_prefill(SnHipModel* m, const int32_t* tokens_dev, int B, int T,
 // first cooperative launch could not be queued at all (nothing ran).
 snhip_status run_persist(SnHipModel* m, const int32_t* tok, int B, int n_steps, bool greedy, int32_t* out_tok,
                          float* logits, bool* launch_failed) {
-    constexpr int kMaxStepsPerLaunch = 1 << 20;   // keeps exchange epochs far from wrapping
-    PersistCall call(m->stream);
-    SNHIP_CHECK(call.enter());
     PersistArgs a{};
     a.layers = m->dlayers;
     a.L = m->L; a.D = m->D; a.I = m->I; a.R = m->R; a.K = m->K; a.kh = m->kh;
@@ -1699,7 +1696,7 @@ snhip_status run_persist(SnHipModel* m, const int32_t* tok, int B, int n_steps, 
     const int blk = persist_blk(m);
     const int grid = B == 1 ? m->persist_wg : B * m->mi_grid[B];
     for (int done = 0; done < n_steps;) {
-        const int n = std::min(n_steps - done, kMaxStepsPerLaunch);
+        const int n = std::min(n_steps - done, kPersistHoldSteps);
         // A launch uses 4 L + 1 exchange epochs and one state epoch per step;
         // before they would wrap, the words start over from zero.
         const uint64_t n_ep = (uint64_t)n * (4 * (uint64_t)m->L + 1) + 2;
@@ -1717,15 +1714,18 @@ snhip_status run_persist(SnHipModel* m, const int32_t* tok, int B, int n_steps, 
         a.out_tok = greedy ? out_tok + (size_t)done * B : nullptr;
         a.logits = done + n == n_steps ? logits : nullptr;
         a.n_steps = n;
-        const snhip_status rc = launch_decode_persist(a, grid, blk, m->stream);
+        PersistCall call(m->stream);
+        SNHIP_CHECK(call.enter());
+        snhip_status rc = launch_decode_persist(a, grid, blk, m->stream);
         if (rc != SNHIP_OK) {
             if (done == 0 && launch_failed) *launch_failed = true;
             return rc;
         }
+        SNHIP_CHECK(call.finish());
+        if ((rc = persist_status(m, B)) != SNHIP_OK) return rc;
         done += n;
     }
-    SNHIP_CHECK(call.finish());
-    return persist_status(m, B);
+    return SNHIP_OK;
 }
 
 // Does a step of B >= 2 sequences run as B instances of the single-sequence

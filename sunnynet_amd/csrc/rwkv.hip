@@ -422,16 +422,13 @@ void setup_rkq_tiles(SnHipRwkv7* m) {
 bool uses_mi(const SnHipRwkv7* m, int B) { return m->p_grid > 0 && m->all_cus && B >= 2 && B <= m->p_mi_max; }
 
 // reps persistent steps of sequences [0, B) on tok (device; B = 1, or
-// 2..p_mi_max on a grid slice each): greedy, one launch of up to kRkPStepsPerLaunch steps at a
+// 2..p_mi_max on a grid slice each): greedy, one launch of up to kPersistHoldSteps steps at a
 // time, otherwise one launch per step; every step has its own epoch. The
 // call waits for them and reports a time-out of an exchange wait as an error.
 // The kernel updates S and shift in place layer by layer, so a time-out
 // leaves them part-stepped: the handle is then refused for stepping until its
 // state is reset or set.
-constexpr int kRkPStepsPerLaunch = 1024;
 snhip_status run_persist(SnHipRwkv7* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps) {
-    PersistCall call(m->stream);
-    SNHIP_CHECK(call.enter());
     RkPArgs a = m->p_args;
     a.stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
     a.logits = logits_out;
@@ -441,7 +438,7 @@ snhip_status run_persist(SnHipRwkv7* m, const int32_t* tok, int B, float* logits
     a.ni = B;
     const int grid = B == 1 ? m->p_grid : B * m->p_mi_grid[B];
     for (int i = 0; i < reps;) {
-        const int n = greedy ? std::min(reps - i, kRkPStepsPerLaunch) : 1;
+        const int n = greedy ? std::min(reps - i, kPersistHoldSteps) : 1;
         if (m->p_epoch > 0xFFFFFFFFu - (unsigned)n) {
             // epochs start over from clean words
             SNHIP_CHECK(hipMemsetAsync(m->p_words, 0, m->p_nwords * sizeof(unsigned long long), m->stream));
@@ -452,17 +449,19 @@ snhip_status run_persist(SnHipRwkv7* m, const int32_t* tok, int B, float* logits
         a.hist0 = i;
         m->p_epoch += (unsigned)n;
         a.tok_in = i == 0 ? tok : m->tok;
+        PersistCall call(m->stream);
+        SNHIP_CHECK(call.enter());
         const snhip_status rc = m->p_exact ? launch_rk_exact(a, grid, m->stream) : launch_rk_persist(a, grid, m->stream);
         if (rc != SNHIP_OK) return rc;
+        SNHIP_CHECK(call.finish());
+        if (*m->h_err) {
+            *m->h_err = 0;
+            m->poisoned = 1;
+            SNHIP_CHECK(hipMemsetAsync(m->p_err, 0, sizeof(unsigned), m->stream));
+            set_last_error("RWKV-7 persistent step: an exchange wait timed out");
+            return SNHIP_E_DEVICE;
+        }
         i += n;
-    }
-    SNHIP_CHECK(call.finish());
-    if (*m->h_err) {
-        *m->h_err = 0;
-        m->poisoned = 1;
-        SNHIP_CHECK(hipMemsetAsync(m->p_err, 0, sizeof(unsigned), m->stream));
-        set_last_error("RWKV-7 persistent step: an exchange wait timed out");
-        return SNHIP_E_DEVICE;
     }
     return SNHIP_OK;
 }

@@ -4,10 +4,12 @@ share the device), and a handle that moves between streams goes on from its stat
 also while its earlier calls are still running."""
 from __future__ import annotations
 
-import ctypes
+import subprocess
+import sys
 import threading
 import time
 from concurrent.futures import ThreadPoolExecutor
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -295,3 +297,50 @@ def test_a_call_does_not_wait_for_foreign_work(gpu, paths):
     assert still, "the second handle's step waited for the first one's stream"
     ha.close()
     hb.close()
+
+
+_CHILD = """
+import sys
+import numpy as np, torch
+sys.path.insert(0, sys.argv[1])
+from sunnynet_amd.config import SMALL as c
+from sunnynet_amd.runtime.model import HipModel
+h = HipModel(sys.argv[2], c.vocab_size, c.dim, c.inner, c.rank, c.taps, c.layers, max_batch=4)
+rng = np.random.default_rng(5)
+toks = [torch.from_numpy(rng.integers(0, h.vocab, 4).astype(np.int32)).cuda() for _ in range(24)]
+torch.cuda.synchronize()
+print("ready", flush=True)
+sys.stdin.readline()
+for _ in range(20):
+    h.reset()
+    out = torch.stack([h.step_batch(t) for t in toks]).cpu().numpy()
+np.save(sys.argv[3], out)
+h.close()
+"""
+
+
+@pytest.mark.parametrize("n,lock_dir", [(2, "shared"), (1, "none")])
+def test_processes(gpu, paths, tmp_path, monkeypatch, n, lock_dir):
+    """Two processes that step on one device at once: each gets what it gets alone.
+    Without a folder for the lock files the launches are cooperative."""
+    print("processes:", n, "lock folder:", lock_dir, flush=True)
+    monkeypatch.setenv("SNHIP_LOCK_DIR", str(tmp_path if lock_dir == "shared" else tmp_path / "missing"))
+    root = str(Path(__file__).resolve().parents[1])
+    ps = [subprocess.Popen([sys.executable, "-c", _CHILD, root, str(paths[0]), str(tmp_path / f"o{i}.npy")],
+                           stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True) for i in range(n)]
+    try:
+        for p in ps:
+            assert p.stdout.readline() == "ready\n"
+        for p in ps:
+            p.stdin.write("\n")
+            p.stdin.flush()
+        assert [p.wait(60) for p in ps] == [0] * n
+    finally:
+        for p in ps:
+            p.kill()
+    assert (len(list(tmp_path.glob("snhip-*.lock*"))) == 2) == (lock_dir == "shared")
+    h = _make("sunny4", paths)
+    want = torch.stack(_run(h, "sunny4", 24, [torch.cuda.current_stream()])).numpy()
+    for i in range(n):
+        assert np.array_equal(np.load(tmp_path / f"o{i}.npy"), want), i
+    h.close()
