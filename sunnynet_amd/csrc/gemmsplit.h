@@ -1,10 +1,18 @@
-// Products of many rows on the fp16 matrix cores at fp32 accuracy (gemmsplit.hip).
+// Products of many rows on the fp16 matrix cores from operands in two fp16 planes
+// (gemmsplit.hip).
 //
 // A row x of K floats is held as 2^s x = h + l in two fp16 planes, s the power of
 // two that takes the row's largest magnitude into [2^14, 2^15): h rounds 2^s x to
 // 11 bits, l the exact remainder to 11 more, so h + l differs from 2^s x by at most
-// 2^-22 of it or 2^-25. A product is X W^T = 2^-(sx + sw) (Hx Hw + Hx Lw + Lx Hw),
-// accumulated in fp32; Lx Lw, below 2^-22 of a term, is left out.
+// 2^-22 of it or 2^-24: 22 bits where fp32 has 24, and fewer for values below 2^-17
+// of their row's largest. A product is X W^T = 2^-(sx + sw) (Hx Hw + (Hx Lw + Lx Hw)),
+// accumulated in fp32, the two parts apart; Lx Lw, below 2^-22 of a term, is left
+// out. What these leave out is less than what the sums round: against 64 bits the
+// outputs are nearer than with the fp32 matrix cores, whose sums are rounded once
+// per two values of k and these once per 16. SunnyNet-100M and -small, 1 to 16
+// prompts of 64 to 2048 tokens, fp32, fp16 and INT4 weights (57 calls of two seeds):
+// the error of logits 0.38 to 0.75 of theirs, of states 0.76 to 0.99. (With one
+// accumulator for the three products it was up to 1.16 of theirs.)
 #pragma once
 
 #include <climits>

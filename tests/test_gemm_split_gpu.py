@@ -4,15 +4,18 @@ widths around the tiles and stages, split K and whole, in each weight format and
 across chunks; with weights of very different magnitudes; and with infinities.
 
 Bar: the prefill's own against the oracle (logits within 2e-5, states within 1e-5);
-both forms round in fp32, so neither is the other's reference."""
+both forms round in fp32, so neither is the other's reference. Against 64 bits the
+planes' error is to be no larger than that of the fp32 matrix cores."""
 from __future__ import annotations
 
 import numpy as np
 import pytest
 import torch
 
+import oracle
+from oracle.torch_ref import TorchSunny, forward_hist_to_step
 from sunnynet_amd.blob import pack_sunny_blob
-from sunnynet_amd.config import SMALL, TINY
+from sunnynet_amd.config import SMALL, SUNNY_100M, TINY
 from sunnynet_amd.runtime.model import HipModel
 from sunnynet_amd.weights import gaussian_matmuls, init_sunnynet
 
@@ -51,6 +54,44 @@ def test_matches_fp32_products(gpu, tmp_path, monkeypatch, cfg, B, T, kw, chunk)
     a, b = _both(monkeypatch, p, cfg, toks, **kw)
     assert np.abs(a[0] - b[0]).max() < TOL
     assert np.abs(a[1] - b[1]).max() < 1e-5 and np.abs(a[2] - b[2]).max() < 1e-5
+
+
+def _in_64_bits(w, toks, block):
+    """Logits, s and hist of the prefill in 64 bits, from what the handle multiplies:
+    decay and W_eff rounded to fp32 as in the blob, INT4 values dequantized."""
+    ref, ref32 = TorchSunny(w, torch.float64), TorchSunny(w, torch.float32)
+
+    def mat(m):
+        m = m.float().contiguous()
+        if block:
+            m = torch.from_numpy(oracle.dequant_i4(*oracle.quant_i4(m.numpy(), block), m.shape[1], block))
+        return m.double()
+    for a, b in zip(ref.layers, ref32.layers):
+        a.delta = b.delta.double()
+        a.V, a.U, a.W_z, a.W_c, a.W_eff = (mat(m) for m in (b.V, b.U, b.W_z, b.W_c, b.W_eff))
+    ref.head = mat(ref32.head)
+    lg, (s, hist) = ref.forward(toks.long().cpu())
+    return lg, s, forward_hist_to_step(hist)
+
+
+@pytest.mark.parametrize("block", [0, 32])
+@pytest.mark.parametrize("B,T", [(4, 200), (1, 999), (16, 64)])
+def test_error_against_64_bits(gpu, tmp_path, monkeypatch, B, T, block):
+    """At the 100M model's width, split K and whole: no output is further from the
+    64-bit result than with the products on the fp32 matrix cores (2-norm)."""
+    print("split products against 64 bits", B, T, block, flush=True)
+    cfg = SUNNY_100M.with_(vocab_size=512, layers=4)
+    w = gaussian_matmuls(init_sunnynet(cfg, 0), seed=8)
+    p = tmp_path / "m.bin"
+    p.write_bytes(pack_sunny_blob(w))
+    toks = torch.from_numpy(np.random.default_rng(T).integers(0, cfg.vocab_size, (B, T)).astype(np.int32)).to(gpu)
+    kw = {"weights": "int4", "block": block} if block else {}
+    split, fp32 = _both(monkeypatch, p, cfg, toks, **kw)
+    for x, y, e in zip(split, fp32, _in_64_bits(w, toks, block)):
+        e = e.numpy()
+        es, ef = (np.linalg.norm(v - e) / np.linalg.norm(e) for v in (x, y))
+        print(f"  planes {es:.3e}, fp32 matrix cores {ef:.3e}", flush=True)
+        assert es <= ef
 
 
 def test_rows_of_any_magnitude(gpu, tmp_path, monkeypatch):
