@@ -54,6 +54,9 @@ __device__ __forceinline__ void split_store(const float (&y)[8], int s, bool bad
         if (bad && fabsf(x) < __builtin_inff()) x = x == 0.0f ? 0.0f : copysignf(1.0f, x);
         h[j] = (_Float16)x;
         l[j] = bad ? (_Float16)0.0f : (_Float16)(x - (float)h[j]);
+        // too small for either plane, but not zero: the smallest value of its sign, so
+        // that it times an infinity is one
+        if ((float)h[j] == 0.0f && (float)l[j] == 0.0f && y[j] != 0.0f) l[j] = (_Float16)copysignf(0x1p-24f, y[j]);
     }
     half8* o = reinterpret_cast<half8*>(pl + (((size_t)(row >> 5) * nk + (k >> 4)) << 10)) + ((k >> 3) & 1) * 32 +
                (row & 31);

@@ -128,3 +128,30 @@ def test_infinite_weights_and_bad_tokens(gpu, tmp_path, monkeypatch, where):
         assert np.array_equal(np.isinf(x), np.isinf(y)) and np.array_equal(x[np.isinf(x)], y[np.isinf(y)])
         fin = np.isfinite(y)
         assert fin.sum() == 0 or np.abs(x[fin] - y[fin]).max() < TOL
+
+
+@pytest.mark.parametrize("where", ["row of W", "row of X"])
+def test_tiny_value_times_infinity(gpu, tmp_path, monkeypatch, where):
+    """A value too small for the planes beside its row's largest, times an infinity,
+    is that infinity and not zero times it: in the vocabulary head, an infinite
+    weight on a channel of 2^-60, and an infinite channel on a weight of 2^-60 (and
+    of 2^-149, fp32's smallest)."""
+    print("split products, tiny times infinity:", where, flush=True)
+    cfg = TINY.with_(layers=1)
+    w = gaussian_matmuls(init_sunnynet(cfg, 0), seed=9)
+    if where == "row of W":
+        w.no_g[3], w.no_c[3] = 2.0 ** -60, 0.0
+        w.embed[7, 3] = float("inf")
+    else:
+        w.no_c[3] = float("inf")
+        w.embed[9, 3], w.embed[11, 3], w.embed[13, 3], w.embed[15, 3] = 2.0 ** -60, -2.0 ** -149, 0.0, -0.0
+    p = tmp_path / "m.bin"
+    p.write_bytes(pack_sunny_blob(w))
+    toks = np.random.default_rng(3).integers(20, cfg.vocab_size, (3, 50)).astype(np.int32)
+    a, b = _both(monkeypatch, p, cfg, torch.from_numpy(toks).to(gpu))
+    assert np.isinf(b[0]).any() and np.isinf(b[0][..., 7 if where == "row of W" else 9]).all()
+    assert np.array_equal(np.isnan(a[0]), np.isnan(b[0]))
+    assert np.array_equal(a[0][np.isinf(b[0])], b[0][np.isinf(b[0])])
+    fin = np.isfinite(b[0])
+    assert np.isfinite(a[0][fin]).all()
+    assert fin.sum() == 0 or np.abs(a[0][fin] - b[0][fin]).max() < TOL
