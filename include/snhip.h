@@ -169,6 +169,13 @@ int32_t snhip_persistent_grid_batch(const SnHipModel* m, int32_t B);
  * steps one sequence at a time (sunnynet.c:212). */
 int32_t snhip_batch_grid(const SnHipModel* m);
 
+/* Bytes of device memory that the handles of this process hold (SunnyNet and
+ * RWKV-7: weights, their copies for the kernels, state and workspaces). With
+ * SNHIP_MEM_LIMIT=<bytes> in the environment, read at every allocation, they
+ * take no more than that in all: what can be done without (weight copies, a
+ * large prefill workspace) is left out, and a call that needs more fails. */
+uint64_t snhip_device_bytes(void);
+
 /* State of sequences [0, B) in the SunnyState layout above, device pointers. */
 snhip_status snhip_get_state_dev(SnHipModel* m, float* s_dev, float* hist_dev, int32_t B);
 snhip_status snhip_set_state_dev(SnHipModel* m, const float* s_dev, const float* hist_dev,

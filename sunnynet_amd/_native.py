@@ -87,6 +87,7 @@ _SIGS = {
     "snhip_persistent_grid": (I32, [V]),
     "snhip_persistent_grid_batch": (I32, [V, I32]),
     "snhip_batch_grid": (I32, [V]),
+    "snhip_device_bytes": (ctypes.c_uint64, []),
     "snhip_step_batch_dev": (I32, [V, V, I32, V]),
     "snhip_step_batch": (I32, [V, V, I32, V]),
     "snhip_decode_greedy_dev": (I32, [V, V, I32, I32, V, V]),

@@ -8,10 +8,12 @@
 #include <mutex>
 #include <set>
 #include <thread>
+#include <unordered_map>
 #include <utility>
 
 #include "common.h"
 #include "devgate.h"
+#include "snhip.h"
 
 namespace snhip {
 namespace {
@@ -24,6 +26,39 @@ int host_threads() {
     if (g_threads > 0) return g_threads;
     const unsigned n = std::thread::hardware_concurrency();
     return n > 0 ? (int)n : 1;
+}
+
+namespace {
+std::mutex g_mem_mu;
+std::unordered_map<void*, size_t> g_mem;
+size_t g_mem_total = 0;
+}  // namespace
+
+void* dev_alloc(size_t bytes) {
+    if (bytes == 0) bytes = 4;
+    std::lock_guard<std::mutex> lock(g_mem_mu);
+    if (const char* e = getenv("SNHIP_MEM_LIMIT"))
+        if (g_mem_total + bytes > strtoull(e, nullptr, 10)) return nullptr;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    g_mem.emplace(p, bytes);
+    g_mem_total += bytes;
+    return p;
+}
+void dev_free(void* p) {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lock(g_mem_mu);
+        const auto it = g_mem.find(p);
+        if (it != g_mem.end()) {
+            g_mem_total -= it->second;
+            g_mem.erase(it);
+        }
+    }
+    (void)hipFree(p);
 }
 
 namespace {
@@ -129,6 +164,11 @@ int32_t snhip_abi_version_string(char* buf, int32_t buflen) { return copy_str(kV
 int32_t snhip_abi_backend_string(char* buf, int32_t buflen) { return copy_str("hip", buf, buflen); }
 int32_t snhip_abi_last_error(char* buf, int32_t buflen) {
     return copy_str(last_error().c_str(), buf, buflen);
+}
+
+uint64_t snhip_device_bytes(void) {
+    std::lock_guard<std::mutex> lock(g_mem_mu);
+    return g_mem_total;
 }
 
 snhip_status snhip_abi_set_threads(int32_t n) {

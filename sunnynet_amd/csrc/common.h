@@ -52,6 +52,13 @@ inline unsigned env_unsigned(const char* name, unsigned dflt, unsigned lo) {
     return v < (long)lo ? lo : (unsigned)v;
 }
 
+// Device memory of the handles. dev_alloc returns null when there is none, and
+// leaves no error behind for the launches that follow; with SNHIP_MEM_LIMIT set
+// (bytes, read per call) also when the handles of the process would hold more than
+// that.
+void* dev_alloc(size_t bytes);
+void dev_free(void* p);
+
 // A call that runs grid-synchronizing persistent kernels on `st`. enter() waits
 // until what is queued on the stream is done and then for the device's gate;
 // finish() waits for the call's kernels and opens the gate (so does the destructor).

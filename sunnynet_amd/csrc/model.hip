@@ -580,8 +580,8 @@ namespace {
 
 template <typename T>
 T* dalloc(SnHipModel* m, size_t n) {
-    void* p = nullptr;
-    if (hipMalloc(&p, n * sizeof(T) > 0 ? n * sizeof(T) : 4) != hipSuccess) return nullptr;
+    void* p = dev_alloc(n * sizeof(T));
+    if (!p) return nullptr;
     m->allocs.push_back(p);
     return static_cast<T*>(p);
 }
@@ -591,7 +591,7 @@ void free_model(SnHipModel* m) {
     if (m->h_err) (void)hipHostFree(m->h_err);
     for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
     if (m->cap) (void)hipStreamDestroy(m->cap);
-    for (void* p : m->allocs) (void)hipFree(p);
+    for (void* p : m->allocs) dev_free(p);
     delete m;
 }
 
@@ -1087,7 +1087,7 @@ SnHipModel* load_model(const char* path, int vocab, int dim, int inner, int rank
     }
     // The transpose staging buffers are no longer needed.
     for (auto it = m->allocs.begin(); it != m->allocs.end();) {
-        if (*it == tmp_in || *it == tmp_out) { (void)hipFree(*it); it = m->allocs.erase(it); }
+        if (*it == tmp_in || *it == tmp_out) { dev_free(*it); it = m->allocs.erase(it); }
         else ++it;
     }
     if (hipMemset(m->s, 0, B * layers * D * sizeof(float)) != hipSuccess ||
@@ -1432,7 +1432,7 @@ snhip_status ensure_prefill_ws(SnHipModel* m, int chunk) {
                       &m->pf_st, &m->pf_z, &m->pf_yn, &m->pf_sfb, &m->pf_send, &m->pf_pa, &m->pf_pb};
     auto drop = [&](void* p) {
         if (!p) return;
-        (void)hipFree(p);
+        dev_free(p);
         for (auto it = m->allocs.begin(); it != m->allocs.end(); ++it)
             if (*it == p) { m->allocs.erase(it); break; }
     };
@@ -1468,7 +1468,6 @@ snhip_status ensure_prefill_ws(SnHipModel* m, int chunk) {
     // Without memory for the planes the products stay on the fp32 matrix cores.
     m->pf_xs.pl = dalloc<uint16_t>(m, split_halfs(rows, std::max({D, I, R})));
     m->pf_xs.ex = dalloc<int>(m, split_rows(rows));
-    if (!m->pf_xs.pl || !m->pf_xs.ex) (void)hipGetLastError();   // not an error of the launches that follow
     m->pf_chunk = chunk;
     return SNHIP_OK;
 }
@@ -1491,10 +1490,7 @@ snhip_status build_split(SnHipModel* m, const std::vector<Mat*>& mats, bool* tri
     }
     uint16_t* pl = dalloc<uint16_t>(m, halfs);
     int* ex = pl ? dalloc<int>(m, rows) : nullptr;
-    if (!ex) {
-        (void)hipGetLastError();
-        return SNHIP_OK;
-    }
+    if (!ex) return SNHIP_OK;
     for (Mat* W : mats) {
         const SplitMat S{pl, ex};
         const snhip_status rc = launch_split_w(gemm_for(m, *W, nullptr, 0, 0, nullptr, 0), S, m->stream);
@@ -1973,10 +1969,10 @@ snhip_status snhip_decode_greedy_dev(SnHipModel* m, const int32_t* tokens_dev, i
         long cap = 256L * m->max_batch;
         while (cap < (long)n_steps * B) cap *= 2;
         if (cap > (1L << 30)) return SNHIP_E_INVAL;
-        int32_t* h = nullptr;
-        SNHIP_CHECK(hipMalloc(&h, (size_t)cap * sizeof(int32_t)));
+        int32_t* h = static_cast<int32_t*>(dev_alloc((size_t)cap * sizeof(int32_t)));
+        if (!h) { set_last_error("out of device memory (token history)"); return SNHIP_E_DEVICE; }
         if (m->tok_hist) {
-            (void)hipFree(m->tok_hist);
+            dev_free(m->tok_hist);
             for (auto it = m->allocs.begin(); it != m->allocs.end(); ++it)
                 if (*it == m->tok_hist) { m->allocs.erase(it); break; }
         }

@@ -146,7 +146,8 @@ struct SnHipRwkv7 {
           *dw = nullptr, *da = nullptr, *dv = nullptr, *g = nullptr, *y = nullptr, *vfirst = nullptr,
           *xk2 = nullptr, *ck = nullptr, *nrm = nullptr, *logits = nullptr;
     int32_t* tok = nullptr;
-    float* pf = nullptr;   // chunked prefill workspace of kPfRows tokens, on first use
+    float* pf = nullptr;   // chunked prefill workspace of pf_rows tokens, on first use
+    int pf_rows = 0;
     unsigned long long* best = nullptr;
     int32_t *counter = nullptr, *done = nullptr, *tok_hist = nullptr;
     int hist_cap = 0;
@@ -186,8 +187,8 @@ namespace {
 
 template <typename T>
 T* ralloc(SnHipRwkv7* m, size_t n) {
-    void* p = nullptr;
-    if (hipMalloc(&p, n * sizeof(T) > 0 ? n * sizeof(T) : 4) != hipSuccess) return nullptr;
+    void* p = dev_alloc(n * sizeof(T));
+    if (!p) return nullptr;
     m->allocs.push_back(p);
     return static_cast<T*>(p);
 }
@@ -197,7 +198,7 @@ void free_rk(SnHipRwkv7* m) {
     for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
     if (m->cap) (void)hipStreamDestroy(m->cap);
     if (m->h_err) (void)hipHostFree(m->h_err);
-    for (void* p : m->allocs) (void)hipFree(p);
+    for (void* p : m->allocs) dev_free(p);
     delete m;
 }
 
@@ -582,7 +583,7 @@ SnHipRwkv7* load_rk(const char* path, int max_batch, int wfmt, int block) {
         return nullptr;
     }
     for (auto it = m->allocs.begin(); it != m->allocs.end();) {
-        if (*it == tmp0 || *it == tmp1) { (void)hipFree(*it); it = m->allocs.erase(it); }
+        if (*it == tmp0 || *it == tmp1) { dev_free(*it); it = m->allocs.erase(it); }
         else ++it;
     }
     const size_t B = max_batch;
@@ -873,8 +874,8 @@ struct PfWs {
     float *x, *X6, *r, *k, *v, *lo, *dw, *da, *dv, *g, *ys, *y, *vfirst, *xk2, *ck, *pack, *dot, *shift;
     int32_t* tok;
 };
-size_t pf_layout(const SnHipRwkv7* m, float* base, PfWs* ws) {
-    const size_t T = kPfRows, D = m->D;
+size_t pf_layout(const SnHipRwkv7* m, int rows, float* base, PfWs* ws) {
+    const size_t T = rows, D = m->D;
     size_t at = 0;
     auto take = [&](float*& p, size_t n) {
         if (base) p = base + at;
@@ -906,7 +907,7 @@ size_t pf_layout(const SnHipRwkv7* m, float* base, PfWs* ws) {
     return at;
 }
 
-// T <= kPfRows tokens (in ws.tok) of sequence 0 from its current state; the
+// T <= m->pf_rows tokens (in ws.tok) of sequence 0 from its current state; the
 // last token's logits to logits_out unless null.
 snhip_status enqueue_chunk(SnHipRwkv7* m, const PfWs& ws, int T, float* logits_out, hipStream_t st) {
     const int D = m->D, NH = m->NH;
@@ -970,14 +971,21 @@ snhip_status enqueue_chunk(SnHipRwkv7* m, const PfWs& ws, int T, float* logits_o
     return enqueue_head(m, 1, logits_out, false, st);
 }
 
+// A workspace for chunks of kPfRows tokens, or of as many as there is memory for;
+// false without one of at least 16.
+bool ensure_prefill_ws(SnHipRwkv7* m) {
+    for (int rows = kPfRows; !m->pf && rows >= 16; rows /= 2) {
+        m->pf = ralloc<float>(m, pf_layout(m, rows, nullptr, nullptr));
+        m->pf_rows = rows;
+    }
+    return m->pf != nullptr;
+}
+
 snhip_status run_prefill(SnHipRwkv7* m, const int32_t* tokens, int n, float* logits_out) {
-    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
-    if (!m->pf) m->pf = ralloc<float>(m, pf_layout(m, nullptr, nullptr));
-    if (!m->pf) { set_last_error("out of device memory (prefill)"); return SNHIP_E_NOMEM; }
     PfWs ws;
-    pf_layout(m, m->pf, &ws);
-    for (int c0 = 0; c0 < n; c0 += kPfRows) {
-        const int T = std::min(kPfRows, n - c0);
+    pf_layout(m, m->pf_rows, m->pf, &ws);
+    for (int c0 = 0; c0 < n; c0 += m->pf_rows) {
+        const int T = std::min(m->pf_rows, n - c0);
         SNHIP_CHECK(hipMemcpyAsync(ws.tok, tokens + c0, T * sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
         const snhip_status rc = enqueue_chunk(m, ws, T, c0 + T == n ? logits_out : nullptr, m->stream);
         if (rc != SNHIP_OK) return rc;
@@ -989,11 +997,13 @@ snhip_status prefill_host(SnHipRwkv7* m, const int32_t* tokens, int n, float* lo
     if (!m || !tokens || n <= 0 || !logits) return SNHIP_E_INVAL;
     if (!tokens_ok(m, tokens, n)) return SNHIP_E_INVAL;
     if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
-    if (n >= kPfMin) {
+    if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
+    if (n >= kPfMin && ensure_prefill_ws(m)) {
         const snhip_status rc = run_prefill(m, tokens, n, m->logits);
         if (rc != SNHIP_OK) return rc;
     } else {
-        // rwkv7.c:362-364: the step, once per token, in order.
+        // rwkv7.c:362-364: the step, once per token, in order (also without memory
+        // for the workspace).
         for (int i = 0; i < n; ++i) {
             SNHIP_CHECK(hipMemcpyAsync(m->tok, tokens + i, sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
             const snhip_status rc = run_steps(m, nullptr, 1, m->logits, false, 1);
@@ -1065,7 +1075,7 @@ snhip_status snhip_rk_dbg(SnHipRwkv7* m, int token, int layer, float* out) {
         rc = SNHIP_E_DEVICE;
     (void)hipStreamSynchronize(m->stream);
     for (auto it = m->allocs.begin(); it != m->allocs.end(); ++it)
-        if (*it == d) { (void)hipFree(d); m->allocs.erase(it); break; }
+        if (*it == d) { dev_free(d); m->allocs.erase(it); break; }
     return rc;
 }
 
@@ -1110,10 +1120,10 @@ snhip_status snhip_rk_decode_greedy_dev(SnHipRwkv7* m, const int32_t* tokens_dev
         long cap = 256L * m->max_batch;
         while (cap < (long)n_steps * B) cap *= 2;
         if (cap > (1L << 30)) return SNHIP_E_INVAL;
-        int32_t* hbuf = nullptr;
-        SNHIP_CHECK(hipMalloc(&hbuf, (size_t)cap * sizeof(int32_t)));
+        int32_t* hbuf = static_cast<int32_t*>(dev_alloc((size_t)cap * sizeof(int32_t)));
+        if (!hbuf) { set_last_error("out of device memory (token history)"); return SNHIP_E_DEVICE; }
         if (m->tok_hist) {
-            (void)hipFree(m->tok_hist);
+            dev_free(m->tok_hist);
             for (auto it = m->allocs.begin(); it != m->allocs.end(); ++it)
                 if (*it == m->tok_hist) { m->allocs.erase(it); break; }
         }

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import oracle
+from sunnynet_amd import _native
 from sunnynet_amd.runtime.rwkv7 import HipRwkv7
 from sunnynet_amd.rwkv7 import RwkvConfig, init_rwkv7, pack_rwkv7_blob
 
@@ -52,3 +53,31 @@ def test_prefill_equals_steps(gpu, tmp_path, monkeypatch, dim, int4, T, env):
     assert (S[1:] == S1).all() and (sh[1:] == sh1).all()     # sequence 1 is untouched
     for t in toks[3 + T:]:                                   # and the steps go on from there
         assert np.array_equal(np.asarray(hm.step(int(t)), np.float32), orc.step([t])[0])
+
+
+@pytest.mark.parametrize("room", [0, 400_000, 3_000_000])
+def test_prefill_without_memory(gpu, tmp_path, monkeypatch, room):
+    """With no memory for the workspace of 512 tokens the prompt runs in shorter
+    chunks, and with none at all token by token: never an error, the same bits."""
+    print("rwkv7 prefill, bytes left:", room, flush=True)
+    cfg = CFGS[128]
+    blob = pack_rwkv7_blob(init_rwkv7(cfg, 3))
+    path = tmp_path / "rk.bin"
+    path.write_bytes(blob)
+    lib = _native.lib()
+    hm = HipRwkv7(path)
+    orc = oracle.RkOracle(blob)
+    toks = [int(t) for t in np.random.default_rng(4).integers(0, cfg.vocab, 90)]
+    before = lib.snhip_device_bytes()
+    monkeypatch.setenv("SNHIP_MEM_LIMIT", str(before + room))
+    got = np.asarray(hm.prefill(toks), np.float32)
+    taken = lib.snhip_device_bytes() - before
+    assert taken <= room and (taken > 0) == (room > 0)
+    for t in toks:
+        ref = orc.step([t])[0]
+    assert np.array_equal(got, ref)
+    So, sho = orc.get_state()
+    S, sh = hm.get_state()
+    assert np.array_equal(S.cpu().numpy(), So) and np.array_equal(sh.cpu().numpy(), sho)
+    hm.close()
+    assert lib.snhip_device_bytes() < before
