@@ -538,7 +538,8 @@ struct SnHipModel {
           *pf_send = nullptr, *pf_pa = nullptr, *pf_pb = nullptr;
     int32_t* pf_tok = nullptr;
     snhip::SplitMat pf_xs;                       // planes of the current product's rows
-    bool split_tried = false, split_head_tried = false;
+    uint16_t* split_pl = nullptr;                // planes of every matrix, in one allocation; null: none
+    int* split_ex = nullptr;
     // Persistent single-sequence decode (persist.hip): grid size, 0 when the
     // model's shape or the device does not allow it.
     int persist_wg = 0;
@@ -584,6 +585,13 @@ T* dalloc(SnHipModel* m, size_t n) {
     if (!p) return nullptr;
     m->allocs.push_back(p);
     return static_cast<T*>(p);
+}
+
+void dfree(SnHipModel* m, void* p) {
+    if (!p) return;
+    dev_free(p);
+    for (auto it = m->allocs.begin(); it != m->allocs.end(); ++it)
+        if (*it == p) { m->allocs.erase(it); break; }
 }
 
 void free_model(SnHipModel* m) {
@@ -976,6 +984,8 @@ bool load_layers_i4(SnHipModel* m, const uint8_t* raw) {
     return ok && store_ok(m, hs) && upload_q(m, m->head, q, sc, (int)D, (int)V, hs, 0);
 }
 
+bool setup_split(SnHipModel* m);
+
 SnHipModel* load_model(const char* path, int vocab, int dim, int inner, int rank, int taps,
                        int layers, int group, int tied, int max_batch, int wfmt, int block) {
     if (!path || vocab <= 0 || dim <= 0 || inner <= 0 || rank <= 0 || taps <= 0 || layers <= 0 ||
@@ -1122,6 +1132,11 @@ SnHipModel* load_model(const char* path, int vocab, int dim, int inner, int rank
     }
     setup_persist(m);
     setup_batch(m);
+    if (!setup_split(m)) {
+        set_last_error("planes of the weights: conversion failed");
+        free_model(m);
+        return nullptr;
+    }
     m->ready = 1;
     return m;
 }
@@ -1424,88 +1439,126 @@ snhip_status run_steps(SnHipModel* m, const int32_t* tok, int B, float* logits_o
     return SNHIP_OK;
 }
 
-// Workspace of the chunked prefill for max_batch x chunk rows.
+// Whether a prefill product of `rows` rows runs from the planes: more rows than the
+// decode paths take.
+constexpr long kSplitMinRows = 65;
+bool split_rows_ok(const SnHipModel* m, const Mat& W, long rows) {
+    return rows >= kSplitMinRows && W.split.pl && m->pf_xs.pl;
+}
+// Whether its rows, read by nothing else, go to the planes as they are computed.
+bool split_fused(const SnHipModel* m, const Mat& W, long rows) {
+    return W.Kd <= kSplitRegs && split_rows_ok(m, W, rows);
+}
+// Whether the gates of every row are computed in parallel before the scan.
+bool gate_rows_ok(const SnHipModel* m, int B, int Tc) {
+    return (size_t)m->max_batch * m->D <= kSplitScanChannels && ring_scan_ok(B, Tc, m->D, m->D);
+}
+
+std::vector<Mat*> split_mats(SnHipModel* m) {
+    std::vector<Mat*> v;
+    for (Layer& A : m->layers)
+        for (Mat* W : {&A.V, &A.U, &A.Wz, &A.Wc, &A.Ws}) v.push_back(W);
+    v.push_back(&m->head);
+    return v;
+}
+void drop_split(SnHipModel* m) {
+    for (Mat* W : split_mats(m)) W->split = SplitMat{};
+    dfree(m, m->split_pl);
+    dfree(m, m->split_ex);
+    m->split_pl = nullptr;
+    m->split_ex = nullptr;
+}
+
+// Planes of every matrix that the prefill multiplies, at load: 4 bytes per weight
+// (SNHIP_GEMM_SPLIT=0: none), left out when there is no memory for them. Built in a
+// first prefill they cost it 0.3 ms of allocation, more than they saved on prompts
+// below 200 tokens.
+bool setup_split(SnHipModel* m) {
+    if (!m->gemm_ok || m->D % 64 || env_unsigned("SNHIP_GEMM_SPLIT", 1, 0) == 0) return true;
+    size_t halfs = 0, rows = 0;
+    for (const Mat* W : split_mats(m)) {
+        halfs += split_halfs(W->M, W->Kd);
+        rows += split_rows(W->M);
+    }
+    uint16_t* pl = m->split_pl = dalloc<uint16_t>(m, halfs);
+    int* ex = m->split_ex = pl ? dalloc<int>(m, rows) : nullptr;
+    if (!ex) {
+        drop_split(m);
+        return true;
+    }
+    for (Mat* W : split_mats(m)) {
+        W->split = SplitMat{pl, ex};
+        if (launch_split_w(gemm_for(m, *W, nullptr, 0, 0, nullptr, 0), W->split, nullptr) != SNHIP_OK) return false;
+        pl += split_halfs(W->M, W->Kd);
+        ex += split_rows(W->M);
+    }
+    return hipStreamSynchronize(nullptr) == hipSuccess;
+}
+
+// Workspace of the chunked prefill for max_batch x chunk rows. When there is no
+// memory for it beside the planes, the planes go.
 snhip_status ensure_prefill_ws(SnHipModel* m, int chunk) {
     if (m->pf_chunk >= chunk) return SNHIP_OK;
     SNHIP_CHECK(hipStreamSynchronize(m->stream));
     float** bufs[] = {&m->pf_x, &m->pf_raw, &m->pf_at, &m->pf_v, &m->pf_q, &m->pf_u,
                       &m->pf_st, &m->pf_z, &m->pf_yn, &m->pf_sfb, &m->pf_send, &m->pf_pa, &m->pf_pb};
-    auto drop = [&](void* p) {
-        if (!p) return;
-        dev_free(p);
-        for (auto it = m->allocs.begin(); it != m->allocs.end(); ++it)
-            if (*it == p) { m->allocs.erase(it); break; }
+    auto drop = [&] {
+        for (float** b : bufs) {
+            dfree(m, *b);
+            *b = nullptr;
+        }
+        dfree(m, m->pf_tok);
+        dfree(m, m->pf_xs.pl);
+        dfree(m, m->pf_xs.ex);
+        m->pf_tok = nullptr;
+        m->pf_xs = SplitMat{};
+        m->pf_chunk = 0;
     };
-    for (float** b : bufs) {
-        drop(*b);
-        *b = nullptr;
-    }
-    drop(m->pf_tok);
-    drop(m->pf_xs.pl);
-    drop(m->pf_xs.ex);
-    m->pf_tok = nullptr;
-    m->pf_xs = SplitMat{};
     const size_t rows = (size_t)m->max_batch * chunk, D = m->D, I = m->I, R = m->R;
-    m->pf_x = dalloc<float>(m, rows * D);
-    m->pf_raw = dalloc<float>(m, rows * D);
-    m->pf_at = dalloc<float>(m, rows * D);
-    m->pf_v = dalloc<float>(m, rows * R);
-    m->pf_q = dalloc<float>(m, rows * 2 * D);
-    m->pf_u = dalloc<float>(m, rows * D);
-    m->pf_st = dalloc<float>(m, rows * D);
-    m->pf_z = dalloc<float>(m, rows * I);
-    m->pf_yn = dalloc<float>(m, rows * I);
-    m->pf_sfb = dalloc<float>(m, rows * D);
-    m->pf_send = dalloc<float>(m, (size_t)m->max_batch * D);
-    // scan inputs of the small-batch path (kSplitScanChannels)
-    const size_t prow = (size_t)m->max_batch * D <= kSplitScanChannels ? rows * D : 1;
-    m->pf_pa = dalloc<float>(m, prow);
-    m->pf_pb = dalloc<float>(m, prow);
-    m->pf_tok = dalloc<int32_t>(m, rows);
-    for (float** b : bufs)
-        if (!*b) { m->pf_chunk = 0; set_last_error("out of device memory (prefill)"); return SNHIP_E_NOMEM; }
-    if (!m->pf_tok) { m->pf_chunk = 0; return SNHIP_E_NOMEM; }
-    // Without memory for the planes the products stay on the fp32 matrix cores.
-    m->pf_xs.pl = dalloc<uint16_t>(m, split_halfs(rows, std::max({D, I, R})));
-    m->pf_xs.ex = dalloc<int>(m, split_rows(rows));
+    auto take = [&] {
+        if (m->split_pl) {
+            m->pf_xs.pl = dalloc<uint16_t>(m, split_halfs(rows, std::max({D, I, R})));
+            m->pf_xs.ex = m->pf_xs.pl ? dalloc<int>(m, split_rows(rows)) : nullptr;
+            if (!m->pf_xs.ex) return false;
+        }
+        // Rows that go to the planes as they are computed are stored only where
+        // the planes are not used: up to kSplitMinRows - 1 of them.
+        auto stored = [&](bool fused) { return fused ? std::min(rows, (size_t)kSplitMinRows - 1) : rows; };
+        const bool planes = m->split_pl != nullptr, planes_d = planes && D <= (size_t)kSplitRegs;
+        m->pf_x = dalloc<float>(m, rows * D);
+        m->pf_raw = dalloc<float>(m, rows * D);
+        m->pf_at = dalloc<float>(m, stored(planes_d) * D);
+        m->pf_v = dalloc<float>(m, rows * R);
+        m->pf_q = dalloc<float>(m, rows * 2 * D);
+        m->pf_u = dalloc<float>(m, stored(planes_d && gate_rows_ok(m, m->max_batch, chunk)) * D);
+        m->pf_st = dalloc<float>(m, rows * D);
+        m->pf_z = dalloc<float>(m, rows * I);
+        m->pf_yn = dalloc<float>(m, stored(planes && I <= (size_t)kSplitRegs) * I);
+        m->pf_sfb = dalloc<float>(m, rows * D);
+        m->pf_send = dalloc<float>(m, (size_t)m->max_batch * D);
+        // prefill rows of the split scan: only when few channels use it
+        const bool few = (size_t)m->max_batch * D <= kSplitScanChannels;
+        m->pf_pa = dalloc<float>(m, few ? rows * D : 1);
+        m->pf_pb = dalloc<float>(m, few ? rows * D : 1);
+        m->pf_tok = dalloc<int32_t>(m, rows);
+        for (float** b : bufs)
+            if (!*b) return false;
+        return m->pf_tok != nullptr;
+    };
+    drop();
+    bool ok = take();
+    if (!ok && m->split_pl) {
+        drop();
+        drop_split(m);
+        ok = take();
+    }
+    if (!ok) {
+        drop();
+        set_last_error("out of device memory (prefill)");
+        return SNHIP_E_NOMEM;
+    }
     m->pf_chunk = chunk;
     return SNHIP_OK;
-}
-
-// Planes of the matrices `mats` in one allocation, once per model; left out when
-// there is no memory for them.
-snhip_status build_split(SnHipModel* m, const std::vector<Mat*>& mats, bool* tried) {
-    if (*tried) return SNHIP_OK;
-    // nothing is allocated under a caller's capture: those products stay as they are
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    SNHIP_CHECK(hipStreamIsCapturing(m->stream, &cap));
-    if (cap != hipStreamCaptureStatusNone) return SNHIP_OK;
-    *tried = true;
-    if (const char* e = getenv("SNHIP_GEMM_SPLIT"))
-        if (atoi(e) == 0) return SNHIP_OK;
-    size_t halfs = 0, rows = 0;
-    for (const Mat* W : mats) {
-        halfs += split_halfs(W->M, W->Kd);
-        rows += split_rows(W->M);
-    }
-    uint16_t* pl = dalloc<uint16_t>(m, halfs);
-    int* ex = pl ? dalloc<int>(m, rows) : nullptr;
-    if (!ex) return SNHIP_OK;
-    for (Mat* W : mats) {
-        const SplitMat S{pl, ex};
-        const snhip_status rc = launch_split_w(gemm_for(m, *W, nullptr, 0, 0, nullptr, 0), S, m->stream);
-        if (rc != SNHIP_OK) return rc;
-        W->split = S;
-        pl += split_halfs(W->M, W->Kd);
-        ex += split_rows(W->M);
-    }
-    return SNHIP_OK;
-}
-
-// Whether a prefill product of `rows` rows runs from the planes: more rows than the
-// decode paths take.
-bool split_rows_ok(const SnHipModel* m, const Mat& W, long rows) {
-    return rows > 64 && W.split.pl && m->pf_xs.pl && m->pf_xs.ex;
 }
 
 // A prefill product; `planes`: those of its rows are in pf_xs already.
@@ -1539,7 +1592,7 @@ snhip_status enqueue_prefill_chunk(SnHipModel* m, int B, int Tc, float* logits_o
         float* h_l = m->hist + (size_t)l * (m->kh ? m->kh : 1) * D;
         launch_ln((int)rows, m->pf_x, D, A.ni_g, A.ni_c, m->pf_raw, D, D, m->eps, st);
         // Rows that only a product reads are split into its planes as they are computed.
-        auto fuse = [&](const Mat& W) { return W.Kd <= kSplitRegs && split_rows_ok(m, W, rows); };
+        auto fuse = [&](const Mat& W) { return split_fused(m, W, rows); };
         const float* at = m->pf_raw;
         bool conv_split = false, gate_split = false;
         if (m->K > 1) {
@@ -1559,7 +1612,7 @@ snhip_status enqueue_prefill_chunk(SnHipModel* m, int B, int Tc, float* logits_o
         if ((rc = run_gemm_rows(m, gemm_for(m, A.V, at, D, (int)rows, m->pf_v, R), A.V, st, conv_split)) != SNHIP_OK)
             return rc;
         if ((rc = run_gemm_rows(m, gemm_for(m, A.U, m->pf_v, R, (int)rows, m->pf_q, 2 * D), A.U, st)) != SNHIP_OK) return rc;
-        if ((size_t)m->max_batch * D <= kSplitScanChannels && ring_scan_ok(B, Tc, D, D)) {
+        if (gate_rows_ok(m, B, Tc)) {
             // Few channels: the gates of every row in parallel, then a scan
             // that only multiplies and adds.
             const long n = rows * D;
@@ -1644,13 +1697,6 @@ snhip_status run_prefill(SnHipModel* m, const int32_t* tokens_dev, int B, int T,
     chunk = std::min(chunk, T);
     snhip_status rc = ensure_prefill_ws(m, chunk);
     if (rc != SNHIP_OK) return rc;
-    if ((long)B * chunk > 64) {
-        std::vector<Mat*> mats;
-        for (Layer& A : m->layers)
-            for (Mat* W : {&A.V, &A.U, &A.Wz, &A.Wc, &A.Ws}) mats.push_back(W);
-        if ((rc = build_split(m, mats, &m->split_tried)) != SNHIP_OK) return rc;
-        if (all_logits && (rc = build_split(m, {&m->head}, &m->split_head_tried)) != SNHIP_OK) return rc;
-    }
     for (int c0 = 0; c0 < T; c0 += chunk) {
         const int Tc = std::min(chunk, T - c0);
         SNHIP_CHECK(hipMemcpy2DAsync(m->pf_tok, (size_t)Tc * sizeof(int32_t), tokens_dev + c0,

@@ -14,8 +14,9 @@ import torch
 
 import oracle
 from oracle.torch_ref import TorchSunny, forward_hist_to_step
+from sunnynet_amd import _native
 from sunnynet_amd.blob import pack_sunny_blob
-from sunnynet_amd.config import SMALL, SUNNY_100M, TINY
+from sunnynet_amd.config import SMALL, SUNNY_100M, TINY, matmul_params
 from sunnynet_amd.runtime.model import HipModel
 from sunnynet_amd.weights import gaussian_matmuls, init_sunnynet
 
@@ -155,3 +156,63 @@ def test_tiny_value_times_infinity(gpu, tmp_path, monkeypatch, where):
     fin = np.isfinite(b[0])
     assert np.isfinite(a[0][fin]).all()
     assert fin.sum() == 0 or np.abs(a[0][fin] - b[0][fin]).max() < TOL
+
+
+def test_planes_and_memory(gpu, tmp_path, monkeypatch):
+    """The weights' planes are made at load, not in the first prefill; without memory
+    for them, at load or beside a prefill's workspace, the products are the fp32 ones;
+    and a prefill that does not fit even so fails and leaves the handle usable."""
+    print("planes and memory", flush=True)
+    cfg, lib = SMALL, _native.lib()
+    p = tmp_path / "m.bin"
+    p.write_bytes(pack_sunny_blob(gaussian_matmuls(init_sunnynet(cfg, 0), seed=4)))
+    toks = torch.from_numpy(np.random.default_rng(5).integers(0, cfg.vocab_size, (1, 200)).astype(np.int32)).to(gpu)
+
+    def load():
+        return HipModel(p, cfg.vocab_size, cfg.dim, cfg.inner, cfg.rank, cfg.taps, cfg.layers)
+
+    def run(h):
+        h.reset()
+        return [x.cpu() for x in (h.prefill_batch(toks), *h.get_state(1))]
+
+    def same(a, b):
+        return all(torch.equal(x, y) for x, y in zip(a, b))
+    base = lib.snhip_device_bytes()
+    monkeypatch.setenv("SNHIP_GEMM_SPLIT", "0")
+    h = load()
+    plain_bytes = lib.snhip_device_bytes() - base
+    plain = run(h)
+    plain_ws = lib.snhip_device_bytes() - base - plain_bytes
+    h.close()
+    assert lib.snhip_device_bytes() == base
+    monkeypatch.delenv("SNHIP_GEMM_SPLIT")
+    h = load()
+    planes_bytes = lib.snhip_device_bytes() - base - plain_bytes
+    assert planes_bytes >= 4 * matmul_params(cfg)
+    split = run(h)
+    ws = lib.snhip_device_bytes() - base - plain_bytes - planes_bytes
+    assert 0 < ws < plain_ws and not same(split, plain)       # no rows stored beside their planes
+    assert same(run(h), split) and lib.snhip_device_bytes() - base == plain_bytes + planes_bytes + ws
+    h.close()
+    # no room for the planes at load
+    monkeypatch.setenv("SNHIP_MEM_LIMIT", str(base + plain_bytes + planes_bytes // 2))
+    h = load()
+    assert lib.snhip_device_bytes() - base == plain_bytes
+    monkeypatch.delenv("SNHIP_MEM_LIMIT")
+    assert same(run(h), plain)
+    h.close()
+    # no room for the workspace beside them
+    h = load()
+    monkeypatch.setenv("SNHIP_MEM_LIMIT", str(base + plain_bytes + planes_bytes + ws // 2))
+    assert same(run(h), plain)
+    assert lib.snhip_device_bytes() - base == plain_bytes + plain_ws
+    h.close()
+    # nor without them
+    h = load()
+    monkeypatch.setenv("SNHIP_MEM_LIMIT", str(base + plain_bytes + plain_ws // 2))
+    with pytest.raises(_native.SnHipError):
+        run(h)
+    monkeypatch.delenv("SNHIP_MEM_LIMIT")
+    assert same(run(h), plain)
+    h.close()
+    assert lib.snhip_device_bytes() == base
