@@ -862,12 +862,14 @@ snhip_status step_host(SnHipRwkv7* m, const int32_t* tokens, int B, float* logit
 }
 
 // Chunked prefill of sequence 0 (rkprefill.hip). Its products use whichever
-// form the matrices have; prompts shorter than kPfMin step token by token.
-// Measured on 12 x 768 INT4 g32, host call: a chunk of 2 to 16 tokens 1.1 ms, a
-// step 0.71 ms, so the line lies at two tokens; 512 tokens 3.4 ms in one chunk
-// against 345 ms stepped.
+// form the matrices have; prompts shorter than pf_min step token by token.
+// 12 x 768 INT4 g32, host call with the logits' copy: a chunk of 2 to 16 tokens
+// 1.40 ms; two steps of the exact one-launch kernel 1.4 (three 2.1), of the
+// per-kernel step 2.5, so the line lies at two tokens; of the opt-in fast kernel
+// 1.22 (three 1.63), so there at three. 512 tokens 4.0 ms in one chunk against 345
+// stepped.
 constexpr int kPfRows = 512;   // tokens per chunk
-constexpr int kPfMin = 2;
+int pf_min(const SnHipRwkv7* m) { return m->p_grid > 0 && m->all_cus && !m->p_exact ? 3 : 2; }
 
 // Floats of the workspace's parts per token, in PfWs's order.
 struct PfWs {
@@ -998,7 +1000,7 @@ snhip_status prefill_host(SnHipRwkv7* m, const int32_t* tokens, int n, float* lo
     if (!tokens_ok(m, tokens, n)) return SNHIP_E_INVAL;
     if (follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
-    if (n >= kPfMin && ensure_prefill_ws(m)) {
+    if (n >= pf_min(m) && ensure_prefill_ws(m)) {
         const snhip_status rc = run_prefill(m, tokens, n, m->logits);
         if (rc != SNHIP_OK) return rc;
     } else {

@@ -98,6 +98,22 @@ def test_persist_matches_oracle_and_per_kernel_step(gpu, tiny, monkeypatch, fmt)
     assert np.abs(S.cpu().numpy() - So).max() < 1e-4 and np.abs(sh.cpu().numpy() - sho).max() < 1e-5
 
 
+@pytest.mark.parametrize("n", [1, 2, 3])
+def test_short_prompts(gpu, tiny, monkeypatch, n):
+    """A prompt of up to two tokens takes the fast steps (a chunk costs more than two
+    of them); a longer one the chunked prefill, which is exact."""
+    print("rwkv7 persistent, prompt of", n, flush=True)
+    _, p32, _ = tiny
+    hp, hg = _pair(p32, monkeypatch)
+    toks = [int(t) for t in np.random.default_rng(12).integers(0, RWKV_TINY.vocab, n)]
+    got = np.asarray(hp.prefill(toks), np.float32)
+    like = hp if n < 3 else hg
+    like.reset()
+    for t in toks:
+        want = np.asarray(like.step(t), np.float32)
+    assert np.array_equal(got, want)
+
+
 def test_persist_greedy_matches_oracle_chain(gpu, tiny):
     w, p32, _ = tiny
     n = 20
