@@ -28,15 +28,16 @@
 // tiles of inputs in registers: the loads for tile i+1 are issued before
 // tile i is processed, a whole tile period ahead of their use. The fast path
 // needs D % 128 == 0 and T % (W TC) == 0 (the reference's block pads T to its
-// scan chunk before it calls the kernel). Any other shape, and few channels, take
-// the split form: the heavy part as an elementwise kernel over all steps at once
+// scan chunk before it calls the kernel). Any other shape, and few channels, of
+// more than a few steps (split_pays_fwd, split_pays_bwd) take the split form: the heavy part as an elementwise kernel over all steps at once
 // (after the chain in the backward), the chain as a ring scan over u and p
 // (forward) or over p and dstate (backward, ds passing through dq). It moves
 // 28 B forward and 48 B backward per channel and step where the fused kernels
 // move 20 and 36, but neither part waits for the other's latency: on 8192
 // channels of 2048 steps the fused kernels' 64 workgroups leave three CUs in four
-// idle. Arrays past the ring's 32-bit offsets and outputs that overlap inputs take
-// a one lane per channel kernel.
+// idle. What is left, few steps of other shapes, arrays past the ring's 32-bit offsets
+// and outputs that overlap inputs, takes a one lane per channel kernel.
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -602,9 +603,21 @@ void k_core_gate_bwd(const float* __restrict__ q, const float* __restrict__ delt
     for (int c = 0; c < 4; ++c) o[c] = acc[c];
 }
 
-// ddelta[d] += sum over the n partial rows of dacc[r, d]: kDdSlots running sums of
-// every kDdSlots-th row in order, then those in order (n <= kDdSlots: the rows in
-// order).
+// ddelta[d] += sum over the n partial rows of dacc[r, d], rows in order: few rows, one
+// lane per channel.
+constexpr int kDdFew = 16;
+__global__ void k_core_ddelta_few(const float* __restrict__ dacc, float* __restrict__ ddelta, int n, int D) {
+    const int d = blockIdx.x * blockDim.x + threadIdx.x;
+    if (d >= D) return;
+    float r = 0.0f;
+#pragma unroll 4
+    for (int i = 0; i < n; ++i) r = add_rn(r, dacc[(size_t)i * D + d]);
+    ddelta[d] = add_rn(ddelta[d], r);
+}
+
+// The same over more rows: kDdSlots running sums of every kDdSlots-th row in order,
+// then those in order (n <= kDdSlots: the rows in order). A backward of 1 x 128 steps
+// x 128 channels, us: 28.9 with it, 27.0 with the one above.
 constexpr int kDdSlots = 64, kDdChans = 16;
 __global__ __launch_bounds__(kDdSlots * kDdChans)
 void k_core_ddelta(const float* __restrict__ dacc, float* __restrict__ ddelta, int n, int D) {
@@ -648,16 +661,27 @@ bool fast_ok(int B, int T, int D, int tile, std::initializer_list<const void*> p
 }
 
 
-// The split form is taken by calls whose shape or alignment the fused kernels do
-// not run, and by long ones with few channels (B D). Split / fused, us, forward
-// and backward, at 2048 steps: 1024 channels 45 / 163 and 58 / 339, 8192 104 / 170
-// and 179 / 343, 12288 148 / 179 and 269 / 346, 16384 188 / 182 and 350 / 345,
-// 32768 366 / 227 and 671 / 417 (the fused kernels read and write each array once);
-// at 8192 channels of 128 steps 14.6 / 14.3 and 32 / 36 (launches), of 256 18 / 24
-// and 34 / 56. Against one lane per channel, 600 channels of 777 steps: 319 -> 24
-// and 450 -> 42.
-bool split_pays(bool fused, int B, int T, int D) {
-    return !fused || ((long)B * D < 16384 && T >= 256);
+// When the split form is taken (us a call). Where the fused kernels run: by long
+// calls with few channels (B D). Split / fused, forward and backward, at 2048 steps:
+// 1024 channels 45 / 163 and 58 / 339, 8192 104 / 170 and 179 / 343, 12288 148 / 179
+// and 269 / 346, 16384 188 / 182 and 350 / 345, 32768 366 / 227 and 671 / 417 (the
+// fused kernels read and write each array once); at 8192 channels of 128 steps 14.6 /
+// 14.3 and 32 / 36 (launches), of 256 18 / 24 and 34 / 56.
+// Where they do not (shape or alignment), against one lane per channel, which costs
+// 0.3 us a step forward and 0.5 backward however few the channels, and less than the
+// split form's launches for few steps: forward from 32 steps on (600 channels: 24
+// steps 13.0 / 10.3, 32 12.9 / 13.2, 777 24 / 319), more beyond 16384 channels (32000:
+// 32 21.5 / 16.0, 48 22.5 / 23.4; 64000: 64 37 / 35, 96 43 / 50; 85760: 100 63 / 56); backward past 48 steps
+// (600: 32 27.3 / 21.3, 48 27.9 / 26.3, 64 26.9 / 33.1, 777 42 / 450), 32 from 8192 and 60
+// from 32768 channels on (16000: 24 26.0 / 21.7, 32 27.0 / 27.5, 48 27.8 / 37.9; 62928: 51
+// 52 / 43; 64000: 48 52.0 / 51.8, 64 56.5 / 61.8).
+bool split_pays_fwd(bool fused, int B, int T, int D) {
+    const long chans = (long)B * D;
+    return fused ? chans < 16384 && T >= 256 : T >= 32 + std::max(0L, (chans - 16384) / 768);
+}
+bool split_pays_bwd(bool fused, int B, int T, int D) {
+    const long chans = (long)B * D;
+    return fused ? chans < 16384 && T >= 256 : T > (chans < 8192 ? 48 : chans <= 32768 ? 32 : 60);
 }
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -699,7 +723,7 @@ snhip_status launch_core_fwd(const float* q, const float* delta, const float* s0
     const size_t n = (size_t)B * T * D, c = (size_t)B * D;
     const int nch = (T + kGateSteps - 1) / kGateSteps;
     unsigned grid = 0;
-    if (split_pays(fused, B, T, D) && ring_scan_ok(B, T, D, D) && split_grid(B, D, nch, &grid) &&
+    if (split_pays_fwd(fused, B, T, D) && ring_scan_ok(B, T, D, D) && split_grid(B, D, nch, &grid) &&
         apart({{uo, n}, {po, n}, {states, n}}, {{q, 2 * n}, {delta, (size_t)D}, {s0, c}}) &&
         apart({{uo, n}}, {{po, n}}) && apart({{states, n}}, {{po, n}, {uo, n}})) {
         if (al16(q) && al16(uo) && al16(po))
@@ -736,7 +760,7 @@ snhip_status core_bwd_ws(const float* q, const float* delta, const float* s0, co
     int parts = B;
     const int nch = bwd_chunks(B, T, D);
     unsigned grid = 0;
-    if (split_pays(fused, B, T, D) && ring_scan_ok(B, T, D, 2 * D) && split_grid(B, D, nch, &grid) &&
+    if (split_pays_bwd(fused, B, T, D) && ring_scan_ok(B, T, D, 2 * D) && split_grid(B, D, nch, &grid) &&
         apart({{dq, 2 * n}, {ds0, c}}, {{q, 2 * n}, {delta, (size_t)D}, {s0, c}, {states, n}, {uo, n}, {po, n},
                                         {dstate, n}, {du_in, n}}) &&
         apart({{dq, 2 * n}}, {{ds0, c}})) {
@@ -760,8 +784,12 @@ snhip_status core_bwd_ws(const float* q, const float* delta, const float* s0, co
                            s0, states, uo, po, dstate, du_in, dq, acc, ds0, B, T, D);
     }
     SNHIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_core_ddelta, dim3((unsigned)((D + kDdChans - 1) / kDdChans)), dim3(kDdSlots * kDdChans),
-                       0, st, acc, ddelta, parts, D);
+    if (parts <= kDdFew)
+        hipLaunchKernelGGL(k_core_ddelta_few, dim3((unsigned)((D + 255) / 256)), dim3(256), 0, st, acc, ddelta, parts,
+                           D);
+    else
+        hipLaunchKernelGGL(k_core_ddelta, dim3((unsigned)((D + kDdChans - 1) / kDdChans)),
+                           dim3(kDdSlots * kDdChans), 0, st, acc, ddelta, parts, D);
     SNHIP_CHECK(hipGetLastError());
     return SNHIP_OK;
 }
@@ -798,10 +826,12 @@ snhip_status scratch_ptr(float** out) {
 snhip_status launch_core_bwd(const float* q, const float* delta, const float* s0, const float* states,
                              const float* uo, const float* po, const float* dstate, const float* du_in,
                              float* dq, float* ddelta, float* ds0, int B, int T, int D, hipStream_t st) {
-    // Partial sums of ddelta's terms, reduced in order afterwards.
+    // Partial sums of ddelta's terms, reduced in order afterwards; a row per batch
+    // row and, in the split form, chunk of time.
+    const bool may_split = split_pays_bwd(true, B, T, D) || split_pays_bwd(false, B, T, D);
+    const size_t rows = (size_t)B * (may_split ? bwd_chunks(B, T, D) : 1);
     float* acc = nullptr;
-    SNHIP_CHECK(hipMallocAsync(reinterpret_cast<void**>(&acc),
-                               (size_t)bwd_chunks(B, T, D) * B * D * sizeof(float), st));
+    SNHIP_CHECK(hipMallocAsync(reinterpret_cast<void**>(&acc), rows * D * sizeof(float), st));
     const snhip_status rc = core_bwd_ws(q, delta, s0, states, uo, po, dstate, du_in, dq, ddelta, ds0,
                                         B, T, D, acc, st);
     const hipError_t f = hipFreeAsync(acc, st);

@@ -529,13 +529,44 @@ hipError_t launch_cfg(const float* a, const float* b, const float* s0, float* ou
 
 bool aligned(const void* p, size_t n) { return (reinterpret_cast<uintptr_t>(p) % n) == 0; }
 
-// Below this many channels (B N; up to it backward) a scan takes the ring form,
-// and at any number where the layout is not the buffer kernels'. Gated, 2048
-// steps, us, ring / buffer kernels: 4096 channels 30 / 58, 8192 35 / 62, 12288
-// 64 / 66, 16384 86 / 70; backward 4096 54 / 118 (961 in the one-lane kernel),
-// 16384 165 / 230, 32768 269 / 262. 16 rows of 2047 channels, 777 steps: ring 72,
-// one-lane-per-channel tiles 138.
+// When the ring form is taken (us a call, ring / the kernel of the layout). Its
+// launch costs 1 to 2 us more than a small scan's, and past 1 us per 8192 channels
+// it loads a whole tile however short T is, so it needs some length to win.
+//
+// Forward, layouts of the buffer kernels: below 16384 channels from more than 128
+// steps (a tile of theirs) on. 1024 channels: 64 steps 5.8 / 5.1, 128 5.6 / 4.8, 192
+// 5.3 / 7.9; 14336: 128 6.5 / 5.6, 192 6.9 / 9.8; at 2048 steps 4096 channels 30 /
+// 58, 8192 35 / 62, 12288 64 / 66, 16384 85 / 74.
+// Other layouts, one channel per lane: from 80 steps on below 4096 channels, 64
+// below 12288, 48 below 24576, 32 beyond. 777 channels: 64 steps 6.4 / 6.0, 96 6.5 / 6.7; 6993: 48
+// 6.9 / 6.2, 64 6.7 / 7.2; 12432: 32 6.7 / 6.0, 48 6.9 / 7.1; 32752: 24 12.3 / 11.9, 32
+// 11.8 / 12.3; 2048 steps, 12012: 75 / 173.
+// Two channels per lane (even widths, 24576 channels on): past one tile of 128
+// steps. 32736 channels: 128 steps 16.9 / 13.3, 160 18.2 / 24.1, 2048 198 / 224; 130944:
+// 128 57.8 / 55.3, 160 58.0 / 90.8, 2048 727 / 898. In the FMA form, where that
+// kernel's workgroups come out even over the CUs, only to 256 steps: 32736
+// channels: 256 22.0 / 23.8, 512 42.9 / 46.8, 1024 97.6 / 93.0; 65472: 256 41.1 / 48.8, 512
+// 104 / 95.8; 130944: 256 97.1 / 96.2, 384 161 / 145; uneven, 49104: 512 68 / 85.
+//
+// Backward: up to 16384 channels from 24 steps on, in other layouts than the buffer
+// kernel's beyond that too, from more steps the more channels. 128 channels: 16 steps
+// 5.3 / 3.7, 24 5.1 / 4.8, 32 5.1 / 5.9; 8192: 16 5.5 / 4.5, 24 5.6 / 5.8; 32736: 32
+// 10.3 / 8.9, 48 10.6 / 18.7; 98256: 64 37 / 28, 96 42 / 41, 128 63 / 96; 130944: 64
+// 47 / 34, 96 62 / 80. At 2048 steps 4096 channels 54 / 961, 16384 165 / 230 (buffer
+// kernel), 32768 269 / 262 (so not there).
 constexpr long kRingChannels = 16384;
+bool ring_pays(bool buf, int cpl, int B, int T, int N, bool gated) {
+    const long chans = (long)B * N;
+    if (buf) return chans < kRingChannels && T > 128;
+    if (cpl == 1) return T >= (chans < 4096 ? 80 : chans < 12288 ? 64 : chans < 24576 ? 48 : 32);
+    const long wgs = (long)B * ((N + 127) / 128);
+    return T > 128 && (gated || T <= 256 || wgs % 256 != 0);
+}
+bool ring_pays_bwd(bool buf, int B, int T, int N) {
+    const long chans = (long)B * N;
+    if (chans <= kRingChannels) return T >= 24;
+    return !buf && T >= std::min(96L, 24 + 24 * chans / 32768);
+}
 // Channels of a ring workgroup: half a wave where that still spreads the call over
 // at most one workgroup per CU. 32 / 64 of them, us: 8192 channels backward 90 /
 // 106, forward 35 / 36; 2331 channels of 333 steps backward 13 / 28; but 12288
@@ -612,9 +643,9 @@ snhip_status launch_ring_ds(const float* p, const float* dstate, float* out, int
 
 // Launch-shape selection. SNHIP_SCAN_SHAPE="kind,cpl,w,tc" (kind "buf", "gen" or
 // "ring"; for "ring" w is the channels of a workgroup) pins one compiled shape for
-// the tuning sweep and tests; otherwise the ring form for few channels, the buffer
-// kernel when the layout allows it, else the ring form again; the generic kernel
-// where an array is past the ring's 32-bit offsets.
+// the tuning sweep and tests; otherwise the ring form where it pays (ring_pays) and
+// its 32-bit offsets reach, else the buffer kernel when the layout allows it, else
+// the generic kernel.
 snhip_status launch_recur_scan(const float* a, const float* b, const float* s0,
                                float* out, float* send, int B, int T, int N,
                                int gated, hipStream_t st) {
@@ -630,9 +661,14 @@ snhip_status launch_recur_scan(const float* a, const float* b, const float* s0,
     char kind = 'g';
     int cpl = 1, w = 8, tc = 16;
     if (N % 2 == 0 && al8 && chans / 128 >= 192) cpl = 2;
-    if (buf_ok(2, 2 * 32) && chans / 128 >= 192) { kind = 'b'; cpl = 2; w = 2; tc = 32; }
+    // Two channels per lane above 16384 channels, and at 16384 while one tile of it
+    // holds every step; us, two / one: 16384 channels, 64 steps 5.1 / 5.6, 128 8.2 / 6.1,
+    // 2048 89 / 74; 18432, 16 steps 4.1 / 5.5, 160 10.4 / 12.5, 2048 90 / 98.
+    if (buf_ok(2, 2 * 32) && chans / 128 >= (T <= 64 ? 128 : 129)) { kind = 'b'; cpl = 2; w = 2; tc = 32; }
     else if (buf_ok(1, 4 * 32)) { kind = 'b'; cpl = 1; w = 4; tc = 32; }
-    if ((chans < kRingChannels || kind == 'g') && ring_scan_ok(B, T, N, N)) { kind = 'r'; cpl = 1; w = ring_ch(chans); tc = 32; }
+    if (ring_pays(kind == 'b', cpl, B, T, N, gated) && ring_scan_ok(B, T, N, N)) {
+        kind = 'r'; cpl = 1; w = ring_ch(chans); tc = 32;
+    }
     if (const char* env = getenv("SNHIP_SCAN_SHAPE")) {
         char k[8] = {0};
         int c = 0, ww = 0, t = 0;
@@ -840,8 +876,10 @@ snhip_status launch_scan_bwd(const float* p, const float* nu, const float* s0, c
     const bool al8 = aligned(p, 8) && aligned(nu, 8) && aligned(s0, 8) && aligned(out, 8) &&
                      aligned(dout, 8) && aligned(dp, 8) && aligned(dnu, 8) && aligned(ds0, 8);
     constexpr int C = 2, WW = 2, TT = 16;
-    const bool buf = N % (64 * C) == 0 && al8 && (long)T * N * 4 < (1L << 31);
-    if (((long)B * N <= kRingChannels || !buf) && ring_scan_ok(B, T, N, N)) {
+    const bool buf_ok = N % (64 * C) == 0 && al8 && (long)T * N * 4 < (1L << 31);
+    const bool ring_ok = ring_scan_ok(B, T, N, N);
+    const bool buf = buf_ok && ((long)B * N >= kRingChannels || !ring_ok);
+    if (ring_ok && ring_pays_bwd(buf_ok, B, T, N)) {
         RingArgs r = ring_args(p, dout, s0, dp, ds0, B, T, N);
         r.x2 = nu; r.x3 = out; r.y1 = dnu;
         r.ch = ring_ch((long)B * N);

@@ -1,8 +1,8 @@
 """The split form of the fused block core (gate kernels over the whole chip, the
 chain as a ring scan) against the oracle: widths and lengths at the edges of its
-lane pairs, chunks of time and ring workgroups, from aligned and unaligned
-storage, where the ddelta partials are limited by their scratch, with saturated
-gates, and with outputs that overlap inputs.
+lane pairs, chunks of time and ring workgroups and of the rules that choose it,
+from aligned and unaligned storage, where the ddelta partials are limited by
+their scratch, with saturated gates, and with outputs that overlap inputs.
 
 Bar: the reference's own (tests/test_architecture.py:738-740, 803-805), 1e-5 on
 states, u and p and 1e-4 on dq, ddelta and ds0 (relative to the largest
@@ -20,7 +20,8 @@ pytestmark = pytest.mark.gpu
 
 FWD_TOL, BWD_TOL = 1e-5, 1e-4
 SHAPES = [(1, 1, 8), (2, 7, 8), (3, 9, 40), (1, 33, 136), (2, 257, 200), (1, 2049, 8), (3, 64, 128),
-          (33, 31, 264), (32, 150, 2048)]
+          (33, 31, 264), (32, 150, 2048), (2, 32, 72), (2, 49, 72), (9, 33, 1000), (3, 49, 8),
+          (2, 75, 264)]
 
 
 def _inputs(B, T, D, seed):
@@ -78,7 +79,7 @@ def test_saturated_gates(gpu):
         assert np.abs(a[fin] - b[fin]).max() < FWD_TOL
 
 
-@pytest.mark.parametrize("B,T,D", [(2, 37, 40), (2, 64, 128)])
+@pytest.mark.parametrize("B,T,D", [(2, 37, 40), (2, 64, 128), (2, 57, 40), (2, 272, 128)])
 def test_outputs_over_inputs(gpu, B, T, D):
     """dq in place of q and ds0 in place of s0 give what separate outputs give."""
     print("core split, in place", B, T, D, flush=True)

@@ -1,7 +1,8 @@
 """The ring form of the recurrence (k_scan_ring: few channels, any width and
 length) against the oracle, bit for bit: forward in both forms and backward, at
-the edges of its 64-channel workgroups, its slots and its tiles, from an
-unaligned view; and with infinities and NaN against the other kernels."""
+the edges of its 64-channel workgroups, its slots and its tiles and of the rules
+that choose it (forward pinned to it and as chosen), from an unaligned view; and with
+infinities and NaN against the other kernels."""
 from __future__ import annotations
 
 import numpy as np
@@ -15,7 +16,9 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 1, 1), (3, 2, 7), (1, 33, 64), (2, 31, 65), (1, 256, 63), (5, 257, 13), (3, 333, 777),
           (2, 511, 128), (1, 513, 1000), (1, 1025, 8),
-          (3, 40, 2731), (9, 65, 2047)]
+          (3, 40, 2731), (9, 65, 2047),
+          (2, 23, 100), (2, 24, 100), (2, 79, 100), (2, 128, 128), (2, 129, 128), (13, 32, 1001),
+          (8, 64, 2048), (9, 65, 2048), (13, 129, 2046)]
 
 
 def _dev(x, off=0):
@@ -30,8 +33,11 @@ def _dev(x, off=0):
 
 @pytest.mark.parametrize("B,T,N", SHAPES)
 @pytest.mark.parametrize("gated", [True, False])
-def test_forward(gpu, B, T, N, gated):
-    print("ring scan", B, T, N, gated, flush=True)
+@pytest.mark.parametrize("pin", [None, "ring,1,32,32", "ring,1,64,32"])
+def test_forward(gpu, monkeypatch, B, T, N, gated, pin):
+    print("ring scan", B, T, N, gated, pin, flush=True)
+    if pin:
+        monkeypatch.setenv("SNHIP_SCAN_SHAPE", pin)
     rng = np.random.default_rng(T * 1000 + N)
     a = rng.random((B, T, N), dtype=np.float32)
     b = rng.standard_normal((B, T, N)).astype(np.float32)
@@ -69,6 +75,7 @@ def test_special_values(gpu, monkeypatch, gated):
     s0 = np.zeros((2, 72), np.float32)
     s0[0, :3] = [np.inf, -np.inf, np.nan]
     args = [_dev(x) for x in (a, b, s0)]
+    monkeypatch.setenv("SNHIP_SCAN_SHAPE", "ring,1,32,32")
     got = runtime.scan(*args, gated=gated)
     monkeypatch.setenv("SNHIP_SCAN_SHAPE", "gen,1,8,16")
     ref = runtime.scan(*args, gated=gated)
