@@ -11,8 +11,10 @@
 // one wave per (token, head). What is left for the recurrence is 8 multiply-adds
 // of the read, one of the update and 8 of the read-out per state element.
 //
-// Measured (12 x 768, INT4 g32, 512-token prompt): 3.4 ms, where the
-// token-by-token prefill took 345 ms (512 one-launch steps of 673 us).
+// Measured (12 x 768, INT4 g32, 512-token prompt): 2.85 ms of kernels (products 1.31,
+// recurrence 1.01, LayerNorms 0.34), 4.0 ms a call with the state read and the host's
+// copy of the logits, where the token-by-token prefill took 345 ms (512 one-launch
+// steps of 673 us).
 #include <algorithm>
 #include <type_traits>
 

@@ -15,8 +15,7 @@
 // * Heads: one wave per (head, sequence), lane i owning state row i.
 // * expf / tanhf: refmath.h (glibc's algorithms).
 #include <algorithm>
-#include <cstdio>
-#include <cstring>
+#include <cstdlib>
 #include <type_traits>
 
 #include "lanesum.h"
@@ -244,7 +243,7 @@ __global__ __launch_bounds__(LT) void k_rkq_ln(RkqLnArgs A) {
 // row-major x in the wave (11 instructions per MFMA), took 28 us for the
 // channel-mix value at B = 64; this one takes 15 (the 4x4x1 chains it replaced:
 // 26). The step at B = 64: 1,350 -> 1,030 us (12 x 768 INT4 g32); a 512-token
-// prefill chunk 4.8 -> 3.4 ms.
+// prefill chunk, kernels, 4.8 -> 3.4 ms (2.9 since the recurrence's interleaving).
 //
 // Weights (BLK): -1, tiled fp32 copies of the layer matrices, made at load
 // (k_rkq_tile); 32 / 64, INT4 codes: byte g of dword i of a group is exactly
@@ -785,6 +784,8 @@ snhip_status launch_rkq_mm(const RkqJob* jobs, int n, int B, int block, hipStrea
         const double cost = rounds * O * S == 1 ? 1.125 : (double)(rounds * O * S);
         if (h == 0 || cost <= best) { shape = h; best = cost; }
     }
+    // SNHIP_RKQ_SHAPE=0..3 pins one (tests).
+    if (const char* e = getenv("SNHIP_RKQ_SHAPE")) shape = std::min(3u, (unsigned)atoi(e));
     const int O = kShape[shape][0], S = kShape[shape][1];
     a.n = n;
     a.B = B;

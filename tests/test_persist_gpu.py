@@ -206,10 +206,9 @@ def test_barrier_timeout_reports_error(gpu, tiny, monkeypatch):
 
 @pytest.mark.parametrize("B", [1, 8])
 def test_ordinary_launch_equals_cooperative(gpu, small, monkeypatch, B):
-    """SNHIP_COOP=0 launches the same co-resident grid without the
-    cooperative flag (for tools that do not handle cooperative launches):
-    the B=1 persistent kernel and the batched one give the same tokens and
-    logits, bit for bit."""
+    """SNHIP_COOP=1 launches the same co-resident grid cooperatively instead of as
+    an ordinary launch (the default): the B=1 persistent kernel and the batched one
+    give the same tokens and logits, bit for bit."""
     w, buf, path = small
     print(f"cooperative vs ordinary launch, B={B}", flush=True)
     start = torch.arange(3, 3 + B, dtype=torch.int32, device=gpu)

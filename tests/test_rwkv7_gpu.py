@@ -261,9 +261,9 @@ def test_cfg4_int4_b1(gpu, cfg4):
 
 
 def _w4(monkeypatch, w4):
-    """SNHIP_RKQ_W4 for the next handle: "1" (default) multiplies the per-kernel
-    products on input-blocked fp32 copies made at load (one independent wave
-    per tile), "0" on the INT4 codes (producer waves dequantizing into LDS)."""
+    """SNHIP_RKQ_W4 for the next handle: "1" (default) multiplies the layers' products
+    on tiled fp32 copies made at load, "0" on the weights as stored (INT4 codes are
+    dequantized in the waves' registers)."""
     monkeypatch.setenv("SNHIP_RKQ_W4", w4)
 
 
@@ -292,12 +292,8 @@ def test_cfg4_int4_b64_exact(gpu, cfg4, monkeypatch, w4, fuse):
 
 @pytest.mark.parametrize("w4", ["1", "0"])
 def test_cfg4_int4_ragged_batch_exact(gpu, cfg4, monkeypatch, w4):
-    """B=37: the r/k/v and LoRA-up launches then take the staged-X form
-    (four consumers per workgroup, 16 sequences of X rows in LDS), with a last
-    sequence tile of 5 rows, and the wide vocabulary head four 16-sequence
-    chains per workgroup (three would cover 37, but only 1, 2 and 4 are
-    built: B = 33..48 once asked for three and the launch was refused);
-    sequences from the first and the partial tile replayed on the oracle,
+    """B=37: three sequence tiles, the last of 5 rows, where a wave takes one, two
+    or four of them; sequences from the first and the partial tile replayed on the oracle,
     three steps, logits identical."""
     p, dq = cfg4
     cfg = RWKV_CFG4
@@ -316,20 +312,57 @@ def test_cfg4_int4_ragged_batch_exact(gpu, cfg4, monkeypatch, w4):
         assert np.array_equal(a[pick], b)
 
 
-@pytest.mark.parametrize("shape", ["1,1", "1,2", "1,4", "2,1", "2,2", "2,4", "4,1", "4,2"])
+# Output x sequence tiles of a wave of the products (SNHIP_RKQ_SHAPE): 1x1, 1x2, 2x2, 2x4
+RKQ_SHAPES = ["0", "1", "2", "3"]
+
+
+@pytest.mark.parametrize("shape", RKQ_SHAPES)
+@pytest.mark.parametrize("fmt", ["tiled", "fp32 rows", "int4 32", "int4 64"])
+def test_product_shapes(gpu, tmp_path, monkeypatch, shape, fmt):
+    """Every shape of the products' waves in every form of the weights, in the layers
+    and the vocabulary head: inputs shorter than the read-ahead (ranks 12 to 68, not
+    multiples of 16, in the fp32 forms), outputs that no tile pair divides, and B = 37,
+    whose last sequence tile is partial and whose last group of tiles is not full; two
+    steps and a prefill, every sequence identical to the oracle's."""
+    print("rwkv7 products, shape", shape, fmt, flush=True)
+    int4 = fmt.startswith("int4")
+    cfg = RwkvConfig(layers=2, dim=192, head_size=64, ff=320, vocab=568,
+                     ranks=(64, 64, 64, 128) if int4 else (32, 68, 12, 100))
+    w = init_rwkv7(cfg, 6)
+    p = tmp_path / "w.bin"
+    p.write_bytes(pack_rwkv7_blob(w))
+    monkeypatch.setenv("SNHIP_RKQ_SHAPE", shape)
+    monkeypatch.setenv("SNHIP_RKQ_FUSE_UPS", "0")
+    monkeypatch.setenv("SNHIP_RK_EXACT", "0")
+    _w4(monkeypatch, "1" if fmt == "tiled" else "0")
+    B = 37
+    kw = {"weights": "int4", "block": int(fmt[5:])} if int4 else {}
+    hm = HipRwkv7(p, max_batch=B, **kw)
+    ref = pack_rwkv7_blob(dequant_weights(w, int(fmt[5:]))) if int4 else p.read_bytes()
+    rng = np.random.default_rng(7)
+    orc = oracle.RkOracle(ref, batch=B)
+    for _ in range(2):
+        toks = rng.integers(0, cfg.vocab, B).astype(np.int32)
+        a = hm.step_batch(torch.from_numpy(toks).cuda()).cpu().numpy()
+        assert np.array_equal(a, orc.step(toks))
+    hm.reset()
+    one = oracle.RkOracle(ref)
+    toks = [int(t) for t in rng.integers(0, cfg.vocab, 37)]
+    a = np.asarray(hm.prefill(toks), np.float32)
+    for t in toks:
+        b = one.step([t])[0]
+    assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape", RKQ_SHAPES)
 def test_cfg4_int4_tiled_product_shapes(gpu, cfg4, monkeypatch, shape):
-    """Every workgroup shape of the tiled fp32 products (S chains of 4
-    sequences per wave, NW waves per workgroup), forced with
-    SNHIP_RKQ_W4_SHAPE wherever it fits (the channel-mix value's K = 3072
-    takes one chain per wave; a shape over 64 KiB of LDS falls back to the
-    chosen one): B = 37, so the last sequence tile is partial and a
-    workgroup's last waves may have no tile; sequences of the first and the
-    partial tile replayed on the oracle, two steps, logits identical."""
+    """The same shapes at the 12-layer model's sizes, on the tiled fp32 weights, B = 37:
+    sequences of the first and the partial tile replayed on the oracle, two steps."""
     p, dq = cfg4
     cfg = RWKV_CFG4
     B = 37
-    print(f"rwkv7 cfg4 int4 g32 B={B}, tiled products forced to S,NW={shape}", flush=True)
-    monkeypatch.setenv("SNHIP_RKQ_W4_SHAPE", shape)
+    print(f"rwkv7 cfg4 int4 g32 B={B}, products' shape {shape}", flush=True)
+    monkeypatch.setenv("SNHIP_RKQ_SHAPE", shape)
     hm = HipRwkv7(p, weights="int4", block=32, max_batch=B)
     pick = [0, 3, 33, 36]
     orc = oracle.RkOracle(dq, batch=len(pick))
@@ -345,9 +378,7 @@ def test_cfg4_int4_tiled_product_shapes(gpu, cfg4, monkeypatch, shape):
 def test_cfg4_int4_every_batch_size(gpu, cfg4, monkeypatch, w4):
     """Every batch size 1..64 of the 12-layer INT4 model (1..8 on the exact
     one-launch kernel, one grid slice per sequence; from 9 on the per-kernel
-    step, whose launch shapes change with B: one or four consumers per
-    workgroup, staged or global X, narrow or wide chains and their counts):
-    one step from the reset state, the first and the last sequence identical
+    step, whose waves' shapes change with B): one step from the reset state, the first and the last sequence identical
     to the oracle's."""
     p, dq = cfg4
     cfg = RWKV_CFG4
