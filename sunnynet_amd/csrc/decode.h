@@ -84,7 +84,7 @@ bool persist_grid_ok(int G, int D, int I, int R, int vocab);
 snhip_status launch_decode_persist(const PersistArgs& a, int nwg, int blk, hipStream_t st);
 
 // Persistent step of a batch of sequences (batch.hip): every layer of one
-// decode step in one cooperative launch, phases separated by grid barriers.
+// decode step in one launch, phases separated by grid barriers.
 // Each phase writes its outputs to buffers no other phase of the launch
 // writes (per-layer slabs), with agent-coherent stores, so a barrier needs no
 // cache fences: a line a workgroup reads after a barrier was not cached by

@@ -1,5 +1,5 @@
 // Persistent decode of one sequence: every layer of every greedy step in one
-// cooperative launch (the B = 1 path of snhip_step / snhip_decode_greedy_dev).
+// launch (the B = 1 path of snhip_step / snhip_decode_greedy_dev).
 //
 // The math is the decode step of sunnynet/runtime/sunnynet.c:212-334 (LayerNorm,
 // depthwise conv, low-rank U V product, competitive and decay gates, state

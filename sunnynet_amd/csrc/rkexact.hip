@@ -1,5 +1,5 @@
 // RWKV-7 decode step for one sequence (or one per equal slice of the grid) as
-// one cooperative launch, rounded in the reference's order
+// one launch, rounded in the reference's order
 // (sunnynet/runtime/rwkv7.c:127-360), so that a step gives the reference's
 // bits. The phases, exchange words, waits and the ordering of the shift
 // vectors' rewrites are rkpersist.hip's:

@@ -1,4 +1,4 @@
-// RWKV-7 decode at one sequence as one cooperative launch per step
+// RWKV-7 decode at one sequence as one launch per step
 // (rkpersist.hip): the shared types between the handle (rwkv.hip) and the
 // kernel.
 #pragma once

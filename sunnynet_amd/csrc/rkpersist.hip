@@ -1,4 +1,4 @@
-// RWKV-7 decode step for one sequence as one cooperative launch
+// RWKV-7 decode step for one sequence as one launch
 // (sunnynet/runtime/rwkv7.c:143-360; the math is the one listed at the top of
 // rwkv.hip).
 //

@@ -1,5 +1,5 @@
 """The persistent batched step (every layer of a step of 3..64 sequences in one
-cooperative launch, each tile waiting on the flags of the tiles it reads)
+launch, each tile waiting on the flags of the tiles it reads)
 against the oracle and the per-kernel step path.
 
 Bar as for every decode path: logits within 2e-5 absolute of the C oracle

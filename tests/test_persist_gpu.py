@@ -1,4 +1,4 @@
-"""The persistent single-sequence decode (one cooperative launch per call,
+"""The persistent single-sequence decode (one launch per call,
 grid barriers between the phases of every layer) against the oracle and the
 per-kernel step path.
 
