@@ -62,10 +62,9 @@ void dev_free(void* p) {
 }
 
 namespace {
-// A gate that another process has not opened for this long is passed with a
-// cooperative launch: the longest hold is a launch of a second or so.
+// How long a call waits for another process to open the gate (the longest hold is a
+// launch of a second or so) before it does without.
 constexpr double kGateSeconds = 60.0;
-thread_local bool t_shared = false;   // this thread's PersistCall holds the gate against its process only
 
 // The device's gate; its files are named by the card's PCI address.
 DeviceGate* gate_of(int dev) {
@@ -83,14 +82,16 @@ DeviceGate* gate_of(int dev) {
 }
 }  // namespace
 
-hipError_t PersistCall::enter() {
+hipError_t PersistCall::enter(bool* alone) {
+    *alone = false;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if ((e = hipStreamSynchronize(st_)) != hipSuccess) return e;
     DeviceGate* g = gate_of(dev);
-    t_shared = !g->enter(kGateSeconds);
-    gate_ = g;
+    const char* limit = getenv("SNHIP_GATE_SECONDS");
+    *alone = g->enter(limit ? atof(limit) : kGateSeconds);
+    if (*alone) gate_ = g;
     return hipSuccess;
 }
 hipError_t PersistCall::finish() {
@@ -98,12 +99,11 @@ hipError_t PersistCall::finish() {
     const hipError_t e = hipStreamSynchronize(st_);
     gate_->leave();
     gate_ = nullptr;
-    t_shared = false;
     return e;
 }
 
 hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st) {
-    if (t_shared || env_unsigned("SNHIP_COOP", 0, 0) != 0)
+    if (env_unsigned("SNHIP_COOP", 0, 0) != 0)
         return hipLaunchCooperativeKernel(k, grid, block, args, 0, st);
     return hipLaunchKernel(k, grid, block, args, 0, st);
 }

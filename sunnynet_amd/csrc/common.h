@@ -69,7 +69,9 @@ class PersistCall {
 public:
     explicit PersistCall(hipStream_t st) : st_(st) {}
     ~PersistCall() { (void)finish(); }
-    hipError_t enter();
+    // *alone: whether other processes are kept out too (see devgate.h); if not, the
+    // gate is not held and the caller takes kernels that need no co-resident grid.
+    hipError_t enter(bool* alone);
     hipError_t finish();
     PersistCall(const PersistCall&) = delete;
     PersistCall& operator=(const PersistCall&) = delete;
@@ -86,8 +88,10 @@ private:
 // call (SunnyNet-100M fp32 B = 1 step 315 -> 258 us). What the cooperative queue
 // also gave, that no two such kernels share the device, the gate keeps, among this
 // process's threads and among the processes that see its files (in SNHIP_LOCK_DIR,
-// by default /tmp; containers that share a card share that folder, or set
-// SNHIP_COOP=1). Without the files, and with SNHIP_COOP=1, the launch is cooperative.
+// by default /tmp: containers that share a card share that folder). Without the
+// files a call takes the per-kernel step. SNHIP_COOP=1 launches cooperatively; the
+// runtime gives the cooperative queue to one process at a time, and the launches
+// of others fail.
 hipError_t launch_persistent(const void* k, dim3 grid, dim3 block, void** args, hipStream_t st);
 
 // Steps of one launch, or of the launches of one hold of the gate, so that other

@@ -30,26 +30,26 @@ public:
     DeviceGate(const DeviceGate&) = delete;
     DeviceGate& operator=(const DeviceGate&) = delete;
 
-    // Waits for the gate. True if it is held against other processes too; false
-    // if only against this one's threads: the files cannot be opened, or a holder
-    // has not let go for `limit` seconds (it is stopped, or hangs).
+    // Waits for the gate. False, and not held, if other processes cannot be kept out:
+    // the files cannot be opened, or a holder has not let go for `limit` seconds (it is
+    // stopped, or hangs; the next calls then do not wait until it has).
     bool enter(double limit) {
         next_.lock();
         hold_.lock();
-        const bool all = enter_files(limit);
+        const bool all = enter_files(stuck_ ? 0.0 : limit);
+        if (!all) hold_.unlock();
         next_.unlock();
         return all;
     }
     void leave() {
-        if (fheld_) (void)flock(fhold_, LOCK_UN);
-        fheld_ = false;
+        (void)flock(fhold_, LOCK_UN);
         hold_.unlock();
     }
 
 private:
     std::mutex next_, hold_;
     const std::string path_;
-    bool opened_ = false, fheld_ = false;   // under hold_
+    bool opened_ = false, stuck_ = false;   // under hold_
     int fnext_ = -1, fhold_ = -1;
 
     // Any user of the device may lock the files: flock needs no write access.
@@ -85,10 +85,11 @@ private:
         if (fnext_ < 0 || fhold_ < 0) return false;
         const auto end = std::chrono::steady_clock::now() +
                          std::chrono::duration_cast<std::chrono::steady_clock::duration>(std::chrono::duration<double>(limit));
-        if (!lock_by(fnext_, end)) return false;
-        fheld_ = lock_by(fhold_, end);
+        stuck_ = !lock_by(fnext_, end);
+        if (stuck_) return false;
+        stuck_ = !lock_by(fhold_, end);
         (void)flock(fnext_, LOCK_UN);
-        return fheld_;
+        return !stuck_;
     }
 };
 

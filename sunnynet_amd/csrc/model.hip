@@ -858,8 +858,8 @@ int setup_persist_mi(SnHipModel* m, int ncu, int cap) {
     return std::max(1, m->mi_max);
 }
 
-// Enables the persistent single-sequence decode when the shape fits it and the
-// device supports cooperative launches (SNHIP_PERSIST=0 turns it off;
+// Enables the persistent single-sequence decode when the shape fits it and its
+// grid co-resides on the device (SNHIP_PERSIST=0 turns it off;
 // SNHIP_PERSIST_WG caps the grid size). The grid is the largest size the
 // kernel accepts for the shape (persist_grid_ok) up to one workgroup per CU
 // and per four channels (fp32 / fp16 rows) or eight (INT4 rows): measured
@@ -904,7 +904,7 @@ void setup_persist(SnHipModel* m) {
 }
 
 // Enables the persistent batched step (batch.hip) when the shape fits it and
-// the device supports cooperative launches (SNHIP_BATCH_PERSIST=0 turns it
+// its grid co-resides on the device (SNHIP_BATCH_PERSIST=0 turns it
 // off). Its per-layer slabs are sized for min(max_batch, batch_max) rows.
 void setup_batch(SnHipModel* m) {
     if (const char* e = getenv("SNHIP_BATCH_PERSIST"))
@@ -1259,12 +1259,14 @@ snhip_status enqueue_layer_gemv(SnHipModel* m, int B, int l, hipStream_t st) {
 // Enqueue one decode step for sequences [0, B) on `st`; tokens in tok (device).
 // greedy: the head also reduces the first maximal logit per sequence and a
 // final kernel writes it to m->tok (the next step's input) and m->tok_hist.
-snhip_status enqueue_step(SnHipModel* m, const int32_t* tok, int B, float* logits_out, bool greedy, hipStream_t st) {
+// batch: as the batched persistent kernel (inside a PersistCall).
+snhip_status enqueue_step(SnHipModel* m, const int32_t* tok, int B, float* logits_out, bool greedy, hipStream_t st,
+                          bool batch = false) {
     const int D = m->D, I = m->I, R = m->R, L = m->L;
     const size_t sbs = (size_t)L * D;                               // s batch stride
     const size_t hbs = (size_t)L * (m->kh ? m->kh : 1) * D;         // hist batch stride
-    if (uses_batch(m, B)) {
-        // Every layer in one cooperative launch (the embedding rows gathered
+    if (batch) {
+        // Every layer in one launch (the embedding rows gathered
         // inside), then the head.
         BatchArgs a{};
         a.layers = m->dlayers;
@@ -1374,9 +1376,49 @@ snhip_status follow_streams(SnHipModel* m) {
     return SNHIP_OK;
 }
 
+// Why a persistent call has not run: the caller takes another path.
+enum NotRun { RAN, NOT_RUN_FAILED, NOT_RUN_SHARED };
+
+// The gate was not to be had after `done` steps of a call.
+snhip_status gate_lost(int done, bool* shared) {
+    *shared = done == 0;
+    if (done == 0) return SNHIP_OK;
+    set_last_error("another process has kept the device from this call's next steps");
+    return SNHIP_E_DEVICE;
+}
+
 // Copies B tokens into m->tok on the caller's stream.
 snhip_status put_tokens(SnHipModel* m, const int32_t* t, int B, hipMemcpyKind kind) {
     SNHIP_CHECK(hipMemcpyAsync(m->tok, t, B * sizeof(int32_t), kind, m->stream));
+    return SNHIP_OK;
+}
+
+// `reps` batched persistent steps on the caller's stream, the first on tok (device):
+// a handful of launches each, queued directly. Returns once they have finished, so
+// that a wait's time-out is reported by this call, not a later one. *shared: the
+// device cannot be kept from other processes, nothing ran.
+snhip_status run_batch(SnHipModel* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps,
+                       bool* shared) {
+    m->persist_stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
+    for (int i = 0; i < reps;) {
+        PersistCall call(m->stream);
+        bool alone = false;
+        SNHIP_CHECK(call.enter(&alone));
+        if (!alone) return gate_lost(i, shared);
+        if (i == 0 && greedy && tok != m->tok) {
+            // greedy steps write the next tokens to m->tok
+            const snhip_status rc = put_tokens(m, tok, B, hipMemcpyDeviceToDevice);
+            if (rc != SNHIP_OK) return rc;
+            tok = m->tok;
+        }
+        for (const int end = std::min(reps, i + kPersistHoldSteps); i < end; ++i) {
+            const snhip_status rc = enqueue_step(m, tok, B, logits_out, greedy, m->stream, true);
+            if (rc != SNHIP_OK) return rc;
+        }
+        SNHIP_CHECK(call.finish());
+        const snhip_status st = persist_status(m, B);
+        if (st != SNHIP_OK) return st;
+    }
     return SNHIP_OK;
 }
 
@@ -1385,30 +1427,17 @@ snhip_status put_tokens(SnHipModel* m, const int32_t* t, int B, hipMemcpyKind ki
 // of about 20 us.) The step's kernels are captured once per (B, logits, greedy)
 // into a HIP graph, which reads m->tok, and replayed.
 snhip_status run_steps(SnHipModel* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps) {
-    const bool batch = uses_batch(m, B);
-    if (tok != m->tok && (!batch || greedy)) {
-        // greedy steps write the next tokens to m->tok
+    if (uses_batch(m, B)) {
+        bool shared = false;
+        const snhip_status rc = run_batch(m, tok, B, logits_out, greedy, reps, &shared);
+        if (!shared) return rc;
+    }
+    if (tok != m->tok) {
         const snhip_status rc = put_tokens(m, tok, B, hipMemcpyDeviceToDevice);
         if (rc != SNHIP_OK) return rc;
         tok = m->tok;
     }
-    if (batch) {
-        // The batched persistent step is a handful of launches per step: they
-        // are queued directly. The call returns once its launches have finished,
-        // so that a barrier time-out is reported by this call, not a later one.
-        m->persist_stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
-        for (int i = 0; i < reps;) {
-            PersistCall call(m->stream);
-            SNHIP_CHECK(call.enter());
-            for (const int end = std::min(reps, i + kPersistHoldSteps); i < end; ++i) {
-                const snhip_status rc = enqueue_step(m, tok, B, logits_out, greedy, m->stream);
-                if (rc != SNHIP_OK) return rc;
-            }
-            SNHIP_CHECK(call.finish());
-            const snhip_status st = persist_status(m, B);
-            if (st != SNHIP_OK) return st;
-        }
-    } else if (!m->use_graphs) {
+    if (!m->use_graphs) {
         for (int i = 0; i < reps; ++i) {
             const snhip_status rc = enqueue_step(m, tok, B, logits_out, greedy, m->stream);
             if (rc != SNHIP_OK) return rc;
@@ -1435,7 +1464,7 @@ snhip_status run_steps(SnHipModel* m, const int32_t* tok, int B, float* logits_o
         }
         for (int i = 0; i < reps; ++i) SNHIP_CHECK(hipGraphLaunch(it->second, m->stream));
     }
-    if (!batch) SNHIP_CHECK(m->order.mark(m->stream));   // (the batched step is done)
+    SNHIP_CHECK(m->order.mark(m->stream));
     return SNHIP_OK;
 }
 
@@ -1719,10 +1748,12 @@ snhip_status run_prefill(SnHipModel* m, const int32_t* tokens_dev, int B, int T,
 // The call returns once the launches have finished and reports an exchange
 // time-out as SNHIP_E_DEVICE. Each workgroup writes its channels' state back
 // after its own last wait, so a time-out can leave the sequences part-stepped:
-// the handle then refuses steps until reset or set. *launch_failed is set when the
-// first cooperative launch could not be queued at all (nothing ran).
+// the handle then refuses steps until reset or set. *not_run tells why
+// nothing ran: the first launch could not be queued, or the device cannot be kept
+// from other processes. The device's gate is given
+// away every kPersistHoldSteps steps.
 snhip_status run_persist(SnHipModel* m, const int32_t* tok, int B, int n_steps, bool greedy, int32_t* out_tok,
-                         float* logits, bool* launch_failed) {
+                         float* logits, NotRun* not_run) {
     PersistArgs a{};
     a.layers = m->dlayers;
     a.L = m->L; a.D = m->D; a.I = m->I; a.R = m->R; a.K = m->K; a.kh = m->kh;
@@ -1757,10 +1788,16 @@ snhip_status run_persist(SnHipModel* m, const int32_t* tok, int B, int n_steps, 
         a.logits = done + n == n_steps ? logits : nullptr;
         a.n_steps = n;
         PersistCall call(m->stream);
-        SNHIP_CHECK(call.enter());
+        bool alone = false, shared = false;
+        SNHIP_CHECK(call.enter(&alone));
+        if (!alone) {
+            const snhip_status rc = gate_lost(done, &shared);
+            if (shared) *not_run = NOT_RUN_SHARED;
+            return rc;
+        }
         snhip_status rc = launch_decode_persist(a, grid, blk, m->stream);
         if (rc != SNHIP_OK) {
-            if (done == 0 && launch_failed) *launch_failed = true;
+            if (done == 0) *not_run = NOT_RUN_FAILED;
             return rc;
         }
         SNHIP_CHECK(call.finish());
@@ -1776,28 +1813,28 @@ bool uses_mi(const SnHipModel* m, int B) { return m->persist_wg > 0 && m->all_cu
 
 // One step of sequences [0, B), B >= 2, on tok (device): the single-sequence
 // persistent kernel on a slice of the grid per sequence when it takes B, else
-// the per-kernel or batched step. A failed cooperative launch turns the
+// the per-kernel or batched step. A launch that fails turns the
 // persistent path for B >= 2 off and falls back.
 snhip_status step_many(SnHipModel* m, const int32_t* tok, int B, float* logits_out) {
     if (uses_mi(m, B)) {
-        bool launch_failed = false;
-        const snhip_status rc = run_persist(m, tok, B, 1, false, nullptr, logits_out, &launch_failed);
-        if (!launch_failed) return rc;
-        m->mi_max = 0;
+        NotRun why = RAN;
+        const snhip_status rc = run_persist(m, tok, B, 1, false, nullptr, logits_out, &why);
+        if (why == RAN) return rc;
+        if (why == NOT_RUN_FAILED) m->mi_max = 0;
         (void)hipGetLastError();
     }
     return run_steps(m, tok, B, logits_out, false, 1);
 }
 
 // One step of sequence 0 on tok (device): the persistent kernel
-// when enabled, else the captured per-kernel step. A failed cooperative launch
+// when enabled, else the captured per-kernel step. A launch that fails
 // turns the persistent path off for this handle and falls back.
 snhip_status step_one(SnHipModel* m, const int32_t* tok, float* logits_out) {
     if (m->persist_wg && m->all_cus) {
-        bool launch_failed = false;
-        const snhip_status rc = run_persist(m, tok, 1, 1, false, nullptr, logits_out, &launch_failed);
-        if (!launch_failed) return rc;
-        m->persist_wg = 0;
+        NotRun why = RAN;
+        const snhip_status rc = run_persist(m, tok, 1, 1, false, nullptr, logits_out, &why);
+        if (why == RAN) return rc;
+        if (why == NOT_RUN_FAILED) m->persist_wg = 0;
         (void)hipGetLastError();
     }
     return run_steps(m, tok, 1, logits_out, false, 1);
@@ -1994,17 +2031,17 @@ snhip_status snhip_decode_greedy_dev(SnHipModel* m, const int32_t* tokens_dev, i
         return SNHIP_E_INVAL;
     if (check_usable(m) != SNHIP_OK || follow_streams(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     if (B == 1 && m->persist_wg && m->all_cus) {
-        bool launch_failed = false;
-        const snhip_status rc = run_persist(m, tokens_dev, 1, n_steps, true, out_tokens_dev, logits_dev, &launch_failed);
-        if (!launch_failed) return rc;
-        m->persist_wg = 0;
+        NotRun why = RAN;
+        const snhip_status rc = run_persist(m, tokens_dev, 1, n_steps, true, out_tokens_dev, logits_dev, &why);
+        if (why == RAN) return rc;
+        if (why == NOT_RUN_FAILED) m->persist_wg = 0;
         (void)hipGetLastError();
     }
     if (uses_mi(m, B)) {
-        bool launch_failed = false;
-        const snhip_status rc = run_persist(m, tokens_dev, B, n_steps, true, out_tokens_dev, logits_dev, &launch_failed);
-        if (!launch_failed) return rc;
-        m->mi_max = 0;
+        NotRun why = RAN;
+        const snhip_status rc = run_persist(m, tokens_dev, B, n_steps, true, out_tokens_dev, logits_dev, &why);
+        if (why == RAN) return rc;
+        if (why == NOT_RUN_FAILED) m->mi_max = 0;
         (void)hipGetLastError();
     }
     if ((long)n_steps * B > (long)m->hist_cap || !m->tok_hist) {

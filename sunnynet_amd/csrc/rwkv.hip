@@ -22,7 +22,7 @@
 // kernel per head for the decay, mixes, normalized kk, the 64 x 64 state
 // update and read-out, group norm, bonus and gate. A step therefore gives the
 // reference's logits bit for bit on the same weights. Single-sequence steps
-// may instead run as one cooperative launch (rkpersist.hip).
+// may instead run as one launch (rkpersist.hip).
 // Weights live row-major (out, in), fp32 or INT4.
 #include <cstdio>
 #include <cstdlib>
@@ -159,7 +159,7 @@ struct SnHipRwkv7 {
     std::map<int, hipGraphExec_t> graphs;   // the captured layers, by batch size
     bool use_graphs = true;
     bool fuse_ups = true;   // LoRA up-projections inside the heads kernel (SNHIP_RKQ_FUSE_UPS=0: apart)
-    // One-sequence steps as one cooperative launch each (rkpersist.hip);
+    // One-sequence steps as one launch each (rkpersist.hip);
     // p_grid = 0 when off (SNHIP_RK_PERSIST=0, or a shape it does not take).
     int p_grid = 0;
     bool p_exact = false;                 // the kernel is k_rk_exact (else k_rk_persist)
@@ -429,7 +429,9 @@ bool uses_mi(const SnHipRwkv7* m, int B) { return m->p_grid > 0 && m->all_cus &&
 // The kernel updates S and shift in place layer by layer, so a time-out
 // leaves them part-stepped: the handle is then refused for stepping until its
 // state is reset or set.
-snhip_status run_persist(SnHipRwkv7* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps) {
+// *shared: the device cannot be kept from other processes, nothing ran.
+snhip_status run_persist(SnHipRwkv7* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps,
+                         bool* shared) {
     RkPArgs a = m->p_args;
     a.stall = env_unsigned("SNHIP_PERSIST_STALL", 0, 0);
     a.logits = logits_out;
@@ -451,7 +453,14 @@ snhip_status run_persist(SnHipRwkv7* m, const int32_t* tok, int B, float* logits
         m->p_epoch += (unsigned)n;
         a.tok_in = i == 0 ? tok : m->tok;
         PersistCall call(m->stream);
-        SNHIP_CHECK(call.enter());
+        bool alone = false;
+        SNHIP_CHECK(call.enter(&alone));
+        if (!alone) {
+            *shared = i == 0;
+            if (*shared) return SNHIP_OK;
+            set_last_error("another process has kept the device from this call's next steps");
+            return SNHIP_E_DEVICE;
+        }
         const snhip_status rc = m->p_exact ? launch_rk_exact(a, grid, m->stream) : launch_rk_persist(a, grid, m->stream);
         if (rc != SNHIP_OK) return rc;
         SNHIP_CHECK(call.finish());
@@ -806,37 +815,38 @@ snhip_status enqueue_head(SnHipRwkv7* m, int B, float* logits_out, bool greedy, 
 snhip_status run_steps(SnHipRwkv7* m, const int32_t* tok, int B, float* logits_out, bool greedy, int reps) {
     if (check_usable(m) != SNHIP_OK) return SNHIP_E_DEVICE;
     if ((B == 1 && m->p_grid > 0 && m->all_cus) || uses_mi(m, B)) {
-        return run_persist(m, tok ? tok : m->tok, B, logits_out, greedy, reps);
-    } else {
-        if (tok) SNHIP_CHECK(hipMemcpyAsync(m->tok, tok, B * sizeof(int32_t), hipMemcpyDeviceToDevice, m->stream));
-        hipGraphExec_t ex = nullptr;
-        if (m->use_graphs) {
-            auto it = m->graphs.find(B);
-            if (it == m->graphs.end()) {
-                if (m->graphs.size() >= 16) {
-                    for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
-                    m->graphs.clear();
-                }
-                hipGraph_t g = nullptr;
-                SNHIP_CHECK(hipStreamBeginCapture(m->cap, hipStreamCaptureModeThreadLocal));
-                const snhip_status rc = enqueue_layers(m, B, m->cap);
-                const hipError_t ec = hipStreamEndCapture(m->cap, &g);
-                if (rc != SNHIP_OK) { if (g) (void)hipGraphDestroy(g); return rc; }
-                SNHIP_CHECK(ec);
-                const hipError_t ei = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-                (void)hipGraphDestroy(g);
-                SNHIP_CHECK(ei);
-                it = m->graphs.emplace(B, ex).first;
+        bool shared = false;
+        const snhip_status rc = run_persist(m, tok ? tok : m->tok, B, logits_out, greedy, reps, &shared);
+        if (!shared) return rc;
+    }
+    if (tok) SNHIP_CHECK(hipMemcpyAsync(m->tok, tok, B * sizeof(int32_t), hipMemcpyDeviceToDevice, m->stream));
+    hipGraphExec_t ex = nullptr;
+    if (m->use_graphs) {
+        auto it = m->graphs.find(B);
+        if (it == m->graphs.end()) {
+            if (m->graphs.size() >= 16) {
+                for (auto& kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
+                m->graphs.clear();
             }
-            ex = it->second;
+            hipGraph_t g = nullptr;
+            SNHIP_CHECK(hipStreamBeginCapture(m->cap, hipStreamCaptureModeThreadLocal));
+            const snhip_status rc = enqueue_layers(m, B, m->cap);
+            const hipError_t ec = hipStreamEndCapture(m->cap, &g);
+            if (rc != SNHIP_OK) { if (g) (void)hipGraphDestroy(g); return rc; }
+            SNHIP_CHECK(ec);
+            const hipError_t ei = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
+            (void)hipGraphDestroy(g);
+            SNHIP_CHECK(ei);
+            it = m->graphs.emplace(B, ex).first;
         }
-        for (int i = 0; i < reps; ++i) {
-            snhip_status rc = SNHIP_OK;
-            if (ex) SNHIP_CHECK(hipGraphLaunch(ex, m->stream));
-            else rc = enqueue_layers(m, B, m->stream);
-            if (rc == SNHIP_OK) rc = enqueue_head(m, B, logits_out, greedy, m->stream);
-            if (rc != SNHIP_OK) return rc;
-        }
+        ex = it->second;
+    }
+    for (int i = 0; i < reps; ++i) {
+        snhip_status rc = SNHIP_OK;
+        if (ex) SNHIP_CHECK(hipGraphLaunch(ex, m->stream));
+        else rc = enqueue_layers(m, B, m->stream);
+        if (rc == SNHIP_OK) rc = enqueue_head(m, B, logits_out, greedy, m->stream);
+        if (rc != SNHIP_OK) return rc;
     }
     SNHIP_CHECK(m->order.mark(m->stream));
     return SNHIP_OK;

@@ -3,8 +3,8 @@
 //       inside it reads, waits and writes back the number in COUNTER plus one
 //   loop PATH SECONDS                  passes it without a pause; prints how often
 //   hold PATH SECONDS                  enters, prints "in", sleeps holding it
-//   try PATH LIMIT                     enters once, prints whether other processes are
-//                                      kept out and how long it took
+//   try PATH LIMIT [N PAUSE]           tries to enter once (N times, PAUSE seconds apart),
+//                                      prints whether it did and how long it took
 #include <unistd.h>
 
 #include <cstdio>
@@ -58,10 +58,14 @@ int main(int argc, char** argv) {
         usleep((useconds_t)(atof(argv[3]) * 1e6));
         gate.leave();
     } else if (mode == "try") {
-        const double t = now();
-        const bool all = gate.enter(atof(argv[3]));
-        printf("%d %.3f\n", all, now() - t);
-        gate.leave();
+        for (int i = 0; i < (argc > 4 ? atoi(argv[4]) : 1); ++i) {
+            if (i) usleep((useconds_t)(atof(argv[5]) * 1e6));
+            const double t = now();
+            const bool in = gate.enter(atof(argv[3]));
+            printf("%d %.3f\n", in, now() - t);
+            fflush(stdout);
+            if (in) gate.leave();
+        }
     }
     return 0;
 }

@@ -52,13 +52,17 @@ def test_a_killed_holder_lets_go(exe, tmp_path):
     assert _run(exe, "try", tmp_path / "gate", 10).stdout.split()[0] == "1"
 
 
-def test_a_stuck_holder_is_not_waited_for_longer_than_the_limit(exe, tmp_path):
+def test_a_stuck_holder_is_waited_for_once(exe, tmp_path):
+    """Up to the limit, and not again until it has let go."""
     p = subprocess.Popen([exe, "hold", tmp_path / "gate", "20"], stdout=subprocess.PIPE, text=True)
     assert p.stdout.readline() == "in\n"
-    ok, took = _run(exe, "try", tmp_path / "gate", 0.3).stdout.split()
+    q = subprocess.Popen([exe, "try", tmp_path / "gate", "0.3", "4", "0.5"], stdout=subprocess.PIPE, text=True)
+    tries = [q.stdout.readline().split() for _ in range(2)]
     p.kill()
     p.wait(20)
-    assert ok == "0" and 0.25 < float(took) < 5
+    tries += [x.split() for x in q.communicate(timeout=20)[0].splitlines()]
+    assert [x[0] for x in tries] == ["0", "0", "1", "1"]
+    assert 0.25 < float(tries[0][1]) < 5 and all(float(x[1]) < 0.2 for x in tries[1:])
 
 
 @pytest.mark.parametrize("what", ["no folder", "a folder", "a fifo", "a link"])

@@ -4,6 +4,8 @@ share the device), and a handle that moves between streams goes on from its stat
 also while its earlier calls are still running."""
 from __future__ import annotations
 
+import ctypes
+import fcntl
 import subprocess
 import sys
 import threading
@@ -303,30 +305,50 @@ _CHILD = """
 import sys
 import numpy as np, torch
 sys.path.insert(0, sys.argv[1])
-from sunnynet_amd.config import SMALL as c
-from sunnynet_amd.runtime.model import HipModel
-h = HipModel(sys.argv[2], c.vocab_size, c.dim, c.inner, c.rank, c.taps, c.layers, max_batch=4)
-rng = np.random.default_rng(5)
-toks = [torch.from_numpy(rng.integers(0, h.vocab, 4).astype(np.int32)).cuda() for _ in range(24)]
+from pathlib import Path
+from tests.test_streams_gpu import _make, _tokens
+h = {k: _make(k, (Path(sys.argv[2]), Path(sys.argv[3]))) for k in sys.argv[5:]}
+toks = {k: _tokens(x) for k, x in h.items()}
 torch.cuda.synchronize()
 print("ready", flush=True)
 sys.stdin.readline()
-for _ in range(20):
-    h.reset()
-    out = torch.stack([h.step_batch(t) for t in toks]).cpu().numpy()
-np.save(sys.argv[3], out)
-h.close()
+out = {}
+for k, x in h.items():
+    for _ in range(10):
+        x.reset()
+        out[k] = torch.stack([x.step_batch(t) for t in toks[k]]).cpu().numpy()
+    x.reset()
+    out[k + " greedy"] = x.decode_greedy(toks[k][0], 8).cpu().numpy()
+np.savez(sys.argv[4], **out)
+for x in h.values():
+    x.close()
 """
 
 
-@pytest.mark.parametrize("n,lock_dir", [(2, "shared"), (1, "none")])
-def test_processes(gpu, paths, tmp_path, monkeypatch, n, lock_dir):
+def _tokens(h):
+    rng = np.random.default_rng(5)
+    return [torch.from_numpy(rng.integers(0, h.vocab, h.max_batch).astype(np.int32)).cuda() for _ in range(24)]
+
+
+@pytest.mark.parametrize("n,locks", [(2, "shared"), (1, "no folder"), (1, "stuck")])
+def test_processes(gpu, paths, tmp_path, monkeypatch, n, locks):
     """Two processes that step on one device at once: each gets what it gets alone.
-    Without a folder for the lock files the launches are cooperative."""
-    print("processes:", n, "lock folder:", lock_dir, flush=True)
-    monkeypatch.setenv("SNHIP_LOCK_DIR", str(tmp_path if lock_dir == "shared" else tmp_path / "missing"))
+    Without a folder for the lock files, and while another process sits on them, the
+    calls take the per-kernel steps."""
+    print("processes:", n, "lock files:", locks, flush=True)
+    kinds = ["sunny1", "sunny4", "sunny20", "rwkv1"]
+    monkeypatch.setenv("SNHIP_LOCK_DIR", str(tmp_path / "missing" if locks == "no folder" else tmp_path))
+    monkeypatch.setenv("SNHIP_GATE_SECONDS", "0.2" if locks == "stuck" else "60")
+    pci = ctypes.create_string_buffer(64)
+    assert _native.lib().hipDeviceGetPCIBusId(pci, 64, 0) == 0
+    lock = tmp_path / f"snhip-{pci.value.decode()}.lock"
+    held = None
+    if locks == "stuck":
+        held = open(lock, "w")
+        fcntl.flock(held, fcntl.LOCK_EX)
     root = str(Path(__file__).resolve().parents[1])
-    ps = [subprocess.Popen([sys.executable, "-c", _CHILD, root, str(paths[0]), str(tmp_path / f"o{i}.npy")],
+    ps = [subprocess.Popen([sys.executable, "-c", _CHILD, root, str(paths[0]), str(paths[1]),
+                            str(tmp_path / f"o{i}.npz"), *kinds],
                            stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True) for i in range(n)]
     try:
         for p in ps:
@@ -338,9 +360,20 @@ def test_processes(gpu, paths, tmp_path, monkeypatch, n, lock_dir):
     finally:
         for p in ps:
             p.kill()
-    assert (len(list(tmp_path.glob("snhip-*.lock*"))) == 2) == (lock_dir == "shared")
-    h = _make("sunny4", paths)
-    want = torch.stack(_run(h, "sunny4", 24, [torch.cuda.current_stream()])).numpy()
-    for i in range(n):
-        assert np.array_equal(np.load(tmp_path / f"o{i}.npy"), want), i
-    h.close()
+        if held:
+            held.close()
+    assert lock.exists() == (locks != "no folder")
+    for k in kinds:
+        h = _make(k, paths)
+        toks = _tokens(h)
+        want = torch.stack([h.step_batch(t) for t in toks]).cpu().numpy()
+        h.reset()
+        greedy = h.decode_greedy(toks[0], 8).cpu().numpy()
+        for i in range(n):
+            o = np.load(tmp_path / f"o{i}.npz")
+            if locks == "shared" or k == "rwkv1":
+                assert np.array_equal(o[k], want), (i, k)
+            else:                                         # another order of the sums
+                assert np.abs(o[k] - want).max() < 2e-5, (i, k)
+            assert np.array_equal(o[k + " greedy"], greedy), (i, k)
+        h.close()
