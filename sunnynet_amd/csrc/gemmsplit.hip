@@ -253,7 +253,7 @@ __device__ float split_bad(const uint16_t* xp, const uint16_t* wp, int m, int n,
 // outputs. A stage is KB blocks of 16 in k: a wave's X fragments are its own and come
 // straight to registers, the W fragments are shared through LDS; the next stage of
 // both is in flight while this one is multiplied. Three fp16 products per fp32 one:
-// N = K = 1024 at 8192 rows takes 55 us, 940 TFLOP/s in fp16 (a large library
+// N = K = 1024 at 8192 rows takes 54 us, 960 TFLOP/s in fp16 (a large library
 // product reaches 1156 on the same card) and 313 in fp32, where the fp32 matrix
 // cores took 183; N = 32000 1.51 ms, 1070 and 357 (5.7 ms). 2 x 4 blocks per wave
 // with half the W reads measured the same (58 us, 1.48 ms).
